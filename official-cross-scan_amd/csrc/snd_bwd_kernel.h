@@ -17,12 +17,15 @@
 //
 // Organisation (not a translation): the same lane = one (channel, state) plane, TE x TE tile walk
 // as the forward (TE = 8 or 7), in reverse.  For each tile a lane recomputes h from the forward's checkpoints (row above
-// from x_v, column to the left from x, s from x_sd), one half of the tile (4 columns, then the rest) at a time into 32
-// registers, and sweeps that half bottom-right to top-left.  The adjoint row handed to the strip
-// above goes through a private global scratch row; the column handed to the tile on the left stays
-// in registers.  dB/dC are reduced over a wave's channels with lane swaps, over the block's waves
+// from x_v, column to the left from x, s from x_sd) into 64 registers and sweeps the tile bottom-right to top-left.  The
+// adjoint row handed to the strip above goes through a private global scratch row; the column handed to the tile on the
+// left stays in registers.  dB/dC are reduced over a wave's channels with lane swaps, over the block's waves
 // through LDS, and leave the block once per tile; du/ddelta are reduced over states by DPP and
 // finished once per pixel by the thread that staged it.
+// What the sweep evaluates per cell (26 vector instructions): the part of a lower row's contribution that does not depend on
+// the row above it is formed where the row is swept, K = G - a/2 * G[right], and G + Gs is carried instead of Gs, since
+//     g = dout*C + G[i,j+1] + K[i+1,j] - a[i,j+1]/2 * G[i+1,j+1]       g + gs = (G + Gs)[i,j+1] + K[i+1,j] - a[i,j+1]/2 * G[i+1,j+1]
+// share their tail and dout*C cancels in the second.
 // As in the forward, tiles are computed in full on zero-padded staging (dout = B = C = 0 outside
 // the plane makes every adjoint there exactly zero), so the inner loops have no bounds checks.
 #pragma once
@@ -58,12 +61,6 @@ __device__ __forceinline__ void rows_scatter4x2(float &b0, float &b1, float &b2,
                  "v_add_f32 %4, %4, %5\n\t"
                  : "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3), "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3));
 }
-#ifndef SND_BWD_WAVES
-#define SND_BWD_WAVES 2
-#endif
-#ifndef SND_KA8
-#define SND_KA8 3
-#endif
 // VEC: the tile's inputs are staged, and du / ddelta stored, four columns at a time with one 16-byte (fp32) or
 // 8-byte (16-bit) access per thread and tensor instead of one access per element - a quarter of the memory
 // instructions and of their address arithmetic.  Needs 8x8 tiles, a width that is a multiple of four and tensors
@@ -72,7 +69,7 @@ __device__ __forceinline__ void rows_scatter4x2(float &b0, float &b1, float &b2,
 // segment's block to the next through the workspace (strip_segments).  A variant of its own, because the few
 // registers it takes are registers the other variants do not have.
 template <typename T, int NP, bool PIPE, int TE, bool VEC, bool SEG = false>
-__global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD_WAVES, SND_BWD_WAVES))) void bwd_kernel(const snd_bwd_params p, const Geo geo) {
+__global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_kernel(const snd_bwd_params p, const Geo geo) {
     static_assert(!VEC || TE == 8, "vector staging needs 8x8 tiles");
     static_assert(!SEG || PIPE, "column segments belong to the strip pipeline");
     constexpr int WPB = NP / 4;                     // waves per block
@@ -85,7 +82,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
     // consecutive banks.  NSD: the dB/dC partial sums, which the 16-lane row q of a wave writes at element q of
     // a state's tile row, so states must start 2 (16 states) or 4 banks apart.
     constexpr int PCH = kTile + (NP == 16 ? 8 : 4);
-    constexpr int PCS = kTile + NP;
+    constexpr int PCS = kTile + (NP < 8 ? NP : 8);
     constexpr int NSD = NP == 16 ? kTile + 2 : kTile + 4;
     constexpr int NBC = 4;
     constexpr int NPX = kTile / NP;
@@ -102,16 +99,18 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
     extern __shared__ __align__(16) float smem[];
     float *sB = smem;                               // [NP][NSTR]
     float *sC = sB + NP * NSTR;
-    float *sdB = sC + NP * NSTR;                    // [NPART][NP][NSD]
-    float *sdC = sdB + NPART * NP * NSD;
-    float *sDl = sdC + NPART * NP * NSD;            // [CB][DLP]
+    constexpr int PART = NP * NSD;
+    float *sdB = sC + NP * NSTR;                    // [NPART][PART]
+    float *sdC = sdB + NPART * PART;
+    float *sDl = sdC + NPART * PART;                // [CB][DLP]
     float *sDu = sDl + CB * DLP;                    // [CB][PCH] delta' * u
+    float *sQ = sDu;                                // sum_n dbu*B: takes the place of a row half's delta' * u once that is swept
     float *sU = sDu + CB * PCH;                     // [CB][PCS]
     float *sDo = sU + CB * PCS;                     // dout
     float *sSg = sDo + CB * PCH;                    // [CB][PCS] d softplus / d raw
-    float *sQ = sSg + CB * PCS;                     // sum_n dbu*B
-    float *sP = sQ + CB * PCH + 4;                  // sum_n A*da*a (4 banks off sQ: a wave writes both in one instruction)
-    float *sRed = sP + CB * PCH;                    // [WPB]
+    float *sP = sSg + CB * PCS + 4;                 // sum_n A*da*a (4 banks off sQ: a wave writes both in one instruction)
+    float *sHold = sP + CB * PCH;                   // dB, dC sums of a pair's right tile, [2][NP][kTile]
+    float *sRed = sHold + 2 * NP * kTile;           // [WPB]
 
     const snd_fwd_params &f = p.f;
     const snd_shape &sh = f.shape;
@@ -126,9 +125,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
     const int64_t nSync = sync_words((int64_t)sh.batch * G * nChunks, geo.nCY);
     bool dead = false;
     int seen = 0;                                   // last progress count read (strip pipeline)
-#ifdef SND_PIPE_TRACE
-    int *trace_ = nullptr, trace_wait_ = 0;
-#endif
     __shared__ int sSeen;                           // (pipelined) progress count of the strip below, as last polled
     __shared__ int sDead;                           // (pipelined) a hand-over wait of this block has timed out
     if (PIPE) {
@@ -151,10 +147,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
             segdone = progress + nPC * geo.nCY;
             colstate = (float *)p.workspace + nSync + (int64_t)sh.batch * Dm * N * geo.Wp + ((int64_t)pc * geo.nCY + I_hi) * kColStateFloats;
         }
-#ifdef SND_PIPE_TRACE
-        trace_ = sync + kSyncHeader + 2 * nPC * geo.nCY + 4 * (pc * geo.nCY + I_hi);
-        if (threadIdx.x == 0) trace_[0] = (int)wall_clock64();
-#endif
     } else if (!xcd_job(blockIdx.x, sh.batch * G, nChunks, pair, chunk)) return;
     const int b = pair / G, g = pair - b * G;
     const int cbase = g * rg + chunk * CB, cend = (g + 1) * rg;
@@ -172,9 +164,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
     const int cc = cvalid ? c : cend - 1, nn = n < N ? n : N - 1;
     const int px = tid & 63, pr = px >> 3, pj = px & 7;
 
-    const float Av = lvalid ? f.A[(int64_t)cc * f.A_d_stride + (int64_t)nn * f.A_dstate_stride] : 0.f;
-    const float A2 = Av * kLog2e;
-    const float ld = f.A_decay ? __log2f(f.A_decay[0]) : 0.f;
+    const float A2 = kLog2e * (lvalid ? f.A[(int64_t)cc * f.A_d_stride + (int64_t)nn * f.A_dstate_stride] : 0.f);
+    const float ld = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f.A_decay ? __log2f(f.A_decay[0]) : 0.f)));
     const float Dv = f.D ? f.D[cc] : 0.f;
     const float bias = f.delta_bias ? f.delta_bias[cc / rd] : 0.f;
     const bool softplus = f.delta_softplus != 0;
@@ -248,7 +239,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
         else { rr = hidx - 16; jj = -1; }
     };
     auto prefetch = [&](int I, int J) {
-        const int r0 = (SND_TILE_ABLATE & 2) ? 0 : I * TE, j0 = (SND_TILE_ABLATE & 2) ? 0 : J * TE;
+        const int r0 = I * TE, j0 = J * TE;
         // The thread's element maps are re-derived here from an opaque copy of the thread id, so that
         // they are a few integer ops per tile instead of dozens of registers kept live across the tile.
         SND_THREAD_MAPS(NP);
@@ -260,23 +251,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                 const int row = min(r0 + (q >> 1), H - 1), col = min(j0 + (q & 1) * 4, W - 4);
                 return (uint32_t)mad24(mrow(row), hB, mcol(col + (fh ? 3 : 0)) * esz);
             };
-            uint32_t z_ = 0;                        // (timing studies) what a load that is switched off leaves in its registers
-            if (SND_TILE_ABLATE & 112) asm volatile("v_mov_b32 %0, 0x3e000000" : "=v"(z_));
-            if (SND_TILE_ABLATE & 16) {
-                for (int e = 0; e < (int)sizeof(T); ++e) { vb.w[e] = z_; vc.w[e] = z_; }
-            } else {
+            {
                 const int sn = min(t_ >> 4, N - 1), q = t_ & 15;
-                ldraw4_b(vb, (const T *)((const char *)Bb + sn * BsB), chunk_off(q, BhB, ESZ));
-                ldraw4_b(vc, (const T *)((const char *)Cb + sn * CsB), chunk_off(q, ChB, ESZ));
+                ldraw4_b(vb, Bb, (uint32_t)sn * (uint32_t)BsB + chunk_off(q, BhB, ESZ));   // (below 2^32: bwd_vec_ok)
+                ldraw4_b(vc, Cb, (uint32_t)sn * (uint32_t)CsB + chunk_off(q, ChB, ESZ));
             }
 #pragma unroll
             for (int k = 0; k < NCH; ++k) {
                 const int q = n + NP * k;
-                if (SND_TILE_ABLATE & 32) {
-                    for (int e = 0; e < (int)sizeof(T); ++e) { vdl[k].w[e] = z_; vu[k].w[e] = z_; }
-                    for (int e = 0; e < 4; ++e) vdo[k][e] = z_;
-                    continue;
-                }
                 ldraw4_b(vdl[k], db, cDb + chunk_off(q, DhB, ESZ));
                 ldraw4_b(vu[k], ub, cUb + chunk_off(q, UhB, ESZ));
                 const char *src = (const char *)dob + (cDob + chunk_off(q, DohB, esz_do));
@@ -293,7 +275,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                 int rr, jj;
                 halo_cell(n + NP * k, rr, jj);
                 const int row = min(max(r0 + rr, 0), H - 1), col = min(max(j0 + jj, 0), W - 1);
-                if (SND_TILE_ABLATE & 64) { vh[k] = z_; continue; }
                 vh[k] = ldraw_b(db, cDb + mad24(mrow(row), DhB, mcol(col) * ESZ));
             }
             return;
@@ -453,45 +434,69 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
     // dB, dC of a tile leave the block (summed over its channels) one tile late, from the partial sums that stay
     // in LDS until the next sweep: between the requests for the next tile's inputs and the wait for them, so that the
     // LDS reads and the address arithmetic of the flush fall under the latency of those loads (B=64, D=192, 56x56:
-    // 1.290 -> 1.258 ms against the flush behind the wait, which -DSND_BWD_FLUSH_LATE restores for timing; with the
+    // 1.290 -> 1.258 ms against the flush behind the wait; with the
     // sums in front of the wait and the atomics behind it the eight values kept across the wait are spilled and
     // nothing more is gained, and the per-pixel epilogue moved to the same place gains nothing either).
     int pI = -1, pJ = 0;                            // the tile whose partial sums are still in LDS
     auto flush_bc = [&](int I_, int J_) __attribute__((always_inline)) {
         SND_THREAD_MAPS(NP);
+        // Two neighbouring 8x8 tiles leave together: the right one's sums are held in LDS and joined to the left one's, so that an
+        // instruction adds 4 rows x 16 columns instead of 8 rows x 8.  An atomic costs its CU 12 ns per 64-byte line it
+        // touches, however few of the line's words it adds to (2 x 192 x 200x336: 1.09 -> 1.07 ms, 256 channels of 512x512:
+        // 2.56 -> 2.51 ms; rows that are no multiple of 64 bytes gain nothing, 7x7 tiles lose 2 % and keep the plain form).
+        const bool holds = TE == 8 && (J_ & 1) && J_ > J_lo, joins = TE == 8 && !(J_ & 1) && J_ < J_hi;
         const int row = I_ * TE + pr, col = J_ * TE + pj;
         const bool in = pr < TE && pj < TE && row < H && col < W;
         const uint32_t o = mad24(mrow(row), W4, mcol(col) * 4);
+        // (joined) lane l: row l / 16 (+ 4), column l % 16 of the pair
+        const int jc = px & 7, jr = px >> 4;
+        const bool right = px & 8;
+        const int jcol = (J_ + (right ? 1 : 0)) * TE + jc;
 #pragma unroll
         for (int k = 0; k < NBC; ++k) {
             const int sn = wave_u + WPB * k;                        // scalar: folded into the base
             float tb = 0.f, tc = 0.f;
 #pragma unroll
             for (int w = 0; w < NPART; ++w) {
-                tb += sdB[w * NP * NSD + sn * NSD + px];
-                tc += sdC[w * NP * NSD + sn * NSD + px];
+                tb += sdB[w * PART + sn * NSD + px];
+                tc += sdC[w * PART + sn * NSD + px];
             }
-            if (in && sn < N && !(SND_TILE_ABLATE & 1)) {
+            if (holds) {
+                sHold[sn * kTile + px] = tb;
+                sHold[(NP + sn) * kTile + px] = tc;
+            } else if (joins) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int src = (4 * h + jr) * kCkX + jc, jrow = I_ * TE + 4 * h + jr;
+                    float vb = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src * 4, __builtin_bit_cast(int, tb)));
+                    float vc = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src * 4, __builtin_bit_cast(int, tc)));
+                    const float hb = sHold[sn * kTile + src], hc_ = sHold[(NP + sn) * kTile + src];
+                    if (right) { vb = hb; vc = hc_; }
+                    if (4 * h + jr < TE && jc < TE && jrow < H && jcol < W && sn < N) {
+                        const uint32_t jo = mad24(mrow(jrow), W4, mcol(jcol) * 4);
+                        glb_add((float *)((char *)dBg + sn * HW4 + jo), vb);
+                        glb_add((float *)((char *)dCg + sn * HW4 + jo), vc);
+                    }
+                }
+            } else if (in && sn < N) {
                 glb_add((float *)((char *)dBg + sn * HW4 + o), tb);
                 glb_add((float *)((char *)dCg + sn * HW4 + o), tc);
-            } else if (SND_TILE_ABLATE & 1) {
-                dbias_acc += tb + tc;               // keeps the values live
             }
         }
     };
     for (int I = I_hi; I >= I_lo; --I) {
         const int r0 = I * TE;
-        float GR[kRows], GsR[kRows];                // G, Gs at the column right of the tile
-        float aR[kRows];                            // a at that column (only ever multiplies G there)
+        float GR[kRows], SR[kRows];                 // G, G + Gs at the column right of the tile
+        float tR[kRows];                            // -a/2 at that column (only ever multiplies G there)
         float GRc = 0.f;                            // G[r0+8][j0+8]
 #pragma unroll
-        for (int r = 0; r < kRows; ++r) { GR[r] = 0.f; GsR[r] = 0.f; aR[r] = 0.f; }
+        for (int r = 0; r < kRows; ++r) { GR[r] = 0.f; SR[r] = 0.f; tR[r] = 0.f; }
         if (SEG && seg > 0) {
-            // a later column segment of the strip: G, Gs, a of the column right of it and the corner G come from the
+            // a later column segment of the strip: G, G + Gs, -a/2 of the column right of it and the corner G come from the
             // block that swept the segment before (written in full before its count moved: see strip_stores_done)
             if (wave == 0) {
                 int seen_ = 0;
-                strip_wait(segdone + I, seg, seen_, sync, dead, geo.spinLimit SND_TRACE_PASS);
+                strip_wait(segdone + I, seg, seen_, sync, dead, geo.spinLimit);
                 if (dead && tid == 0) sDead = 1;
             }
             __syncthreads();
@@ -500,15 +505,15 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
 #pragma unroll
             for (int r = 0; r < kRows; r += 2) {
                 ld2_coherent(src + (r >> 1) * 512, GR[r], GR[r + 1]);
-                ld2_coherent(src + (4 + (r >> 1)) * 512, GsR[r], GsR[r + 1]);
-                ld2_coherent(src + (8 + (r >> 1)) * 512, aR[r], aR[r + 1]);
+                ld2_coherent(src + (4 + (r >> 1)) * 512, SR[r], SR[r + 1]);
+                ld2_coherent(src + (8 + (r >> 1)) * 512, tR[r], tR[r + 1]);
             }
             float pad_;
             ld2_coherent(src + 12 * 512, GRc, pad_);
             if (bad) {
                 GRc = __builtin_nanf("");
 #pragma unroll
-                for (int r = 0; r < kRows; ++r) GR[r] = GsR[r] = __builtin_nanf("");
+                for (int r = 0; r < kRows; ++r) GR[r] = SR[r] = __builtin_nanf("");
             }
         }
 
@@ -519,7 +524,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
             float hu[kCkX], hlft[kRows], slft[kRows], hc = 0.f;   // h row above, h/s column to the left
             float Gd[kCkX];                                        // G of the row below
             if (I > 0) {
-                const char *src = xv + ((SND_TILE_ABLATE & 8) ? 1 : ((int64_t)(I - 1) * geo.nCX + J)) * DN8 * 4;
+                const char *src = xv + ((int64_t)(I - 1) * geo.nCX + J) * DN8 * 4;
                 const float4 v0 = ck4(src, 0), v1 = ck4(src, DN4);
                 hu[0] = v0.x; hu[1] = v0.y; hu[2] = v0.z; hu[3] = v0.w;
                 hu[4] = v1.x; hu[5] = v1.y; hu[6] = v1.z; hu[7] = v1.w;
@@ -530,8 +535,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                 for (int j = 0; j < kCkX; ++j) hu[j] = 0.f;
             }
             if (J > 0) {
-                const char *sh_ = xh + ((SND_TILE_ABLATE & 8) ? 0 : ((int64_t)(J - 1) * geo.nCY + I)) * DN8 * 4;
-                const char *ss_ = xs + ((SND_TILE_ABLATE & 8) ? 0 : ((int64_t)(J - 1) * geo.nCY + I)) * DN8 * 4;
+                const char *sh_ = xh + ((int64_t)(J - 1) * geo.nCY + I) * DN8 * 4;
+                const char *ss_ = xs + ((int64_t)(J - 1) * geo.nCY + I) * DN8 * 4;
                 const float4 h0 = ck4(sh_, 0), h1 = ck4(sh_, DN4);
                 const float4 s0 = ck4(ss_, 0), s1 = ck4(ss_, DN4);
                 hlft[0] = h0.x; hlft[1] = h0.y; hlft[2] = h0.z; hlft[3] = h0.w;
@@ -564,18 +569,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                 }
             }
             prefetch(I, J);                         // no loads in flight across the register-hungry sweep
-#ifndef SND_BWD_FLUSH_LATE
             if (pI >= 0) flush_bc(pI, pJ);          // the previous tile's dB, dC, under the latency of the loads just requested
             commit(I, J);
-#else                                               // (timing study: the flush behind the wait, as it was; same results)
-            commit(I, J);
-            if (pI >= 0) flush_bc(pI, pJ);
-#endif
             pI = I; pJ = J;
             // strip pipeline: the strip below must have handed over tile J.  One wave polls; the
             // others wait at the barrier.
             if (handed && wave == 0) {
-                strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit SND_TRACE_PASS);
+                strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit);
                 if (tid == 0) { sSeen = seen; if (dead) sDead = 1; }   // read at the top of later tiles
             }
             __syncthreads();
@@ -603,154 +603,121 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
             }
             const float gd_old0 = Gd[0];            // G[r0+8][j0]: the corner of the tile on the left
 
-            // The tile is swept as two 8x4 halves, right then left, so that only 32 values of h
-            // are held at a time.  The right half starts from h, s at column 3, which a plain
-            // forward pass over the left half provides first (that half is recomputed when it is
-            // swept: 32 extra cell updates per tile buy about 60 registers).
-            float hmid[kRows] = {}, smid[kRows] = {}, amid[kRows] = {};   // h, s, a at column 3
+            // ---- recompute h on the whole tile, and s at column 3 of every row (the sweep takes a row's right half first)
+            float hT[TE][TE], smid[TE];
+            // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
+            // the tile loop (a spilled register is two vector memory instructions per tile: the 16-bit variant and the one with
+            // column segments are 2 to 4 % faster with none)
+            constexpr int KA = TE == 7 ? 4 : sizeof(T) == 4 && !SEG ? 3 : 0;
+            float aT[KA ? TE : 1][KA ? KA : 1];
             {
-                float aprev[4], hprev[4], dlr[4];
-                dl_row4(-1, 0, dlr);
+                float aprev[8], hprev[8], dlr[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) { aprev[j] = EXPA(dlr[j]); hprev[j] = hu[j]; }
+                for (int c0 = 0; c0 < 8; c0 += 4) {
+                    dl_row4(-1, c0, dlr);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (c0 + j < TE) { aprev[c0 + j] = EXPA(dlr[j]); hprev[c0 + j] = hu[c0 + j]; }
+                }
                 float diag0 = hc;
 #pragma unroll
                 for (int r = 0; r < TE; ++r) {
                     float al = AEXP(r, -1), left = hlft[r], sl = slft[r], diag = diag0;
                     diag0 = hlft[r];
-                    dl_row4(r, 0, dlr);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float a = EXPA(dlr[j]);
-                        const float bu = myB[r * kCkX + j] * myDu[r * kCkX + j];
-                        const float up = hprev[j];
-                        const float X = fmaf(-0.5f * (aprev[j] + al), diag, up);
-                        const float h = fmaf(a, left + X, bu);
-                        sl = fmaf(a, sl, bu);
-                        hprev[j] = h;
-                        diag = up; left = h; al = a; aprev[j] = a;
-                    }
-                    hmid[r] = left; smid[r] = sl; amid[r] = al;
-                }
-            }
-
-            // One half: recompute h on rows 0..7, columns C0..C0+3, then sweep it bottom-right to
-            // top-left.  top/corner: h of the row above; hL/sL: h, s of the column to the left;
-            // GR/GsR (in/out): G, Gs of the column to the right, replaced by those of column C0;
-            // GdH (in/out): G of the row below, replaced by G of row 0; gdiag0: G[8][C0+4].
-            auto sweep_half = [&](auto C0_, const float *top, float corner, const float (&hL)[kRows],
-                                  const float (&sL)[kRows], float *GdH, float gdiag0) {
-                constexpr int C0 = decltype(C0_)::value;
-                constexpr int HW = C0 == 0 ? 4 : TE - 4;        // columns of this half inside the tile
-                float hT[kRows][4];
-                // the left half keeps a of its first KA columns from this pass for the sweep (as many as
-                // fit under 256 registers without spilling); everything else is recomputed there
-                constexpr int KA = C0 == 0 ? (TE == 7 ? 4 : SND_KA8) : 0;
-                float aT[KA ? kRows : 1][KA ? KA : 1];
-                {
-                    float aprev[4], hprev[4], dlr[4];
-                    dl_row4(-1, C0, dlr);
+                    for (int c0 = 0; c0 < 8; c0 += 4) {
+                        dl_row4(r, c0, dlr);
+                        const float4 b4 = *(const float4 *)(myB + r * kCkX + c0), u4 = *(const float4 *)(myDu + r * kCkX + c0);
+                        const float aB[4] = {b4.x, b4.y, b4.z, b4.w}, aU[4] = {u4.x, u4.y, u4.z, u4.w};
 #pragma unroll
-                    for (int j = 0; j < HW; ++j) { aprev[j] = EXPA(dlr[j]); hprev[j] = top[j]; }
-                    float diag0 = corner;
-#pragma unroll
-                    for (int r = 0; r < TE; ++r) {
-                        float al = C0 == 0 ? AEXP(r, C0 - 1) : amid[r], left = hL[r], diag = diag0;
-                        diag0 = hL[r];
-                        dl_row4(r, C0, dlr);
-#pragma unroll
-                        for (int j = 0; j < HW; ++j) {
+                        for (int j = 0; j < 4; ++j) {
+                            const int c_ = c0 + j;
+                            if (c_ >= TE) continue;
                             const float a = EXPA(dlr[j]);
-                            const float bu = myB[r * kCkX + C0 + j] * myDu[r * kCkX + C0 + j];
-                            const float up = hprev[j];
-                            const float X = fmaf(-0.5f * (aprev[j] + al), diag, up);
+                            const float bu = aB[j] * aU[j];
+                            const float up = hprev[c_];
+                            const float X = fmaf(-0.5f * (aprev[c_] + al), diag, up);
                             const float h = fmaf(a, left + X, bu);
-                            hT[r][j] = h;
-                            if (j < KA) aT[r][j] = a;
-                            hprev[j] = h;
-                            diag = up; left = h; al = a; aprev[j] = a;
+                            if (c0 == 0) sl = fmaf(a, sl, bu);
+                            hT[r][c_] = h;
+                            if (c_ < KA) aT[KA ? r : 0][KA ? c_ : 0] = a;
+                            hprev[c_] = h;
+                            diag = up; left = h; al = a; aprev[c_] = a;
                         }
                     }
+                    smid[r] = sl;
                 }
-                float adn[4];
-                float Gd8 = gdiag0;
-                {
-                    float dlr[4];
-                    dl_row4(TE, C0, dlr);
+            }
+            // ---- reverse sweep, bottom-right to top-left.  K[j] = G[j] - 0.5*a[j]*G[j+1] of the row below: the part of its
+            // contribution to g that does not depend on this row.
+            float Kd[8];
+            asm volatile("" ::: "memory");
+            {
+                float dlr[4];
 #pragma unroll
-                    for (int j = 0; j < HW; ++j) adn[j] = EXPA(dlr[j]);
+                for (int c0 = 0; c0 < 8; c0 += 4) {
+                    dl_row4(TE, c0, dlr);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (c0 + j < TE) Kd[c0 + j] = fmaf(-0.5f * EXPA(dlr[j]), c0 + j + 1 < TE ? Gd[c0 + j + 1 < 8 ? c0 + j + 1 : 7] : GRc, Gd[c0 + j]);
                 }
-                // The five LDS operands of a row (delta', B, C, delta'*u, dout; 16 bytes each) are requested one row ahead.
-                // With 7x7 tiles, 16 states and whole-plane blocks the request sits behind the row's cell updates and in front of its
-                // cross-lane sums (the registers of the row just finished are free there, and the reads complete under
-                // the sums: 64 x 768 channels of 14x14, bf16, 0.347 -> 0.336 ms); every other variant has no register
-                // left for that (12 to 16 spilled, nothing gained) and requests the next row behind the sums.
-                constexpr bool ROWPF = TE == 7 && NP == 16 && !PIPE;
-                float4 nD4, nB4, nC4, nU4, nO4;
-                auto request_row = [&](int r) __attribute__((always_inline)) {
-                    nD4 = *(const float4 *)(myDl + (r + 1) * HG + DLO + C0);
-                    nB4 = *(const float4 *)(myB + r * kCkX + C0);
-                    nU4 = *(const float4 *)(myDu + r * kCkX + C0);
-                    nC4 = *(const float4 *)(myC + r * kCkX + C0); nO4 = *(const float4 *)(myDo + r * kCkX + C0);
-                };
-                request_row(TE - 1);
+            }
+            float Gd8 = GRc;                        // G[r+1][j0+TE]
 #pragma unroll
-                for (int r = TE - 1; r >= 0; --r) {
+            for (int r = TE - 1; r >= 0; --r) {
+                float Gr = GR[r], Sr = SR[r], Gdiag = Gd8, tr = tR[r];
+#pragma unroll
+                for (int C0 = 4; C0 >= 0; C0 -= 4) {
                     __builtin_amdgcn_sched_barrier(0);
-                    float arow[5], s[4], buv[4];
-                    const float dlr[4] = {nD4.x, nD4.y, nD4.z, nD4.w};
-#pragma unroll
-                    for (int j = 0; j < HW; ++j) arow[j] = j < KA ? aT[KA ? r : 0][j < KA ? j : 0] : EXPA(dlr[j]);
-                    arow[HW] = aR[r];
-                    const float aB[4] = {nB4.x, nB4.y, nB4.z, nB4.w}, aC[4] = {nC4.x, nC4.y, nC4.z, nC4.w};
+                    const int HW = C0 == 0 ? 4 : TE - 4;        // columns of this half inside the tile
+                    const float4 nD4 = *(const float4 *)(myDl + (r + 1) * HG + DLO + C0), nB4 = *(const float4 *)(myB + r * kCkX + C0);
+                    const float4 nU4 = *(const float4 *)(myDu + r * kCkX + C0), nC4 = *(const float4 *)(myC + r * kCkX + C0);
+                    const float4 nO4 = *(const float4 *)(myDo + r * kCkX + C0);
+                    const float dlr[4] = {nD4.x, nD4.y, nD4.z, nD4.w}, aB[4] = {nB4.x, nB4.y, nB4.z, nB4.w}, aC[4] = {nC4.x, nC4.y, nC4.z, nC4.w};
                     const float aU[4] = {nU4.x, nU4.y, nU4.z, nU4.w}, aO[4] = {nO4.x, nO4.y, nO4.z, nO4.w};
-                    {
-                        float sp = sL[r];
+                    float arow[4], s[4], buv[4];
+                    float sp = C0 ? smid[r] : slft[r];
 #pragma unroll
-                        for (int j = 0; j < HW; ++j) {
+                    for (int j = 0; j < 4; ++j)
+                        if (j < HW) {
+                            arow[j] = C0 + j < KA ? aT[KA ? r : 0][C0 + j < KA ? C0 + j : 0] : EXPA(dlr[j]);
                             buv[j] = aB[j] * aU[j];
                             sp = fmaf(arow[j], sp, buv[j]);
                             s[j] = sp;
                         }
-                    }
-                    float Gr = GR[r], Gsr = GsR[r], Gdiag = Gd8;
                     float q[4] = {}, pp_[4] = {}, vB[4] = {}, vC[4] = {}, dsum[4] = {};
 #pragma unroll
-                    for (int j = HW - 1; j >= 0; --j) {
-                        const float dov = aO[j];
-                        const float Bv = aB[j], Cv = aC[j];
-                        const float duv = aU[j];
-                        const float bu = buv[j];
-                        const float dyC = dov * Cv;
-                        const float a = arow[j];
-                        const float g_ = fmaf(-0.5f * (arow[j + 1] + adn[j]), Gdiag, dyC + Gr + GdH[j]);
-                        const float gs = Gsr - dyC;
-                        const float dbu = fmaf(0.25f, dyC, g_ + gs);
-                        const float h_l = (j == 0) ? hL[r] : hT[r][j - 1 < 0 ? 0 : j - 1];
-                        const float h_u = (r == 0) ? top[j] : hT[r - 1 < 0 ? 0 : r - 1][j];
+                    for (int j = 3; j >= 0; --j) {
+                        if (j >= HW) continue;
+                        const int cj = C0 + j;
+                        const float dov = aO[j], duv = aU[j], bu = buv[j], a = arow[j];
+                        const float dyC = dov * aC[j];
+                        const float w = fmaf(tr, Gdiag, Kd[cj]);
+                        const float g_ = (w + Gr) + dyC, gg = w + Sr;   // g, and g + gs (dyC cancels)
+                        const float dbu = fmaf(0.25f, dyC, gg);
+                        const float h_l = cj == 0 ? hlft[r] : hT[r][cj - 1 < 0 ? 0 : cj - 1];
+                        const float h_u = r == 0 ? hu[cj] : hT[r - 1 < 0 ? 0 : r - 1][cj];
                         // g(h - bu) + gs(s - bu) = g(h - s) + (g + gs)(s - bu)
-                        const float hs = hT[r][j] - s[j], sb = s[j] - bu;
-                        const float cross = fmaf(GdH[j], h_l, Gr * h_u);
-                        const float da = fmaf(-0.5f * a, cross, fmaf(g_, hs, (g_ + gs) * sb));
+                        const float hs = hT[r][cj] - s[j], sb = s[j] - bu;
+                        const float cross = fmaf(Gd[cj], h_l, Gr * h_u);
+                        const float t = -0.5f * a;
+                        const float da = fmaf(t, cross, fmaf(g_, hs, gg * sb));
                         dA_acc = fmaf(dlr[j], da, dA_acc);
                         dsum[j] = da;
                         const float Gn = a * g_;
-                        Gdiag = GdH[j];
-                        GdH[j] = Gn;
+                        Gdiag = Gd[cj];
+                        Kd[cj] = fmaf(t, Gr, Gn);
+                        Gd[cj] = Gn;
                         Gr = Gn;
-                        Gsr = a * gs;
-                        q[j] = dbu * Bv;                           // per-pixel terms, summed over states below
-                        pp_[j] = Av * da;
+                        Sr = a * gg;
+                        tr = t;
+                        q[j] = dbu * aB[j];                        // per-pixel terms, summed over states below
+                        pp_[j] = A2 * da;
+                        const float z = fmaf(0.25f, bu, hs);
                         vB[j] = dbu * duv;                         // dB, dC contributions
-                        vC[j] = dov * fmaf(0.25f, bu, hs);
+                        vC[j] = dov * z;
                     }
-                    // The two running sums are pinned to their row: left to itself the compiler sinks the whole chain of
-                    // multiply-adds to the end of the tile and keeps delta' and da of all 64 cells in registers until then.
                     if (want_decay) dec_acc += (dsum[0] + dsum[1]) + (dsum[2] + dsum[3]);
-                    if (ROWPF) {
-                        if (r > 0) request_row(r - 1);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
                     if (NP == 16) {
                         // sums over the channel's 16 states: quads 0,1 of the lane group end with
                         // q[0..1], q[2..3], quads 2,3 with pp_[0..1], pp_[2..3]
@@ -779,18 +746,12 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                             mydC[r * kCkX + C0 + qrow] = tc;
                         }
                     }
-                    if (!ROWPF && r > 0) request_row(r - 1);
-                    Gd8 = GR[r];                    // G[r][C0+4]: diagonal neighbour for the row above
-                    GR[r] = Gr;                     // G[r][C0]: right neighbour for the half on the left
-                    GsR[r] = Gsr;
-                    aR[r] = arow[0];
-#pragma unroll
-                    for (int j = 0; j < HW; ++j) adn[j] = arow[j];
                 }
-            };
-            const float gd_old4 = Gd[4];            // G[r0+8][j0+4]: corner of the left half
-            sweep_half(std::integral_constant<int, 4>{}, hu + 4, hu[3], hmid, smid, Gd + 4, GRc);
-            sweep_half(std::integral_constant<int, 0>{}, hu, hc, hlft, slft, Gd, gd_old4);
+                Gd8 = GR[r];                        // G[r][j0+TE]: diagonal neighbour for the row above
+                GR[r] = Gr;                         // G[r][j0]: right neighbour for the tile on the left
+                SR[r] = Sr;
+                tR[r] = tr;
+            }
             GRc = gd_old0;
             const bool hands_over = PIPE && I == I_lo && I > 0;   // top strip of a band: another block takes the row
             if (I > 0 && lvalid) {                  // adjoint row for the strip above
@@ -826,7 +787,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         duv[e] = fmaf(Dv, ao[e], al[e] * aq[e]);
-                        ddl[e] = fmaf(au[e], aq[e], ap[e]) * ag[e];
+                        ddl[e] = fmaf(kLn2, ap[e], au[e] * aq[e]) * ag[e];
                     }
                     if (cvalid && row < H && col < W) {
 #pragma unroll
@@ -841,12 +802,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                             ddl[0] = ddl[3]; ddl[1] = ddl[2]; ddl[2] = b1; ddl[3] = b0;
                         }
                         const uint32_t o = cGb + mad24(mrow(row), WB, mcol(col + (fh ? 3 : 0)) * ESZ);
-                        if (!(SND_TILE_ABLATE & 4)) {
-                            stg4_b(dub, o, duv);
-                            stg4_b(ddb, o, ddl);
-                        } else {
-                            dD_acc += duv[0] + ddl[0];  // keeps the values live
-                        }
+                        stg4_b(dub, o, duv);
+                        stg4_b(ddb, o, ddl);
                     }
                 }
             } else {
@@ -858,18 +815,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
                 const float dl = sDl[cl * DLP + ((pp >> 3) + 1) * HG + DLO + (pp & 7)];
                 const float uv = sU[cl * PCS + pp], dov = sDo[cl * PCH + pp], sg = sSg[cl * PCS + pp];
                 const float duv = fmaf(Dv, dov, dl * qv);
-                const float ddl = fmaf(uv, qv, pv) * sg;
+                const float ddl = fmaf(kLn2, pv, uv * qv) * sg;
                 if (cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W) {
                     dD_acc = fmaf(dov, uv, dD_acc);
                     dw_acc = fmaf(duv, uv, dw_acc);
                     dbias_acc += ddl;
                     const uint32_t o = cGb + mad24(mrow(row), WB, mcol(col) * ESZ);
-                    if (!(SND_TILE_ABLATE & 4)) {
-                        stg_b(dub, o, duv);
-                        stg_b(ddb, o, ddl);
-                    } else {
-                        dD_acc += duv;              // keeps the values live
-                    }
+                    stg_b(dub, o, duv);
+                    stg_b(ddb, o, ddl);
                 }
             }
             }
@@ -882,8 +835,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
 #pragma unroll
             for (int r = 0; r < kRows; r += 2) {
                 st2_coherent(dst + (r >> 1) * 512, GR[r], GR[r + 1]);
-                st2_coherent(dst + (4 + (r >> 1)) * 512, GsR[r], GsR[r + 1]);
-                st2_coherent(dst + (8 + (r >> 1)) * 512, aR[r], aR[r + 1]);
+                st2_coherent(dst + (4 + (r >> 1)) * 512, SR[r], SR[r + 1]);
+                st2_coherent(dst + (8 + (r >> 1)) * 512, tR[r], tR[r + 1]);
             }
             st2_coherent(dst + 12 * 512, GRc, 0.f);
             strip_stores_done();
@@ -896,9 +849,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
 #undef AEXP
 #undef EXPA
 
-#ifdef SND_PIPE_TRACE
-    if (PIPE && threadIdx.x == 0) { trace_[1] = (int)wall_clock64(); trace_[2] = trace_wait_; }
-#endif
     // ---- per-lane / per-channel sums leave the kernel
     if (lvalid) glb_add(p.dA + (int64_t)c * N + n, dA_acc);
     dD_acc = group_sum<NP>(dD_acc);
@@ -928,8 +878,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(SND_BWD
 
 // Dynamic LDS of one backward block (more than the 64 KB a kernel gets without asking).
 template <int NP> constexpr size_t bwd_lds_bytes() {
-    constexpr int PCH = kTile + (NP == 16 ? 8 : 4), PCS = kTile + NP, NSD = NP == 16 ? kTile + 2 : kTile + 4;
-    return sizeof(float) * (2 * NP * (kTile + 4) + 2 * (NP / 4) * NP * NSD + 16 * 120 + 16 * (4 * PCH + 2 * PCS) + 4 + NP / 4);
+    constexpr int PCH = kTile + (NP == 16 ? 8 : 4), PCS = kTile + (NP < 8 ? NP : 8), NSD = NP == 16 ? kTile + 2 : kTile + 4;
+    return sizeof(float) * (2 * NP * (kTile + 4) + 2 * (NP / 4) * NP * NSD + 16 * 120 + 16 * (3 * PCH + 2 * PCS) + 4 + 2 * NP * kTile + NP / 4);
 }
 // Raise the dynamic LDS limit of every backward instantiation of one input dtype on the current device.
 // hipFuncSetAttribute is not stream-ordered and must not run under a stream capture, which is why it is

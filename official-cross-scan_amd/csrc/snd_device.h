@@ -289,22 +289,9 @@ constexpr int kErrorWord = 1, kTicketWord = 4, kSyncHeader = 12;
 constexpr int kSpinLimit = 1 << 21;                 // default polls (a memory round trip each) before giving up
 // The limit launches use: kSpinLimit unless snd_debug_set_spin_limit() lowered it (tests of the time-out path).
 int spin_limit();
-// Timing studies of the tile kernels only (-DSND_TILE_ABLATE=<bits>, results wrong, never shipped): one memory
-// stream of a kernel is switched off or pointed at one hot tile, and the time that goes away prices it.
-// Forward: 1 no out stores, 2 staging loads from tile (0,0), 4 no checkpoint stores, 8 row-above loads from one
-// tile.  Backward: 1 no dB/dC atomics, 2 staging loads from tile (0,0), 4 no du/ddelta stores, 8 checkpoint loads
-// from one tile; (vector staging) 16 no loads of B and C, 32 none of delta, u and dout, 64 none of the halo of
-// delta - their registers hold a constant instead.
-#ifndef SND_TILE_ABLATE
-#define SND_TILE_ABLATE 0
-#endif
 __host__ __device__ inline int64_t sync_words(int64_t nPlaneChunks, int nStrips) {
     // per (plane chunk, strip): tiles handed over, then column segments finished
-#ifdef SND_PIPE_TRACE   // timing study only: 4 extra words per job (start, end, time spent waiting, -)
-    return (kSyncHeader + 6 * nPlaneChunks * nStrips + 3) / 4 * 4;
-#else
     return (kSyncHeader + 2 * nPlaneChunks * nStrips + 3) / 4 * 4;
-#endif
 }
 
 // Data handed from one block to another inside a launch is written and read with agent-scope
@@ -344,25 +331,14 @@ __device__ __forceinline__ void strip_stores_done() { asm volatile("s_waitcnt vm
 __device__ __forceinline__ void strip_signal(int *count) {
     if (threadIdx.x == 0) __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-#ifdef SND_PIPE_TRACE
-#define SND_TRACE_ARG , int &trace_wait_
-#define SND_TRACE_PASS , trace_wait_
-#define g_wait_ticks trace_wait_
-#else
-#define SND_TRACE_ARG
-#define SND_TRACE_PASS
-#endif
 // Wait until *count >= need.  `seen` caches the last value read (counts only grow), so a consumer
 // that runs well behind its producer polls once per strip, not once per tile.  Bounded: after
 // `limit` polls the error word (sync word kErrorWord) is set and the wave goes on so that the grid
 // always drains; `dead` then disables further waits.  A block that gave up replaces every row it
 // should have been handed by NaN (see the callers), so the outputs downstream of a timed-out wait are
 // NaN and never plausible-looking numbers; the error word says why (snd_workspace_error reads it).
-__device__ __forceinline__ void strip_wait(const int *count, int need, int &seen, int *sync, bool &dead, int limit SND_TRACE_ARG) {
+__device__ __forceinline__ void strip_wait(const int *count, int need, int &seen, int *sync, bool &dead, int limit) {
     if (dead || seen >= need) return;
-#ifdef SND_PIPE_TRACE
-    const long long t0_ = wall_clock64();
-#endif
     int polls = 0;
     while ((seen = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < need) {
         __builtin_amdgcn_s_sleep(SND_POLL_SLEEP);
@@ -373,9 +349,6 @@ __device__ __forceinline__ void strip_wait(const int *count, int need, int &seen
         }
     }
     asm volatile("" ::: "memory");
-#ifdef SND_PIPE_TRACE
-    g_wait_ticks += (int)(wall_clock64() - t0_);
-#endif
 }
 // Take the next job.  Jobs are (plane chunk, band) in band-major order, so the job a block waits for
 // always holds an earlier ticket of the same queue: it is running or finished.  With many (batch, group)

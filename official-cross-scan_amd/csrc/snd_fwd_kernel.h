@@ -73,9 +73,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     int *sync = (int *)p.workspace, *progress = nullptr;
     bool dead = false;
     int seen = 0;                                   // last progress count read (strip pipeline)
-#ifdef SND_PIPE_TRACE
-    int *trace_ = nullptr, trace_wait_ = 0;
-#endif
     __shared__ int sDead;                           // (pipelined) a hand-over wait of this block has timed out
     if (SAVE && blockIdx.x == 0 && threadIdx.x == 0 && geo.tag) *(uint32_t *)geo.tag = kTagTile;   // which family wrote this state
     if (PIPE) {
@@ -84,16 +81,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
         // top band first; band k covers strips ceil(k*nCY/nBands) .. ceil((k+1)*nCY/nBands)-1.
         int band;
         if (!draw_job(sync, sh.batch * G, nChunks, geo.nBands, geo.nQueues, pair, chunk, band)) return;
-        const int nPC = sh.batch * G * nChunks;
         const int pc = pair * nChunks + chunk;
         I_begin = (band * geo.nCY + geo.nBands - 1) / geo.nBands;
         I_end = ((band + 1) * geo.nCY + geo.nBands - 1) / geo.nBands;
-        (void)nPC;
         progress = sync + kSyncHeader + pc * geo.nCY;
-#ifdef SND_PIPE_TRACE
-        trace_ = sync + kSyncHeader + 2 * nPC * geo.nCY + 4 * (pc * geo.nCY + I_begin);
-        if (threadIdx.x == 0) trace_[0] = (int)wall_clock64();
-#endif
     } else if (!xcd_job(blockIdx.x, sh.batch * G, nChunks, pair, chunk)) return;
     const int b = pair / G, g = pair - b * G;
     const int cbase = g * rg + chunk * CB, cend = (g + 1) * rg;
@@ -171,7 +162,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     Stage st0, st1;                                 // tile J uses st0 when J is even (or always), st1 when odd
     float qxv[kCkX], qcorner = 0.f;                 // h of the row above the next tile (from x_v)
     auto load_tile = [&](Stage &q, int I, int J) {
-        const int r0 = (SND_TILE_ABLATE & 2) ? 0 : I * TE, j0 = (SND_TILE_ABLATE & 2) ? 0 : J * TE;
+        const int r0 = I * TE, j0 = J * TE;
         // The thread's element maps are re-derived here from an opaque copy of the thread id, so that
         // they are a few integer ops per tile instead of dozens of registers kept live across the tile.
         SND_THREAD_MAPS(NP);
@@ -227,7 +218,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     // schedule; every strip of a pipelined band but its first)
     auto prefetch_xv = [&](int I, int J) {
         if ((!PIPE || I > I_begin) && I > 0 && geo.nCX > 1) {   // with one column tile the row comes from registers
-            const float *src = xv + ((SND_TILE_ABLATE & 8) ? 1 : ((int64_t)(I - 1) * geo.nCX + J)) * DN8;
+            const float *src = xv + ((int64_t)(I - 1) * geo.nCX + J) * DN8;
             const float4 v0 = ld4_stream(src), v1 = ld4_stream(src + DN4);
             qxv[0] = v0.x; qxv[1] = v0.y; qxv[2] = v0.z; qxv[3] = v0.w;
             qxv[4] = v1.x; qxv[5] = v1.y; qxv[6] = v1.z; qxv[7] = v1.w;
@@ -356,7 +347,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             // first strip of a pipelined band: the row above comes from another block
             const bool handed = PIPE && I == I_begin && I > 0;
             if (handed && wave == 0) {
-                strip_wait(progress + I - 1, J + 1, seen, sync, dead, geo.spinLimit SND_TRACE_PASS);
+                strip_wait(progress + I - 1, J + 1, seen, sync, dead, geo.spinLimit);
                 if (dead && tid == 0) sDead = 1;
             }
             __syncthreads();
@@ -468,10 +459,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             if (lvalid) {
                 // row checkpoint / carry to the next strip: h at the strip's last row
                 float *dst = xv + ((int64_t)I * geo.nCX + J) * DN8;
-                if (!(SND_TILE_ABLATE & 4)) {
-                    st4_stream(dst, hup[0], hup[1], hup[2], hup[3]);
-                    st4_stream(dst + DN4, hup[4], hup[5], hup[6], hup[7]);
-                }
+                st4_stream(dst, hup[0], hup[1], hup[2], hup[3]);
+                st4_stream(dst + DN4, hup[4], hup[5], hup[6], hup[7]);
                 if (PIPE && I + 1 == I_end && I + 1 < geo.nCY) {   // and the hand-over copy for the block of the strip below
                     float *ho = hrow + (int64_t)J * DN8;
 #pragma unroll
@@ -480,7 +469,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             }
             const bool hands_over = PIPE && I + 1 == I_end && I + 1 < geo.nCY;
             if (hands_over) strip_stores_done();
-            if (lvalid && SAVE && J + 1 < geo.nCX && !(SND_TILE_ABLATE & 4)) {   // column checkpoints: only if a tile follows
+            if (lvalid && SAVE && J + 1 < geo.nCX) {   // column checkpoints: only if a tile follows
                 float *dh = xh + ((int64_t)J * geo.nCY + I) * DN8;
                 float *ds = xs + ((int64_t)J * geo.nCY + I) * DN8;
                 st4_stream(dh, hl[0], hl[1], hl[2], hl[3]);
@@ -500,7 +489,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 for (int k = 0; k < NPX; ++k) {
                     const int pp = VEC ? 4 * (n + NP * (k >> 2)) + (k & 3) : n + NP * k;
                     const int row = r0 + (pp >> 3), col = j0 + (pp & 7);
-                    if (cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W && !(SND_TILE_ABLATE & 1)) {
+                    if (cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W) {
                         const float v = fmaf(sDu[cl * PCH + pp], sS[pp], sY[cl * PCH + pp] + dukeep[k]);
                         const uint32_t o = cOb + mad24(mrow(row), OhB, mcol(col) << sh_out);
                         if (merge) glb_add((float *)((char *)outb + o), wm * v);
@@ -539,7 +528,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                     for (int idx = tid; idx < CB * kRows * Q4; idx += 16 * NP) {
                         const int ch = idx / (kRows * Q4), rr = (idx / Q4) & 7, c4 = (idx & (Q4 - 1)) * 4;
                         const int row = r0 + rr;
-                        if (row < H && c4 < ncols && cbase + ch < cend && !(SND_TILE_ABLATE & 1)) {
+                        if (row < H && c4 < ncols && cbase + ch < cend) {
                             const float4 v = *(const float4 *)(sOut + ch * OCH + rr * OROW + c4);
                             float a4[4] = {v.x, v.y, v.z, v.w};
                             if (fh) { a4[0] = v.w; a4[1] = v.z; a4[2] = v.y; a4[3] = v.x; }   // scan order -> memory order
@@ -555,7 +544,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 for (int idx = tid; idx < CB * PER_CH; idx += 16 * NP) {
                     const int ch = idx / PER_CH, rr = (idx / QC) & 7, c32 = idx & (QC - 1);
                     const int row = r0 + rr;
-                    if (rr < TE && row < H && c32 < ncols && cbase + ch < cend && !(SND_TILE_ABLATE & 1)) {
+                    if (rr < TE && row < H && c32 < ncols && cbase + ch < cend) {
                         const uint32_t o = (uint32_t)(cbase + ch - mshift) * (uint32_t)p.out_d_stride * esz_out +
                                            mad24(mrow(row), OhB, mcol(c0 + c32) << sh_out);
                         if (merge) glb_add((float *)((char *)outb + o), sOut[ch * OCH + rr * OROW + c32]);
@@ -575,9 +564,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             for (int J = 0; J < geo.nCX; ++J) do_tile(J, st0, true);
         }
     }
-#ifdef SND_PIPE_TRACE
-    if (PIPE && threadIdx.x == 0) { trace_[1] = (int)wall_clock64(); trace_[2] = trace_wait_; }
-#endif
 }
 
 template <typename T, int NP, int TE, bool VEC>

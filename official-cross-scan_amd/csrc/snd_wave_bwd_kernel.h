@@ -28,12 +28,6 @@
 #include <type_traits>
 #include "snd_device.h"
 
-// Timing studies only (-DSND_WAVE_ABLATE=<bits>, results wrong): 64 no dB / dC atomics, 128 no du / ddelta stores,
-// 256 (column groups) nothing left for the group on the left, 512 nothing taken from the group on the right.
-#ifndef SND_WAVE_ABLATE
-#define SND_WAVE_ABLATE 0
-#endif
-
 namespace snd {
 
 constexpr int kWaveShareWaves = 8;                   // waves of a block whose channels share their dB / dC atomics
@@ -235,8 +229,8 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     const float *ebase = EXT ? wg.bcol + (plane0 + (el / R) % NS) * wave_bcol_plane(wg)
                                + (int64_t)min(gq + 1, wave_groups(wg.nsegAll) - 1) * 3 * wg.Hp + eq * wg.Hp : nullptr;
     float *eout = EXT ? wg.bcol + plane0 * wave_bcol_plane(wg) + (int64_t)gq * 3 * wg.Hp : nullptr;
-    const bool ext_in = EXT && (SPL ? half == 1 : wg.extR != 0) && w == nseg - 1 && !(SND_WAVE_ABLATE & 512),
-               ext_out = EXT && (SPL ? half == 0 : wg.extL != 0) && w == 0 && !(SND_WAVE_ABLATE & 256);
+    const bool ext_in = EXT && (SPL ? half == 1 : wg.extR != 0) && w == nseg - 1,
+               ext_out = EXT && (SPL ? half == 0 : wg.extL != 0) && w == 0;
     // (split planes) the tagged words of the plane's first state
     float *eouttag = SPL ? wg.bcol + plane0 * wave_split_words(wg) : nullptr;
 
@@ -505,7 +499,7 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                     if (CHB > 1) {
                         sX[kXBuf == 2 ? step & 1 : 0][wi][(r * NS + n) * 2][lane] = active ? ya[0] : 0.f;
                         sX[kXBuf == 2 ? step & 1 : 0][wi][(r * NS + n) * 2 + 1][lane] = active ? ys[0] : 0.f;
-                    } else if (!(SND_WAVE_ABLATE & 64) || ya[0] == 1234.5f) {
+                    } else {
 #pragma unroll
                         for (int e = 0; e < CPL; ++e) {                                // memory order
                             const int t = fh ? e : CPL - 1 - e;
@@ -547,7 +541,7 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                         float t_ = duv[0]; duv[0] = duv[CPL - 1]; duv[CPL - 1] = t_;
                         t_ = ddl[0]; ddl[0] = ddl[CPL - 1]; ddl[CPL - 1] = t_;
                     }
-                    if (!(SND_WAVE_ABLATE & 128) || duv[0] == 1234.5f) {
+                    {
                         wave_st_buf<T, CPL, VEC>(rdu, in_plane ? og : kBufOOB, duv);
                         wave_st_buf<T, CPL, VEC>(rdd, in_plane ? og : kBufOOB, ddl);
                     }
@@ -560,7 +554,6 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
             // Wave kc of a segment adds up rows kc, kc + CHB, ... of what the segment's CHB waves left and issues
             // their atomics.
             lds_barrier();
-            if (!(SND_WAVE_ABLATE & 64))
 #pragma unroll
             for (int m = 0; m < kItems / CHB; ++m) {
                 const int it = m * CHB + kc, r = it / (2 * NS), n = (it >> 1) % NS;

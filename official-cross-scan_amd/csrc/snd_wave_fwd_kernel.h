@@ -26,12 +26,6 @@
 #include <type_traits>
 #include "snd_device.h"
 
-// Timing studies only (-DSND_WAVE_ABLATE=<bits>, results wrong): 1 no out stores, 2 no block barriers,
-// 4 no softplus, 8 no scan, 16 no checkpoint stores, 32 no hand-over through LDS.
-#ifndef SND_WAVE_ABLATE
-#define SND_WAVE_ABLATE 0
-#endif
-
 namespace snd {
 
 // PK > 1: narrow planes packed PK to a wave (wave_pack() in snd_device.h): lane l works on column l % (64 / PK) of
@@ -64,10 +58,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     static_assert(R % RC == 0, "a band ends on a checkpoint row");
     static_assert(PK == 1 || CPL == 1, "packed planes: one column per lane");
     constexpr int S = 64 / PK;                       // lanes per plane
-#ifndef SND_WAVE_RD
-#define SND_WAVE_RD 4
-#endif
-    constexpr int RD = SND_WAVE_RD < R ? SND_WAVE_RD : R;   // rows per wavefront step
+    constexpr int RD = R < 4 ? R : 4;                // rows per wavefront step
     static_assert(R % RD == 0, "a band is a whole number of steps");
     // what a wave leaves for the wave on its right: {h, s, a, -} at its last column, per step parity, row and
     // state.  Wave w writes slot w+1 and reads slot w; slot 0 stays zero (nothing enters the first segment).
@@ -229,7 +220,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
             // put it: the group's first wave fills its own slot, one word per lane, and the rows read it as ever
             if (EXT && r % RD == 0 && ext_in && lane < kExtLanes && er / RD == r / RD)
                 ((float *)&sHO[(step + 1) & 1][0][er % RD][(el / wave_fwd_rows(NS)) % NS])[eq] = cur.e;
-            if (r % RD == 0 && HOIST_IN && !ONE && !(SND_WAVE_ABLATE & 32)) {
+            if (r % RD == 0 && HOIST_IN && !ONE) {
 #pragma unroll
                 for (int q = 0; q < RD; ++q)
 #pragma unroll
@@ -247,7 +238,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                         float dsp;
                         // always evaluated, then selected: a branch around it (the flag is uniform) costs a wave more
                         // issue time than the select, and every model in practice asks for the softplus
-                        float sp = (SND_WAVE_ABLATE & 4) ? raw : softplus20(raw, dsp);
+                        float sp = softplus20(raw, dsp);
                         asm volatile("" : "+v"(sp));
                         dlb[q][k] = softplus ? sp : raw;
                         dub_[q][k] = dlb[q][k] * ub_[q][k];
@@ -262,7 +253,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
 #pragma unroll
                 for (int n = 0; n < NS; ++n) {
                     // what the segment on the left left for this row: h, s, a at column S*w-1
-                    const float4 in = ((SND_WAVE_ABLATE & 32) || ONE) ? make_float4(0.f, 0.f, 0.f, 0.f)
+                    const float4 in = ONE ? make_float4(0.f, 0.f, 0.f, 0.f)
                                       : HOIST_IN ? inb[HOIST_IN ? r % RD : 0][n] : sHO[(step + 1) & 1][w][r % RD][n];
                     float a[CPL], bu[CPL], cv[CPL], y[CPL], h[CPL], s[CPL];
                     unpack(cur.b[r][n], bu);
@@ -281,12 +272,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                         const float X = fmaf(-0.5f * (aprev[n][k] + al), hd, hprev[n][k]);
                         y[k] = fmaf(a[k], X, bu[k]);
                     }
-                    if (SND_WAVE_ABLATE & 8) {
-#pragma unroll
-                        for (int k = 0; k < CPL; ++k) { h[k] = y[k]; s[k] = bu[k]; }
-                    } else {
-                        wave_row_solve<CPL, PK>(a, y, bu, in.x, in.y, h, s);
-                    }
+                    wave_row_solve<CPL, PK>(a, y, bu, in.x, in.y, h, s);
 #pragma unroll
                     for (int k = 0; k < CPL; ++k) {
                         acc[k] = fmaf(cv[k], fmaf(0.25f, bu[k], h[k] - s[k]), acc[k]);
@@ -294,7 +280,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                         aprev[n][k] = a[k];
                     }
                     hdiag[n] = in.x;
-                    if (!ONE && !(SND_WAVE_ABLATE & 32)) {
+                    if (!ONE) {
                         wr[(r % RD) * NS + n] = make_float4(h[CPL - 1], s[CPL - 1], a[CPL - 1], 0.f);
                     }
                     if (EXT && ext_out && lane == 63) {   // what enters the column group on the right
@@ -310,7 +296,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                         ca[n] = mine ? in.z : ca[n];
                     }
                 }
-                if (jin && act && (!(SND_WAVE_ABLATE & 1) || acc[0] == 1234.5f)) {
+                if (jin && act) {
                     float o[CPL];
 #pragma unroll
                     for (int k = 0; k < CPL; ++k) o[k] = fmaf(Dv, u[k], acc[k]);
@@ -328,7 +314,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                 if (r % RC == RC - 1) {
 #pragma unroll
                     for (int n = 0; n < NS; ++n) {
-                        if (EVEN || (act && !bar && !(SND_WAVE_ABLATE & 16))) {
+                        if (EVEN || (act && !bar)) {
                             float *dst = xv + (int64_t)n * wave_xv_plane(wg) + (int64_t)(band * (R / RC) + r / RC) * wg.Wp;
                             if (CPL == 2) {
                                 const wave_f2 v = {hprev[n][0], hprev[n][CPL - 1]};
@@ -340,10 +326,10 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                     }
                 }
             }
-            if (multi && r % RD == RD - 1) { if (!(SND_WAVE_ABLATE & 2)) lds_barrier(); ++step; }
+            if (multi && r % RD == RD - 1) { lds_barrier(); ++step; }
         }
         // column checkpoints: lanes 0..R-1 hold what entered the segment on the band's rows
-        if (SAVE && w > 0 && lane < R && band * R + lane < wg.Hp && !(SND_WAVE_ABLATE & 16)) {
+        if (SAVE && w > 0 && lane < R && band * R + lane < wg.Hp) {
 #pragma unroll
             for (int n = 0; n < NS; ++n) {
                 const int64_t o = (int64_t)n * wave_x_plane(wg) + band * R + lane;
