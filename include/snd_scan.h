@@ -143,7 +143,9 @@ typedef struct snd_fwd_params {
     void *out;
     float *x, *x_v, *x_sd;         /* saved state sized by snd_make_plan, 16-byte aligned.  x_v is always
                                       required (it also carries h from one row strip to the next);
-                                      x and x_sd may both be null = inference only (bwd impossible) */
+                                      x and x_sd may both be null = inference only (bwd impossible): x_v is
+                                      then scratch, of which the first x_v_elems / n_chunks_y *
+                                      min(4, n_chunks_y) floats are used (none by the row-segment kernels) */
     int64_t u_batch_stride, u_d_stride, u_h_stride;
     int64_t delta_batch_stride, delta_d_stride, delta_h_stride;
     int64_t A_d_stride, A_dstate_stride;

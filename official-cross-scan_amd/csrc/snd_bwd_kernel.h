@@ -969,7 +969,15 @@ static int launch_bwd_np(const snd_bwd_params &p, hipStream_t stream) {
 // One instantiation per input dtype, each in its own translation unit.
 template <typename T>
 int launch_bwd_t(const snd_bwd_params &p, hipStream_t stream) {
-    const int N = p.f.shape.dstate;
+    const snd_shape &sh = p.f.shape;
+    const int N = sh.dstate;
+    if (N > 4 && N <= 8) {
+        const Geo geo = make_geo(sh.nrows, sh.ncols);
+        const int nChunks = (sh.dim / sh.n_groups + 15) / 16;
+        const int64_t pairs = (int64_t)sh.batch * sh.n_groups;
+        const int jobs = bwd_band_count(p.f.schedule, pairs, nChunks, geo.nCY, p.workspace, N, geo.nCX);
+        if (launch_underfilled(pairs * nChunks, jobs, geo.nCY, geo.nCX)) return launch_bwd_np<T, 16>(p, stream);
+    }
     return N > 8 ? launch_bwd_np<T, 16>(p, stream) : N > 4 ? launch_bwd_np<T, 8>(p, stream) : launch_bwd_np<T, 4>(p, stream);
 }
 

@@ -493,6 +493,9 @@ __host__ inline int band_count(int schedule, int64_t nPairs, int nChunks, int nS
     if (schedule == kSchedBands) return best > 1 ? best : 2;
     return best > 1 ? best : 0;
 }
+// Rows of h per plane a forward without saved state keeps in x_v (one per band of the most bands band_count() makes)
+constexpr int kInferSlabs = 4;
+__host__ __device__ inline int infer_slabs(int nCY) { return nCY < kInferSlabs ? nCY : kInferSlabs; }
 // Blocks per CU by the state-lane count of the kernels (16, 8 or 4 lanes per channel): the backward is held
 // to 2, 3, 4 by its LDS, the forward to 3, 6, 6.
 __host__ inline int64_t bwd_slots(int dstate) { return dstate > 8 ? 512 : dstate > 4 ? 768 : 1024; }
@@ -501,6 +504,16 @@ __host__ inline int bwd_band_count(int schedule, int64_t nPairs, int nChunks, in
 }
 __host__ inline int fwd_band_count(int schedule, int64_t nPairs, int nChunks, int nStrips, const void *sync, int dstate, int nTilesX = 0) {
     return band_count(schedule, nPairs, nChunks, nStrips, sync, dstate > 8 ? 768 : 1536, nTilesX, bwd_slots(dstate));
+}
+
+// Whether a launch of `nPC` plane chunks leaves CUs without a block: `jobs` per chunk as the launch makes them (strips of a
+// plane run side by side nStrips*nTilesX / (nStrips + nTilesX - 1) at a time).  What such a launch takes is one block's time
+// per tile times the tiles of its longest chain, so 5-8 states run on the 16-lane kernels there: half the lanes idle, but
+// four waves stage a tile instead of two.  Measured (8 states, fwd / bwd, 8 -> 16 lanes): 3 x 152 x 61x83 (176 blocks at a
+// time) 0.123 / 0.256 -> 0.111 / 0.225 ms, 4 x 192 x 56x56 (181) 0.084 / 0.167 -> 0.078 / 0.152, 8 x 384 x 14x14 (192)
+// 0.024 / 0.050 -> 0.020 / 0.042; 8 x 152 x 61x83 (470) 0.144 / 0.287 -> 0.146 / 0.330.
+__host__ inline bool launch_underfilled(int64_t nPC, int jobs, int nStrips, int nTilesX) {
+    return jobs == nStrips && jobs > 1 ? nPC * nStrips * nTilesX <= 256 * ((int64_t)nStrips + nTilesX - 1) : nPC * (jobs > 1 ? jobs : 1) <= 256;
 }
 
 

@@ -70,6 +70,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     const int nChunks = (rg + CB - 1) / CB;
     int pair, chunk;
     int I_begin = 0, I_end = geo.nCY;               // strips this block walks
+    // (no state saved) the row carried from strip to strip goes through one slab of x_v per block - a tile's row is read
+    // before the tile's own takes its place - which stays in the L2 instead of streaming to memory: slab `band`, at most
+    // kInferSlabs of them (one strip per job: the row is handed over through the workspace, nothing is stored here)
+    int slab = 0;
     int *sync = (int *)p.workspace, *progress = nullptr;
     bool dead = false;
     int seen = 0;                                   // last progress count read (strip pipeline)
@@ -82,6 +86,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
         int band;
         if (!draw_job(sync, sh.batch * G, nChunks, geo.nBands, geo.nQueues, pair, chunk, band)) return;
         const int pc = pair * nChunks + chunk;
+        slab = band;
         I_begin = (band * geo.nCY + geo.nBands - 1) / geo.nBands;
         I_end = ((band + 1) * geo.nCY + geo.nBands - 1) / geo.nBands;
         progress = sync + kSyncHeader + pc * geo.nCY;
@@ -139,7 +144,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     const int64_t DN8 = (int64_t)Dm * N * 8;
     const int64_t DN4 = DN8 / 2;                    // the lane's values 0-3 of every lane, then values 4-7
     const int64_t lane_off = ((int64_t)cc * N + nn) * 4;
-    float *xv = p.x_v + (int64_t)b * geo.nCY * geo.nCX * DN8 + lane_off;
+    float *xv = p.x_v + (int64_t)b * (SAVE ? geo.nCY : infer_slabs(geo.nCY)) * geo.nCX * DN8 + lane_off;
+    auto xv_row = [&](int I, int J) { return xv + ((int64_t)(SAVE ? I : slab) * geo.nCX + J) * DN8; };   // the row below strip I's tile J
     float *xh = SAVE ? p.x + (int64_t)b * geo.nCX * geo.nCY * DN8 + lane_off : nullptr;
     float *xs = SAVE ? p.x_sd + (int64_t)b * geo.nCX * geo.nCY * DN8 + lane_off : nullptr;
 
@@ -218,8 +224,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     // schedule; every strip of a pipelined band but its first)
     auto prefetch_xv = [&](int I, int J) {
         if ((!PIPE || I > I_begin) && I > 0 && geo.nCX > 1) {   // with one column tile the row comes from registers
-            const float *src = xv + ((int64_t)(I - 1) * geo.nCX + J) * DN8;
-            const float4 v0 = ld4_stream(src), v1 = ld4_stream(src + DN4);
+            const float *src = xv_row(I - 1, J);
+            const float4 v0 = SAVE ? ld4_stream(src) : *(const float4 *)src, v1 = SAVE ? ld4_stream(src + DN4) : *(const float4 *)(src + DN4);
             qxv[0] = v0.x; qxv[1] = v0.y; qxv[2] = v0.z; qxv[3] = v0.w;
             qxv[4] = v1.x; qxv[5] = v1.y; qxv[6] = v1.z; qxv[7] = v1.w;
             qcorner = src[J > 0 ? ((TE - 1) >> 2) * DN4 + ((TE - 1) & 3) - DN8 : 0];   // last column of the tile on the left (if any: masked at its use)
@@ -458,9 +464,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0)
             if (lvalid) {
                 // row checkpoint / carry to the next strip: h at the strip's last row
-                float *dst = xv + ((int64_t)I * geo.nCX + J) * DN8;
-                st4_stream(dst, hup[0], hup[1], hup[2], hup[3]);
-                st4_stream(dst + DN4, hup[4], hup[5], hup[6], hup[7]);
+                float *dst = xv_row(I, J);
+                if (SAVE) {
+                    st4_stream(dst, hup[0], hup[1], hup[2], hup[3]);
+                    st4_stream(dst + DN4, hup[4], hup[5], hup[6], hup[7]);
+                } else if (I + 1 < I_end && geo.nCX > 1) {
+                    *(float4 *)dst = make_float4(hup[0], hup[1], hup[2], hup[3]);
+                    *(float4 *)(dst + DN4) = make_float4(hup[4], hup[5], hup[6], hup[7]);
+                }
                 if (PIPE && I + 1 == I_end && I + 1 < geo.nCY) {   // and the hand-over copy for the block of the strip below
                     float *ho = hrow + (int64_t)J * DN8;
 #pragma unroll
@@ -630,7 +641,15 @@ template <typename T>
 int launch_fwd_t(const snd_fwd_params &p, hipStream_t stream) {
     // (four lanes per channel for N <= 4 work here too, but measure slower than eight: one-wave blocks
     // with 16 staged pixels per thread; the backward does use them)
-    return p.shape.dstate > 8 ? launch_fwd_np<T, 16>(p, stream) : launch_fwd_np<T, 8>(p, stream);
+    const snd_shape &sh = p.shape;
+    if (sh.dstate > 4 && sh.dstate <= 8) {
+        const Geo geo = make_geo(sh.nrows, sh.ncols);
+        const int nChunks = (sh.dim / sh.n_groups + 15) / 16;
+        const int64_t pairs = (int64_t)sh.batch * sh.n_groups;
+        const int jobs = fwd_band_count(p.schedule, pairs, nChunks, geo.nCY, p.workspace, sh.dstate, geo.nCX);
+        if (launch_underfilled(pairs * nChunks, jobs, geo.nCY, geo.nCX)) return launch_fwd_np<T, 16>(p, stream);
+    }
+    return sh.dstate > 8 ? launch_fwd_np<T, 16>(p, stream) : launch_fwd_np<T, 8>(p, stream);
 }
 
 }  // namespace snd

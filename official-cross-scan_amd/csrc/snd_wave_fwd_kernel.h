@@ -132,7 +132,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
 
     // saved state of this plane set
     const int64_t plane0 = ((int64_t)b * Dm + c) * N;
-    float *xv = p.x_v + plane0 * wave_xv_plane(wg) + j0;
+    float *xv = SAVE ? p.x_v + plane0 * wave_xv_plane(wg) + j0 : nullptr;
     float *xh = SAVE ? p.x + plane0 * wave_x_plane(wg) + (int64_t)sg * 2 * wg.Hp : nullptr;
     float *xs = SAVE ? p.x_sd + plane0 * wave_x_plane(wg) + (int64_t)sg * 2 * wg.Hp : nullptr;
     // (column groups) lane (q*NS + n)*R + r fetches h (q = 0), s (1), a (2) entering segment sg on row r of a band, state n
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                 oo += OhB;
                 // row checkpoint: h on the last row of a band of the backward (what its next band starts from; the
                 // last row of the plane is nobody's, and a ragged last band leaves none)
-                if (r % RC == RC - 1) {
+                if (SAVE && r % RC == RC - 1) {
 #pragma unroll
                     for (int n = 0; n < NS; ++n) {
                         if (EVEN || (act && !bar)) {
