@@ -274,6 +274,34 @@ void snd_debug_set_strip_slots(int slots);
 int snd_bwd_static(const snd_bwd_params *params, snd_stream_t stream);
 int64_t snd_static_workspace_bytes(void);
 
+/* The passes a host binding makes around a call - clearing what the kernels accumulate into before it, folding and casting
+ * what they leave after it (selective_scan_oflex.cpp:395-403,432-438) - as up to 8 jobs of ONE launch.
+ *   SND_JOB_CLEAR         zero `outer` BYTES at out (16-byte aligned, a multiple of 4)
+ *   SND_JOB_SUM           out[o*cols + i] = sum over r < rows of in[(o*rows + r)*cols + i], o < outer, added up in fp32
+ *                         (rows = 1: a cast); in_dtype -> out_dtype, which is in_dtype unless in is fp32
+ *   SND_JOB_WEIGHT        out[i] = in[i] / w(in2[i]), outer * cols elements, fp32: d merge_weights from snd_bwd's dmerge
+ *   SND_JOB_WEIGHT_GROUP  out[o] = sum over i < cols of in[o*cols + i] / w(in2[o*cols + i]): the same per group
+ *   SND_JOB_WEIGHT_FLOOR  out[i] = w(in[i])
+ * w(x) is x, or SND_MERGE_WEIGHT_FLOOR where |x| is below it: the merge weights a backward takes.  snd_bwd returns
+ * weight * d(weight), and dividing by a weight of exactly 0 would lose d(weight), which does not vanish with the weight;
+ * with the floor the other gradients of such a channel come out scaled by 1e-20 instead of 0. */
+#define SND_MERGE_WEIGHT_FLOOR 1e-20f
+enum { SND_JOB_CLEAR = 0, SND_JOB_SUM = 1, SND_JOB_WEIGHT = 2, SND_JOB_WEIGHT_GROUP = 3, SND_JOB_WEIGHT_FLOOR = 4 };
+typedef struct {
+    const void *in, *in2;
+    void *out;
+    int64_t outer, cols;
+    int32_t rows, kind, in_dtype, out_dtype;
+} snd_job;
+int snd_run_jobs(const snd_job *jobs, int n, snd_stream_t stream);
+
+/* Bytes at the start of the workspace that snd_fwd / snd_bwd, given one, clear in a launch of their own before the kernel
+ * (hand-over counts and words; 0 where the schedule hands nothing over), and the two calls for a host that has cleared
+ * them already - among its own SND_JOB_CLEARs, on the same stream - and saves that launch. */
+int64_t snd_clear_bytes(const snd_shape *shape, int schedule, int backward);
+int snd_fwd_cleared(const snd_fwd_params *params, snd_stream_t stream);
+int snd_bwd_cleared(const snd_bwd_params *params, snd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

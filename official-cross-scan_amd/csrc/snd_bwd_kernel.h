@@ -937,7 +937,7 @@ static int launch_bwd_te(const snd_bwd_params &p, const Geo &geo, hipStream_t st
     if (int st = ensure_device_ready(); st != SND_OK) return st;
     if (pipe) {
         if (nPC * geo.nCY >= (int64_t)1 << 31) return SND_ERR_SHAPE;
-        if (zero_words((int *)p.workspace, sync_words(nPC, geo.nCY), stream) != SND_OK) return SND_ERR_LAUNCH;
+        if (clear_sync_words((int *)p.workspace, sync_words(nPC, geo.nCY), stream) != SND_OK) return SND_ERR_LAUNCH;
         Geo gb = geo;
         gb.spinLimit = spin_limit();
         gb.nBands = bands;

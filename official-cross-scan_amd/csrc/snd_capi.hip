@@ -41,6 +41,8 @@ __global__ void zero_words_kernel(int *p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
 }
+static thread_local bool t_sync_cleared = false;    // this thread is inside snd_fwd_cleared / snd_bwd_cleared
+int clear_sync_words(int *p, int64_t n, hipStream_t stream) { return t_sync_cleared ? SND_OK : zero_words(p, n, stream); }
 int zero_words(int *p, int64_t n, hipStream_t stream) {
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, p, n);
     return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
@@ -428,6 +430,37 @@ static int bwd_checked(const snd_bwd_params *params, snd_stream_t stream) {
 }
 
 int snd_bwd(const snd_bwd_params *params, snd_stream_t stream) { return bwd_checked(params, stream); }
+
+int64_t snd_clear_bytes(const snd_shape *shape, int schedule, int backward) {
+    if (!shape || check_shape(*shape) != SND_OK || schedule < SND_SCHED_AUTO || schedule > SND_SCHED_WAVEFRONT) return 0;
+    const snd_shape &s = *shape;
+    const int wave = use_wavefront(s, schedule);
+    if (wave < 0) return 0;
+    if (wave) {
+        if (!backward || snd::wave_wide(s.ncols, s.dstate) || !snd::wave_bwd_split(s.batch, s.dim, s.ncols, s.dstate)) return 0;
+        return group_ws_offset(s) + (int64_t)s.batch * s.dim * s.dstate * snd::wave_split_words(snd::make_wave_geo(s.nrows, s.ncols, s.dstate)) * (int64_t)sizeof(float);
+    }
+    const snd::Geo g = snd::make_geo(s.nrows, s.ncols);
+    const int64_t pairs = (int64_t)s.batch * s.n_groups;
+    const int nChunks = (s.dim / s.n_groups + 15) / 16;
+    const int jobs = backward ? snd::bwd_band_count(schedule, pairs, nChunks, g.nCY, shape, s.dstate, g.nCX)
+                              : snd::fwd_band_count(schedule, pairs, nChunks, g.nCY, shape, s.dstate, g.nCX);
+    return jobs > 0 ? snd::sync_words(plane_chunks(s), g.nCY) * (int64_t)sizeof(int) : 0;
+}
+
+int snd_fwd_cleared(const snd_fwd_params *params, snd_stream_t stream) {
+    snd::t_sync_cleared = true;
+    const int st = snd_fwd(params, stream);
+    snd::t_sync_cleared = false;
+    return st;
+}
+
+int snd_bwd_cleared(const snd_bwd_params *params, snd_stream_t stream) {
+    snd::t_sync_cleared = true;
+    const int st = snd_bwd(params, stream);
+    snd::t_sync_cleared = false;
+    return st;
+}
 
 int snd_init(int device) {
     int cur = 0;

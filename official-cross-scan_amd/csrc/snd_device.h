@@ -418,6 +418,8 @@ int strip_segments(int64_t nPlaneChunks, int nStrips, int nTilesX, int64_t slots
 constexpr int kColStateFloats = 13 * 2 * 256;
 // Enqueue a fill kernel that zeroes n int32 words (defined with the C entry points).
 int zero_words(int *p, int64_t n, hipStream_t stream);
+// The same for a workspace's sync words, left out where the caller has cleared them (snd_fwd_cleared, snd_bwd_cleared).
+int clear_sync_words(int *p, int64_t n, hipStream_t stream);
 // Per-device set-up (kernel attributes, the address of the static scratch array), done by snd_init() or
 // by the first call that needs it on a device.  Returns an snd_status.
 int ensure_device_ready();

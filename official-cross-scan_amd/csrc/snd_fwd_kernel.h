@@ -586,7 +586,7 @@ static int launch_fwd_te(const snd_fwd_params &p, const Geo &geo, hipStream_t st
     const int bands = fwd_band_count(p.schedule, (int64_t)sh.batch * sh.n_groups, nChunks, geo.nCY, p.workspace, sh.dstate, geo.nCX);
     if (bands > 0) {
         if (nPC * geo.nCY >= (int64_t)1 << 31) return SND_ERR_SHAPE;
-        if (zero_words((int *)p.workspace, sync_words(nPC, geo.nCY), stream) != SND_OK) return SND_ERR_LAUNCH;
+        if (clear_sync_words((int *)p.workspace, sync_words(nPC, geo.nCY), stream) != SND_OK) return SND_ERR_LAUNCH;
         const int grid = (int)(nPC * bands);
         Geo gs = geo;
         gs.spinLimit = spin_limit();

@@ -13,6 +13,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <vector>
@@ -167,69 +168,254 @@ void check_merge(const Checked &c, bool merge, const c10::optional<at::Tensor> &
     }
 }
 
-std::vector<at::Tensor> selective_scan_fwd(const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
-                                           const at::Tensor &B, const at::Tensor &C,
-                                           const c10::optional<at::Tensor> &D_,
-                                           const c10::optional<at::Tensor> &delta_bias_, bool delta_softplus,
-                                           bool out_float, const c10::optional<at::Tensor> &A_decay_,
-                                           int64_t directions, int64_t schedule, bool merge,
-                                           const c10::optional<at::Tensor> &merge_weights_) {
-    TORCH_CHECK(directions == SND_DIR_TOPLEFT || directions == SND_DIR_CORNERS, "directions must be 0 (top-left) or 1 (four corners)");
-    const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
-    check_merge(c, merge, merge_weights_, u);
-    TORCH_CHECK(!merge || out_float, "the fused merge accumulates in float32: out_float must be true");
-    at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
-    const auto f32 = u.options().dtype(at::ScalarType::Float);
-    // merged: one fp32 channel per feature, zero-filled, to which every group adds its weighted result
-    at::Tensor out = merge ? torch::zeros({c.batch, c.dim / c.n_groups, c.nrows, c.ncols}, f32)
-                           : torch::empty({c.batch, c.dim, c.nrows, c.ncols},
-                                          u.options().dtype(out_float ? at::ScalarType::Float : u.scalar_type()));
-    at::Tensor x = torch::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_x, c.plan.x_inner}, f32);
-    at::Tensor x_v = torch::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_y, c.plan.xv_inner}, f32);
-    at::Tensor x_sd = torch::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_x, c.plan.x_inner}, f32);
+// Everything a scan call takes beside its tensors.
+struct Options {
+    bool delta_softplus = false, out_float = true;
+    int64_t directions = 0;
+    int sched = SND_SCHED_AUTO;
+    bool merge = false;
+};
+typedef c10::optional<at::Tensor> OptTensor;
 
+snd_job clear_job(void *ptr, int64_t bytes) {
+    snd_job j{};
+    j.kind = SND_JOB_CLEAR;
+    j.out = ptr;
+    j.outer = bytes;
+    return j;
+}
+// out[o][i] = sum over the rows of in[o][row][i] (one row: a cast)
+snd_job sum_job(const at::Tensor &in, int64_t outer, int rows, int64_t cols, const at::Tensor &out) {
+    snd_job j{};
+    j.kind = SND_JOB_SUM;
+    j.in = in.data_ptr();
+    j.out = out.data_ptr();
+    j.outer = outer; j.rows = rows; j.cols = cols;
+    j.in_dtype = dtype_code(in.scalar_type());
+    j.out_dtype = dtype_code(out.scalar_type());
+    return j;
+}
+void run_jobs(const snd_job *jobs, int n, hipStream_t stream, const char *what) {
+    if (n > 0) check_status(snd_run_jobs(jobs, n, (snd_stream_t)stream), what);
+}
+at::Tensor floats(int64_t n, const at::Tensor &like) { return at::empty({n}, like.options().dtype(at::kFloat)); }
+
+// The forward launch: clears what it accumulates into, and runs the kernel.  x == nullptr: no state is saved (x_v is then
+// scratch of this call).
+at::Tensor launch_fwd(const Checked &c, const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A, const at::Tensor &B,
+                      const at::Tensor &C, const OptTensor &D_, const OptTensor &delta_bias_, const OptTensor &A_decay_,
+                      const Options &o, const OptTensor &merge_weights_, float *x, float *x_v, float *x_sd) {
+    const auto f32 = u.options().dtype(at::kFloat);
+    // merged: one fp32 channel per feature, zero-filled, to which every group adds its weighted result
+    at::Tensor out = o.merge ? at::empty({c.batch, c.dim / c.n_groups, c.nrows, c.ncols}, f32)
+                             : at::empty({c.batch, c.dim, c.nrows, c.ncols}, o.out_float ? f32 : u.options());
+    auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
     snd_fwd_params p;
-    fill_fwd(p, c, u, delta, A, B, C, D_, delta_bias_, A_decay_, delta_softplus);
+    fill_fwd(p, c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o.delta_softplus);
     p.out = out.data_ptr();
     p.out_dtype = dtype_code(out.scalar_type());
     p.out_batch_stride = out.stride(0); p.out_d_stride = out.stride(1); p.out_h_stride = out.stride(2);
-    p.x = x.data_ptr<float>(); p.x_v = x_v.data_ptr<float>(); p.x_sd = x_sd.data_ptr<float>();
-    // scratch for the strip-pipelined schedule (only when it will be used); released to the caching
-    // allocator in stream order
-    const int sched = resolve_schedule(schedule);
-    p.schedule = sched;
-    at::Tensor ws;
-    if (pipelined(sched, c.plan.auto_schedule)) {
-        ws = torch::empty({(c.plan.fwd_workspace_bytes + 3) / 4}, f32);
+    p.schedule = o.sched;
+    p.directions = (int32_t)o.directions;
+    p.merge = o.merge ? 1 : 0;
+    p.merge_weights = o.merge && merge_weights_.has_value() ? merge_weights_.value().data_ptr<float>() : nullptr;
+    // scratch for the pipelined schedules, and for wide planes without saved state (only when it will be used); released to
+    // the caching allocator in stream order
+    const bool wave = wavefront(o.sched, c.plan);
+    const bool need_ws = wave ? !x && c.plan.wavefront_workspace : pipelined(o.sched, c.plan.auto_schedule);
+    at::Tensor ws, scratch;
+    if (need_ws) {
+        ws = floats((c.plan.fwd_workspace_bytes + 3) / 4, u);
         p.workspace = ws.data_ptr();
         p.workspace_bytes = c.plan.fwd_workspace_bytes;
     }
-    p.directions = (int32_t)directions;
-    p.merge = merge ? 1 : 0;
-    p.merge_weights = merge && merge_weights_.has_value() ? merge_weights_.value().data_ptr<float>() : nullptr;
-    auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-    check_status(snd_fwd(&p, (snd_stream_t)stream), "fwd");
+    if (!x) {                                       // (the row-segment kernels carry the row in registers and touch none of it)
+        const int64_t slabs = std::min(4, (int)c.plan.n_chunks_y);
+        scratch = floats(wave ? 4 : c.plan.x_v_elems / c.plan.n_chunks_y * slabs, u);
+        x_v = scratch.data_ptr<float>();
+    }
+    p.x = x; p.x_v = x_v; p.x_sd = x_sd;
+    snd_job jobs[2];
+    int nj = 0;
+    if (o.merge) jobs[nj++] = clear_job(out.data_ptr(), out.numel() * 4);
+    if (need_ws && !wave) jobs[nj++] = clear_job(ws.data_ptr(), snd_clear_bytes(&c.shape, o.sched, 0));
+    run_jobs(jobs, nj, stream, "fwd");
+    check_status(snd_fwd_cleared(&p, (snd_stream_t)stream), "fwd");
     check_pipeline(ws, stream, "fwd");
-    return {out, x, x_v, x_sd};
+    return out;
 }
 
-std::vector<at::Tensor> selective_scan_bwd(const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
-                                           const at::Tensor &B, const at::Tensor &C,
-                                           const c10::optional<at::Tensor> &D_,
-                                           const c10::optional<at::Tensor> &delta_bias_, const at::Tensor &dout,
-                                           const c10::optional<at::Tensor> &x_, const c10::optional<at::Tensor> &x_v_,
-                                           bool delta_softplus, const c10::optional<at::Tensor> &A_decay_,
-                                           const c10::optional<at::Tensor> &x_sd_, int64_t directions, int64_t schedule,
-                                           bool merge, const c10::optional<at::Tensor> &merge_weights_) {
+void check_call(const Options &o) {
+    TORCH_CHECK(o.directions == SND_DIR_TOPLEFT || o.directions == SND_DIR_CORNERS, "directions must be 0 (top-left) or 1 (four corners)");
+    TORCH_CHECK(!o.merge || o.out_float, "the fused merge accumulates in float32: out_float must be true");
+}
+
+std::vector<at::Tensor> selective_scan_fwd(const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
+                                           const at::Tensor &B, const at::Tensor &C, const OptTensor &D_,
+                                           const OptTensor &delta_bias_, bool delta_softplus, bool out_float,
+                                           const OptTensor &A_decay_, int64_t directions, int64_t schedule, bool merge,
+                                           const OptTensor &merge_weights_) {
+    Options o{delta_softplus, out_float, directions, SND_SCHED_AUTO, merge};
     TORCH_CHECK(directions == SND_DIR_TOPLEFT || directions == SND_DIR_CORNERS, "directions must be 0 (top-left) or 1 (four corners)");
     const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
     check_merge(c, merge, merge_weights_, u);
-    const int batch_size = c.batch, dim = c.dim, nrows = c.nrows, ncols = c.ncols, dstate = c.dstate;
+    check_call(o);
+    o.sched = resolve_schedule(schedule);
+    at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
+    const auto f32 = u.options().dtype(at::kFloat);
+    at::Tensor x = at::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_x, c.plan.x_inner}, f32);
+    at::Tensor x_v = at::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_y, c.plan.xv_inner}, f32);
+    at::Tensor x_sd = at::empty({c.batch, c.dim, c.dstate, c.plan.n_chunks_x, c.plan.x_inner}, f32);
+    at::Tensor out = launch_fwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o, merge_weights_, x.data_ptr<float>(),
+                                x_v.data_ptr<float>(), x_sd.data_ptr<float>());
+    return {out, x, x_v, x_sd};
+}
+
+struct Grads {
+    at::Tensor du, ddelta, dA, dB, dC, dD, ddelta_bias, dA_decay, dmerge, dweights;
+};
+
+// The backward launch with its passes before (accumulators and sync words cleared, merge weights floored) and after it
+// (dB / dC cast to the input dtype, du folded over the groups that share u and ddelta over the channels that share a
+// delta, host.cpp:432-438; d merge_weights), each side one launch.
+// want_weights: dweights = d merge_weights, of `weight_numel` elements (per channel, or per group), and the weights enter
+// floored (SND_MERGE_WEIGHT_FLOOR); otherwise they enter as they are and only dmerge = weight * d(weight) is returned.
+Grads launch_bwd(const Checked &c, const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A, const at::Tensor &B,
+                 const at::Tensor &C, const OptTensor &D_, const OptTensor &delta_bias_, const OptTensor &A_decay_, const at::Tensor &dout,
+                 const float *x, const float *x_v, const float *x_sd, const Options &o, const OptTensor &merge_weights_,
+                 bool floor_weights, int64_t weight_numel) {
+    const int64_t dim = c.dim, HW = (int64_t)c.nrows * c.ncols;
+    auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    Grads g;
+    g.du = at::empty({c.batch, dim, c.nrows, c.ncols}, u.options());
+    g.ddelta = at::empty({c.batch, dim, c.nrows, c.ncols}, u.options());
+    // the accumulated gradients are zero-filled as host.cpp:395-403 does.  dB and dC share one buffer; the small ones (dA, dD,
+    // ddelta_bias, dA_decay) share another, so that a parameter gradient kept by the optimizer never pins the large buffer.
+    const int64_t nA = dim * c.dstate, nBC = B.numel();
+    auto round64 = [](int64_t v) { return (v + 63) / 64 * 64; };
+    // dB and dC are accumulated at equal offsets at the same time.  Where that matters (the row-segment kernels on
+    // tensors of 2 MiB and more) dC starts a chosen distance past the 2 MiB-rounded end of dB (snd_plan.dC_skew_bytes:
+    // not a multiple of 2 MiB apart); everywhere else it follows dB directly.
+    const bool spread = c.plan.auto_schedule == SND_SCHED_WAVEFRONT && nBC * 4 >= (int64_t)(2 << 20);
+    const int64_t oC = spread ? (round_2mib(nBC * 4) + c.plan.dC_skew_bytes) / 4 : round64(nBC);
+    at::Tensor accBC = floats(oC + nBC, u);
+    g.dB = accBC.narrow(0, 0, nBC).view(B.sizes());
+    g.dC = accBC.narrow(0, oC, nBC).view(C.sizes());
+    const bool merge = o.merge, weights = merge && merge_weights_.has_value();
+    const int64_t oD = round64(nA), oBias = oD + round64(dim), oDec = oBias + round64(dim), oMerge = oDec + 64, nP = oMerge + (merge ? round64(dim) : 0);
+    at::Tensor accP = floats(nP, u);
+    g.dA = accP.narrow(0, 0, nA).view({dim, c.dstate});
+    if (D_.has_value()) g.dD = accP.narrow(0, oD, dim);
+    if (delta_bias_.has_value()) g.ddelta_bias = accP.narrow(0, oBias, dim);
+    if (A_decay_.has_value()) g.dA_decay = accP.narrow(0, oDec, 1);
+    if (merge) g.dmerge = accP.narrow(0, oMerge, dim);   // weight * d(weight) per channel
+    at::Tensor ws, wfloor;                          // (the row-segment kernels need no workspace, except for planes taken in column groups or halves)
+    if (!wavefront(o.sched, c.plan) || c.plan.wavefront_workspace) ws = floats((c.plan.bwd_workspace_bytes + 3) / 4, u);
+
+    snd_job jobs[8];
+    int nj = 0;
+    // one job over both accumulators where the gap between them is small beside them
+    if ((oC - nBC) * 4 <= nBC) {
+        jobs[nj++] = clear_job(accBC.data_ptr(), (oC + nBC) * 4);
+    } else {
+        jobs[nj++] = clear_job(g.dB.data_ptr(), nBC * 4);
+        jobs[nj++] = clear_job(g.dC.data_ptr(), nBC * 4);
+    }
+    jobs[nj++] = clear_job(accP.data_ptr(), nP * 4);
+    if (ws.defined()) jobs[nj++] = clear_job(ws.data_ptr(), snd_clear_bytes(&c.shape, o.sched, 1));
+    if (weights && floor_weights) {
+        wfloor = floats(dim, u);
+        snd_job j{};
+        j.kind = SND_JOB_WEIGHT_FLOOR;
+        j.in = merge_weights_.value().data_ptr();
+        j.out = wfloor.data_ptr();
+        j.outer = 1; j.cols = dim; j.rows = 1;
+        jobs[nj++] = j;
+    }
+    run_jobs(jobs, nj, stream, "bwd");
+
+    snd_bwd_params p;
+    memset(&p, 0, sizeof(p));
+    fill_fwd(p.f, c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o.delta_softplus);
+    p.f.x = const_cast<float *>(x); p.f.x_v = const_cast<float *>(x_v); p.f.x_sd = const_cast<float *>(x_sd);
+    p.dout = dout.data_ptr();
+    p.dout_dtype = dtype_code(dout.scalar_type());
+    p.dout_batch_stride = dout.stride(0); p.dout_d_stride = dout.stride(1); p.dout_h_stride = dout.stride(2);
+    p.du = g.du.data_ptr(); p.ddelta = g.ddelta.data_ptr();
+    p.dA = g.dA.data_ptr<float>(); p.dB = g.dB.data_ptr<float>(); p.dC = g.dC.data_ptr<float>();
+    p.dD = g.dD.defined() ? g.dD.data_ptr<float>() : nullptr;
+    p.ddelta_bias = g.ddelta_bias.defined() ? g.ddelta_bias.data_ptr<float>() : nullptr;
+    p.dA_decay = g.dA_decay.defined() ? g.dA_decay.data_ptr<float>() : nullptr;
+    p.workspace = ws.defined() ? ws.data_ptr() : nullptr;
+    p.workspace_bytes = ws.defined() ? c.plan.bwd_workspace_bytes : 0;
+    p.f.schedule = o.sched;
+    p.f.directions = (int32_t)o.directions;
+    p.f.merge = merge ? 1 : 0;
+    p.f.merge_weights = wfloor.defined() ? wfloor.data_ptr<float>() : weights ? merge_weights_.value().data_ptr<float>() : nullptr;
+    p.dmerge = merge ? g.dmerge.data_ptr<float>() : nullptr;
+    check_status(snd_bwd_cleared(&p, (snd_stream_t)stream), "bwd");
+    if (o.sched == SND_SCHED_STRIPS || o.sched == SND_SCHED_BANDS || (o.sched == SND_SCHED_AUTO && c.plan.auto_bwd_jobs != 0))
+        check_pipeline(ws, stream, "bwd");
+
+    nj = 0;
+    if (B.scalar_type() != at::kFloat) {
+        at::Tensor cast = at::empty({2 * round64(nBC)}, B.options());
+        at::Tensor dBc = cast.narrow(0, 0, nBC).view(B.sizes()), dCc = cast.narrow(0, round64(nBC), nBC).view(C.sizes());
+        jobs[nj++] = sum_job(g.dB, 1, 1, nBC, dBc);
+        jobs[nj++] = sum_job(g.dC, 1, 1, nBC, dCc);
+        g.dB = dBc;
+        g.dC = dCc;
+    }
+    at::Tensor du_all, dd_all, db_all;              // (kept until the launch below is enqueued)
+    if (dim != c.delta_dim) {
+        const int rep = dim / c.delta_dim;
+        dd_all = g.ddelta;
+        g.ddelta = at::empty({c.batch, c.delta_dim, c.nrows, c.ncols}, u.options());
+        jobs[nj++] = sum_job(dd_all, (int64_t)c.batch * c.delta_dim, rep, HW, g.ddelta);
+        if (delta_bias_.has_value()) {
+            db_all = g.ddelta_bias;
+            g.ddelta_bias = floats(c.delta_dim, u);
+            jobs[nj++] = sum_job(db_all, c.delta_dim, rep, 1, g.ddelta_bias);
+        }
+    }
+    if (c.u_shared) {   // one feature map scanned by every group: its gradient is the sum over the groups
+        du_all = g.du;
+        g.du = at::empty({c.batch, dim / c.n_groups, c.nrows, c.ncols}, u.options());
+        jobs[nj++] = sum_job(du_all, c.batch, c.n_groups, dim / c.n_groups * HW, g.du);
+    }
+    if (weights && weight_numel > 0) {
+        g.dweights = floats(weight_numel, u);
+        snd_job j{};
+        j.kind = weight_numel == dim ? SND_JOB_WEIGHT : SND_JOB_WEIGHT_GROUP;
+        j.in = g.dmerge.data_ptr(); j.in2 = merge_weights_.value().data_ptr(); j.out = g.dweights.data_ptr();
+        j.outer = c.n_groups; j.cols = dim / c.n_groups; j.rows = 1;
+        jobs[nj++] = j;
+    }
+    run_jobs(jobs, nj, stream, "bwd");
+    return g;
+}
+
+void check_dout(const Checked &c, const at::Tensor &u, const at::Tensor &dout, bool merge) {
+    const int batch_size = c.batch, dim = c.dim, nrows = c.nrows, ncols = c.ncols;
     TORCH_CHECK(dout.scalar_type() == u.scalar_type() || dout.scalar_type() == at::ScalarType::Float,
                 "dout must be float32 or the input dtype");
     TORCH_CHECK(dout.is_cuda());
     TORCH_CHECK(dout.stride(-1) == 1 || dout.size(-1) == 1, "dout must be contiguous in its last dimension");
     CHECK_SHAPE(dout, batch_size, merge ? dim / c.n_groups : dim, nrows, ncols);   // merged: the gradient of the merged output
+}
+
+std::vector<at::Tensor> selective_scan_bwd(const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
+                                           const at::Tensor &B, const at::Tensor &C, const OptTensor &D_,
+                                           const OptTensor &delta_bias_, const at::Tensor &dout, const OptTensor &x_,
+                                           const OptTensor &x_v_, bool delta_softplus, const OptTensor &A_decay_,
+                                           const OptTensor &x_sd_, int64_t directions, int64_t schedule, bool merge,
+                                           const OptTensor &merge_weights_) {
+    Options o{delta_softplus, true, directions, SND_SCHED_AUTO, merge};
+    check_call(o);
+    const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
+    check_merge(c, merge, merge_weights_, u);
+    const int batch_size = c.batch, dim = c.dim, dstate = c.dstate;
+    check_dout(c, u, dout, merge);
     // the saved state is required: gradients computed without it would belong to another function
     TORCH_CHECK(x_.has_value() && x_v_.has_value() && x_sd_.has_value(),
                 "bwd needs the x, x_v and x_sd tensors returned by fwd");
@@ -243,88 +429,100 @@ std::vector<at::Tensor> selective_scan_bwd(const at::Tensor &u, const at::Tensor
     CHECK_SHAPE(x, batch_size, dim, dstate, nChunksX, x_inner);
     CHECK_SHAPE(x_sd, batch_size, dim, dstate, nChunksX, x_inner);
     CHECK_SHAPE(x_v, batch_size, dim, dstate, nChunksY, xv_inner);
-
+    o.sched = resolve_schedule(schedule);
     at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
-    const auto f32 = u.options().dtype(at::ScalarType::Float);
-    at::Tensor du = torch::empty({batch_size, dim, nrows, ncols}, u.options());
-    at::Tensor ddelta = torch::empty({batch_size, dim, nrows, ncols}, u.options());
-    // the accumulated gradients are zero-filled as host.cpp:395-403 does.  dB and dC share one buffer (one
-    // fill kernel for the two large tensors); the small ones (dA, dD, ddelta_bias, dA_decay) share another,
-    // so that a parameter gradient kept by the optimizer never pins the large buffer.
-    const int64_t nA = (int64_t)dim * dstate, nBC = B.numel();
-    auto round64 = [](int64_t v) { return (v + 63) / 64 * 64; };
-    // dB and dC are accumulated at equal offsets at the same time.  Where that matters (the row-segment kernels on
-    // tensors of 2 MiB and more) dC starts a chosen distance past the 2 MiB-rounded end of dB (snd_plan.dC_skew_bytes:
-    // not a multiple of 2 MiB apart); everywhere else it follows dB directly and nothing beyond the two is filled.
-    const bool spread = c.plan.auto_schedule == SND_SCHED_WAVEFRONT && nBC * 4 >= (int64_t)(2 << 20);
-    const int64_t oC = spread ? (round_2mib(nBC * 4) + c.plan.dC_skew_bytes) / 4 : round64(nBC);
-    // one fill (and, for 16-bit inputs, one cast) over both where the gap between them is small beside them, else one
-    // per tensor
-    const bool whole = (oC - nBC) * 4 <= nBC;
-    at::Tensor accBC = whole ? torch::zeros({oC + nBC}, f32) : torch::empty({oC + nBC}, f32);
-    at::Tensor dB = accBC.narrow(0, 0, nBC).view(B.sizes());
-    at::Tensor dC = accBC.narrow(0, oC, nBC).view(C.sizes());
-    if (!whole) { dB.zero_(); dC.zero_(); }         // (not the gap between them)
-    const int64_t oD = round64(nA), oBias = oD + round64(dim), oDec = oBias + round64(dim), oMerge = oDec + 64;
-    at::Tensor accP = torch::zeros({oMerge + (merge ? round64(dim) : 0)}, f32);
-    at::Tensor dA = accP.narrow(0, 0, nA).view({dim, dstate});
-    at::Tensor dD, ddelta_bias, dA_decay;
-    if (D_.has_value()) dD = accP.narrow(0, oD, dim);
-    if (delta_bias_.has_value()) ddelta_bias = accP.narrow(0, oBias, dim);
-    if (A_decay_.has_value()) dA_decay = accP.narrow(0, oDec, 1);
-    at::Tensor dmerge;                              // weight * d(weight) per channel (the caller divides)
-    if (merge) dmerge = accP.narrow(0, oMerge, dim);
-    const int sched = resolve_schedule(schedule);
-    at::Tensor ws;                                  // the wavefront kernels need none, except for planes taken in column groups
-    if (!wavefront(sched, c.plan) || c.plan.wavefront_workspace) ws = torch::empty({(c.plan.bwd_workspace_bytes + 3) / 4}, f32);
-
-    snd_bwd_params p;
-    memset(&p, 0, sizeof(p));
-    fill_fwd(p.f, c, u, delta, A, B, C, D_, delta_bias_, A_decay_, delta_softplus);
-    p.f.x = x.data_ptr<float>(); p.f.x_v = x_v.data_ptr<float>(); p.f.x_sd = x_sd.data_ptr<float>();
-    p.dout = dout.data_ptr();
-    p.dout_dtype = dtype_code(dout.scalar_type());
-    p.dout_batch_stride = dout.stride(0); p.dout_d_stride = dout.stride(1); p.dout_h_stride = dout.stride(2);
-    p.du = du.data_ptr(); p.ddelta = ddelta.data_ptr();
-    p.dA = dA.data_ptr<float>(); p.dB = dB.data_ptr<float>(); p.dC = dC.data_ptr<float>();
-    p.dD = dD.defined() ? dD.data_ptr<float>() : nullptr;
-    p.ddelta_bias = ddelta_bias.defined() ? ddelta_bias.data_ptr<float>() : nullptr;
-    p.dA_decay = dA_decay.defined() ? dA_decay.data_ptr<float>() : nullptr;
-    p.workspace = ws.defined() ? ws.data_ptr() : nullptr;
-    p.workspace_bytes = ws.defined() ? c.plan.bwd_workspace_bytes : 0;
-    p.f.schedule = sched;
-    p.f.directions = (int32_t)directions;
-    p.f.merge = merge ? 1 : 0;
-    p.f.merge_weights = merge && merge_weights_.has_value() ? merge_weights_.value().data_ptr<float>() : nullptr;
-    p.dmerge = dmerge.defined() ? dmerge.data_ptr<float>() : nullptr;
-    auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-    check_status(snd_bwd(&p, (snd_stream_t)stream), "bwd");
-    if (sched == SND_SCHED_STRIPS || sched == SND_SCHED_BANDS || (sched == SND_SCHED_AUTO && c.plan.auto_bwd_jobs != 0))
-        check_pipeline(ws, stream, "bwd");
-
-    // host.cpp:432-438: cast dB/dC to the input dtype, fold channel groups that share a delta
-    // (16-bit inputs: one cast kernel for the two tensors, which share a buffer)
-    at::Tensor dBo = dB, dCo = dC;
-    if (B.scalar_type() != at::ScalarType::Float) {
-        if (!whole) {                               // two casts of the live ranges, not one of the gap as well
-            dBo = dB.to(B.dtype());
-            dCo = dC.to(C.dtype());
-        } else {
-            const at::Tensor cast = accBC.to(B.dtype());
-            dBo = cast.narrow(0, 0, nBC).view(B.sizes());
-            dCo = cast.narrow(0, oC, nBC).view(C.sizes());
-        }
-    }
-    std::vector<at::Tensor> result = {du, ddelta, dA, dBo, dCo, dD, ddelta_bias, dA_decay};
-    if (dim != c.delta_dim) {
-        const int rep = dim / c.delta_dim;
-        result[1] = ddelta.view({batch_size, c.delta_dim, rep, nrows, ncols}).sum(2);
-        if (delta_bias_.has_value()) result[6] = ddelta_bias.view({c.delta_dim, rep}).sum(1);
-    }
-    if (c.u_shared)   // one feature map scanned by every group: its gradient is the sum over the groups
-        result[0] = du.view({batch_size, c.n_groups, dim / c.n_groups, nrows, ncols}).sum(1);
-    if (merge) result.push_back(dmerge);
+    Grads g = launch_bwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, dout, x.data_ptr<float>(), x_v.data_ptr<float>(),
+                         x_sd.data_ptr<float>(), o, merge_weights_, false, 0);
+    std::vector<at::Tensor> result = {g.du, g.ddelta, g.dA, g.dB, g.dC, g.dD, g.ddelta_bias, g.dA_decay};
+    if (merge) result.push_back(g.dmerge);
     return result;
+}
+
+at::Tensor rows_contiguous(const at::Tensor &t) { return t.stride(-1) == 1 || t.size(-1) == 1 ? t : t.contiguous(); }
+OptTensor optional_of(const at::Tensor &t) { return t.defined() ? OptTensor(t) : OptTensor(); }
+
+// The differentiable scan.  The saved state is one buffer [x | x_sd | x_v] that only the backward reads.
+// The block mapping is resolved once, in the forward, and the backward runs the same one: the two kernel families keep
+// different saved-state layouts, so a default changed between a forward and its backward must not reach it.
+struct ScanFn : public torch::autograd::Function<ScanFn> {
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
+                              const at::Tensor &B, const at::Tensor &C, const OptTensor &D_, const OptTensor &delta_bias_,
+                              const OptTensor &A_decay_, const OptTensor &weights_, bool delta_softplus, bool out_float,
+                              int64_t directions, bool merge) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        Options o{delta_softplus, out_float, directions, resolve_schedule(-1), merge};
+        OptTensor w;
+        const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
+        if (weights_.has_value())                   // [G], [G, 1] or [G, D/G] -> one per channel
+            w = weights_.value().to(at::kFloat).reshape({c.n_groups, -1}).expand({c.n_groups, c.dim / c.n_groups}).contiguous().view(-1);
+        check_merge(c, merge, w, u);
+        check_call(o);
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
+        const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        at::Tensor state = floats(2 * nx + c.plan.x_v_elems, u);
+        float *st = state.data_ptr<float>();
+        at::Tensor out = launch_fwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o, w, st, st + 2 * nx, st + nx);
+        ctx->save_for_backward({u, delta, A, B, C, D_.value_or(at::Tensor()), delta_bias_.value_or(at::Tensor()), A_decay_.value_or(at::Tensor()),
+                                w.value_or(at::Tensor()), state});
+        ctx->saved_data["softplus"] = delta_softplus;
+        ctx->saved_data["directions"] = directions;
+        ctx->saved_data["sched"] = (int64_t)o.sched;
+        ctx->saved_data["merge"] = merge;
+        if (weights_.has_value()) {
+            ctx->saved_data["w_shape"] = weights_.value().sizes().vec();
+            ctx->saved_data["w_dtype"] = (int64_t)weights_.value().scalar_type();
+        }
+        return out;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &u = saved[0], &delta = saved[1], &A = saved[2], &B = saved[3], &C = saved[4], &state = saved[9];
+        const OptTensor D_ = optional_of(saved[5]), delta_bias_ = optional_of(saved[6]), A_decay_ = optional_of(saved[7]), w = optional_of(saved[8]);
+        torch::autograd::variable_list r(13);
+        if (!grads[0].defined()) return r;
+        Options o{ctx->saved_data["softplus"].toBool(), true, ctx->saved_data["directions"].toInt(), (int)ctx->saved_data["sched"].toInt(),
+                  ctx->saved_data["merge"].toBool()};
+        const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
+        const at::Tensor dout = rows_contiguous(grads[0]);
+        check_dout(c, u, dout, o.merge);
+        const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        const float *st = state.data_ptr<float>();
+        int64_t wn = 0;
+        if (w.has_value()) {
+            wn = 1;
+            for (int64_t s : ctx->saved_data["w_shape"].toIntVector()) wn *= s;
+        }
+        Grads g = launch_bwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, dout, st, st + 2 * nx, st + nx, o, w, true, wn);
+        r[0] = g.du; r[1] = g.ddelta; r[2] = g.dA; r[3] = g.dB; r[4] = g.dC; r[5] = g.dD; r[6] = g.ddelta_bias; r[7] = g.dA_decay;
+        if (wn > 0) r[8] = g.dweights.view(ctx->saved_data["w_shape"].toIntVector()).to((at::ScalarType)ctx->saved_data["w_dtype"].toInt());
+        return r;
+    }
+};
+
+// selective_nd_scan / selective_nd_scan_merged: the differentiable function where a gradient can be asked for, the forward
+// that saves no state where none can.
+at::Tensor scan(const at::Tensor &u_, const at::Tensor &delta_, const at::Tensor &A, const at::Tensor &B_, const at::Tensor &C_,
+                const OptTensor &D_, const OptTensor &delta_bias_, bool delta_softplus, bool out_float, const OptTensor &A_decay_,
+                int64_t directions, bool merge, const OptTensor &weights_) {
+    TORCH_CHECK(u_.dim() == 4 && delta_.dim() == 4 && A.dim() == 2 && B_.dim() == 5 && C_.dim() == 5, "expected u, delta 4-D; A 2-D; B, C 5-D");
+    const at::Tensor u = rows_contiguous(u_), delta = rows_contiguous(delta_), B = rows_contiguous(B_), C = rows_contiguous(C_);
+    bool grad = false;
+    if (at::GradMode::is_enabled()) {
+        for (const at::Tensor *t : {&u, &delta, &A, &B, &C}) grad = grad || t->requires_grad();
+        for (const OptTensor *t : {&D_, &delta_bias_, &A_decay_, &weights_}) grad = grad || (t->has_value() && t->value().requires_grad());
+    }
+    if (grad) return ScanFn::apply(u, delta, A, B, C, D_, delta_bias_, A_decay_, weights_, delta_softplus, out_float, directions, merge);
+    at::AutoDispatchBelowADInplaceOrView below;
+    Options o{delta_softplus, out_float, directions, resolve_schedule(-1), merge};
+    const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
+    OptTensor w;
+    if (weights_.has_value())
+        w = weights_.value().to(at::kFloat).reshape({c.n_groups, -1}).expand({c.n_groups, c.dim / c.n_groups}).contiguous().view(-1);
+    check_merge(c, merge, w, u);
+    check_call(o);
+    at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
+    return launch_fwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o, w, nullptr, nullptr, nullptr);
 }
 
 }  // namespace
@@ -344,6 +542,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("B"), py::arg("C"), py::arg("D"), py::arg("delta_bias"), py::arg("dout"), py::arg("x"), py::arg("x_v"),
           py::arg("delta_softplus"), py::arg("A_decay"), py::arg("x_sd"), py::arg("directions") = 0, py::arg("schedule") = -1,
           py::arg("merge") = false, py::arg("merge_weights") = py::none());
+    m.def("scan", &scan, "selective_nd_scan / selective_nd_scan_merged (differentiable)", py::arg("u"), py::arg("delta"), py::arg("A"),
+          py::arg("B"), py::arg("C"), py::arg("D"), py::arg("delta_bias"), py::arg("delta_softplus"), py::arg("out_float"),
+          py::arg("A_decay"), py::arg("directions"), py::arg("merge"), py::arg("merge_weights"));
     m.def("set_schedule", [](int mode) {
         TORCH_CHECK(mode >= SND_SCHED_AUTO && mode <= SND_SCHED_WAVEFRONT, "schedule must be 0 (auto), 1 (plane), 2 (strips), 3 (bands) or 4 (row-segment wavefront)");
         g_schedule.store(mode);

@@ -705,7 +705,7 @@ static int launch_wave_bwd_split(const snd_bwd_params &p, WaveGeo wg, float *gro
     constexpr bool F32 = std::is_same<T, float>::value;
     constexpr bool K = NS <= 2;                      // (the kernel exists for one and two states)
     const int64_t words = (int64_t)((char *)group_ws - (char *)p.workspace) / 4 + (int64_t)sh.batch * sh.dim * sh.dstate * wave_split_words(wg);
-    if (zero_words((int *)p.workspace, words, stream) != SND_OK) return SND_ERR_LAUNCH;
+    if (clear_sync_words((int *)p.workspace, words, stream) != SND_OK) return SND_ERR_LAUNCH;
     wg.bcol = group_ws;
     wg.sync = (int *)p.workspace;
     wg.spinLimit = spin_limit();

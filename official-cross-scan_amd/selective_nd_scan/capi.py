@@ -49,6 +49,15 @@ class BwdParams(C.Structure):
                 [("workspace_bytes", i64), ("dmerge", vp)])
 
 
+class Job(C.Structure):
+    """snd_job: one pass of snd_run_jobs."""
+    _fields_ = [("src", vp), ("src2", vp), ("out", vp), ("outer", C.c_int64), ("cols", C.c_int64), ("rows", C.c_int32), ("kind", C.c_int32),
+                ("in_dtype", C.c_int32), ("out_dtype", C.c_int32)]
+
+
+JOB_CLEAR, JOB_SUM, JOB_WEIGHT, JOB_WEIGHT_GROUP, JOB_WEIGHT_FLOOR = range(5)
+
+
 def declared_symbols():
     """Every function include/snd_scan.h declares."""
     text = open(HEADER).read()
@@ -74,6 +83,11 @@ def lib():
         _lib.snd_bwd_static.argtypes = [C.POINTER(BwdParams), vp]
         _lib.snd_static_workspace_bytes.restype = C.c_int64
         _lib.snd_init.argtypes = [C.c_int]
+        _lib.snd_fwd_cleared.argtypes = [C.POINTER(FwdParams), vp]
+        _lib.snd_bwd_cleared.argtypes = [C.POINTER(BwdParams), vp]
+        _lib.snd_clear_bytes.argtypes = [C.POINTER(Shape), C.c_int, C.c_int]
+        _lib.snd_clear_bytes.restype = C.c_int64
+        _lib.snd_run_jobs.argtypes = [C.POINTER(Job), C.c_int, vp]
         _lib.snd_workspace_error.argtypes = [vp, vp]
         _lib.snd_debug_set_spin_limit.argtypes = [C.c_int]
         _lib.snd_debug_set_spin_limit.restype = None

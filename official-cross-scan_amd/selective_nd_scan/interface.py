@@ -1,8 +1,8 @@
 """Python face of the 2D-CrossScan selective scan on MI355X.
 
 The reference ships only the pybind pair `fwd` / `bwd`
-(kernels/selective_nd_scan/src/cusoflex/selective_scan_oflex.cpp:442-445); the Python function and
-autograd.Function that backbones call are authored here on top of the same pair, with the argument
+(kernels/selective_nd_scan/src/cusoflex/selective_scan_oflex.cpp:442-445); the Python function that
+backbones call is authored here, on a native autograd function over the same pair, with the argument
 order of those bindings (selective_scan_oflex.cpp:179-187).
 
     out = selective_nd_scan(u, delta, A, B, C, D=None, delta_bias=None,
@@ -19,8 +19,6 @@ With directions=0 every group is scanned from the top-left corner, as the refere
 (selective_scan_fwd_kernel_oflex.cuh:140).  directions=1 starts group g at corner g % 4 inside the
 kernels (no flipped copies); cross_scan.py builds the four-corner block on top of it.
 """
-import torch
-
 from ._ext import ext
 
 
@@ -71,97 +69,31 @@ def init(device=0):
     ext().init(int(device))
 
 
-def _last_dim_contiguous(t):
-    return t if (t is None or t.stride(-1) == 1 or t.size(-1) == 1) else t.contiguous()
-
-
-class SelectiveNdScanFn(torch.autograd.Function):
-    @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True,
-                A_decay=None, directions=0):
-        u, delta, B, C = map(_last_dim_contiguous, (u, delta, B, C))
-        # The block mapping is resolved once, here, and the backward is told the same one: the two kernel families keep
-        # different saved-state layouts, so a default changed between a forward and its backward must not reach it.
-        ctx.schedule = get_schedule()
-        out, x, x_v, x_sd = fwd(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, ctx.schedule)
-        ctx.delta_softplus = delta_softplus
-        ctx.directions = directions
-        ctx.has = (D is not None, delta_bias is not None, A_decay is not None)
-        ctx.save_for_backward(u, delta, A, B, C, D, delta_bias, A_decay, x, x_v, x_sd)
-        return out
+class SelectiveNdScanFn:
+    """selective_nd_scan under the name and call form of an autograd.Function (the function itself, forward and
+    backward, is native code in the extension)."""
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, dout):
-        u, delta, A, B, C, D, delta_bias, A_decay, x, x_v, x_sd = ctx.saved_tensors
-        dout = _last_dim_contiguous(dout)
-        du, ddelta, dA, dB, dC, dD, ddelta_bias, dA_decay = bwd(
-            u, delta, A, B, C, D, delta_bias, dout, x, x_v, ctx.delta_softplus, A_decay, x_sd, ctx.directions, ctx.schedule)
-        has_D, has_bias, has_decay = ctx.has
-        return (du, ddelta, dA, dB, dC, dD if has_D else None, ddelta_bias if has_bias else None,
-                None, None, dA_decay if has_decay else None, None)
+    def apply(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True, A_decay=None,
+              directions=0):
+        return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
 
 
 def selective_nd_scan(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True,
                       A_decay=None, directions=0):
     """Differentiable 2D-CrossScan selective scan (forward and backward run on the HIP kernels).
-    directions=1: group g of B/C (and its dim/G channels) is scanned from corner g % 4."""
-    return SelectiveNdScanFn.apply(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions)
+    directions=1: group g of B/C (and its dim/G channels) is scanned from corner g % 4.
+    Where no gradient can be asked for (no_grad, or no input that requires one) the forward saves no state."""
+    return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
 
 
-# Magnitude below which a merge weight enters the backward as +-1e-20 instead of itself.  The kernels return
-# weight * d(weight) (every gradient of the op is linear in the weighted dout, so the weight is applied once,
-# where dout is staged); dividing by a weight of exactly 0 would lose d(weight), which is <dout, result> and does
-# not vanish with the weight.  With the floor, the other gradients of such a channel come out scaled by 1e-20
-# instead of 0: far below one ulp of anything they are added to.
-_MERGE_WEIGHT_FLOOR = 1e-20
-
-
-class SelectiveNdScanMergedFn(torch.autograd.Function):
+class SelectiveNdScanMergedFn:
     """The scan with the CrossMerge fused into its output stores: out [B, D/G, H, W] fp32 is the sum over the
     G groups of merge_weights[g, i] * (result of channel g*(D/G) + i)."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, u, delta, A, B, C, D, delta_bias, delta_softplus, A_decay, directions, merge_weights):
-        u, delta, B, C = map(_last_dim_contiguous, (u, delta, B, C))
-        w = None
-        if merge_weights is not None:
-            G = B.shape[1]
-            w = merge_weights.detach().to(torch.float32).reshape(G, -1).expand(G, A.shape[0] // G).contiguous().view(-1)
-        ctx.schedule = get_schedule()               # (resolved once for the pair: see SelectiveNdScanFn.forward)
-        out, x, x_v, x_sd = fwd(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, ctx.schedule, True, w)
-        ctx.delta_softplus = delta_softplus
-        ctx.directions = directions
-        ctx.has = (D is not None, delta_bias is not None, A_decay is not None)
-        ctx.w_shape = None if merge_weights is None else tuple(merge_weights.shape)
-        ctx.w_dtype = None if merge_weights is None else merge_weights.dtype
-        ctx.save_for_backward(u, delta, A, B, C, D, delta_bias, A_decay, x, x_v, x_sd, w)
-        return out
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, dout):
-        u, delta, A, B, C, D, delta_bias, A_decay, x, x_v, x_sd, w = ctx.saved_tensors
-        dout = _last_dim_contiguous(dout)
-        wb = None
-        if w is not None:
-            floor = torch.full_like(w, _MERGE_WEIGHT_FLOOR)
-            wb = torch.where(w.abs() < _MERGE_WEIGHT_FLOOR, floor, w)
-        du, ddelta, dA, dB, dC, dD, ddelta_bias, dA_decay, wdw = bwd(
-            u, delta, A, B, C, D, delta_bias, dout, x, x_v, ctx.delta_softplus, A_decay, x_sd, ctx.directions, ctx.schedule,
-            True, wb)
-        dw = None
-        if w is not None and ctx.needs_input_grad[10]:
-            G = B.shape[1]
-            dw = (wdw / wb).view(G, -1)
-            if ctx.w_shape != tuple(dw.shape):       # weights were given per group ([G] or [G, 1]): sum the features
-                dw = dw.sum(1).view(ctx.w_shape)
-            dw = dw.to(ctx.w_dtype)
-        has_D, has_bias, has_decay = ctx.has
-        return (du, ddelta, dA, dB, dC, dD if has_D else None, ddelta_bias if has_bias else None,
-                None, dA_decay if has_decay else None, None, dw)
+    def apply(u, delta, A, B, C, D, delta_bias, delta_softplus, A_decay, directions, merge_weights):
+        return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)
 
 
 def selective_nd_scan_merged(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, A_decay=None,
@@ -177,5 +109,4 @@ def selective_nd_scan_merged(u, delta, A, B, C, D=None, delta_bias=None, delta_s
                 raise ValueError("merge_weights must have shape [G], [G, 1] or [G, D/G]")
         elif tuple(merge_weights.shape) not in ((G, 1), (G, A.shape[0] // G)):
             raise ValueError("merge_weights must have shape [G], [G, 1] or [G, D/G]")
-    return SelectiveNdScanMergedFn.apply(u, delta, A, B, C, D, delta_bias, delta_softplus, A_decay, directions,
-                                         merge_weights)
+    return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)
