@@ -22,7 +22,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .cross_scan import cross_merge, four_corner_scan
+from .cross_scan import cross_merge, cross_scan_2d
 
 
 class SS2DCrossScan(nn.Module):
@@ -34,7 +34,7 @@ class SS2DCrossScan(nn.Module):
         self.d_model, self.d_state = d_model, d_state
         self.d_inner = int(ssm_ratio * d_model)
         self.dt_rank = math.ceil(d_model / 16) if dt_rank == "auto" else dt_rank
-        self.scan_fn = scan_fn or four_corner_scan
+        self.scan_fn = scan_fn          # None: the scan with the merge fused into it
         K, Di, N, R = self.K, self.d_inner, d_state, self.dt_rank
 
         self.in_proj = nn.Linear(d_model, 2 * Di, bias=bias)
@@ -68,8 +68,11 @@ class SS2DCrossScan(nn.Module):
         x, z = xz.chunk(2, dim=-1)
         x = F.silu(self.conv2d(x.permute(0, 3, 1, 2).contiguous()))
         u, delta, A, Bs, Cs, Ds, dt_bias = self.scan_inputs(x)
-        ys = self.scan_fn(u, delta, A, Bs, Cs, Ds, dt_bias, True, True)              # [B, K*Di, H, W] fp32
-        y = cross_merge(ys, self.merge_weights)                                       # [B, Di, H, W]
+        if self.scan_fn is None:                                                      # [B, Di, H, W] fp32
+            y = cross_scan_2d(u, delta, A, Bs, Cs, Ds, dt_bias, True, self.merge_weights)
+        else:
+            ys = self.scan_fn(u, delta, A, Bs, Cs, Ds, dt_bias, True, True)          # [B, K*Di, H, W] fp32
+            y = cross_merge(ys, self.merge_weights)
         y = self.out_norm(y.permute(0, 2, 3, 1)).to(z.dtype)
         return self.out_proj(y * F.silu(z))
 
