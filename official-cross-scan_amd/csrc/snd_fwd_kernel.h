@@ -161,13 +161,22 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     // flight: a line is fetched from HBM twice per strip instead of four times.
     // (Only where it pays and fits: the 16-state whole-plane kernels, which are bandwidth-bound.)
     constexpr bool PAIR = NP == 16;
+    // A strip runs one tile behind the strip above it, and what one strip's tile takes longer, for whatever reason, every strip
+    // below it waits for: 200 x 336 planes spent 6.0 us per tile in the first strip and 10.3 us in the last.  The requests for a
+    // pair of tiles, 10 scattered loads on the queue of a CU's memory path, took 2 us of that between the arrival of the
+    // row above and the walk; one or two before each row of the walk they cost nothing there.  2 x 192 x 200x336: 594 -> 550
+    // us (with the row handed over ahead of the checkpoint stores), 256 channels of 512x512 bf16: 1143 -> 1095 us.  Where the
+    // next pair is wanted right after the tile - planes of one pair, walked whole - the loads have to go first, and element-wise
+    // staging (34 loads) gains nothing.
+    constexpr bool INSIDE = PIPE && VEC;
     constexpr int NHL = (kCkX + NP - 1) / NP;       // halo-row elements per thread (1; 2 with four lanes per channel)
     struct StageE { uint32_t qb[NBC], qc[NBC], qdl[NPX], qu[NPX], qhalo[NHL]; };   // raw: masked and converted at commit
     struct StageV { Raw4<T> vb, vc, vdl[NCH], vu[NCH]; uint32_t qhalo[NHL]; };       // (VEC) one chunk of B and C, NCH of delta and u
     typedef typename std::conditional<VEC, StageV, StageE>::type Stage;
     Stage st0, st1;                                 // tile J uses st0 when J is even (or always), st1 when odd
     float qxv[kCkX], qcorner = 0.f;                 // h of the row above the next tile (from x_v)
-    auto load_tile = [&](Stage &q, int I, int J) {
+    // (part 0: B and C, 1: delta and u, 2: the halo row)
+    auto load_part = [&](Stage &q, int I, int J, int part) __attribute__((always_inline)) {
         const int r0 = I * TE, j0 = J * TE;
         // The thread's element maps are re-derived here from an opaque copy of the thread id, so that
         // they are a few integer ops per tile instead of dozens of registers kept live across the tile.
@@ -180,13 +189,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 const int row = min(r0 + (c >> 1), H - 1), col = min(j0 + (c & 1) * 4, W - 4);
                 return (uint32_t)mad24(mrow(row), hB, mcol(col + (fh ? 3 : 0)) * ESZ);
             };
-            {
+            if (part == 0) {
                 const int sn = min(t_ >> 4, N - 1), c = t_ & 15;
                 ldraw4_b(q.vb, (const T *)((const char *)Bb + sn * BsB), chunk_off(c, BhB));
                 ldraw4_b(q.vc, (const T *)((const char *)Cb + sn * CsB), chunk_off(c, ChB));
             }
 #pragma unroll
-            for (int k = 0; k < NCH; ++k) {
+            for (int k = 0; k < (part == 1 ? NCH : 0); ++k) {
                 ldraw4_b(q.vdl[k], db, cDb + chunk_off(n + NP * k, DhB));
                 ldraw4_b(q.vu[k], ub, cUb + chunk_off(n + NP * k, UhB));
             }
@@ -195,13 +204,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             const int mr = mrow(min(row, H - 1)), mcB = mcol(min(col, W - 1)) * ESZ;
             const uint32_t ob = mad24(mr, BhB, mcB), oc = mad24(mr, ChB, mcB);
 #pragma unroll
-            for (int k = 0; k < NBC; ++k) {
+            for (int k = 0; k < (part == 0 ? NBC : 0); ++k) {
                 const int sn = wave_u + WPB * k, sc = min(sn, N - 1);       // scalar: folded into the base
                 q.qb[k] = ldraw_b((const T *)((const char *)Bb + sc * BsB), ob);
                 q.qc[k] = ldraw_b((const T *)((const char *)Cb + sc * CsB), oc);
             }
 #pragma unroll
-            for (int k = 0; k < NPX; ++k) {
+            for (int k = 0; k < (part == 1 ? NPX : 0); ++k) {
                 const int pp = n + NP * k;
                 const int row_ = r0 + (pp >> 3), col_ = j0 + (pp & 7);
                 const int mr_ = mrow(min(row_, H - 1)), mcB_ = mcol(min(col_, W - 1)) * ESZ;
@@ -210,10 +219,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             }
         }
 #pragma unroll
-        for (int k = 0; k < NHL; ++k) {     // halo row r0-1 (needed for a[i-1,j] of the strip's first row)
+        for (int k = 0; k < (part == 2 ? NHL : 0); ++k) {     // halo row r0-1 (needed for a[i-1,j] of the strip's first row)
             const int row = r0 - 1, col = j0 + min(n + NP * k, TE - 1);
             q.qhalo[k] = ldraw_b(db, cDb + mad24(mrow(max(row, 0)), DhB, mcol(min(col, W - 1)) * ESZ));
         }
+    };
+    auto load_tile = [&](Stage &q, int I, int J) __attribute__((always_inline)) {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) load_part(q, I, J, part);
     };
     // the pair of tiles that starts at (I, J), J even (or the single tile when not pairing)
     auto load_pair = [&](int I, int J) {
@@ -345,9 +358,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
 #pragma unroll
         for (int r = 0; r < kRows; ++r) { hl[r] = 0.f; sl[r] = 0.f; al[r] = 0.f; }
 
-        // one tile; `mine` holds its staged inputs, `last_of_pair` says that both register sets are
-        // free once it is committed, so the next pair's loads can be issued under its compute
-        auto do_tile = [&](const int J, const Stage &mine, const bool last_of_pair) {
+        // one tile; `mine` holds its staged inputs.  Once it is committed and both register sets are free the next pair's loads
+        // are issued under its compute: `inside`, between the rows of the walk, or `ahead` of it.
+        auto do_tile = [&](const int J, const Stage &mine, const bool ahead, const bool inside) __attribute__((always_inline)) {
             const int j0 = J * TE;
             commit(mine, I, J);
             // first strip of a pipelined band: the row above comes from another block
@@ -383,14 +396,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
 #pragma unroll
                 for (int j = 0; j < kCkX; ++j) hup[j] = (I > 0) ? qxv[j] : 0.f;
             }
-            {   // issue the next loads now; they complete while this tile is computed
-                int In = I, Jn = J + 1;
-                if (Jn == geo.nCX) { Jn = 0; In = I + 1; }
-                if (In < I_end) {
-                    prefetch_xv(In, Jn);
-                    if (last_of_pair) load_pair(In, Jn);
-                }
-            }
+            // issue the next loads now; they complete while this tile is computed
+            int In = I, Jn = J + 1;
+            if (Jn == geo.nCX) { Jn = 0; In = I + 1; }
+            if (In < I_end) {
+                prefetch_xv(In, Jn);
+                if (ahead) load_pair(In, Jn);
+            } else if (INSIDE) { In = I; Jn = J; }  // (the block's last tile: loads that nobody reads, of a tile that exists)
+            const int Jn1 = min(Jn + 1, geo.nCX - 1);
             if (handed) {                           // the corner is the previous fetch's last column
                 corner = J > 0 ? xv_last : 0.f;
                 xv_last = hup[TE - 1];
@@ -407,6 +420,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
 
 #pragma unroll
             for (int r = 0; r < TE; ++r) {
+                if (inside) {
+                    if (r < 3) load_part(st0, In, Jn, r);
+                    else if (PAIR && r < 6) load_part(st1, In, Jn1, r - 3);
+                }
                 float left = hl[r], sleft = sl[r], aleft = al[r];
                 float diag = corner;
                 corner = hl[r];                     // h[r0+r][j0-1] is the next row's corner
@@ -462,6 +479,15 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             // acknowledgement of those stores (one counter counts both, and it is not decremented in order across
             // loads and stores).
             __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0)
+            const bool hands_over = PIPE && I + 1 == I_end && I + 1 < geo.nCY;
+            if (hands_over) {                       // the copy for the block of the strip below, ahead of everything else this tile stores
+                if (lvalid) {
+                    float *ho = hrow + (int64_t)J * DN8;
+#pragma unroll
+                    for (int k = 0; k < kCkX; k += 2) st2_coherent(ho + (k >> 1) * DN2, hup[k], hup[k + 1]);
+                }
+                strip_stores_done();
+            }
             if (lvalid) {
                 // row checkpoint / carry to the next strip: h at the strip's last row
                 float *dst = xv_row(I, J);
@@ -472,14 +498,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                     *(float4 *)dst = make_float4(hup[0], hup[1], hup[2], hup[3]);
                     *(float4 *)(dst + DN4) = make_float4(hup[4], hup[5], hup[6], hup[7]);
                 }
-                if (PIPE && I + 1 == I_end && I + 1 < geo.nCY) {   // and the hand-over copy for the block of the strip below
-                    float *ho = hrow + (int64_t)J * DN8;
-#pragma unroll
-                    for (int k = 0; k < kCkX; k += 2) st2_coherent(ho + (k >> 1) * DN2, hup[k], hup[k + 1]);
-                }
             }
-            const bool hands_over = PIPE && I + 1 == I_end && I + 1 < geo.nCY;
-            if (hands_over) strip_stores_done();
             if (lvalid && SAVE && J + 1 < geo.nCX) {   // column checkpoints: only if a tile follows
                 float *dh = xh + ((int64_t)J * geo.nCY + I) * DN8;
                 float *ds = xs + ((int64_t)J * geo.nCY + I) * DN8;
@@ -568,11 +587,11 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
         if (PAIR) {
             for (int J = 0; J < geo.nCX; J += 2) {
                 const bool single = J + 1 >= geo.nCX;
-                do_tile(J, st0, single);
-                if (!single) do_tile(J + 1, st1, true);
+                do_tile(J, st0, single, false);
+                if (!single) do_tile(J + 1, st1, !INSIDE, INSIDE);
             }
         } else {
-            for (int J = 0; J < geo.nCX; ++J) do_tile(J, st0, true);
+            for (int J = 0; J < geo.nCX; ++J) do_tile(J, st0, !INSIDE, INSIDE);
         }
     }
 }
