@@ -175,7 +175,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     typedef typename std::conditional<VEC, StageV, StageE>::type Stage;
     Stage st0, st1;                                 // tile J uses st0 when J is even (or always), st1 when odd
     float qxv[kCkX], qcorner = 0.f;                 // h of the row above the next tile (from x_v)
-    // (part 0: B and C, 1: delta and u, 2: the halo row)
+    // (part 0: B and C, 1: delta and u, 2: the halo row, kAll: all three)
+    constexpr int kAll = -1;
     auto load_part = [&](Stage &q, int I, int J, int part) __attribute__((always_inline)) {
         const int r0 = I * TE, j0 = J * TE;
         // The thread's element maps are re-derived here from an opaque copy of the thread id, so that
@@ -189,13 +190,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 const int row = min(r0 + (c >> 1), H - 1), col = min(j0 + (c & 1) * 4, W - 4);
                 return (uint32_t)mad24(mrow(row), hB, mcol(col + (fh ? 3 : 0)) * ESZ);
             };
-            if (part == 0) {
+            if (part == 0 || part == kAll) {
                 const int sn = min(t_ >> 4, N - 1), c = t_ & 15;
                 ldraw4_b(q.vb, (const T *)((const char *)Bb + sn * BsB), chunk_off(c, BhB));
                 ldraw4_b(q.vc, (const T *)((const char *)Cb + sn * CsB), chunk_off(c, ChB));
             }
 #pragma unroll
-            for (int k = 0; k < (part == 1 ? NCH : 0); ++k) {
+            for (int k = 0; k < (part == 1 || part == kAll ? NCH : 0); ++k) {
                 ldraw4_b(q.vdl[k], db, cDb + chunk_off(n + NP * k, DhB));
                 ldraw4_b(q.vu[k], ub, cUb + chunk_off(n + NP * k, UhB));
             }
@@ -204,13 +205,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             const int mr = mrow(min(row, H - 1)), mcB = mcol(min(col, W - 1)) * ESZ;
             const uint32_t ob = mad24(mr, BhB, mcB), oc = mad24(mr, ChB, mcB);
 #pragma unroll
-            for (int k = 0; k < (part == 0 ? NBC : 0); ++k) {
+            for (int k = 0; k < (part == 0 || part == kAll ? NBC : 0); ++k) {
                 const int sn = wave_u + WPB * k, sc = min(sn, N - 1);       // scalar: folded into the base
                 q.qb[k] = ldraw_b((const T *)((const char *)Bb + sc * BsB), ob);
                 q.qc[k] = ldraw_b((const T *)((const char *)Cb + sc * CsB), oc);
             }
 #pragma unroll
-            for (int k = 0; k < (part == 1 ? NPX : 0); ++k) {
+            for (int k = 0; k < (part == 1 || part == kAll ? NPX : 0); ++k) {
                 const int pp = n + NP * k;
                 const int row_ = r0 + (pp >> 3), col_ = j0 + (pp & 7);
                 const int mr_ = mrow(min(row_, H - 1)), mcB_ = mcol(min(col_, W - 1)) * ESZ;
@@ -219,19 +220,15 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             }
         }
 #pragma unroll
-        for (int k = 0; k < (part == 2 ? NHL : 0); ++k) {     // halo row r0-1 (needed for a[i-1,j] of the strip's first row)
+        for (int k = 0; k < (part == 2 || part == kAll ? NHL : 0); ++k) {     // halo row r0-1 (needed for a[i-1,j] of the strip's first row)
             const int row = r0 - 1, col = j0 + min(n + NP * k, TE - 1);
             q.qhalo[k] = ldraw_b(db, cDb + mad24(mrow(max(row, 0)), DhB, mcol(min(col, W - 1)) * ESZ));
         }
     };
-    auto load_tile = [&](Stage &q, int I, int J) __attribute__((always_inline)) {
-#pragma unroll
-        for (int part = 0; part < 3; ++part) load_part(q, I, J, part);
-    };
     // the pair of tiles that starts at (I, J), J even (or the single tile when not pairing)
     auto load_pair = [&](int I, int J) {
-        load_tile(st0, I, J);
-        if (PAIR && J + 1 < geo.nCX) load_tile(st1, I, J + 1);
+        load_part(st0, I, J, kAll);
+        if (PAIR && J + 1 < geo.nCX) load_part(st1, I, J + 1, kAll);
     };
     // h of the row above tile (I, J), one tile ahead, where this block wrote it itself (whole-plane
     // schedule; every strip of a pipelined band but its first)
