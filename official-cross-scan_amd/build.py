@@ -20,7 +20,7 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libsnd_scan.so")
 
 HIP_SOURCES = ["snd_bwd_f32.hip", "snd_bwd_bf16.hip", "snd_bwd_f16.hip", "snd_wave_bwd_f32.hip", "snd_wave_bwd_bf16.hip", "snd_wave_bwd_f16.hip", "snd_wave_fwd_f32.hip", "snd_wave_fwd_bf16.hip", "snd_wave_fwd_f16.hip", "snd_fwd_f32.hip", "snd_fwd_bf16.hip",
-               "snd_fwd_f16.hip", "snd_jobs.hip", "snd_capi.hip"]
+               "snd_fwd_f16.hip", "snd_jobs.hip", "snd_block.hip", "snd_capi.hip"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
     # packed-FP32 VALU forms are switched off for every device function

@@ -1,0 +1,886 @@
+// The passes of a VSS block around its scan: token LayerNorm, depthwise convolution + SiLU, the step-size projection, output
+// LayerNorm + gate, and the weight gradients of the two projections.  All of them are bound by memory: what they move is
+// read once from it (halos and second passes come from the L2) and written once, in the layout its reader wants - tokens by
+// channels for the linear layers, channels by pixels for the scan - with the transposition done in LDS on the way.
+// Measured on a block of width 96 (inner 192, rank 6) at 8 x 56 x 56, bf16, us forward / backward, against the torch layers
+// they replace: convolution + SiLU 90 / 420 -> 31 / 63 (layout copies, im2col per image for the weight), projections 100 / 400
+// -> 30 / 90 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 32 / 58,
+// token norm 33 / 70 -> 9 / 26 each, weight gradient of a linear layer 93 + 20 -> 20; the block's training step 2940 -> 1616.
+#include <algorithm>
+#include <initializer_list>
+#include <type_traits>
+
+#include "snd_block.h"
+#include "snd_device.h"
+
+namespace snd {
+namespace {
+
+__device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
+__device__ __forceinline__ float dsilu(float x) {
+    const float s = 1.f / (1.f + __expf(-x));
+    return s * fmaf(x, 1.f - s, 1.f);
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    v = group_sum<16>(v);
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+}
+
+// The value as a tensor of type T holds it.  Parameters and intermediate results are rounded where the chain of torch layers
+// these passes stand for rounds them under autocast, so that both compute with the same numbers.
+template <typename T> __device__ __forceinline__ float rnd(float x) {
+    T v;
+    stg(&v, 0, x);
+    return ldg(&v, 0);
+}
+
+// ---------------------------------------------------------------- LayerNorm over tokens
+// One wave per token, the token's channels in registers (CPL per lane).  TX: type of x and dx, TY: of y and dy.
+template <typename TX, typename TY, int CPL>
+__global__ __launch_bounds__(256) void norm_fwd_kernel(const TX *x, const float *gamma, const float *beta, float eps, int64_t tokens, int C, TY *y,
+                                                       float *stats) {
+    const int lane = threadIdx.x & 63;
+    const int64_t tok = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (tok >= tokens) return;
+    float v[CPL], sum = 0.f, var = 0.f;
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) v[k] = ldg(x + tok * C, min(lane + 64 * k, C - 1));
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+        v[k] = lane + 64 * k < C ? v[k] : 0.f;
+        sum += v[k];
+    }
+    const float mean = wave_sum(sum) / (float)C;
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+        v[k] = lane + 64 * k < C ? v[k] - mean : 0.f;
+        var = fmaf(v[k], v[k], var);
+    }
+    const float rstd = rsqrtf(wave_sum(var) / (float)C + eps);
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+        const int c = lane + 64 * k;
+        if (c < C) stg(y + tok * C, c, fmaf(v[k] * rstd, gamma[c], beta[c]));
+    }
+    if (stats && lane == 0) *(float2 *)(stats + 2 * tok) = make_float2(mean, rstd);
+}
+// Each wave takes TPW neighbouring tokens, then those 4 * TPW * gridDim.x further on, with the loads of all TPW in flight, and keeps
+// its channels' dgamma, dbeta in registers.
+template <typename TX, typename TY, int CPL>
+__global__ __launch_bounds__(256) void norm_bwd_kernel(const TY *dy, const TX *x, const float *gamma, const float *stats, int64_t tokens, int C, TX *dx,
+                                                       float *dgamma, float *dbeta) {
+    constexpr int TPW = CPL <= 4 ? 4 : 1;
+    __shared__ float sG[4][64 * CPL], sB[4][64 * CPL];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float g[CPL], dg[CPL], db[CPL];
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+        g[k] = lane + 64 * k < C ? gamma[lane + 64 * k] : 0.f;
+        dg[k] = db[k] = 0.f;
+    }
+    for (int64_t t0 = ((int64_t)blockIdx.x * 4 + wave) * TPW; t0 < tokens; t0 += (int64_t)gridDim.x * 4 * TPW) {
+        float xh[TPW][CPL], d[TPW][CPL];
+        float2 st[TPW];
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            const int64_t tok = min(t0 + i, tokens - 1);
+            st[i] = *(const float2 *)(stats + 2 * tok);
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) {
+                xh[i][k] = ldg(x + tok * C, min(lane + 64 * k, C - 1));
+                d[i][k] = ldg(dy + tok * C, min(lane + 64 * k, C - 1));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            const bool tin = t0 + i < tokens;
+            float m1 = 0.f, m2 = 0.f;
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) {
+                const bool in = tin && lane + 64 * k < C;
+                xh[i][k] = in ? (xh[i][k] - st[i].x) * st[i].y : 0.f;
+                d[i][k] = in ? d[i][k] : 0.f;
+                dg[k] = fmaf(d[i][k], xh[i][k], dg[k]);
+                db[k] += d[i][k];
+                d[i][k] *= g[k];
+                m1 += d[i][k];
+                m2 = fmaf(d[i][k], xh[i][k], m2);
+            }
+            m1 = wave_sum(m1) / (float)C;
+            m2 = wave_sum(m2) / (float)C;
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) {
+                const int c = lane + 64 * k;
+                if (tin && c < C) stg(dx + (t0 + i) * C, c, st[i].y * (d[i][k] - m1 - xh[i][k] * m2));
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) { sG[wave][lane + 64 * k] = dg[k]; sB[wave][lane + 64 * k] = db[k]; }
+    __syncthreads();
+    for (int c = threadIdx.x; c < C; c += 256) {
+        glb_add(dgamma + c, sG[0][c] + sG[1][c] + sG[2][c] + sG[3][c]);
+        glb_add(dbeta + c, sB[0][c] + sB[1][c] + sB[2][c] + sB[3][c]);
+    }
+}
+
+// ---------------------------------------------------------------- depthwise 3x3 + SiLU
+// A block takes 32 channels of 4 rows x 32 columns.  The 6 x 34 pixels around them go through LDS, channels innermost at an
+// odd pitch, so that both sides of the transposition (lanes along channels of a token, along pixels of a channel) are free of
+// bank conflicts.
+constexpr int kCvC = 32, kCvR = 4, kCvX = 32, kCvP = kCvC + 1, kCvRow = (kCvX + 2) * kCvP, kCvTile = (kCvR + 2) * kCvRow;
+constexpr int kCvN = (kCvR + 2) * (kCvX + 2) * kCvC, kCvB = 13;     // elements of a tile; loads a thread has in flight
+static_assert((kCvN + 255) / 256 == 2 * kCvB, "two batches of loads per thread");
+// All loads are of valid addresses (clamped coordinates) and unconditional, so that a batch is requested before any is waited
+// for; what lies outside the image becomes zero afterwards.
+template <typename T>
+__device__ __forceinline__ void conv_stage_x(float *sX, const T *xb, int h0, int w0, int c0, int H, int W, int Di) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        float v[kCvB];
+#pragma unroll
+        for (int k = 0; k < kCvB; ++k) {
+            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), ch = i & 31, p = i >> 5, r = p / (kCvX + 2), x = p - r * (kCvX + 2);
+            const int h = min(max(h0 + r - 1, 0), H - 1), q = min(max(w0 + x - 1, 0), W - 1);
+            v[k] = ldg(xb + ((int64_t)h * W + q) * 2 * Di, min(c0 + ch, Di - 1));
+        }
+#pragma unroll
+        for (int k = 0; k < kCvB; ++k) {
+            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), ch = i & 31, p = i >> 5, r = p / (kCvX + 2), x = p - r * (kCvX + 2);
+            const int h = h0 + r - 1, q = w0 + x - 1;
+            sX[r * kCvRow + x * kCvP + ch] = h >= 0 && h < H && q >= 0 && q < W && c0 + ch < Di ? v[k] : 0.f;
+        }
+    }
+}
+// dpre = du * silu'(pre); du, pre: the planes of channel c0
+template <typename T>
+__device__ __forceinline__ void conv_stage_d(float *sD, const T *du, const T *pre, int h0, int w0, int c0, int H, int W, int Di) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        float v[kCvB], a[kCvB];
+#pragma unroll
+        for (int k = 0; k < kCvB; ++k) {
+            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), p = i / (kCvX + 2), x = i - p * (kCvX + 2), ch = p / (kCvR + 2), r = p - ch * (kCvR + 2);
+            const int h = min(max(h0 + r - 1, 0), H - 1), q = min(max(w0 + x - 1, 0), W - 1);
+            const int64_t o = ((int64_t)min(ch, Di - 1 - c0) * H + h) * W + q;
+            v[k] = ldg(du + o, 0);
+            a[k] = ldg(pre + o, 0);
+        }
+#pragma unroll
+        for (int k = 0; k < kCvB; ++k) {
+            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), p = i / (kCvX + 2), x = i - p * (kCvX + 2), ch = p / (kCvR + 2), r = p - ch * (kCvR + 2);
+            const int h = h0 + r - 1, q = w0 + x - 1;
+            sD[r * kCvRow + x * kCvP + ch] = h >= 0 && h < H && q >= 0 && q < W && c0 + ch < Di ? rnd<T>(v[k] * dsilu(a[k])) : 0.f;
+        }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void conv_fwd_kernel(snd_block_shape s, const T *xz, const float *w, const float *bias, T *pre, T *u) {
+    __shared__ float sX[kCvTile];
+    const int H = s.nrows, W = s.ncols, Di = s.inner, t = threadIdx.x;
+    const int nX = (W + kCvX - 1) / kCvX, h0 = (blockIdx.x / nX) * kCvR, w0 = (blockIdx.x % nX) * kCvX, c0 = blockIdx.y * kCvC, b = blockIdx.z;
+    const T *xb = xz + (int64_t)b * H * W * 2 * Di;
+    conv_stage_x(sX, xb, h0, w0, c0, H, W, Di);
+    __syncthreads();
+    const int x = t & 31;
+    if (w0 + x >= W) return;
+#pragma unroll
+    for (int ch = t >> 5; ch < kCvC; ch += 8) {
+        const int c = c0 + ch;
+        if (c >= Di) break;
+        float wt[9], acc[kCvR];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) wt[k] = rnd<T>(w[c * 9 + k]);
+        const float bv = bias ? rnd<T>(bias[c]) : 0.f;
+#pragma unroll
+        for (int r = 0; r < kCvR; ++r) acc[r] = 0.f;
+#pragma unroll
+        for (int r = 0; r < kCvR + 2; ++r)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const float v = sX[r * kCvRow + (x + j) * kCvP + ch];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    if (r - i >= 0 && r - i < kCvR) acc[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0] = fmaf(wt[i * 3 + j], v, acc[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0]);
+            }
+        const int64_t o = ((int64_t)b * Di + c) * H * W + w0 + x;
+#pragma unroll
+        for (int r = 0; r < kCvR; ++r)
+            if (h0 + r < H) {
+                const float v = rnd<T>(rnd<T>(acc[r]) + bv);
+                if (pre) stg(pre + o + (int64_t)(h0 + r) * W, 0, v);
+                stg(u + o + (int64_t)(h0 + r) * W, 0, silu(v));
+            }
+    }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const T *du, const T *pre, const T *xz, const float *w, T *dxz, float *dw,
+                                                       float *dbias) {
+    __shared__ float sX[kCvTile], sD[kCvTile];
+    const int H = s.nrows, W = s.ncols, Di = s.inner, t = threadIdx.x;
+    const int nX = (W + kCvX - 1) / kCvX, h0 = (blockIdx.x / nX) * kCvR, w0 = (blockIdx.x % nX) * kCvX, c0 = blockIdx.y * kCvC, b = blockIdx.z;
+    const T *xb = xz + (int64_t)b * H * W * 2 * Di;
+    const int64_t plane = ((int64_t)b * Di + c0) * H * W;
+    conv_stage_x(sX, xb, h0, w0, c0, H, W, Di);
+    conv_stage_d(sD, du + plane, pre + plane, h0, w0, c0, H, W, Di);
+    __syncthreads();
+    const int ch = t & 31, c = c0 + ch;
+    float wt[9], gw[9], gb = 0.f;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) { wt[k] = c < Di ? rnd<T>(w[c * 9 + k]) : 0.f; gw[k] = 0.f; }
+    for (int x = t >> 5; x < kCvX; x += 8) {
+        float dx[kCvR] = {};
+#pragma unroll
+        for (int r = 0; r < kCvR + 2; ++r)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {           // dx[h, q] = sum w[i][j] dpre[h - i + 1, q - j + 1]
+                const float d = sD[r * kCvRow + (x + 2 - j) * kCvP + ch];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const int o = r - 2 + i;        // r = o + 2 - i
+                    if (o >= 0 && o < kCvR) dx[o < 0 ? 0 : o < kCvR ? o : 0] = fmaf(wt[i * 3 + j], d, dx[o < 0 ? 0 : o < kCvR ? o : 0]);
+                }
+            }
+        float d[kCvR];
+#pragma unroll
+        for (int r = 0; r < kCvR; ++r) { d[r] = sD[(r + 1) * kCvRow + (x + 1) * kCvP + ch]; gb += d[r]; }
+#pragma unroll
+        for (int r = 0; r < kCvR + 2; ++r)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {           // dw[i][j] = sum dpre[h, q] x[h + i - 1, q + j - 1]
+                const float v = sX[r * kCvRow + (x + j) * kCvP + ch];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    if (r - i >= 0 && r - i < kCvR) gw[i * 3 + j] = fmaf(d[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0], v, gw[i * 3 + j]);
+            }
+        if (w0 + x < W && c < Di)
+#pragma unroll
+            for (int r = 0; r < kCvR; ++r)
+                if (h0 + r < H) stg(dxz + (((int64_t)b * H + h0 + r) * W + w0 + x) * 2 * Di, c, dx[r]);
+    }
+    __syncthreads();
+    float *red = sX;                                // [8][10][32]
+#pragma unroll
+    for (int k = 0; k < 9; ++k) red[((t >> 5) * 10 + k) * 32 + ch] = gw[k];
+    red[((t >> 5) * 10 + 9) * 32 + ch] = gb;
+    __syncthreads();
+    for (int i = t; i < 320; i += 256) {
+        float v = 0.f;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) v += red[p * 320 + i];
+        const int k = i >> 5, cc = c0 + (i & 31);
+        if (cc < Di) {
+            if (k < 9) glb_add(dw + cc * 9 + k, v);
+            else if (dbias) glb_add(dbias + cc, v);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- output LayerNorm + gate
+// A block takes 64 pixels of an image with all their channels: y is read along pixels (twice for mean and variance, then in
+// tiles of 32 channels that LDS turns to channels along lanes), z and out along channels.
+constexpr int kGtP = 64, kGtPitch = kGtP + 1;
+__device__ __forceinline__ void gate_tile(const float *yb, int64_t HW, int c0, int Di, int px, float *sY) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int ch = (threadIdx.x >> 6) + 4 * k;
+        sY[ch * kGtPitch + px] = yb[(int64_t)min(c0 + ch, Di - 1) * HW];    // (channels and pixels beyond the edge: never used)
+    }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void gate_fwd_kernel(snd_block_shape s, const float *y, const T *xz, const float *gamma, const float *beta, float eps,
+                                                       T *out, float *stats) {
+    __shared__ float sY[32 * kGtPitch], sR[4][kGtP], sMean[kGtP], sStd[kGtP];
+    const int64_t HW = (int64_t)s.nrows * s.ncols;
+    const int Di = s.inner, t = threadIdx.x, px = t & 63, wave = t >> 6, b = blockIdx.y;
+    const int64_t p0 = (int64_t)blockIdx.x * kGtP;
+    const bool pin = p0 + px < HW;
+    const float *yb = y + (int64_t)b * Di * HW + (pin ? p0 + px : 0);
+    float a = 0.f;
+#pragma unroll 8
+    for (int c = wave; c < Di; c += 4) a += yb[(int64_t)c * HW];
+    sR[wave][px] = a;
+    __syncthreads();
+    const float mean = (sR[0][px] + sR[1][px] + sR[2][px] + sR[3][px]) / (float)Di;
+    __syncthreads();
+    a = 0.f;
+#pragma unroll 8
+    for (int c = wave; c < Di; c += 4) {
+        const float d = yb[(int64_t)c * HW] - mean;
+        a = fmaf(d, d, a);
+    }
+    sR[wave][px] = a;
+    __syncthreads();
+    const float rstd = rsqrtf((sR[0][px] + sR[1][px] + sR[2][px] + sR[3][px]) / (float)Di + eps);
+    if (wave == 0) {
+        sMean[px] = mean;
+        sStd[px] = rstd;
+        if (stats && pin) *(float2 *)(stats + 2 * (b * HW + p0 + px)) = make_float2(mean, rstd);
+    }
+    for (int c0 = 0; c0 < Di; c0 += 32) {
+        __syncthreads();
+        gate_tile(yb, HW, c0, Di, px, sY);
+        __syncthreads();
+        const int ch = t & 31, c = c0 + ch;
+        if (c < Di) {
+            const float g = gamma[c], be = beta[c];
+            float z[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) z[k] = ldg(xz + (b * HW + min(p0 + (t >> 5) + 8 * k, HW - 1)) * 2 * Di + Di, c);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int q = (t >> 5) + 8 * k;
+                const float nv = rnd<T>(fmaf((sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], g, be));
+                if (p0 + q < HW) stg(out + (b * HW + p0 + q) * Di, c, nv * rnd<T>(silu(z[k])));
+            }
+        }
+    }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const T *dout, const float *y, const T *xz, const float *gamma,
+                                                       const float *beta, const float *stats, float *dy, T *dxz, float *dgamma, float *dbeta) {
+    __shared__ float sY[32 * kGtPitch], sMean[kGtP], sStd[kGtP], sM1[kGtP], sM2[kGtP], sG[8][32], sB[8][32];
+    const int64_t HW = (int64_t)s.nrows * s.ncols;
+    const int Di = s.inner, t = threadIdx.x, px = t & 63, b = blockIdx.y, ch = t & 31, pg = t >> 5;
+    const int64_t p0 = (int64_t)blockIdx.x * kGtP;
+    const bool pin = p0 + px < HW;
+    const int64_t yo = (int64_t)b * Di * HW + (pin ? p0 + px : 0);
+    if (t < kGtP) {
+        const float2 st = pin ? *(const float2 *)(stats + 2 * (b * HW + p0 + px)) : make_float2(0.f, 0.f);
+        sMean[px] = st.x;
+        sStd[px] = st.y;
+    }
+    float m1[8] = {}, m2[8] = {};
+    for (int c0 = 0; c0 < Di; c0 += 32) {           // the two means over channels the LayerNorm's gradient takes
+        __syncthreads();
+        gate_tile(y + yo, HW, c0, Di, px, sY);
+        __syncthreads();
+        const int c = c0 + ch;
+        if (c < Di) {
+            const float g = gamma[c];
+            float z[8], d[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int64_t tok = b * HW + min(p0 + pg + 8 * k, HW - 1);
+                z[k] = ldg(xz + tok * 2 * Di + Di, c);
+                d[k] = ldg(dout + tok * Di, c);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int q = pg + 8 * k;
+                const float dn = rnd<T>(d[k] * rnd<T>(silu(z[k]))) * g;
+                m1[k] += dn;
+                m2[k] = fmaf(dn, (sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], m2[k]);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) { m1[k] += __shfl_xor(m1[k], o); m2[k] += __shfl_xor(m2[k], o); }
+        if (ch == 0) { sM1[pg + 8 * k] = m1[k] / (float)Di; sM2[pg + 8 * k] = m2[k] / (float)Di; }
+    }
+    for (int c0 = 0; c0 < Di; c0 += 32) {
+        __syncthreads();
+        gate_tile(y + yo, HW, c0, Di, px, sY);
+        __syncthreads();
+        const int c = c0 + ch;
+        float gg = 0.f, gb = 0.f;
+        if (c < Di) {
+            const float g = gamma[c], be = beta[c];
+            float z[8], d[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int64_t tok = b * HW + min(p0 + pg + 8 * k, HW - 1);
+                z[k] = ldg(xz + tok * 2 * Di + Di, c);
+                d[k] = ldg(dout + tok * Di, c);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int q = pg + 8 * k;
+                const float yh = (sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], dn = rnd<T>(d[k] * rnd<T>(silu(z[k])));
+                if (p0 + q < HW) {
+                    stg(dxz + (b * HW + p0 + q) * 2 * Di + Di, c, rnd<T>(d[k] * rnd<T>(fmaf(yh, g, be))) * dsilu(z[k]));
+                    gg = fmaf(dn, yh, gg);
+                    gb += dn;
+                }
+                sY[ch * kGtPitch + q] = sStd[q] * (dn * g - sM1[q] - yh * sM2[q]);
+            }
+        }
+        sG[pg][ch] = gg;
+        sB[pg][ch] = gb;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int cc = (t >> 6) + 4 * k;
+            if (pin && c0 + cc < Di) dy[yo + (int64_t)(c0 + cc) * HW] = sY[cc * kGtPitch + px];
+        }
+        if (t < 64 && c0 + ch < Di) {
+            float v = 0.f;
+#pragma unroll
+            for (int p = 0; p < 8; ++p) v += t < 32 ? sG[p][ch] : sB[p][ch];
+            glb_add((t < 32 ? dgamma : dbeta) + c0 + ch, v);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- step-size projection (a product with one side of `rank`)
+// The weights of up to kDtW channels at a time in LDS, padded to RP per channel and read by all lanes at one address; two
+// pixels per thread where rows of the maps start on even elements (V), so that a store covers 4 bytes of 16-bit values.
+constexpr int kDtFloats = 4096;
+template <typename T, int V> __device__ __forceinline__ void ld_px(const T *p, float (&o)[V]) {
+    if constexpr (V == 2 && sizeof(T) == 2) {
+        const uint32_t r = *(const uint32_t *)p;
+        o[0] = raw_to_f32((const T *)nullptr, r & 0xffffu);
+        o[1] = raw_to_f32((const T *)nullptr, r >> 16);
+    } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) o[v] = ldg(p, v);
+    }
+}
+template <typename T, int V> __device__ __forceinline__ void st_px(T *p, const float (&x)[V]) {
+    if constexpr (V == 2 && sizeof(T) == 2) {
+        T a[2];
+        stg(a, 0, x[0]);
+        stg(a, 1, x[1]);
+        *(uint32_t *)p = __builtin_bit_cast(uint32_t, a);
+    } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) stg(p, v, x[v]);
+    }
+}
+template <typename T, int RP> __device__ __forceinline__ void dt_stage(float *sW, const float *w, int d0, int n, int R) {
+    for (int i = threadIdx.x; i < n * RP; i += 256) {
+        const int d = i / RP, r = i - d * RP;
+        const float v = w[(int64_t)(d0 + d) * R + min(r, R - 1)];
+        sW[i] = r < R ? rnd<T>(v) : 0.f;
+    }
+}
+// blockIdx.z takes a share of the channels
+template <typename T, int RP, int V>
+__global__ __launch_bounds__(256) void dt_fwd_kernel(snd_block_shape s, const T *proj, const float *w, T *delta) {
+    __shared__ __align__(16) float sW[kDtFloats];
+    const int64_t HW = (int64_t)s.nrows * s.ncols, p = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V, pc = min(p, HW - V);
+    const int Di = s.inner, R = s.rank, bg = blockIdx.y, g = bg % s.n_groups;
+    const T *src = proj + (int64_t)bg * (R + 2 * s.dstate) * HW + pc;
+    float x[RP][V];
+#pragma unroll
+    for (int r = 0; r < RP; ++r) ld_px<T, V>(src + (int64_t)min(r, R - 1) * HW, x[r]);     // (the weights of r >= R are 0)
+    const int per = (Di + gridDim.z - 1) / gridDim.z, d1 = min((int)(blockIdx.z + 1) * per, Di);
+    T *dst = delta + (int64_t)bg * Di * HW + pc;
+    for (int d0 = blockIdx.z * per; d0 < d1; d0 += kDtFloats / RP) {
+        const int n = min(kDtFloats / RP, d1 - d0);
+        __syncthreads();
+        dt_stage<T, RP>(sW, w + (int64_t)g * Di * R, d0, n, R);
+        __syncthreads();
+#pragma unroll 4
+        for (int d = 0; d < n; ++d) {
+            float acc[V] = {};
+#pragma unroll
+            for (int r = 0; r < RP; ++r)
+#pragma unroll
+                for (int v = 0; v < V; ++v) acc[v] = fmaf(sW[d * RP + r], x[r][v], acc[v]);
+            if (p < HW) st_px<T, V>(dst + (int64_t)(d0 + d) * HW, acc);
+        }
+    }
+}
+// 64 * V pixels per block, the channels dealt to its four waves.
+template <typename T, int RP, int V>
+__global__ __launch_bounds__(256) void dt_bwd_kernel(snd_block_shape s, const T *ddelta, const T *dB, const T *dC, const float *w, T *dproj) {
+    __shared__ __align__(16) float sW[kDtFloats], sA[4][8][64 * V];
+    const int64_t HW = (int64_t)s.nrows * s.ncols;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t p = ((int64_t)blockIdx.x * 64 + lane) * V, pc = min(p, HW - V);
+    const int Di = s.inner, R = s.rank, N = s.dstate, bg = blockIdx.y, g = bg % s.n_groups;
+    float acc[RP][V] = {};
+    const T *src = ddelta + (int64_t)bg * Di * HW + pc;
+    for (int d0 = 0; d0 < Di; d0 += kDtFloats / RP) {
+        const int n = min(kDtFloats / RP, Di - d0);
+        __syncthreads();
+        dt_stage<T, RP>(sW, w + (int64_t)g * Di * R, d0, n, R);
+        __syncthreads();
+#pragma unroll 8
+        for (int d = wave; d < n; d += 4) {
+            float v[V];
+            ld_px<T, V>(src + (int64_t)(d0 + d) * HW, v);
+#pragma unroll
+            for (int r = 0; r < RP; ++r)
+#pragma unroll
+                for (int k = 0; k < V; ++k) acc[r][k] = fmaf(sW[d * RP + r], v[k], acc[r][k]);
+        }
+    }
+    T *dst = dproj + (int64_t)bg * (R + 2 * N) * HW + pc;
+#pragma unroll
+    for (int r0 = 0; r0 < RP; r0 += 8) {            // the waves' sums, eight rows at a time
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+#pragma unroll
+            for (int k = 0; k < V; ++k) sA[wave][r][lane * V + k] = acc[r0 + r][k];
+        __syncthreads();
+        for (int r = wave; r < 8 && r0 + r < R; r += 4) {
+            float v[V];
+#pragma unroll
+            for (int k = 0; k < V; ++k) v[k] = sA[0][r][lane * V + k] + sA[1][r][lane * V + k] + sA[2][r][lane * V + k] + sA[3][r][lane * V + k];
+            if (p < HW) st_px<T, V>(dst + (int64_t)(r0 + r) * HW, v);
+        }
+    }
+    const int64_t o = (int64_t)bg * N * HW + pc;
+#pragma unroll 4
+    for (int n = wave; n < N; n += 4) {
+        float vb[V], vc[V];
+        ld_px<T, V>(dB + o + (int64_t)n * HW, vb);
+        ld_px<T, V>(dC + o + (int64_t)n * HW, vc);
+        if (p < HW) {
+            st_px<T, V>(dst + (int64_t)(R + n) * HW, vb);
+            st_px<T, V>(dst + (int64_t)(R + N + n) * HW, vc);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- weight gradients
+// Both operands have the summed axis (pixels) innermost, which is the layout of either operand of a matrix instruction: a
+// lane holds 8 (fp32: 4) consecutive pixels of one row, and rows come straight from memory in 64-byte runs.  The sum is
+// long and the result small (a few thousand values), so the pixels are split over the grid and the parts added with atomics.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+template <typename T> struct Frag { typedef uint16_t E; E v[8]; static constexpr int K = 8; };
+template <> struct Frag<float> { typedef float E; E v[4]; static constexpr int K = 4; };
+__device__ __forceinline__ f32x4 mma(const Frag<float> &a, const Frag<float> &b, f32x4 c) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[k], b.v[k], c, 0, 0, 0);
+    return c;
+}
+__device__ __forceinline__ f32x4 mma(const Frag<bf16_t> &a, const Frag<bf16_t> &b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mma(const Frag<f16_t> &a, const Frag<f16_t> &b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+// VEC: rows start on 16-byte boundaries and hold whole fragments
+template <typename T, bool VEC> __device__ __forceinline__ void ld_frag(Frag<T> &f, const T *row, int64_t k, int64_t K) {
+    typedef typename Frag<T>::E E;
+    const E *src = (const E *)row;
+    if (VEC) {
+        const uint4 v = k < K ? *(const uint4 *)(src + k) : make_uint4(0, 0, 0, 0);
+        __builtin_memcpy(f.v, &v, 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < Frag<T>::K; ++j) f.v[j] = k + j < K ? src[k + j] : (E)0;
+    }
+}
+// MT x NT tiles of 16 x 16 per wave, WM x WN waves; blockIdx.x: tiles, y: image and share of its pixels, z: group
+template <typename T, int MT, int NT, int WM, int WN, bool VEC>
+__global__ __launch_bounds__(256) void wgrad_kernel(const T *a, int64_t ab, int64_t ag, const T *c, int64_t cb, int64_t cg, int M, int N, int64_t P,
+                                                    int splits, float *out) {
+    constexpr int STEP = 4 * Frag<T>::K, UNROLL = VEC ? 2 : 1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nN = (N + 16 * NT * WN - 1) / (16 * NT * WN), mt = blockIdx.x / nN, nt = blockIdx.x - mt * nN;
+    const int m0 = (mt * WM + wave / WN) * 16 * MT, n0 = (nt * WN + wave % WN) * 16 * NT;
+    const int b = blockIdx.y / splits, sp = blockIdx.y - b * splits, g = blockIdx.z;
+    const int64_t per = ((P + splits - 1) / splits + STEP - 1) / STEP * STEP, k0 = sp * per, k1 = min(k0 + per, P);
+    const T *ar[MT], *cr[NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) ar[i] = a + b * ab + g * ag + (int64_t)min(m0 + 16 * i + (lane & 15), M - 1) * P;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) cr[i] = c + b * cb + g * cg + (int64_t)min(n0 + 16 * i + (lane & 15), N - 1) * P;
+    f32x4 acc[MT][NT] = {};
+    if (m0 < M && n0 < N && k0 < k1) {
+#pragma unroll UNROLL
+        for (int64_t k = k0; k < k1; k += STEP) {
+            const int64_t kl = k + (lane >> 4) * Frag<T>::K;
+            Frag<T> fa[MT], fc[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) ld_frag<T, VEC>(fa[i], ar[i], kl, k1);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) ld_frag<T, VEC>(fc[i], cr[i], kl, k1);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = mma(fa[i], fc[j], acc[i][j]);
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int m = m0 + 16 * i + (lane >> 4) * 4 + e, n = n0 + 16 * j + (lane & 15);
+                    if (m < M && n < N) glb_add(out + ((int64_t)g * M + m) * N + n, acc[i][j][e]);
+                }
+    }
+}
+
+// The weight gradient of a linear layer on 16-bit tokens: out[m][n] += sum_t a[t][m] * c[t][n], and bias[m] += sum_t a[t][m].
+// Here the summed axis is the outer one, so stages of 64 tokens x 64 channels of either operand are transposed on their way
+// into LDS: a thread takes two channels of two tokens, swaps the inner halves, and stores two token pairs.  Threads are
+// dealt 8 channel pairs x 8 token pairs to a wave: 32-byte runs of memory, and both the stores and the fragment reads
+// (16 bytes at a pitch of 36 words) spread over all LDS banks.  The next stage's loads are in flight during the products.
+// The library's product has M * N / 4096 blocks and walks all tokens in each (25088 x 384 x 96: 93 us); here the tokens are
+// split over the grid.
+template <typename T>
+__global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *c, int64_t tokens, int M, int N, int splits, float *out, float *bias) {
+    constexpr int KT = 64, PW = KT / 2 + 4;         // tokens per stage; words per channel row
+    __shared__ __align__(16) uint32_t sA[64 * PW], sC[64 * PW];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int nN = (N + 63) / 64, m0 = (blockIdx.x / nN) * 64, n0 = (blockIdx.x % nN) * 64;
+    const int64_t per = ((tokens + splits - 1) / splits + KT - 1) / KT * KT, k0 = blockIdx.y * per, k1 = min(k0 + per, tokens);
+    if (k0 >= k1) return;
+    // item k of this thread: channel pair cp, token pair tp = lane bits 3-5 + 8 * k; the wave index selects 8 of the 32 channel pairs
+    const int cp = (lane & 7) + 8 * wave, tb = lane >> 3;
+    const int ca = min(m0 + 2 * cp, M - 2), cc = min(n0 + 2 * cp, N - 2);       // (clamped channels: rows of the result that are not stored)
+    uint32_t ra[4][2], rc[4][2];
+    auto load = [&](int64_t k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int64_t tok = min(k + 2 * (tb + 8 * i) + h, tokens - 1);
+                ra[i][h] = *(const uint32_t *)(a + tok * M + ca);
+                rc[i][h] = *(const uint32_t *)(c + tok * N + cc);
+            }
+    };
+    f32x4 acc[2][2] = {};
+    float bsum[2] = {};
+    const bool sums = bias != nullptr && n0 == 0;
+    load(k0);
+    for (int64_t k = k0; k < k1; k += KT) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int tp = tb + 8 * i;
+            const int64_t tok = k + 2 * tp;
+            const uint32_t keep = (tok < k1 ? 0xffffu : 0u) | (tok + 1 < k1 ? 0xffff0000u : 0u);
+            // (low half of each word: the even channel) -> words of two tokens per channel
+            const uint32_t e = ((ra[i][0] & 0xffffu) | (ra[i][1] << 16)) & keep, o = ((ra[i][0] >> 16) | (ra[i][1] & 0xffff0000u)) & keep;
+            sA[(2 * cp) * PW + tp] = e;
+            sA[(2 * cp + 1) * PW + tp] = o;
+            sC[(2 * cp) * PW + tp] = ((rc[i][0] & 0xffffu) | (rc[i][1] << 16)) & keep;
+            sC[(2 * cp + 1) * PW + tp] = ((rc[i][0] >> 16) | (rc[i][1] & 0xffff0000u)) & keep;
+            if (sums) {
+                bsum[0] += raw_to_f32((const T *)nullptr, e & 0xffffu) + raw_to_f32((const T *)nullptr, e >> 16);
+                bsum[1] += raw_to_f32((const T *)nullptr, o & 0xffffu) + raw_to_f32((const T *)nullptr, o >> 16);
+            }
+        }
+        __syncthreads();
+        load(min(k + KT, tokens - 1));
+#pragma unroll
+        for (int ks = 0; ks < KT; ks += 32) {
+            Frag<T> fa[2], fc[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int w = (ks + (lane >> 4) * 8) / 2;
+                __builtin_memcpy(fa[i].v, &sA[((wave >> 1) * 32 + 16 * i + (lane & 15)) * PW + w], 16);
+                __builtin_memcpy(fc[i].v, &sC[((wave & 1) * 32 + 16 * i + (lane & 15)) * PW + w], 16);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mma(fa[i], fc[j], acc[i][j]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = m0 + (wave >> 1) * 32 + 16 * i + (lane >> 4) * 4 + e, n = n0 + (wave & 1) * 32 + 16 * j + (lane & 15);
+                if (m < M && n < N) glb_add(out + (int64_t)m * N + n, acc[i][j][e]);
+            }
+    if (sums) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float v = bsum[h];
+            v += __shfl_xor(v, 8);
+            v += __shfl_xor(v, 16);
+            v += __shfl_xor(v, 32);
+            if (lane < 8 && m0 + 2 * cp + h < M) glb_add(bias + m0 + 2 * cp + h, v);
+        }
+    }
+}
+
+bool shape_ok(const snd_block_shape *s) {
+    return s && s->batch > 0 && s->nrows > 0 && s->ncols > 0 && s->inner > 0 && s->n_groups > 0 && s->dstate > 0 && s->rank > 0 &&
+           s->rank <= SND_BLOCK_MAX_RANK && (int64_t)s->batch * s->n_groups < 65536 && (s->dtype == SND_F32 || s->dtype == SND_F16 || s->dtype == SND_BF16);
+}
+int launched() { return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH; }
+// f(T *) with the element type of `dtype`
+template <typename F> int by_type(int dtype, F f) {
+    if (dtype == SND_F32) f((float *)nullptr);
+    else if (dtype == SND_BF16) f((bf16_t *)nullptr);
+    else if (dtype == SND_F16) f((f16_t *)nullptr);
+    else return SND_ERR_DTYPE;
+    return launched();
+}
+template <typename F> int by_types(int a, int b, F f) {
+    int st = SND_ERR_DTYPE;
+    by_type(a, [&](auto ea) { st = by_type(b, [&](auto eb) { f(ea, eb); }); });
+    return st;
+}
+template <typename F> void by_channels(int C, F f) {
+    if (C <= 128) f(std::integral_constant<int, 2>());
+    else if (C <= 256) f(std::integral_constant<int, 4>());
+    else if (C <= 512) f(std::integral_constant<int, 8>());
+    else f(std::integral_constant<int, 16>());
+}
+template <typename F> void by_rank(int R, F f) {
+    if (R <= 8) f(std::integral_constant<int, 8>());
+    else if (R <= 16) f(std::integral_constant<int, 16>());
+    else if (R <= 32) f(std::integral_constant<int, 32>());
+    else f(std::integral_constant<int, 64>());
+}
+// Whether pixel maps of HW elements can be taken two pixels at a time (every row of every tensor starts on an even element).
+bool px_pairs(int64_t HW, std::initializer_list<const void *> ptrs) {
+    bool ok = HW % 2 == 0;
+    for (const void *p : ptrs) ok = ok && ((uintptr_t)p & 3) == 0;
+    return ok;
+}
+#define ELT(x) typename std::remove_pointer<decltype(x)>::type
+
+}  // namespace
+}  // namespace snd
+
+using namespace snd;
+
+int snd_block_norm_fwd(const void *x, int x_dtype, const float *gamma, const float *beta, float eps, int64_t tokens, int channels, void *y, int y_dtype,
+                       float *stats, snd_stream_t stream) {
+    if (!x || !y || !gamma || !beta) return SND_ERR_NULL;
+    if (tokens <= 0 || channels <= 0 || channels > SND_BLOCK_MAX_NORM || (tokens + 3) / 4 >= ((int64_t)1 << 31)) return SND_ERR_SHAPE;
+    return by_types(x_dtype, y_dtype, [&](auto ex, auto ey) {
+        typedef ELT(ex) TX;
+        typedef ELT(ey) TY;
+        by_channels(channels, [&](auto cpl) {
+            hipLaunchKernelGGL((norm_fwd_kernel<TX, TY, decltype(cpl)::value>), dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+                               (const TX *)x, gamma, beta, eps, tokens, channels, (TY *)y, stats);
+        });
+    });
+}
+int snd_block_norm_bwd(const void *dy, int dy_dtype, const void *x, int x_dtype, const float *gamma, const float *stats, int64_t tokens, int channels,
+                       void *dx, float *dgamma, float *dbeta, snd_stream_t stream) {
+    if (!dy || !x || !gamma || !stats || !dx || !dgamma || !dbeta) return SND_ERR_NULL;
+    if (tokens <= 0 || channels <= 0 || channels > SND_BLOCK_MAX_NORM) return SND_ERR_SHAPE;
+    const int grid = (int)std::min<int64_t>((tokens + 31) / 32, 1024);      // eight tokens per wave at least: each block ends in 2 * channels atomics
+    return by_types(x_dtype, dy_dtype, [&](auto ex, auto ey) {
+        typedef ELT(ex) TX;
+        typedef ELT(ey) TY;
+        by_channels(channels, [&](auto cpl) {
+            hipLaunchKernelGGL((norm_bwd_kernel<TX, TY, decltype(cpl)::value>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const TY *)dy, (const TX *)x,
+                               gamma, stats, tokens, channels, (TX *)dx, dgamma, dbeta);
+        });
+    });
+}
+static dim3 conv_grid(const snd_block_shape &s) {
+    return dim3((unsigned)(((s.nrows + kCvR - 1) / kCvR) * ((s.ncols + kCvX - 1) / kCvX)), (unsigned)((s.inner + kCvC - 1) / kCvC), (unsigned)s.batch);
+}
+int snd_block_conv_fwd(const snd_block_shape *s, const void *xz, const float *w, const float *bias, void *pre, void *u, snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!xz || !w || !u) return SND_ERR_NULL;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        hipLaunchKernelGGL((conv_fwd_kernel<T>), conv_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, (const T *)xz, w, bias, (T *)pre, (T *)u);
+    });
+}
+int snd_block_conv_bwd(const snd_block_shape *s, const void *du, const void *pre, const void *xz, const float *w, void *dxz, float *dw, float *dbias,
+                       snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!du || !pre || !xz || !w || !dxz || !dw) return SND_ERR_NULL;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        hipLaunchKernelGGL((conv_bwd_kernel<T>), conv_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, (const T *)du, (const T *)pre, (const T *)xz, w,
+                           (T *)dxz, dw, dbias);
+    });
+}
+static dim3 gate_grid(const snd_block_shape &s) { return dim3((unsigned)(((int64_t)s.nrows * s.ncols + kGtP - 1) / kGtP), (unsigned)s.batch); }
+int snd_block_gate_fwd(const snd_block_shape *s, const float *y, const void *xz, const float *gamma, const float *beta, float eps, void *out, float *stats,
+                       snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!y || !xz || !gamma || !beta || !out) return SND_ERR_NULL;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        hipLaunchKernelGGL((gate_fwd_kernel<T>), gate_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, y, (const T *)xz, gamma, beta, eps, (T *)out, stats);
+    });
+}
+int snd_block_gate_bwd(const snd_block_shape *s, const void *dout, const float *y, const void *xz, const float *gamma, const float *beta, const float *stats,
+                       float *dy, void *dxz, float *dgamma, float *dbeta, snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!dout || !y || !xz || !gamma || !beta || !stats || !dy || !dxz || !dgamma || !dbeta) return SND_ERR_NULL;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        hipLaunchKernelGGL((gate_bwd_kernel<T>), gate_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, (const T *)dout, y, (const T *)xz, gamma, beta, stats,
+                           dy, (T *)dxz, dgamma, dbeta);
+    });
+}
+int snd_block_dt_fwd(const snd_block_shape *s, const void *proj, const float *w, void *delta, snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!proj || !w || !delta) return SND_ERR_NULL;
+    const int64_t HW = (int64_t)s->nrows * s->ncols;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        by_rank(s->rank, [&](auto rp) {
+            auto go = [&](auto kernel, int V) {
+                const int64_t bx = (HW + 256 * V - 1) / (256 * V), blocks = bx * s->batch * s->n_groups;
+                const int share = (int)std::min<int64_t>(std::max<int64_t>(1, 2048 / blocks), std::max(1, s->inner / 16));
+                hipLaunchKernelGGL(kernel, dim3((unsigned)bx, (unsigned)(s->batch * s->n_groups), (unsigned)share), dim3(256), 0, (hipStream_t)stream, *s,
+                                   (const T *)proj, w, (T *)delta);
+            };
+            px_pairs(HW, {proj, delta}) ? go(dt_fwd_kernel<T, decltype(rp)::value, 2>, 2) : go(dt_fwd_kernel<T, decltype(rp)::value, 1>, 1);
+        });
+    });
+}
+int snd_block_dt_bwd(const snd_block_shape *s, const void *ddelta, const void *dB, const void *dC, const float *w, void *dproj, snd_stream_t stream) {
+    if (!shape_ok(s)) return SND_ERR_SHAPE;
+    if (!ddelta || !dB || !dC || !w || !dproj) return SND_ERR_NULL;
+    const int64_t HW = (int64_t)s->nrows * s->ncols;
+    return by_type(s->dtype, [&](auto e) {
+        typedef ELT(e) T;
+        by_rank(s->rank, [&](auto rp) {
+            auto go = [&](auto kernel, int V) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)((HW + 64 * V - 1) / (64 * V)), (unsigned)(s->batch * s->n_groups)), dim3(256), 0, (hipStream_t)stream,
+                                   *s, (const T *)ddelta, (const T *)dB, (const T *)dC, w, (T *)dproj);
+            };
+            px_pairs(HW, {ddelta, dB, dC, dproj}) ? go(dt_bwd_kernel<T, decltype(rp)::value, 2>, 2) : go(dt_bwd_kernel<T, decltype(rp)::value, 1>, 1);
+        });
+    });
+}
+int snd_block_wgrad(const void *a, int64_t a_batch, int64_t a_group, const void *c, int64_t c_batch, int64_t c_group, int batch, int groups, int M, int N,
+                    int64_t pixels, int dtype, float *out, snd_stream_t stream) {
+    if (!a || !c || !out) return SND_ERR_NULL;
+    if (batch <= 0 || groups <= 0 || groups > 65535 || M <= 0 || N <= 0 || pixels <= 0) return SND_ERR_SHAPE;
+    return by_type(dtype, [&](auto e) {
+        typedef ELT(e) T;
+        constexpr int FK = Frag<T>::K;
+        const bool vec = (((uintptr_t)a | (uintptr_t)c) & 15) == 0 && pixels % FK == 0 && a_batch % FK == 0 && a_group % FK == 0 && c_batch % FK == 0 &&
+                         c_group % FK == 0;
+        // a narrow side (the rank of the step-size projection) takes one column of tiles
+        const bool narrow = N <= 16;
+        const int tiles = ((M + 63) / 64) * (narrow ? 1 : (N + 63) / 64);
+        // pixels are split until the grid has about four blocks per CU, in shares of 256 and more
+        int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 1024 / ((int64_t)tiles * batch * groups)), std::max<int64_t>(1, pixels / 256));
+        while ((int64_t)splits * batch > 65535 && splits > 1) --splits;
+        const dim3 grid((unsigned)tiles, (unsigned)(batch * splits), (unsigned)groups);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const T *)a, a_batch, a_group, (const T *)c, c_batch, c_group, M, N, pixels,
+                               splits, out);
+        };
+        if (narrow) vec ? go(wgrad_kernel<T, 1, 1, 4, 1, true>) : go(wgrad_kernel<T, 1, 1, 4, 1, false>);
+        else vec ? go(wgrad_kernel<T, 2, 2, 2, 2, true>) : go(wgrad_kernel<T, 2, 2, 2, 2, false>);
+    });
+}
+int snd_block_linear_wgrad(const void *dy, const void *x, int64_t tokens, int M, int N, int dtype, float *dw, float *dbias, snd_stream_t stream) {
+    if (!dy || !x || !dw) return SND_ERR_NULL;
+    if (tokens <= 0 || M <= 0 || N <= 0 || M % 2 || N % 2 || (((uintptr_t)dy | (uintptr_t)x) & 3)) return SND_ERR_SHAPE;
+    if (dtype != SND_BF16 && dtype != SND_F16) return SND_ERR_DTYPE;
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    if (tiles >= (int64_t)1 << 31) return SND_ERR_SHAPE;
+    const int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 768 / tiles), (tokens + 255) / 256);
+    const dim3 grid((unsigned)tiles, (unsigned)splits);
+    if (dtype == SND_BF16)
+        hipLaunchKernelGGL((wgrad_tokens_kernel<bf16_t>), grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t *)dy, (const bf16_t *)x, tokens, M, N, splits, dw, dbias);
+    else
+        hipLaunchKernelGGL((wgrad_tokens_kernel<f16_t>), grid, dim3(256), 0, (hipStream_t)stream, (const f16_t *)dy, (const f16_t *)x, tokens, M, N, splits, dw, dbias);
+    return launched();
+}

@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "snd_block.h"
 #include "snd_scan.h"
 
 namespace {
@@ -525,6 +526,228 @@ at::Tensor scan(const at::Tensor &u_, const at::Tensor &delta_, const at::Tensor
     return launch_fwd(c, u, delta, A, B, C, D_, delta_bias_, A_decay_, o, w, nullptr, nullptr, nullptr);
 }
 
+// ---------------------------------------------------------------- the passes of a VSS block around its scan
+hipStream_t current_stream() { return at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
+at::Tensor f32c(const at::Tensor &t) { return t.to(at::kFloat).contiguous(); }
+const float *ptr_or_null(const OptTensor &t) { return t.has_value() ? t.value().data_ptr<float>() : nullptr; }
+
+// LayerNorm over the last axis, its result in `out_dtype` (what the next layer reads under autocast).
+struct NormFn : public torch::autograd::Function<NormFn> {
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &gamma_, const at::Tensor &beta_, double eps,
+                              int64_t out_dtype) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
+        const at::Tensor x = x_.contiguous(), gamma = f32c(gamma_), beta = f32c(beta_);
+        const int64_t C = x.size(-1), tokens = x.numel() / C;
+        at::Tensor y = at::empty(x.sizes(), x.options().dtype((at::ScalarType)out_dtype)), stats = floats(2 * tokens, x);
+        check_status(snd_block_norm_fwd(x.data_ptr(), dtype_code(x.scalar_type()), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, tokens, (int)C,
+                                        y.data_ptr(), dtype_code(y.scalar_type()), stats.data_ptr<float>(), (snd_stream_t)current_stream()), "norm");
+        ctx->save_for_backward({x, gamma, stats});
+        ctx->saved_data["g"] = (int64_t)gamma_.scalar_type();
+        ctx->saved_data["b"] = (int64_t)beta_.scalar_type();
+        return y;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &x = saved[0], &gamma = saved[1], &stats = saved[2];
+        torch::autograd::variable_list r(5);
+        if (!grads[0].defined()) return r;
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
+        const at::Tensor dy = grads[0].contiguous();
+        const int64_t C = x.size(-1), tokens = x.numel() / C;
+        at::Tensor dx = at::empty_like(x), acc = at::zeros({2, C}, x.options().dtype(at::kFloat));
+        check_status(snd_block_norm_bwd(dy.data_ptr(), dtype_code(dy.scalar_type()), x.data_ptr(), dtype_code(x.scalar_type()), gamma.data_ptr<float>(),
+                                        stats.data_ptr<float>(), tokens, (int)C, dx.data_ptr(), acc.data_ptr<float>(), acc.data_ptr<float>() + C,
+                                        (snd_stream_t)current_stream()), "norm");
+        r[0] = dx;
+        r[1] = acc[0].to((at::ScalarType)ctx->saved_data["g"].toInt());
+        r[2] = acc[1].to((at::ScalarType)ctx->saved_data["b"].toInt());
+        return r;
+    }
+};
+at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps, const at::Tensor &like) {
+    return NormFn::apply(x, gamma, beta, eps, (int64_t)like.scalar_type());
+}
+
+// A linear layer in the 16-bit type `dtype` (what autocast makes of F.linear) whose weight and bias gradients are summed over
+// the tokens by the extension's kernel where the library's product would leave most of the chip idle (linear_wgrad_pays).
+// The line lies where the library's product has blocks for half the CUs by itself: weight and bias gradient of 25088 tokens,
+// kernel of the extension / library, us: 384 x 96 20 / 119, 768 x 192 40 / 160, 1536 x 384 147 / 175 (12544 x 3072 x 768: the
+// library is ahead; few tokens cost either their launches).
+bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) { return M % 2 == 0 && N % 2 == 0 && M * N <= (int64_t)1 << 19; }
+struct LinearFn : public torch::autograd::Function<LinearFn> {
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &w_, const OptTensor &b_, int64_t dtype) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const auto T = (at::ScalarType)dtype;
+        const at::Tensor x = x_.to(T).contiguous(), w = w_.to(T).contiguous();
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["x"] = (int64_t)x_.scalar_type();
+        ctx->saved_data["w"] = (int64_t)w_.scalar_type();
+        ctx->saved_data["b"] = b_.has_value() ? (int64_t)b_.value().scalar_type() : (int64_t)-1;
+        return at::linear(x, w, b_.has_value() ? OptTensor(b_.value().to(T)) : OptTensor());
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const at::Tensor &x = sv[0], &w = sv[1];
+        torch::autograd::variable_list r(4);
+        if (!grads[0].defined()) return r;
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
+        const int64_t M = w.size(0), N = w.size(1), tokens = x.numel() / N, btype = ctx->saved_data["b"].toInt();
+        const auto wtype = (at::ScalarType)ctx->saved_data["w"].toInt();
+        const at::Tensor dy = grads[0].to(x.scalar_type()).contiguous().view({tokens, M}), x2 = x.view({tokens, N});
+        if (ctx->needs_input_grad(0)) r[0] = at::mm(dy, w).view(x.sizes()).to((at::ScalarType)ctx->saved_data["x"].toInt());
+        if (linear_wgrad_pays(tokens, M, N)) {
+            const int64_t nw = (M * N + 15) / 16 * 16;
+            at::Tensor acc = at::zeros({nw + M}, x.options().dtype(at::kFloat));
+            float *p = acc.data_ptr<float>();
+            check_status(snd_block_linear_wgrad(dy.data_ptr(), x2.data_ptr(), tokens, (int)M, (int)N, dtype_code(x.scalar_type()), p, btype >= 0 ? p + nw : nullptr,
+                                                (snd_stream_t)current_stream()), "linear");
+            r[1] = acc.narrow(0, 0, M * N).view({M, N}).to(wtype);
+            if (btype >= 0) r[2] = acc.narrow(0, nw, M).to((at::ScalarType)btype);
+        } else {
+            r[1] = at::mm(dy.t(), x2).to(wtype);
+            if (btype >= 0) r[2] = dy.sum(0).to((at::ScalarType)btype);
+        }
+        return r;
+    }
+};
+at::Tensor block_linear(const at::Tensor &x, const at::Tensor &w, const OptTensor &b, const at::Tensor &like) {
+    return LinearFn::apply(x, w, b, (int64_t)like.scalar_type());
+}
+
+// Everything between in_proj and out_proj of SS2DCrossScan: xz [B, H, W, 2 * inner] -> [B, H, W, inner].
+struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
+    static snd_block_shape shape_of(const at::Tensor &xz, const at::Tensor &wx, const at::Tensor &wdt) {
+        snd_block_shape s;
+        s.batch = (int)xz.size(0); s.nrows = (int)xz.size(1); s.ncols = (int)xz.size(2); s.inner = (int)(xz.size(3) / 2);
+        s.n_groups = (int)wx.size(0); s.rank = (int)wdt.size(2); s.dstate = (int)(wx.size(1) - wdt.size(2)) / 2;
+        s.dtype = dtype_code(xz.scalar_type());
+        return s;
+    }
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &xz_, const at::Tensor &conv_w_, const OptTensor &conv_b_,
+                              const at::Tensor &wx_, const at::Tensor &wdt_, const at::Tensor &dt_bias_, const at::Tensor &A_logs_, const at::Tensor &D_,
+                              const OptTensor &mw_, const at::Tensor &gamma_, const at::Tensor &beta_, double eps, bool grad) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{xz_.device()};
+        const snd_stream_t stream = (snd_stream_t)current_stream();
+        const at::Tensor xz = xz_.contiguous(), conv_w = f32c(conv_w_), wdt = f32c(wdt_), gamma = f32c(gamma_), beta = f32c(beta_), Dv = f32c(D_);
+        const at::Tensor dt_bias = f32c(dt_bias_).view(-1), A = f32c(A_logs_).exp().neg_();
+        const OptTensor conv_b = conv_b_.has_value() ? OptTensor(f32c(conv_b_.value())) : OptTensor();
+        const snd_block_shape s = shape_of(xz, wx_, wdt_);
+        const int64_t B = s.batch, H = s.nrows, W = s.ncols, Di = s.inner, K = s.n_groups, N = s.dstate, R = s.rank, M = R + 2 * N, HW = H * W;
+        at::Tensor u = at::empty({B, Di, H, W}, xz.options()), pre = grad ? at::empty({B, Di, H, W}, xz.options()) : at::Tensor();
+        check_status(snd_block_conv_fwd(&s, xz.data_ptr(), conv_w.data_ptr<float>(), ptr_or_null(conv_b), grad ? pre.data_ptr() : nullptr, u.data_ptr(), stream),
+                     "block");
+        const at::Tensor wx = wx_.to(xz.scalar_type()).reshape({1, K * M, Di});
+        const at::Tensor proj = at::bmm(wx.expand({B, K * M, Di}), u.view({B, Di, HW}));                 // [B, K * (R + 2N), HW]
+        at::Tensor delta = at::empty({B, K * Di, H, W}, xz.options());
+        check_status(snd_block_dt_fwd(&s, proj.data_ptr(), wdt.data_ptr<float>(), delta.data_ptr(), stream), "block");
+        const at::Tensor p5 = proj.view({B, K, M, H, W}), Bs = p5.narrow(2, R, N), Cs = p5.narrow(2, R + N, N);
+        OptTensor w;
+        if (mw_.has_value()) w = f32c(mw_.value()).reshape({K, -1}).expand({K, Di}).contiguous().view(-1);
+        Options o{true, true, SND_DIR_CORNERS, resolve_schedule(-1), true};
+        const Checked c = check_inputs(u, delta, A, Bs, Cs, Dv, dt_bias, OptTensor());
+        check_merge(c, true, w, u);
+        const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        at::Tensor state;
+        float *st = nullptr;
+        if (grad) {
+            state = floats(2 * nx + c.plan.x_v_elems, u);
+            st = state.data_ptr<float>();
+        }
+        const at::Tensor y = launch_fwd(c, u, delta, A, Bs, Cs, Dv, dt_bias, OptTensor(), o, w, st, st ? st + 2 * nx : nullptr, st ? st + nx : nullptr);
+        at::Tensor out = at::empty({B, H, W, Di}, xz.options()), stats = grad ? floats(2 * B * HW, u) : at::Tensor();
+        check_status(snd_block_gate_fwd(&s, y.data_ptr<float>(), xz.data_ptr(), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, out.data_ptr(),
+                                        grad ? stats.data_ptr<float>() : nullptr, stream), "block");
+        if (!grad) return out;
+        ctx->save_for_backward({xz, conv_w, conv_b.value_or(at::Tensor()), wx_, wdt, dt_bias, A, Dv, w.value_or(at::Tensor()), gamma, beta, u, pre, proj, delta, y,
+                                stats, state});
+        ctx->saved_data["sched"] = (int64_t)o.sched;
+        if (mw_.has_value()) ctx->saved_data["mw_shape"] = mw_.value().sizes().vec();
+        const at::Tensor *params[] = {&conv_w_, conv_b_.has_value() ? &conv_b_.value() : nullptr, &wx_, &wdt_, &dt_bias_, &A_logs_, &D_,
+                                      mw_.has_value() ? &mw_.value() : nullptr, &gamma_, &beta_};
+        std::vector<int64_t> types;
+        for (const at::Tensor *t : params) types.push_back(t ? (int64_t)t->scalar_type() : -1);
+        ctx->saved_data["types"] = types;
+        return out;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        torch::autograd::variable_list r(13);
+        if (!grads[0].defined()) return r;
+        const at::Tensor &xz = sv[0], &conv_w = sv[1], &wx_ = sv[3], &wdt = sv[4], &dt_bias = sv[5], &A = sv[6], &Dv = sv[7], &gamma = sv[9], &beta = sv[10],
+                         &u = sv[11], &pre = sv[12], &proj = sv[13], &delta = sv[14], &y = sv[15], &stats = sv[16], &state = sv[17];
+        const OptTensor conv_b = optional_of(sv[2]), w = optional_of(sv[8]);
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{xz.device()};
+        const snd_stream_t stream = (snd_stream_t)current_stream();
+        const snd_block_shape s = shape_of(xz, wx_, wdt);
+        const int64_t B = s.batch, H = s.nrows, W = s.ncols, Di = s.inner, K = s.n_groups, N = s.dstate, R = s.rank, M = R + 2 * N, HW = H * W;
+        const at::Tensor dout = grads[0].to(xz.scalar_type()).contiguous();
+        // the accumulated parameter gradients: conv weight and bias, the two projections, gamma, beta
+        const int64_t sizes[] = {Di * 9, Di, K * M * Di, K * Di * R, Di, Di};
+        int64_t off[7] = {0};
+        for (int i = 0; i < 6; ++i) off[i + 1] = off[i] + (sizes[i] + 15) / 16 * 16;
+        at::Tensor acc = at::zeros({off[6]}, xz.options().dtype(at::kFloat));
+        float *ap = acc.data_ptr<float>();
+        at::Tensor dy = at::empty_like(y), dxz = at::empty_like(xz);
+        check_status(snd_block_gate_bwd(&s, dout.data_ptr(), y.data_ptr<float>(), xz.data_ptr(), gamma.data_ptr<float>(), beta.data_ptr<float>(),
+                                        stats.data_ptr<float>(), dy.data_ptr<float>(), dxz.data_ptr(), ap + off[4], ap + off[5], stream), "block");
+        const at::Tensor p5 = proj.view({B, K, M, H, W}), Bs = p5.narrow(2, R, N), Cs = p5.narrow(2, R + N, N);
+        Options o{true, true, SND_DIR_CORNERS, (int)ctx->saved_data["sched"].toInt(), true};
+        const Checked c = check_inputs(u, delta, A, Bs, Cs, Dv, dt_bias, OptTensor());
+        const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        const float *st = state.data_ptr<float>();
+        int64_t wn = 0;
+        if (w.has_value()) {
+            wn = 1;
+            for (int64_t v : ctx->saved_data["mw_shape"].toIntVector()) wn *= v;
+        }
+        Grads g = launch_bwd(c, u, delta, A, Bs, Cs, Dv, dt_bias, OptTensor(), dy, st, st + 2 * nx, st + nx, o, w, true, wn);
+        at::Tensor dproj = at::empty_like(proj);
+        check_status(snd_block_dt_bwd(&s, g.ddelta.data_ptr(), g.dB.data_ptr(), g.dC.data_ptr(), wdt.data_ptr<float>(), dproj.data_ptr(), stream), "block");
+        check_status(snd_block_wgrad(g.ddelta.data_ptr(), K * Di * HW, Di * HW, proj.data_ptr(), K * M * HW, M * HW, (int)B, (int)K, (int)Di, (int)R, HW, s.dtype,
+                                     ap + off[3], stream), "block");
+        check_status(snd_block_wgrad(dproj.data_ptr(), K * M * HW, 0, u.data_ptr(), Di * HW, 0, (int)B, 1, (int)(K * M), (int)Di, HW, s.dtype, ap + off[2],
+                                     stream), "block");
+        const at::Tensor wxt = wx_.to(xz.scalar_type()).reshape({K * M, Di}).t().contiguous();
+        const at::Tensor du = at::baddbmm(g.du.view({B, Di, HW}), wxt.unsqueeze(0).expand({B, Di, K * M}), dproj);
+        check_status(snd_block_conv_bwd(&s, du.data_ptr(), pre.data_ptr(), xz.data_ptr(), conv_w.data_ptr<float>(), dxz.data_ptr(), ap + off[0],
+                                        conv_b.has_value() ? ap + off[1] : nullptr, stream), "block");
+        const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
+        auto part = [&](int i, at::IntArrayRef shape, int type) { return acc.narrow(0, off[i], sizes[i]).view(shape).to((at::ScalarType)types[type]); };
+        r[0] = dxz;
+        r[1] = part(0, {Di, 1, 3, 3}, 0);
+        if (conv_b.has_value()) r[2] = part(1, {Di}, 1);
+        r[3] = part(2, {K, M, Di}, 2);
+        r[4] = part(3, {K, Di, R}, 3);
+        r[5] = g.ddelta_bias.view({K, Di}).to((at::ScalarType)types[4]);
+        r[6] = g.dA.mul_(A).to((at::ScalarType)types[5]);
+        r[7] = g.dD.to((at::ScalarType)types[6]);
+        if (wn > 0) r[8] = g.dweights.view(ctx->saved_data["mw_shape"].toIntVector()).to((at::ScalarType)types[7]);
+        r[9] = part(4, {Di}, 8);
+        r[10] = part(5, {Di}, 9);
+        return r;
+    }
+};
+at::Tensor ss2d(const at::Tensor &xz, const at::Tensor &conv_w, const OptTensor &conv_b, const at::Tensor &wx, const at::Tensor &wdt, const at::Tensor &dt_bias,
+                const at::Tensor &A_logs, const at::Tensor &D, const OptTensor &mw, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
+    TORCH_CHECK(xz.is_cuda() && xz.dim() == 4 && xz.size(3) % 2 == 0, "ss2d: xz must be a GPU tensor [batch, rows, cols, 2 * inner]");
+    const int64_t Di = xz.size(3) / 2;
+    TORCH_CHECK(wx.dim() == 3 && wdt.dim() == 3, "ss2d: projections are 3-D");
+    const int64_t K = wx.size(0), R = wdt.size(2), N = A_logs.size(1);
+    TORCH_CHECK(wx.size(1) == R + 2 * N && wx.size(2) == Di && wdt.size(0) == K && wdt.size(1) == Di && dt_bias.numel() == K * Di && A_logs.size(0) == K * Di &&
+                    D.numel() == K * Di && gamma.numel() == Di && beta.numel() == Di && conv_w.numel() == Di * 9 &&
+                    (!conv_b.has_value() || conv_b.value().numel() == Di),
+                "ss2d: parameter shapes do not fit");
+    for (const at::Tensor *t : {&conv_w, &wx, &wdt, &dt_bias, &A_logs, &D, &gamma, &beta}) TORCH_CHECK(t->device() == xz.device(), "ss2d: parameters must be on xz's device");
+    bool grad = false;
+    if (at::GradMode::is_enabled()) {
+        for (const at::Tensor *t : {&xz, &conv_w, &wx, &wdt, &dt_bias, &A_logs, &D, &gamma, &beta}) grad = grad || t->requires_grad();
+        for (const OptTensor *t : {&conv_b, &mw}) grad = grad || (t->has_value() && t->value().requires_grad());
+    }
+    return Ss2dFn::apply(xz, conv_w, conv_b, wx, wdt, dt_bias, A_logs, D, mw, gamma, beta, eps, grad);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -545,6 +768,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("scan", &scan, "selective_nd_scan / selective_nd_scan_merged (differentiable)", py::arg("u"), py::arg("delta"), py::arg("A"),
           py::arg("B"), py::arg("C"), py::arg("D"), py::arg("delta_bias"), py::arg("delta_softplus"), py::arg("out_float"),
           py::arg("A_decay"), py::arg("directions"), py::arg("merge"), py::arg("merge_weights"));
+    m.def("block_norm", &block_norm, "LayerNorm over the last axis, in the type of `like`", py::arg("x"), py::arg("gamma"), py::arg("beta"), py::arg("eps"), py::arg("like"));
+    m.def("block_linear", &block_linear, "A linear layer in the 16-bit type of `like`", py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("like"));
+    m.def("ss2d", &ss2d, "SS2DCrossScan between its in and out projections", py::arg("xz"), py::arg("conv_w"), py::arg("conv_b"), py::arg("x_proj"),
+          py::arg("dt_proj"), py::arg("dt_bias"), py::arg("A_logs"), py::arg("D"), py::arg("merge_weights"), py::arg("gamma"), py::arg("beta"), py::arg("eps"));
     m.def("set_schedule", [](int mode) {
         TORCH_CHECK(mode >= SND_SCHED_AUTO && mode <= SND_SCHED_WAVEFRONT, "schedule must be 0 (auto), 1 (plane), 2 (strips), 3 (bands) or 4 (row-segment wavefront)");
         g_schedule.store(mode);

@@ -13,8 +13,9 @@ follows the upstream VMamba SS2D layout of that caller so the op can be dropped 
 Because the scan origins are handled inside the kernels, every tensor stays in its natural
 orientation: the projections are pointwise, so no flipped (or even repeated) copy of the feature
 map is ever built - the four direction groups read the same u.
-Everything outside the scan is plain PyTorch (GEMMs / elementwise); `scan_fn` can be replaced for
-testing.
+On the GPU everything between the two outer linear layers runs in the extension (snd_block.hip: convolution + SiLU, the
+step-size projection, output norm + gate, weight gradients; the wide products are library GEMMs), forward and backward;
+elsewhere, and with another `scan_fn`, it is plain PyTorch.
 """
 import math
 
@@ -23,6 +24,35 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .cross_scan import cross_merge, cross_scan_2d
+from .interface import ext
+
+_FLOATS = (torch.float32, torch.bfloat16, torch.float16)
+
+
+def _autocast_like(x):
+    """An empty tensor of the type a layer would compute in: autocast's, or x's own."""
+    return x.new_empty(0, dtype=torch.get_autocast_dtype("cuda")) if torch.is_autocast_enabled("cuda") else x
+
+
+class TokenNorm(nn.LayerNorm):
+    """LayerNorm whose result, under autocast on the GPU, has the type the following linear layer would cast it to."""
+
+    def forward(self, x):
+        if not (x.is_cuda and x.dtype in _FLOATS and len(self.normalized_shape) == 1 and self.normalized_shape[0] <= 1024 and self.bias is not None
+                and x.numel() > 0 and self.weight.is_cuda):
+            return super().forward(x)
+        return ext().block_norm(x, self.weight, self.bias, self.eps, _autocast_like(x))
+
+
+class TokenLinear(nn.Linear):
+    """Linear layer whose weight gradient, in a 16-bit type on the GPU, is split over the tokens."""
+
+    def forward(self, x):
+        like = _autocast_like(x) if x.is_cuda else x
+        if not (x.is_cuda and like.dtype in _FLOATS[1:] and x.dtype in _FLOATS and x.numel() > 0 and self.weight.is_cuda
+                and (like is not x or self.weight.dtype == x.dtype) and torch.is_grad_enabled()):
+            return super().forward(x)
+        return ext().block_linear(x, self.weight, self.bias, like)
 
 
 class SS2DCrossScan(nn.Module):
@@ -37,7 +67,7 @@ class SS2DCrossScan(nn.Module):
         self.scan_fn = scan_fn          # None: the scan with the merge fused into it
         K, Di, N, R = self.K, self.d_inner, d_state, self.dt_rank
 
-        self.in_proj = nn.Linear(d_model, 2 * Di, bias=bias)
+        self.in_proj = TokenLinear(d_model, 2 * Di, bias=bias)
         self.conv2d = nn.Conv2d(Di, Di, d_conv, padding=(d_conv - 1) // 2, groups=Di, bias=conv_bias)
         # per-direction projections, stacked on a leading K axis
         self.x_proj_weight = nn.Parameter(torch.empty(K, R + 2 * N, Di))
@@ -49,7 +79,7 @@ class SS2DCrossScan(nn.Module):
         self.Ds = nn.Parameter(torch.ones(K * Di))
         self.merge_weights = nn.Parameter(torch.ones(K, Di)) if merge == "weighted" else None
         self.out_norm = nn.LayerNorm(Di)
-        self.out_proj = nn.Linear(Di, d_model, bias=bias)
+        self.out_proj = TokenLinear(Di, d_model, bias=bias)
 
     def scan_inputs(self, x):
         """x [B, Di, H, W] (after conv + activation) -> (u, delta, A, B, C, D, delta_bias) of the op."""
@@ -65,6 +95,11 @@ class SS2DCrossScan(nn.Module):
     def forward(self, x):
         """x [B, H, W, d_model] -> [B, H, W, d_model]."""
         xz = self.in_proj(x)
+        conv = self.conv2d
+        if (self.scan_fn is None and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16
+                and conv.kernel_size == (3, 3) and conv.weight.is_cuda):
+            return self.out_proj(ext().ss2d(xz, conv.weight, conv.bias, self.x_proj_weight, self.dt_projs_weight, self.dt_projs_bias, self.A_logs,
+                                            self.Ds, self.merge_weights, self.out_norm.weight, self.out_norm.bias, self.out_norm.eps))
         x, z = xz.chunk(2, dim=-1)
         x = F.silu(self.conv2d(x.permute(0, 3, 1, 2).contiguous()))
         u, delta, A, Bs, Cs, Ds, dt_bias = self.scan_inputs(x)
@@ -82,13 +117,13 @@ class VSSBlock(nn.Module):
 
     def __init__(self, d_model, d_state=16, ssm_ratio=2.0, mlp_ratio=4.0, **ss2d_kwargs):
         super().__init__()
-        self.norm = nn.LayerNorm(d_model)
+        self.norm = TokenNorm(d_model)
         self.op = SS2DCrossScan(d_model, d_state=d_state, ssm_ratio=ssm_ratio, **ss2d_kwargs)
         self.mlp = None
         if mlp_ratio > 0:
             hidden = int(mlp_ratio * d_model)
-            self.norm2 = nn.LayerNorm(d_model)
-            self.mlp = nn.Sequential(nn.Linear(d_model, hidden), nn.GELU(), nn.Linear(hidden, d_model))
+            self.norm2 = TokenNorm(d_model)
+            self.mlp = nn.Sequential(TokenLinear(d_model, hidden), nn.GELU(), TokenLinear(hidden, d_model))
 
     def forward(self, x):
         x = x + self.op(self.norm(x))
