@@ -164,7 +164,8 @@ typedef struct snd_fwd_params {
                                       out, du and every other tensor keep their dim-wide layouts. */
     int32_t merge;                 /* 0: out is [batch, dim, nrows, ncols] (the reference's layout).
                                       1: CrossMerge fused into the output stores: out is fp32
-                                      [batch, dim / n_groups, nrows, ncols], zero-filled by the caller, and
+                                      [batch, dim / n_groups, nrows, ncols], zero-filled by the caller (except
+                                      where snd_fwd_merge_stores() says it need not be), and
                                       channel g*(dim/n_groups) + i adds merge_weights[that channel] * (its result)
                                       to out channel i with a float atomic, so out ends as the weighted sum of
                                       the n_groups results per feature (the summation order, hence the last
@@ -300,6 +301,9 @@ int snd_run_jobs(const snd_job *jobs, int n, snd_stream_t stream);
  * them already - among its own SND_JOB_CLEARs, on the same stream - and saves that launch. */
 int64_t snd_clear_bytes(const snd_shape *shape, int schedule, int backward);
 int snd_fwd_cleared(const snd_fwd_params *params, snd_stream_t stream);
+/* 1 if a forward with merge = 1 of this shape, schedule and directions stores every element of out: the groups of a feature
+ * are added up inside the kernel and out need not be zero-filled.  0: it adds to out. */
+int snd_fwd_merge_stores(const snd_shape *shape, int schedule, int directions);
 int snd_bwd_cleared(const snd_bwd_params *params, snd_stream_t stream);
 
 #ifdef __cplusplus

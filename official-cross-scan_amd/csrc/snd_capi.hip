@@ -448,6 +448,12 @@ int64_t snd_clear_bytes(const snd_shape *shape, int schedule, int backward) {
     return jobs > 0 ? snd::sync_words(plane_chunks(s), g.nCY) * (int64_t)sizeof(int) : 0;
 }
 
+int snd_fwd_merge_stores(const snd_shape *shape, int schedule, int directions) {
+    if (!shape || check_shape(*shape) != SND_OK || schedule < SND_SCHED_AUTO || schedule > SND_SCHED_WAVEFRONT) return 0;
+    const snd_shape &s = *shape;
+    return directions == SND_DIR_CORNERS && use_wavefront(s, schedule) > 0 && snd::wave_fold_shape(s.nrows, s.ncols, s.dstate, s.n_groups) ? 1 : 0;
+}
+
 int snd_fwd_cleared(const snd_fwd_params *params, snd_stream_t stream) {
     snd::t_sync_cleared = true;
     const int st = snd_fwd(params, stream);

@@ -658,6 +658,17 @@ __host__ inline void wave_geo_channels(WaveGeo &g, int batch, int dim, int n_gro
     for (int k = 0; k < 16; ++k)
         if (n_groups == 1 << k) g.gshift = k;
 }
+// Whether the fused merge of a forward is done in LDS (the FOLD instantiation of the wave kernels): the four corners, planes
+// of one segment, and two sums of as many packed planes as a wave takes within the 64 KB a kernel gets without asking: two
+// blocks per CU at the least (16 x 256 channels of 120x64, 61 KB: 112 -> 91 us; one block of four waves could not hide its loads).
+constexpr int kFoldBytes = 65536;
+__host__ inline bool wave_fold_shape(int H, int W, int N, int groups) {
+    const WaveGeo g = make_wave_geo(H, W, N);
+    return groups == kOneWaves && g.nsegAll == 1 && g.cpl == 1 && 2 * (int64_t)wave_pack(g, W) * H * W * 4 <= kFoldBytes;
+}
+__host__ inline bool wave_fold(const snd_fwd_params &p) {
+    return p.merge && p.directions == SND_DIR_CORNERS && p.out_dtype == SND_F32 && wave_fold_shape(p.shape.nrows, p.shape.ncols, p.shape.dstate, p.shape.n_groups);
+}
 // (batch, group) of a pair
 __device__ __forceinline__ void wave_pair_split(const WaveGeo &g, int pair, int G, int &b, int &grp) {
     b = g.gshift >= 0 ? pair >> g.gshift : pair / G;

@@ -207,7 +207,7 @@ at::Tensor launch_fwd(const Checked &c, const at::Tensor &u, const at::Tensor &d
                       const at::Tensor &C, const OptTensor &D_, const OptTensor &delta_bias_, const OptTensor &A_decay_,
                       const Options &o, const OptTensor &merge_weights_, float *x, float *x_v, float *x_sd) {
     const auto f32 = u.options().dtype(at::kFloat);
-    // merged: one fp32 channel per feature, zero-filled, to which every group adds its weighted result
+    // merged: one fp32 channel per feature, to which every group adds its weighted result
     at::Tensor out = o.merge ? at::empty({c.batch, c.dim / c.n_groups, c.nrows, c.ncols}, f32)
                              : at::empty({c.batch, c.dim, c.nrows, c.ncols}, o.out_float ? f32 : u.options());
     auto stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
@@ -238,7 +238,7 @@ at::Tensor launch_fwd(const Checked &c, const at::Tensor &u, const at::Tensor &d
     p.x = x; p.x_v = x_v; p.x_sd = x_sd;
     snd_job jobs[2];
     int nj = 0;
-    if (o.merge) jobs[nj++] = clear_job(out.data_ptr(), out.numel() * 4);
+    if (o.merge && !snd_fwd_merge_stores(&c.shape, o.sched, (int)o.directions)) jobs[nj++] = clear_job(out.data_ptr(), out.numel() * 4);
     if (need_ws && !wave) jobs[nj++] = clear_job(ws.data_ptr(), snd_clear_bytes(&c.shape, o.sched, 0));
     run_jobs(jobs, nj, stream, "fwd");
     check_status(snd_fwd_cleared(&p, (snd_stream_t)stream), "fwd");

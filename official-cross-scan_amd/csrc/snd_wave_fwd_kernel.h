@@ -48,9 +48,18 @@ namespace snd {
 // EVEN: the plane is a whole number of this kernel's bands high and of 64-column segments wide: no row and no lane is
 // skipped, so no branch surrounds a row or its stores and the waits the compiler derives for the prefetched loads are
 // exact (as in the backward's instantiation of the same name).  256 planes of 512x512, one state: 0.186 -> 0.174 ms.
-template <typename T, int NS, int CPL, bool VEC, bool SAVE, bool OUT32, int PK, int EU, bool ONE, bool EXT = false, bool EVEN = false>
+// FOLD: the fused merge of the four corners where a plane is one segment wide and fits in LDS (wave_fold): a block's four
+// waves are the four groups of one feature (or PK features), which add up in LDS and leave as plain stores.  Without it each
+// group adds its result to out with atomics, and those bound the kernel: 4 bytes per pixel and group at the 1.3 TB/s that
+// atomics reach.  Floating-point atomics in LDS are no way out (a wave's takes its CU longer than the rest of a row: 288 ->
+// 401 us), so the groups that start at one side, left or right, share a sum: one of the two comes down the plane and one up,
+// a barrier per band keeps them in step, and they meet once; who comes to a row first stores, who comes second adds.
+// 64 x 384 x 56x56, one state, bf16: 288 -> 190 us, 64 x 768 x 28x28 178 -> 87, 64 x 1536 x 7x7 52 -> 28; out needs no
+// clearing before (18 us at the first of these).
+template <typename T, int NS, int CPL, bool VEC, bool SAVE, bool OUT32, int PK, int EU, bool ONE, bool EXT = false, bool EVEN = false, bool FOLD = false>
 __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__((amdgpu_waves_per_eu(EU))) void wave_fwd_kernel(const snd_fwd_params p, const WaveGeo wg) {
     static_assert(ONE || PK == 1, "packed planes are one segment wide");
+    static_assert(!FOLD || (ONE && OUT32 && CPL == 1), "merge in LDS: one segment, fp32 out");
     static_assert(!EVEN || (!ONE && PK == 1 && CPL == 1 && !EXT), "whole planes: several segments, one column per lane");
     static_assert(!EXT || (!ONE && PK == 1 && CPL == 1), "column groups: whole segments, one column per lane");
     constexpr int R = wave_fwd_rows(NS);             // rows per band of this kernel = rows per load group
@@ -72,9 +81,10 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     const int H = sh.nrows, W = sh.ncols, N = sh.dstate, Dm = sh.dim, G = sh.n_groups;
     const int rg = wg.rg, rd = wg.rd;
     int pair, chunk;
-    if (!wave_job2(wg, sh.batch * G, pair, chunk)) return;
+    if (!wave_job2(wg, FOLD ? sh.batch : sh.batch * G, pair, chunk)) return;   // (FOLD: the whole block, pair = batch image)
+    const int fchunk = chunk;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), w = ONE ? 0 : wv;
-    if (ONE) {                                       // (independent waves: one past the group's last channel just leaves)
+    if (ONE && !FOLD) {                              // (independent waves: one past the group's last channel just leaves)
         chunk = chunk * kOneWaves + wv;
         if (chunk * PK >= rg) return;
     }
@@ -83,7 +93,8 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     const bool act = PK == 1 || chunk < rg;          // a wave past the last channel of its group repeats it and stores nothing
     if (PK > 1) chunk = min(chunk, rg - 1);
     int b, g;
-    wave_pair_split(wg, pair, G, b, g);
+    if (FOLD) { b = pair; g = wv; }
+    else wave_pair_split(wg, pair, G, b, g);
     const int c = g * rg + chunk, cd = rd == 1 ? c : c / rd;   // channel of u, of delta
     // channel offsets: in the scalar base pointers, or (packed) in the lanes' offsets
     const int cB = PK > 1 ? 0 : c, chB = PK > 1 ? 0 : chunk, cL = PK > 1 ? c : 0, chL = PK > 1 ? chunk : 0;
@@ -129,6 +140,11 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     const uint32_t colU = colB + (uint32_t)(p.u_shared ? chL : cL) * (uint32_t)p.u_d_stride * ESZ,
                    colD = colB + (uint32_t)(PK > 1 ? cd : 0) * (uint32_t)p.delta_d_stride * ESZ,
                    colO = (uint32_t)mc * OSZ + (uint32_t)(merge ? chL : cL) * (uint32_t)p.out_d_stride * OSZ;
+
+    // (FOLD) the sums of groups 0 and 2 and of groups 1 and 3, memory order
+    extern __shared__ __align__(16) float sFold[];
+    const int HW = H * W;
+    float *const fold = FOLD ? sFold + (g & 1) * PK * HW : nullptr;
 
     // saved state of this plane set
     const int64_t plane0 = ((int64_t)b * Dm + c) * N;
@@ -203,6 +219,9 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                                                     // default one: 256 planes of 512x512, one state: 0.192 -> 0.186 ms)
         const int i0 = band * R;
         uint32_t oo = mad24(mad24(i0, rs, r0m), OhB * rs, colO);
+        const bool fold_tie = FOLD && H - 1 >= 2 * R * band && H - 1 <= 2 * R * (band + 1) - 2;   // both groups of a sum at one row
+        if (fold_tie && fv) lds_barrier();
+        int fo = mad24(mad24(i0, rs, r0m), W, (PK > 1 ? lane / S : 0) * HW + mc);
         // What the rows need that does not depend on the rows above them - softplus, delta' * u - for the RD rows
         // of a wavefront step at once: independent chains of transcendentals that fill each other's latencies,
         // instead of one such chain in front of every row's scan.  (Per step, not per band: the waves of a block
@@ -301,7 +320,14 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
 #pragma unroll
                     for (int k = 0; k < CPL; ++k) o[k] = fmaf(Dv, u[k], acc[k]);
                     if (CPL == 2 && fh) { const float t = o[0]; o[0] = o[CPL - 1]; o[CPL - 1] = t; }
-                    if (OUT32 && MERGE) {
+                    if (FOLD) {
+                        // the band in which the other group of this sum comes to this row: later (or second): it finds the value
+                        const int other = (H - 1 - (i0 + r)) / R;
+                        const bool first = band < other || (band == other && !fv);
+                        const float v = wm * o[0];
+                        if (first) fold[fo] = v;
+                        else fold[fo] += v;
+                    } else if (OUT32 && MERGE) {
 #pragma unroll
                         for (int k = 0; k < CPL; ++k) glb_add((float *)((char *)outb + oo) + k, wm * o[k]);
                     } else {
@@ -309,6 +335,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                     }
                 }
                 oo += OhB;
+                fo += rs * W;
                 // row checkpoint: h on the last row of a band of the backward (what its next band starts from; the
                 // last row of the plane is nobody's, and a ragged last band leaves none)
                 if (SAVE && r % RC == RC - 1) {
@@ -328,6 +355,8 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
             }
             if (multi && r % RD == RD - 1) { lds_barrier(); ++step; }
         }
+        if (fold_tie && !fv) lds_barrier();
+        if (FOLD) lds_barrier();
         // column checkpoints: lanes 0..R-1 hold what entered the segment on the band's rows
         if (SAVE && w > 0 && lane < R && band * R + lane < wg.Hp) {
 #pragma unroll
@@ -350,7 +379,7 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     if (!ONE) lds_barrier();                         // the zeroed slot
     if (multi)
         for (int e = 0; e < w; ++e) lds_barrier(); // the waves on the left go first
-    if (OUT32 && merge) {
+    if (OUT32 && !FOLD && merge) {
         for (int band = 0; band < nFB; band += 2) {
             do_band(std::true_type{}, sA, sB, band);
             if (band + 1 < nFB) do_band(std::true_type{}, sB, sA, band + 1);
@@ -363,6 +392,15 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
     }
     if (multi)
         for (int e = 0; e < nseg - 1 - w; ++e) lds_barrier();
+    if (FOLD) {
+        const int f0 = fchunk * PK;    // the block's first feature
+        float *dst = (float *)p.out + (int64_t)b * p.out_batch_stride + (int64_t)f0 * p.out_d_stride;
+        for (int q = 0; q < PK && f0 + q < rg; ++q) {
+            // a row per 64 lanes: rows of out may be spaced
+            for (int r = wv; r < H; r += kOneWaves)
+                if (lane < W) dst[(int64_t)q * p.out_d_stride + (int64_t)r * p.out_h_stride + lane] = sFold[q * HW + r * W + lane] + sFold[(PK + q) * HW + r * W + lane];
+        }
+    }
 }
 
 // Whether every row of a tensor starts at a multiple of `bytes` (so that a lane's CPL elements come with one access)
@@ -380,6 +418,17 @@ static int launch_wave_fwd_o(const snd_fwd_params &p, const WaveGeo &wg, hipStre
     const int waves = (rg + PK - 1) / PK;            // per (batch, group) pair
     const dim3 grid = wave_grid2(sh.batch * sh.n_groups, ONE ? (waves + kOneWaves - 1) / kOneWaves : waves), block(ONE ? 64 * kOneWaves : 64 * wg.nseg);
     const bool save = p.x != nullptr, out32 = p.out_dtype == SND_F32;
+    if constexpr (ONE && CPL == 1) {
+        if (wave_fold(p)) {
+            WaveGeo wf = wg;
+            wf.xcd = wave_grid_xcd(sh.batch) ? 1 : 0;
+            const dim3 fgrid = wave_grid2(sh.batch, waves);
+            const size_t lds = sizeof(float) * 2 * PK * sh.nrows * sh.ncols;
+            if (save) hipLaunchKernelGGL((wave_fwd_kernel<T, NS, CPL, VEC, true, true, PK, EU, true, false, false, true>), fgrid, block, lds, stream, p, wf);
+            else hipLaunchKernelGGL((wave_fwd_kernel<T, NS, CPL, VEC, false, true, PK, EU, true, false, false, true>), fgrid, block, lds, stream, p, wf);
+            return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
+        }
+    }
     constexpr bool F = std::is_same<T, float>::value;
     // (whole bands and whole segments, the usual training call - state saved, fp32 out: the instantiation without
     // a branch around a row or a lane)

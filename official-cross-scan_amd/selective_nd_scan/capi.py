@@ -85,6 +85,7 @@ def lib():
         _lib.snd_init.argtypes = [C.c_int]
         _lib.snd_fwd_cleared.argtypes = [C.POINTER(FwdParams), vp]
         _lib.snd_bwd_cleared.argtypes = [C.POINTER(BwdParams), vp]
+        _lib.snd_fwd_merge_stores.argtypes = [C.POINTER(Shape), C.c_int, C.c_int]
         _lib.snd_clear_bytes.argtypes = [C.POINTER(Shape), C.c_int, C.c_int]
         _lib.snd_clear_bytes.restype = C.c_int64
         _lib.snd_run_jobs.argtypes = [C.POINTER(Job), C.c_int, vp]

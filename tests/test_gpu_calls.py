@@ -112,3 +112,24 @@ def test_lanes_per_channel_for_five_to_eight_states(gpu_device, Bt, H, W, N, dty
     for nm, a, w in zip(["du", "ddelta", "dA", "dB", "dC", "dD", "ddelta_bias"], [b.du, b.ddelta, b.dA, b.dB, b.dC, b.dD, b.dbias], gref):
         tol = 1e-2 if (half and nm in ("du", "ddelta", "dB", "dC")) else 1e-4
         assert relerr(a.float().cpu().numpy(), w) <= tol, (nm, relerr(a.float().cpu().numpy(), w))
+
+
+@pytest.mark.parametrize("H,W,N,rg", [(1, 1, 1, 9), (4, 64, 1, 2), (5, 17, 3, 3), (9, 33, 2, 1), (8, 16, 4, 6), (13, 7, 1, 10), (128, 64, 2, 1), (127, 63, 4, 2), (3, 8, 2, 5)])
+@pytest.mark.parametrize("save", [True, False])
+def test_merge_in_lds(gpu_device, H, W, N, rg, save):
+    """One-segment planes merged from the four corners inside the kernel: every element of out is stored (none was cleared)."""
+    import ctypes as C
+    d = O.make_inputs(2, 4 * rg, H, W, N=N, K=4, seed=6)
+    t = {k: torch.from_numpy(v).to(gpu_device) for k, v in d.items()}
+    u = t["u"][:, :rg].contiguous()
+    w = torch.linspace(-1.0, 2.0, 4 * rg, device=gpu_device)
+    args = (u, t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"], True, True, None)
+    f = capi.FwdCall(*args, save, capi.SCHED_WAVEFRONT, capi.DIR_CORNERS, True, w)
+    assert capi.lib().snd_fwd_merge_stores(C.byref(f.params.shape), capi.SCHED_WAVEFRONT, capi.DIR_CORNERS) == 1
+    f.out.fill_(float("nan"))
+    f.launch()
+    f0 = capi.FwdCall(*args, True, capi.SCHED_WAVEFRONT, capi.DIR_CORNERS)
+    f0.launch()
+    torch.cuda.synchronize()
+    want = (f0.out.double() * w.double().view(1, -1, 1, 1)).view(2, 4, rg, H, W).sum(1)
+    assert relerr(f.out.cpu().numpy(), want.cpu().numpy()) <= 1e-5
