@@ -110,6 +110,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     float *sSg = sDo + CB * PCH;                    // [CB][PCS] d softplus / d raw
     float *sP = sSg + CB * PCS + 4;                 // sum_n A*da*a (4 banks off sQ: a wave writes both in one instruction)
     float *sHold = sP + CB * PCH;                   // dB, dC sums of a pair's right tile, [2][NP][kTile]
+    // (TS) sum over a wave's channels of dout * delta' * u / 4, [WPB][kTile], and sum over the states of B*C / 4, [kTile]: where
+    // sHold is, which 7x7 tiles have no use for
+    constexpr bool TS = TE == 7;
+    float *sT = sHold, *sS = sT + WPB * kTile;
     float *sRed = sHold + 2 * NP * kTile;           // [WPB]
 
     const snd_fwd_params &f = p.f;
@@ -437,6 +441,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // 1.290 -> 1.258 ms against the flush behind the wait; with the
     // sums in front of the wait and the atomics behind it the eight values kept across the wait are spilled and
     // nothing more is gained, and the per-pixel epilogue moved to the same place gains nothing either).
+    // (TS) The terms in dout*C/4 and bu/4 are left out of the sweep: summed over channels (states) they are products of B or C
+    // with per-pixel sums that all states (channels) share,
+    //     dB: C * T,  dC: B * T,  T = sum_c dout*delta'*u / 4        sum_n dbu*B: dout * S,  S = sum_n B*C / 4
+    // That and s - bu = a * s[left] take four instructions per cell out of the sweep.  Only where the eight registers B and C of
+    // the flushed tile take until then are free: 7x7 tiles (64 x 768 x 14x14 bf16 312 -> 303 us, 32 x 768 x 28x28 609 -> 600);
+    // 8x8 tiles spill 12 to 14 registers and lose 4 %.  (All schedules alike, so that their results agree bit for bit; in a
+    // pipeline of two strips the sums in front of the sweep cost as much as it saves: 2 x 384 x 14x14 33.9 -> 34.4 us.)
+    float pB[TS ? NBC : 1], pC[TS ? NBC : 1];       // this thread's B, C of that tile
     int pI = -1, pJ = 0;                            // the tile whose partial sums are still in LDS
     auto flush_bc = [&](int I_, int J_) __attribute__((always_inline)) {
         SND_THREAD_MAPS(NP);
@@ -452,10 +464,15 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const int jc = px & 7, jr = px >> 4;
         const bool right = px & 8;
         const int jcol = (J_ + (right ? 1 : 0)) * TE + jc;
+        float tsum = 0.f;
+        if (TS) {
+#pragma unroll
+            for (int w = 0; w < WPB; ++w) tsum += sT[w * kTile + px];
+        }
 #pragma unroll
         for (int k = 0; k < NBC; ++k) {
             const int sn = wave_u + WPB * k;                        // scalar: folded into the base
-            float tb = 0.f, tc = 0.f;
+            float tb = TS ? pC[TS ? k : 0] * tsum : 0.f, tc = TS ? pB[TS ? k : 0] * tsum : 0.f;
 #pragma unroll
             for (int w = 0; w < NPART; ++w) {
                 tb += sdB[w * PART + sn * NSD + px];
@@ -603,6 +620,22 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             const float gd_old0 = Gd[0];            // G[r0+8][j0]: the corner of the tile on the left
 
+            if (TS) {
+                // T of this wave's channels (only this wave touches their delta' * u, whose place the sweep reuses), and S:
+                // the pixels dealt over the waves, the states over the lanes of a pixel
+                const int lane = tid & 63;
+                float t = 0.f, v = 0.f;
+#pragma unroll
+                for (int k = 0; k < CB / WPB; ++k) t = fmaf(sDu[(wave_u * (CB / WPB) + k) * PCH + lane], sDo[(wave_u * (CB / WPB) + k) * PCH + lane], t);
+                sT[wave_u * kTile + lane] = 0.25f * t;
+                constexpr int PXW = kTile / WPB;
+                const int spx = PXW * wave_u + lane % PXW;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v = fmaf(sB[(lane / PXW * 4 + k) * NSTR + spx], sC[(lane / PXW * 4 + k) * NSTR + spx], v);
+#pragma unroll
+                for (int m = PXW; m < 64; m <<= 1) v += __shfl_xor(v, m);
+                if (lane < PXW) sS[spx] = 0.25f * v;
+            }
             // ---- recompute h on the whole tile, and s at column 3 of every row (the sweep takes a row's right half first)
             float hT[TE][TE], smid[TE];
             // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
@@ -675,14 +708,19 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     const float4 nO4 = *(const float4 *)(myDo + r * kCkX + C0);
                     const float dlr[4] = {nD4.x, nD4.y, nD4.z, nD4.w}, aB[4] = {nB4.x, nB4.y, nB4.z, nB4.w}, aC[4] = {nC4.x, nC4.y, nC4.z, nC4.w};
                     const float aU[4] = {nU4.x, nU4.y, nU4.z, nU4.w}, aO[4] = {nO4.x, nO4.y, nO4.z, nO4.w};
-                    float arow[4], s[4], buv[4];
+                    float arow[4], s[4], buv[4] = {}, sbv[4] = {};
                     float sp = C0 ? smid[r] : slft[r];
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (j < HW) {
                             arow[j] = C0 + j < KA ? aT[KA ? r : 0][C0 + j < KA ? C0 + j : 0] : EXPA(dlr[j]);
-                            buv[j] = aB[j] * aU[j];
-                            sp = fmaf(arow[j], sp, buv[j]);
+                            if (TS) {
+                                sbv[j] = arow[j] * sp;             // s - bu
+                                sp = fmaf(aB[j], aU[j], sbv[j]);
+                            } else {
+                                buv[j] = aB[j] * aU[j];
+                                sp = fmaf(arow[j], sp, buv[j]);
+                            }
                             s[j] = sp;
                         }
                     float q[4] = {}, pp_[4] = {}, vB[4] = {}, vC[4] = {}, dsum[4] = {};
@@ -691,14 +729,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         if (j >= HW) continue;
                         const int cj = C0 + j;
                         const float dov = aO[j], duv = aU[j], bu = buv[j], a = arow[j];
-                        const float dyC = dov * aC[j];
+                        const float dyC = TS ? 0.f : dov * aC[j];
                         const float w = fmaf(tr, Gdiag, Kd[cj]);
-                        const float g_ = (w + Gr) + dyC, gg = w + Sr;   // g, and g + gs (dyC cancels)
-                        const float dbu = fmaf(0.25f, dyC, gg);
+                        const float g_ = TS ? fmaf(dov, aC[j], w + Gr) : (w + Gr) + dyC, gg = w + Sr;   // g, and g + gs (dyC cancels)
+                        const float dbu = TS ? gg : fmaf(0.25f, dyC, gg);
                         const float h_l = cj == 0 ? hlft[r] : hT[r][cj - 1 < 0 ? 0 : cj - 1];
                         const float h_u = r == 0 ? hu[cj] : hT[r - 1 < 0 ? 0 : r - 1][cj];
                         // g(h - bu) + gs(s - bu) = g(h - s) + (g + gs)(s - bu)
-                        const float hs = hT[r][cj] - s[j], sb = s[j] - bu;
+                        const float hs = hT[r][cj] - s[j], sb = TS ? sbv[j] : s[j] - bu;
                         const float cross = fmaf(Gd[cj], h_l, Gr * h_u);
                         const float t = -0.5f * a;
                         const float da = fmaf(t, cross, fmaf(g_, hs, gg * sb));
@@ -713,7 +751,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         tr = t;
                         q[j] = dbu * aB[j];                        // per-pixel terms, summed over states below
                         pp_[j] = A2 * da;
-                        const float z = fmaf(0.25f, bu, hs);
+                        const float z = TS ? hs : fmaf(0.25f, bu, hs);
                         vB[j] = dbu * duv;                         // dB, dC contributions
                         vC[j] = dov * z;
                     }
@@ -769,6 +807,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __syncthreads();
             if (hands_over) strip_signal(progress + I);   // tile J is handed over to the strip above
 
+            if (TS) {
+#pragma unroll
+                for (int k = 0; k < NBC; ++k) {     // (another wave may stage the next tile's B, C by the time the flush needs these)
+                    pB[TS ? k : 0] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
+                    pC[TS ? k : 0] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
+                }
+            }
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
             {
             SND_THREAD_MAPS(NP);
@@ -811,9 +856,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (int k = 0; k < NPX; ++k) {
                 const int pp = n + NP * k;
                 const int row = r0 + (pp >> 3), col = j0 + (pp & 7);
-                const float qv = sQ[cl * PCH + pp], pv = sP[cl * PCH + pp];
+                const float pv = sP[cl * PCH + pp];
                 const float dl = sDl[cl * DLP + ((pp >> 3) + 1) * HG + DLO + (pp & 7)];
                 const float uv = sU[cl * PCS + pp], dov = sDo[cl * PCH + pp], sg = sSg[cl * PCS + pp];
+                const float qv = TS ? fmaf(dov, sS[pp], sQ[cl * PCH + pp]) : sQ[cl * PCH + pp];
                 const float duv = fmaf(Dv, dov, dl * qv);
                 const float ddl = fmaf(kLn2, pv, uv * qv) * sg;
                 if (cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W) {
