@@ -19,6 +19,9 @@ int snd_block_norm_fwd(const void *x, int x_dtype, const float *gamma, const flo
 int snd_block_norm_bwd(const void *dy, int dy_dtype, const void *x, int x_dtype, const float *gamma, const float *stats, int64_t tokens,
                        int channels, void *dx, float *dgamma, float *dbeta, snd_stream_t stream);
 
+/* A = -exp(A_logs) (nA values); w = wx [rows, cols] in `dtype` and (if not null) its transpose wt. */
+int snd_block_params(const float *A_logs, int nA, const float *wx, int rows, int cols, int dtype, float *A, void *w, void *wt, snd_stream_t stream);
+
 /* Depthwise 3x3 convolution + bias + SiLU: x = the first `inner` channels of xz [batch, nrows, ncols, 2 * inner] ->
  * u [batch, inner, nrows, ncols]; pre (may be null): the value before SiLU.  Backward: du -> the first half of dxz. */
 int snd_block_conv_fwd(const snd_block_shape *s, const void *xz, const float *w, const float *bias, void *pre, void *u, snd_stream_t stream);

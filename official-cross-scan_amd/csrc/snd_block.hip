@@ -21,12 +21,6 @@ __device__ __forceinline__ float dsilu(float x) {
     const float s = 1.f / (1.f + __expf(-x));
     return s * fmaf(x, 1.f - s, 1.f);
 }
-__device__ __forceinline__ float wave_sum(float v) {
-    v = group_sum<16>(v);
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
-}
-
 // The value as a tensor of type T holds it.  Parameters and intermediate results are rounded where the chain of torch layers
 // these passes stand for rounds them under autocast, so that both compute with the same numbers.
 template <typename T> __device__ __forceinline__ float rnd(float x) {
@@ -36,92 +30,106 @@ template <typename T> __device__ __forceinline__ float rnd(float x) {
 }
 
 // ---------------------------------------------------------------- LayerNorm over tokens
-// One wave per token, the token's channels in registers (CPL per lane).  TX: type of x and dx, TY: of y and dy.
-template <typename TX, typename TY, int CPL>
+// GL lanes per token (16 up to 256 channels: no lane is idle at a width of 96, and the sums over a token stay inside one DPP
+// row; 64 beyond), the token's channels in registers, CPL per lane.  TX: type of x and dx, TY: of y and dy.
+template <int GL> __device__ __forceinline__ float token_sum(float v) {
+    v = group_sum<16>(v);
+    if (GL == 64) {
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+    }
+    return v;
+}
+template <typename TX, typename TY, int GL, int CPL>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const TX *x, const float *gamma, const float *beta, float eps, int64_t tokens, int C, TY *y,
                                                        float *stats) {
-    const int lane = threadIdx.x & 63;
-    const int64_t tok = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (tok >= tokens) return;
+    const int l = threadIdx.x % GL;
+    const int64_t tok = (int64_t)blockIdx.x * (256 / GL) + threadIdx.x / GL, tc = min(tok, tokens - 1);
+    const bool tin = tok < tokens;
     float v[CPL], sum = 0.f, var = 0.f;
 #pragma unroll
-    for (int k = 0; k < CPL; ++k) v[k] = ldg(x + tok * C, min(lane + 64 * k, C - 1));
+    for (int k = 0; k < CPL; ++k) v[k] = ldg(x + tc * C, min(l + GL * k, C - 1));
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
-        v[k] = lane + 64 * k < C ? v[k] : 0.f;
+        v[k] = l + GL * k < C ? v[k] : 0.f;
         sum += v[k];
     }
-    const float mean = wave_sum(sum) / (float)C;
+    const float mean = token_sum<GL>(sum) / (float)C;
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
-        v[k] = lane + 64 * k < C ? v[k] - mean : 0.f;
+        v[k] = l + GL * k < C ? v[k] - mean : 0.f;
         var = fmaf(v[k], v[k], var);
     }
-    const float rstd = rsqrtf(wave_sum(var) / (float)C + eps);
+    const float rstd = rsqrtf(token_sum<GL>(var) / (float)C + eps);
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
-        const int c = lane + 64 * k;
-        if (c < C) stg(y + tok * C, c, fmaf(v[k] * rstd, gamma[c], beta[c]));
+        const int c = l + GL * k;
+        if (tin && c < C) stg(y + tc * C, c, fmaf(v[k] * rstd, gamma[c], beta[c]));
     }
-    if (stats && lane == 0) *(float2 *)(stats + 2 * tok) = make_float2(mean, rstd);
+    if (stats && tin && l == 0) *(float2 *)(stats + 2 * tc) = make_float2(mean, rstd);
 }
-// Each wave takes TPW neighbouring tokens, then those 4 * TPW * gridDim.x further on, with the loads of all TPW in flight, and keeps
-// its channels' dgamma, dbeta in registers.
-template <typename TX, typename TY, int CPL>
-__global__ __launch_bounds__(256) void norm_bwd_kernel(const TY *dy, const TX *x, const float *gamma, const float *stats, int64_t tokens, int C, TX *dx,
+// A lane group takes every NG * gridDim.x-th token and keeps its channels' dgamma, dbeta in registers.  Every block ends in an
+// atomic per channel, all blocks to the same few lines, one after the other: with blocks of 16 waves (where their sums fit in LDS)
+// there are 256 of them (25088 x 96: 26 -> 12 us).
+constexpr int norm_threads(int GL) { return GL == 16 ? 1024 : 256; }
+template <typename TX, typename TY, int GL, int CPL>
+__global__ __launch_bounds__(norm_threads(GL)) void norm_bwd_kernel(const TY *dy, const TX *x, const float *gamma, const float *stats, int64_t tokens, int C, TX *dx,
                                                        float *dgamma, float *dbeta) {
-    constexpr int TPW = CPL <= 4 ? 4 : 1;
-    __shared__ float sG[4][64 * CPL], sB[4][64 * CPL];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NT = norm_threads(GL), NG = NT / GL, CW = GL * CPL, NW = NT / 64;
+    __shared__ float sG[NW][CW], sB[NW][CW];
+    const int l = threadIdx.x % GL, wave = threadIdx.x >> 6;
     float g[CPL], dg[CPL], db[CPL];
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
-        g[k] = lane + 64 * k < C ? gamma[lane + 64 * k] : 0.f;
+        g[k] = gamma[min(l + GL * k, C - 1)];
         dg[k] = db[k] = 0.f;
     }
-    for (int64_t t0 = ((int64_t)blockIdx.x * 4 + wave) * TPW; t0 < tokens; t0 += (int64_t)gridDim.x * 4 * TPW) {
-        float xh[TPW][CPL], d[TPW][CPL];
-        float2 st[TPW];
+    for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < tokens; t0 += (int64_t)gridDim.x * NG) {
+        const int64_t tok = t0 + threadIdx.x / GL, tc = min(tok, tokens - 1);
+        const bool tin = tok < tokens;
+        const float2 st = *(const float2 *)(stats + 2 * tc);
+        float xh[CPL], d[CPL], m1 = 0.f, m2 = 0.f;
 #pragma unroll
-        for (int i = 0; i < TPW; ++i) {
-            const int64_t tok = min(t0 + i, tokens - 1);
-            st[i] = *(const float2 *)(stats + 2 * tok);
-#pragma unroll
-            for (int k = 0; k < CPL; ++k) {
-                xh[i][k] = ldg(x + tok * C, min(lane + 64 * k, C - 1));
-                d[i][k] = ldg(dy + tok * C, min(lane + 64 * k, C - 1));
-            }
+        for (int k = 0; k < CPL; ++k) {
+            xh[k] = ldg(x + tc * C, min(l + GL * k, C - 1));
+            d[k] = ldg(dy + tc * C, min(l + GL * k, C - 1));
         }
 #pragma unroll
-        for (int i = 0; i < TPW; ++i) {
-            const bool tin = t0 + i < tokens;
-            float m1 = 0.f, m2 = 0.f;
+        for (int k = 0; k < CPL; ++k) {
+            const bool in = tin && l + GL * k < C;
+            xh[k] = in ? (xh[k] - st.x) * st.y : 0.f;
+            d[k] = in ? d[k] : 0.f;
+            dg[k] = fmaf(d[k], xh[k], dg[k]);
+            db[k] += d[k];
+            d[k] *= g[k];
+            m1 += d[k];
+            m2 = fmaf(d[k], xh[k], m2);
+        }
+        m1 = token_sum<GL>(m1) / (float)C;
+        m2 = token_sum<GL>(m2) / (float)C;
 #pragma unroll
-            for (int k = 0; k < CPL; ++k) {
-                const bool in = tin && lane + 64 * k < C;
-                xh[i][k] = in ? (xh[i][k] - st[i].x) * st[i].y : 0.f;
-                d[i][k] = in ? d[i][k] : 0.f;
-                dg[k] = fmaf(d[i][k], xh[i][k], dg[k]);
-                db[k] += d[i][k];
-                d[i][k] *= g[k];
-                m1 += d[i][k];
-                m2 = fmaf(d[i][k], xh[i][k], m2);
-            }
-            m1 = wave_sum(m1) / (float)C;
-            m2 = wave_sum(m2) / (float)C;
-#pragma unroll
-            for (int k = 0; k < CPL; ++k) {
-                const int c = lane + 64 * k;
-                if (tin && c < C) stg(dx + (t0 + i) * C, c, st[i].y * (d[i][k] - m1 - xh[i][k] * m2));
-            }
+        for (int k = 0; k < CPL; ++k) {
+            const int c = l + GL * k;
+            if (tin && c < C) stg(dx + tc * C, c, st.y * (d[k] - m1 - xh[k] * m2));
         }
     }
 #pragma unroll
-    for (int k = 0; k < CPL; ++k) { sG[wave][lane + 64 * k] = dg[k]; sB[wave][lane + 64 * k] = db[k]; }
+    for (int k = 0; k < CPL; ++k) {
+        if (GL == 16) {                             // over the wave's four tokens
+            dg[k] += __shfl_xor(dg[k], 16);
+            dg[k] += __shfl_xor(dg[k], 32);
+            db[k] += __shfl_xor(db[k], 16);
+            db[k] += __shfl_xor(db[k], 32);
+        }
+        if ((threadIdx.x & 63) < GL) { sG[wave][l + GL * k] = dg[k]; sB[wave][l + GL * k] = db[k]; }
+    }
     __syncthreads();
-    for (int c = threadIdx.x; c < C; c += 256) {
-        glb_add(dgamma + c, sG[0][c] + sG[1][c] + sG[2][c] + sG[3][c]);
-        glb_add(dbeta + c, sB[0][c] + sB[1][c] + sB[2][c] + sB[3][c]);
+    for (int c = threadIdx.x; c < C; c += NT) {
+        float a = 0.f, b = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) { a += sG[w][c]; b += sB[w][c]; }
+        glb_add(dgamma + c, a);
+        glb_add(dbeta + c, b);
     }
 }
 
@@ -279,42 +287,42 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const 
 }
 
 // ---------------------------------------------------------------- output LayerNorm + gate
-// A block takes 64 pixels of an image with all their channels: y is read along pixels (twice for mean and variance, then in
+// A block of 8 waves takes 64 pixels of an image with all their channels: y is read along pixels (twice for mean and variance, then in
 // tiles of 32 channels that LDS turns to channels along lanes), z and out along channels.
-constexpr int kGtP = 64, kGtPitch = kGtP + 1;
+constexpr int kGtT = 512, kGtP = 64, kGtPitch = kGtP + 1, kGtK = 4;    // threads; pixels; values per thread of a 32-channel tile
 __device__ __forceinline__ void gate_tile(const float *yb, int64_t HW, int c0, int Di, int px, float *sY) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int ch = (threadIdx.x >> 6) + 4 * k;
+    for (int k = 0; k < kGtK; ++k) {
+        const int ch = (threadIdx.x >> 6) + 8 * k;
         sY[ch * kGtPitch + px] = yb[(int64_t)min(c0 + ch, Di - 1) * HW];    // (channels and pixels beyond the edge: never used)
     }
 }
 template <typename T>
-__global__ __launch_bounds__(256) void gate_fwd_kernel(snd_block_shape s, const float *y, const T *xz, const float *gamma, const float *beta, float eps,
+__global__ __launch_bounds__(kGtT) void gate_fwd_kernel(snd_block_shape s, const float *y, const T *xz, const float *gamma, const float *beta, float eps,
                                                        T *out, float *stats) {
-    __shared__ float sY[32 * kGtPitch], sR[4][kGtP], sMean[kGtP], sStd[kGtP];
+    __shared__ float sY[32 * kGtPitch], sR[8][kGtP], sMean[kGtP], sStd[kGtP];
     const int64_t HW = (int64_t)s.nrows * s.ncols;
-    const int Di = s.inner, t = threadIdx.x, px = t & 63, wave = t >> 6, b = blockIdx.y;
+    const int Di = s.inner, t = threadIdx.x, px = t & 63, cg = t >> 6, b = blockIdx.y;
     const int64_t p0 = (int64_t)blockIdx.x * kGtP;
     const bool pin = p0 + px < HW;
     const float *yb = y + (int64_t)b * Di * HW + (pin ? p0 + px : 0);
     float a = 0.f;
 #pragma unroll 8
-    for (int c = wave; c < Di; c += 4) a += yb[(int64_t)c * HW];
-    sR[wave][px] = a;
+    for (int c = cg; c < Di; c += 8) a += yb[(int64_t)c * HW];
+    sR[cg][px] = a;
     __syncthreads();
-    const float mean = (sR[0][px] + sR[1][px] + sR[2][px] + sR[3][px]) / (float)Di;
+    const float mean = (((sR[0][px] + sR[1][px]) + (sR[2][px] + sR[3][px])) + ((sR[4][px] + sR[5][px]) + (sR[6][px] + sR[7][px]))) / (float)Di;
     __syncthreads();
     a = 0.f;
 #pragma unroll 8
-    for (int c = wave; c < Di; c += 4) {
+    for (int c = cg; c < Di; c += 8) {
         const float d = yb[(int64_t)c * HW] - mean;
         a = fmaf(d, d, a);
     }
-    sR[wave][px] = a;
+    sR[cg][px] = a;
     __syncthreads();
-    const float rstd = rsqrtf((sR[0][px] + sR[1][px] + sR[2][px] + sR[3][px]) / (float)Di + eps);
-    if (wave == 0) {
+    const float rstd = rsqrtf((((sR[0][px] + sR[1][px]) + (sR[2][px] + sR[3][px])) + ((sR[4][px] + sR[5][px]) + (sR[6][px] + sR[7][px]))) / (float)Di + eps);
+    if (cg == 0) {
         sMean[px] = mean;
         sStd[px] = rstd;
         if (stats && pin) *(float2 *)(stats + 2 * (b * HW + p0 + px)) = make_float2(mean, rstd);
@@ -326,12 +334,12 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(snd_block_shape s, const 
         const int ch = t & 31, c = c0 + ch;
         if (c < Di) {
             const float g = gamma[c], be = beta[c];
-            float z[8];
+            float z[kGtK];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) z[k] = ldg(xz + (b * HW + min(p0 + (t >> 5) + 8 * k, HW - 1)) * 2 * Di + Di, c);
+            for (int k = 0; k < kGtK; ++k) z[k] = ldg(xz + (b * HW + min(p0 + (t >> 5) + 16 * k, HW - 1)) * 2 * Di + Di, c);
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int q = (t >> 5) + 8 * k;
+            for (int k = 0; k < kGtK; ++k) {
+                const int q = (t >> 5) + 16 * k;
                 const float nv = rnd<T>(fmaf((sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], g, be));
                 if (p0 + q < HW) stg(out + (b * HW + p0 + q) * Di, c, nv * rnd<T>(silu(z[k])));
             }
@@ -339,9 +347,9 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(snd_block_shape s, const 
     }
 }
 template <typename T>
-__global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const T *dout, const float *y, const T *xz, const float *gamma,
+__global__ __launch_bounds__(kGtT) void gate_bwd_kernel(snd_block_shape s, const T *dout, const float *y, const T *xz, const float *gamma,
                                                        const float *beta, const float *stats, float *dy, T *dxz, float *dgamma, float *dbeta) {
-    __shared__ float sY[32 * kGtPitch], sMean[kGtP], sStd[kGtP], sM1[kGtP], sM2[kGtP], sG[8][32], sB[8][32];
+    __shared__ float sY[32 * kGtPitch], sMean[kGtP], sStd[kGtP], sM1[kGtP], sM2[kGtP], sG[16][32], sB[16][32];
     const int64_t HW = (int64_t)s.nrows * s.ncols;
     const int Di = s.inner, t = threadIdx.x, px = t & 63, b = blockIdx.y, ch = t & 31, pg = t >> 5;
     const int64_t p0 = (int64_t)blockIdx.x * kGtP;
@@ -352,7 +360,7 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const 
         sMean[px] = st.x;
         sStd[px] = st.y;
     }
-    float m1[8] = {}, m2[8] = {};
+    float m1[kGtK] = {}, m2[kGtK] = {};
     for (int c0 = 0; c0 < Di; c0 += 32) {           // the two means over channels the LayerNorm's gradient takes
         __syncthreads();
         gate_tile(y + yo, HW, c0, Di, px, sY);
@@ -360,16 +368,16 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const 
         const int c = c0 + ch;
         if (c < Di) {
             const float g = gamma[c];
-            float z[8], d[8];
+            float z[kGtK], d[kGtK];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int64_t tok = b * HW + min(p0 + pg + 8 * k, HW - 1);
+            for (int k = 0; k < kGtK; ++k) {
+                const int64_t tok = b * HW + min(p0 + pg + 16 * k, HW - 1);
                 z[k] = ldg(xz + tok * 2 * Di + Di, c);
                 d[k] = ldg(dout + tok * Di, c);
             }
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int q = pg + 8 * k;
+            for (int k = 0; k < kGtK; ++k) {
+                const int q = pg + 16 * k;
                 const float dn = rnd<T>(d[k] * rnd<T>(silu(z[k]))) * g;
                 m1[k] += dn;
                 m2[k] = fmaf(dn, (sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], m2[k]);
@@ -377,10 +385,10 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const 
         }
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < kGtK; ++k) {
 #pragma unroll
         for (int o = 1; o < 32; o <<= 1) { m1[k] += __shfl_xor(m1[k], o); m2[k] += __shfl_xor(m2[k], o); }
-        if (ch == 0) { sM1[pg + 8 * k] = m1[k] / (float)Di; sM2[pg + 8 * k] = m2[k] / (float)Di; }
+        if (ch == 0) { sM1[pg + 16 * k] = m1[k] / (float)Di; sM2[pg + 16 * k] = m2[k] / (float)Di; }
     }
     for (int c0 = 0; c0 < Di; c0 += 32) {
         __syncthreads();
@@ -390,16 +398,16 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const 
         float gg = 0.f, gb = 0.f;
         if (c < Di) {
             const float g = gamma[c], be = beta[c];
-            float z[8], d[8];
+            float z[kGtK], d[kGtK];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int64_t tok = b * HW + min(p0 + pg + 8 * k, HW - 1);
+            for (int k = 0; k < kGtK; ++k) {
+                const int64_t tok = b * HW + min(p0 + pg + 16 * k, HW - 1);
                 z[k] = ldg(xz + tok * 2 * Di + Di, c);
                 d[k] = ldg(dout + tok * Di, c);
             }
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int q = pg + 8 * k;
+            for (int k = 0; k < kGtK; ++k) {
+                const int q = pg + 16 * k;
                 const float yh = (sY[ch * kGtPitch + q] - sMean[q]) * sStd[q], dn = rnd<T>(d[k] * rnd<T>(silu(z[k])));
                 if (p0 + q < HW) {
                     stg(dxz + (b * HW + p0 + q) * 2 * Di + Di, c, rnd<T>(d[k] * rnd<T>(fmaf(yh, g, be))) * dsilu(z[k]));
@@ -413,14 +421,14 @@ __global__ __launch_bounds__(256) void gate_bwd_kernel(snd_block_shape s, const 
         sB[pg][ch] = gb;
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int cc = (t >> 6) + 4 * k;
+        for (int k = 0; k < 4; ++k) {
+            const int cc = (t >> 6) + 8 * k;
             if (pin && c0 + cc < Di) dy[yo + (int64_t)(c0 + cc) * HW] = sY[cc * kGtPitch + px];
         }
         if (t < 64 && c0 + ch < Di) {
             float v = 0.f;
 #pragma unroll
-            for (int p = 0; p < 8; ++p) v += t < 32 ? sG[p][ch] : sB[p][ch];
+            for (int p = 0; p < 16; ++p) v += t < 32 ? sG[p][ch] : sB[p][ch];
             glb_add((t < 32 ? dgamma : dbeta) + c0 + ch, v);
         }
     }
@@ -703,6 +711,21 @@ __global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *
     }
 }
 
+// What the block's parameters are taken as: A = -exp(A_logs), the projection's weights in the activations' type and, for the
+// backward, their transpose.  One launch instead of five.
+template <typename T>
+__global__ __launch_bounds__(256) void params_kernel(const float *A_logs, int nA, const float *wx, int rows, int cols, float *A, T *w, T *wt) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < nA) A[i] = -__expf(A_logs[i]);
+    if (i < rows * cols) {
+        stg(w, i, wx[i]);
+        if (wt) {                                   // (reads spaced by a row: a few ten thousand elements, all in the L2)
+            const int c = i / rows, r = i - c * rows;
+            stg(wt, i, wx[(int64_t)r * cols + c]);
+        }
+    }
+}
+
 bool shape_ok(const snd_block_shape *s) {
     return s && s->batch > 0 && s->nrows > 0 && s->ncols > 0 && s->inner > 0 && s->n_groups > 0 && s->dstate > 0 && s->rank > 0 &&
            s->rank <= SND_BLOCK_MAX_RANK && (int64_t)s->batch * s->n_groups < 65536 && (s->dtype == SND_F32 || s->dtype == SND_F16 || s->dtype == SND_BF16);
@@ -721,11 +744,15 @@ template <typename F> int by_types(int a, int b, F f) {
     by_type(a, [&](auto ea) { st = by_type(b, [&](auto eb) { f(ea, eb); }); });
     return st;
 }
+// f(lanes per token, channels per lane)
 template <typename F> void by_channels(int C, F f) {
-    if (C <= 128) f(std::integral_constant<int, 2>());
-    else if (C <= 256) f(std::integral_constant<int, 4>());
-    else if (C <= 512) f(std::integral_constant<int, 8>());
-    else f(std::integral_constant<int, 16>());
+    std::integral_constant<int, 16> narrow;
+    std::integral_constant<int, 64> wide;
+    if (C <= 64) f(narrow, std::integral_constant<int, 4>());
+    else if (C <= 128) f(narrow, std::integral_constant<int, 8>());
+    else if (C <= 256) f(narrow, std::integral_constant<int, 16>());
+    else if (C <= 512) f(wide, std::integral_constant<int, 8>());
+    else f(wide, std::integral_constant<int, 16>());
 }
 template <typename F> void by_rank(int R, F f) {
     if (R <= 8) f(std::integral_constant<int, 8>());
@@ -753,8 +780,9 @@ int snd_block_norm_fwd(const void *x, int x_dtype, const float *gamma, const flo
     return by_types(x_dtype, y_dtype, [&](auto ex, auto ey) {
         typedef ELT(ex) TX;
         typedef ELT(ey) TY;
-        by_channels(channels, [&](auto cpl) {
-            hipLaunchKernelGGL((norm_fwd_kernel<TX, TY, decltype(cpl)::value>), dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+        by_channels(channels, [&](auto gl, auto cpl) {
+            constexpr int NG = 256 / decltype(gl)::value;
+            hipLaunchKernelGGL((norm_fwd_kernel<TX, TY, decltype(gl)::value, decltype(cpl)::value>), dim3((unsigned)((tokens + NG - 1) / NG)), dim3(256), 0, (hipStream_t)stream,
                                (const TX *)x, gamma, beta, eps, tokens, channels, (TY *)y, stats);
         });
     });
@@ -763,14 +791,24 @@ int snd_block_norm_bwd(const void *dy, int dy_dtype, const void *x, int x_dtype,
                        void *dx, float *dgamma, float *dbeta, snd_stream_t stream) {
     if (!dy || !x || !gamma || !stats || !dx || !dgamma || !dbeta) return SND_ERR_NULL;
     if (tokens <= 0 || channels <= 0 || channels > SND_BLOCK_MAX_NORM) return SND_ERR_SHAPE;
-    const int grid = (int)std::min<int64_t>((tokens + 31) / 32, 1024);      // eight tokens per wave at least: each block ends in 2 * channels atomics
     return by_types(x_dtype, dy_dtype, [&](auto ex, auto ey) {
         typedef ELT(ex) TX;
         typedef ELT(ey) TY;
-        by_channels(channels, [&](auto cpl) {
-            hipLaunchKernelGGL((norm_bwd_kernel<TX, TY, decltype(cpl)::value>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const TY *)dy, (const TX *)x,
+        by_channels(channels, [&](auto gl, auto cpl) {
+            constexpr int GL = decltype(gl)::value, NT = norm_threads(GL), NG = NT / GL;
+            const int grid = (int)std::min<int64_t>((tokens + NG - 1) / NG, 256 * 1024 / NT);
+            hipLaunchKernelGGL((norm_bwd_kernel<TX, TY, GL, decltype(cpl)::value>), dim3(grid), dim3(NT), 0, (hipStream_t)stream, (const TY *)dy, (const TX *)x,
                                gamma, stats, tokens, channels, (TX *)dx, dgamma, dbeta);
         });
+    });
+}
+int snd_block_params(const float *A_logs, int nA, const float *wx, int rows, int cols, int dtype, float *A, void *w, void *wt, snd_stream_t stream) {
+    if (!A_logs || !wx || !A || !w) return SND_ERR_NULL;
+    if (nA <= 0 || rows <= 0 || cols <= 0 || (int64_t)rows * cols >= (int64_t)1 << 31) return SND_ERR_SHAPE;
+    return by_type(dtype, [&](auto e) {
+        typedef ELT(e) T;
+        hipLaunchKernelGGL((params_kernel<T>), dim3((unsigned)((std::max((int64_t)nA, (int64_t)rows * cols) + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                           A_logs, nA, wx, rows, cols, A, (T *)w, (T *)wt);
     });
 }
 static dim3 conv_grid(const snd_block_shape &s) {
@@ -801,7 +839,7 @@ int snd_block_gate_fwd(const snd_block_shape *s, const float *y, const void *xz,
     if (!y || !xz || !gamma || !beta || !out) return SND_ERR_NULL;
     return by_type(s->dtype, [&](auto e) {
         typedef ELT(e) T;
-        hipLaunchKernelGGL((gate_fwd_kernel<T>), gate_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, y, (const T *)xz, gamma, beta, eps, (T *)out, stats);
+        hipLaunchKernelGGL((gate_fwd_kernel<T>), gate_grid(*s), dim3(kGtT), 0, (hipStream_t)stream, *s, y, (const T *)xz, gamma, beta, eps, (T *)out, stats);
     });
 }
 int snd_block_gate_bwd(const snd_block_shape *s, const void *dout, const float *y, const void *xz, const float *gamma, const float *beta, const float *stats,
@@ -810,7 +848,7 @@ int snd_block_gate_bwd(const snd_block_shape *s, const void *dout, const float *
     if (!dout || !y || !xz || !gamma || !beta || !stats || !dy || !dxz || !dgamma || !dbeta) return SND_ERR_NULL;
     return by_type(s->dtype, [&](auto e) {
         typedef ELT(e) T;
-        hipLaunchKernelGGL((gate_bwd_kernel<T>), gate_grid(*s), dim3(256), 0, (hipStream_t)stream, *s, (const T *)dout, y, (const T *)xz, gamma, beta, stats,
+        hipLaunchKernelGGL((gate_bwd_kernel<T>), gate_grid(*s), dim3(kGtT), 0, (hipStream_t)stream, *s, (const T *)dout, y, (const T *)xz, gamma, beta, stats,
                            dy, (T *)dxz, dgamma, dbeta);
     });
 }

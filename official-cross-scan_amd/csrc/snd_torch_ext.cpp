@@ -579,12 +579,23 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &w_, const OptTensor &b_, int64_t dtype) {
         at::AutoDispatchBelowADInplaceOrView below;
         const auto T = (at::ScalarType)dtype;
-        const at::Tensor x = x_.to(T).contiguous(), w = w_.to(T).contiguous();
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
+        const at::Tensor x = x_.to(T).contiguous();
+        at::Tensor w = w_, b = b_.value_or(at::Tensor());
+        if (b.defined() && w.scalar_type() == at::kFloat && b.scalar_type() == at::kFloat && w.is_contiguous() && b.is_contiguous()) {
+            w = at::empty(w_.sizes(), x.options());  // both casts in one launch
+            b = at::empty(b_.value().sizes(), x.options());
+            const snd_job jobs[] = {sum_job(w_, 1, 1, w_.numel(), w), sum_job(b_.value(), 1, 1, b.numel(), b)};
+            run_jobs(jobs, 2, current_stream(), "linear");
+        } else {
+            w = w.to(T).contiguous();
+            if (b.defined()) b = b.to(T);
+        }
         ctx->save_for_backward({x, w});
         ctx->saved_data["x"] = (int64_t)x_.scalar_type();
         ctx->saved_data["w"] = (int64_t)w_.scalar_type();
         ctx->saved_data["b"] = b_.has_value() ? (int64_t)b_.value().scalar_type() : (int64_t)-1;
-        return at::linear(x, w, b_.has_value() ? OptTensor(b_.value().to(T)) : OptTensor());
+        return at::linear(x, w, optional_of(b));
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
         const auto sv = ctx->get_saved_variables();
@@ -617,10 +628,10 @@ at::Tensor block_linear(const at::Tensor &x, const at::Tensor &w, const OptTenso
 
 // Everything between in_proj and out_proj of SS2DCrossScan: xz [B, H, W, 2 * inner] -> [B, H, W, inner].
 struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
-    static snd_block_shape shape_of(const at::Tensor &xz, const at::Tensor &wx, const at::Tensor &wdt) {
+    static snd_block_shape shape_of(const at::Tensor &xz, const at::Tensor &wdt, const at::Tensor &A) {
         snd_block_shape s;
         s.batch = (int)xz.size(0); s.nrows = (int)xz.size(1); s.ncols = (int)xz.size(2); s.inner = (int)(xz.size(3) / 2);
-        s.n_groups = (int)wx.size(0); s.rank = (int)wdt.size(2); s.dstate = (int)(wx.size(1) - wdt.size(2)) / 2;
+        s.n_groups = (int)wdt.size(0); s.rank = (int)wdt.size(2); s.dstate = (int)A.size(1);
         s.dtype = dtype_code(xz.scalar_type());
         return s;
     }
@@ -631,14 +642,16 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{xz_.device()};
         const snd_stream_t stream = (snd_stream_t)current_stream();
         const at::Tensor xz = xz_.contiguous(), conv_w = f32c(conv_w_), wdt = f32c(wdt_), gamma = f32c(gamma_), beta = f32c(beta_), Dv = f32c(D_);
-        const at::Tensor dt_bias = f32c(dt_bias_).view(-1), A = f32c(A_logs_).exp().neg_();
+        const at::Tensor dt_bias = f32c(dt_bias_).view(-1), A_logs = f32c(A_logs_), wx32 = f32c(wx_);
         const OptTensor conv_b = conv_b_.has_value() ? OptTensor(f32c(conv_b_.value())) : OptTensor();
-        const snd_block_shape s = shape_of(xz, wx_, wdt_);
+        const snd_block_shape s = shape_of(xz, wdt, A_logs);
         const int64_t B = s.batch, H = s.nrows, W = s.ncols, Di = s.inner, K = s.n_groups, N = s.dstate, R = s.rank, M = R + 2 * N, HW = H * W;
         at::Tensor u = at::empty({B, Di, H, W}, xz.options()), pre = grad ? at::empty({B, Di, H, W}, xz.options()) : at::Tensor();
         check_status(snd_block_conv_fwd(&s, xz.data_ptr(), conv_w.data_ptr<float>(), ptr_or_null(conv_b), grad ? pre.data_ptr() : nullptr, u.data_ptr(), stream),
                      "block");
-        const at::Tensor wx = wx_.to(xz.scalar_type()).reshape({1, K * M, Di});
+        at::Tensor A = at::empty_like(A_logs), wx = at::empty({1, K * M, Di}, xz.options()), wxt = grad ? at::empty({1, Di, K * M}, xz.options()) : at::Tensor();
+        check_status(snd_block_params(A_logs.data_ptr<float>(), (int)A.numel(), wx32.data_ptr<float>(), (int)(K * M), (int)Di, s.dtype, A.data_ptr<float>(),
+                                      wx.data_ptr(), grad ? wxt.data_ptr() : nullptr, stream), "block");
         const at::Tensor proj = at::bmm(wx.expand({B, K * M, Di}), u.view({B, Di, HW}));                 // [B, K * (R + 2N), HW]
         at::Tensor delta = at::empty({B, K * Di, H, W}, xz.options());
         check_status(snd_block_dt_fwd(&s, proj.data_ptr(), wdt.data_ptr<float>(), delta.data_ptr(), stream), "block");
@@ -660,7 +673,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         check_status(snd_block_gate_fwd(&s, y.data_ptr<float>(), xz.data_ptr(), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, out.data_ptr(),
                                         grad ? stats.data_ptr<float>() : nullptr, stream), "block");
         if (!grad) return out;
-        ctx->save_for_backward({xz, conv_w, conv_b.value_or(at::Tensor()), wx_, wdt, dt_bias, A, Dv, w.value_or(at::Tensor()), gamma, beta, u, pre, proj, delta, y,
+        ctx->save_for_backward({xz, conv_w, conv_b.value_or(at::Tensor()), wxt, wdt, dt_bias, A, Dv, w.value_or(at::Tensor()), gamma, beta, u, pre, proj, delta, y,
                                 stats, state});
         ctx->saved_data["sched"] = (int64_t)o.sched;
         if (mw_.has_value()) ctx->saved_data["mw_shape"] = mw_.value().sizes().vec();
@@ -675,12 +688,12 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         const auto sv = ctx->get_saved_variables();
         torch::autograd::variable_list r(13);
         if (!grads[0].defined()) return r;
-        const at::Tensor &xz = sv[0], &conv_w = sv[1], &wx_ = sv[3], &wdt = sv[4], &dt_bias = sv[5], &A = sv[6], &Dv = sv[7], &gamma = sv[9], &beta = sv[10],
+        const at::Tensor &xz = sv[0], &conv_w = sv[1], &wxt = sv[3], &wdt = sv[4], &dt_bias = sv[5], &A = sv[6], &Dv = sv[7], &gamma = sv[9], &beta = sv[10],
                          &u = sv[11], &pre = sv[12], &proj = sv[13], &delta = sv[14], &y = sv[15], &stats = sv[16], &state = sv[17];
         const OptTensor conv_b = optional_of(sv[2]), w = optional_of(sv[8]);
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{xz.device()};
         const snd_stream_t stream = (snd_stream_t)current_stream();
-        const snd_block_shape s = shape_of(xz, wx_, wdt);
+        const snd_block_shape s = shape_of(xz, wdt, A);
         const int64_t B = s.batch, H = s.nrows, W = s.ncols, Di = s.inner, K = s.n_groups, N = s.dstate, R = s.rank, M = R + 2 * N, HW = H * W;
         const at::Tensor dout = grads[0].to(xz.scalar_type()).contiguous();
         // the accumulated parameter gradients: conv weight and bias, the two projections, gamma, beta
@@ -709,8 +722,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
                                      ap + off[3], stream), "block");
         check_status(snd_block_wgrad(dproj.data_ptr(), K * M * HW, 0, u.data_ptr(), Di * HW, 0, (int)B, 1, (int)(K * M), (int)Di, HW, s.dtype, ap + off[2],
                                      stream), "block");
-        const at::Tensor wxt = wx_.to(xz.scalar_type()).reshape({K * M, Di}).t().contiguous();
-        const at::Tensor du = at::baddbmm(g.du.view({B, Di, HW}), wxt.unsqueeze(0).expand({B, Di, K * M}), dproj);
+        const at::Tensor du = at::baddbmm(g.du.view({B, Di, HW}), wxt.expand({B, Di, K * M}), dproj);
         check_status(snd_block_conv_bwd(&s, du.data_ptr(), pre.data_ptr(), xz.data_ptr(), conv_w.data_ptr<float>(), dxz.data_ptr(), ap + off[0],
                                         conv_b.has_value() ? ap + off[1] : nullptr, stream), "block");
         const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
