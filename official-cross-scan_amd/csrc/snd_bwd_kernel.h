@@ -568,34 +568,41 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // pipelined band - by another block.  It is requested here if it is known to be there (own
             // rows; rows whose hand-over an earlier poll has already seen), else after the wait below.
             const bool handed = PIPE && I == I_hi && I + 1 < geo.nCY;
+            auto take_row = [&](int J_) __attribute__((always_inline)) {   // (pipelined schedules: through coherent words)
+                if (I + 1 < geo.nCY && lvalid) {
+                    const char *src = gdown + (int64_t)J_ * DN8 * 4;
+#pragma unroll
+                    for (int k = 0; k < kCkX; k += 2) ld2_coherent((const float *)(src + (k >> 1) * DN2 * 4 + laneG), Gd[k], Gd[k + 1]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kCkX; ++j) Gd[j] = 0.f;
+                }
+            };
             const bool late = handed && __builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) < geo.nCX - J;
             if (!late) {
-                if (I + 1 < geo.nCY && lvalid) {
+                if (PIPE) take_row(J);
+                else if (I + 1 < geo.nCY && lvalid) {
                     const char *src = gdown + (int64_t)J * DN8 * 4;
-                    if (PIPE) {
-#pragma unroll
-                        for (int k = 0; k < kCkX; k += 2) ld2_coherent((const float *)(src + (k >> 1) * DN2 * 4 + laneG), Gd[k], Gd[k + 1]);
-                    } else {
-                        const float4 v0 = *(const float4 *)(src + laneG), v1 = *(const float4 *)(src + DN4 * 4 + laneG);
-                        Gd[0] = v0.x; Gd[1] = v0.y; Gd[2] = v0.z; Gd[3] = v0.w;
-                        Gd[4] = v1.x; Gd[5] = v1.y; Gd[6] = v1.z; Gd[7] = v1.w;
-                    }
+                    const float4 v0 = *(const float4 *)(src + laneG), v1 = *(const float4 *)(src + DN4 * 4 + laneG);
+                    Gd[0] = v0.x; Gd[1] = v0.y; Gd[2] = v0.z; Gd[3] = v0.w;
+                    Gd[4] = v1.x; Gd[5] = v1.y; Gd[6] = v1.z; Gd[7] = v1.w;
                 } else {
 #pragma unroll
                     for (int j = 0; j < kCkX; ++j) Gd[j] = 0.f;
                 }
             }
+            int peek = 0;                           // wave 0: the count as it is now, there when the staged inputs are
+            if (late && wave == 0) peek = __hip_atomic_load(progress + I + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             prefetch(I, J);                         // no loads in flight across the register-hungry sweep
             if (pI >= 0) flush_bc(pI, pJ);          // the previous tile's dB, dC, under the latency of the loads just requested
             commit(I, J);
             pI = I; pJ = J;
-            // strip pipeline: the strip below must have handed over tile J.  One wave polls; the
-            // others wait at the barrier.
-            if (handed && wave == 0) {
-                strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit);
-                if (tid == 0) { sSeen = seen; if (dead) sDead = 1; }   // read at the top of later tiles
+            if (late && wave == 0) {
+                seen = __builtin_amdgcn_readfirstlane(peek);
+                if (tid == 0) lds_poke(&sSeen, dead ? geo.nCX : seen);
             }
             __syncthreads();
+            const bool soon = late && __builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) >= geo.nCX - J;
             // The sweep runs at a raised wave priority, everything else (loads, commit to LDS, per-pixel epilogue) at the
             // default: the two waves a SIMD holds belong to two blocks, and with equal priority they drift into the same
             // phase and stall together; with the wave that is in its dependent arithmetic chain preferred, the other's
@@ -603,22 +610,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // c3 1.199 -> 1.181, c4 2.765 -> 2.664; priorities 1, 2, 3 alike, the reverse assignment half as much, a fixed
             // priority per block nothing.
             __builtin_amdgcn_s_setprio(3);
-
-            if (late) {                             // only after the wait above
-                if (I + 1 < geo.nCY && lvalid) {
-                    const char *src = gdown + (int64_t)J * DN8 * 4;
-#pragma unroll
-                    for (int k = 0; k < kCkX; k += 2) ld2_coherent((const float *)(src + (k >> 1) * DN2 * 4 + laneG), Gd[k], Gd[k + 1]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < kCkX; ++j) Gd[j] = 0.f;
-                }
-            }
-            if (handed && lds_peek(&sDead)) {   // the wait timed out: poison everything downstream
-#pragma unroll
-                for (int j = 0; j < kCkX; ++j) Gd[j] = __builtin_nanf("");
-            }
-            const float gd_old0 = Gd[0];            // G[r0+8][j0]: the corner of the tile on the left
 
             if (TS) {
                 // T of this wave's channels (only this wave touches their delta' * u, whose place the sweep reuses), and S:
@@ -639,9 +630,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // ---- recompute h on the whole tile, and s at column 3 of every row (the sweep takes a row's right half first)
             float hT[TE][TE], smid[TE];
             // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
-            // the tile loop (a spilled register is two vector memory instructions per tile: the 16-bit variant and the one with
-            // column segments are 2 to 4 % faster with none)
-            constexpr int KA = TE == 7 ? 4 : sizeof(T) == 4 && !SEG ? 3 : 0;
+            // the tile loop (a spilled register is two vector memory instructions per tile, 2 to 4 % of the kernel); the column
+            // segments' bookkeeping leaves room for two.  In the pipelined schedules the row below is loaded late in this pass or
+            // behind it, which is where the registers for five come from.
+            constexpr int KA = TE == 7 ? 4 : SEG ? 2 : 5;
             float aT[KA ? TE : 1][KA ? KA : 1];
             {
                 float aprev[8], hprev[8], dlr[4];
@@ -655,6 +647,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 float diag0 = hc;
 #pragma unroll
                 for (int r = 0; r < TE; ++r) {
+                    if (PIPE && r == 4 && soon) take_row(J);    // it arrives under the rest of the recomputation
                     float al = AEXP(r, -1), left = hlft[r], sl = slft[r], diag = diag0;
                     diag0 = hlft[r];
 #pragma unroll
@@ -681,6 +674,38 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     smid[r] = sl;
                 }
             }
+            // strip pipeline: the strip below must have handed over tile J - wanted here, behind the recomputation, and no sooner.
+            // One wave polls the count in memory (more pollers only slow it down), the others the word it leaves in LDS.
+            // Waiting ahead of the recomputation cost 1.5-7 % of the pipelined backwards: 1 x 256 x 512^2 bf16, 16 states
+            // 2396 -> 2328 us; 2 x 192 x 200x336 fp32 1063 -> 1040; 3 x 152 x 61x83 fp16, 8 states 225 -> 209 (unpipelined: same).
+            if (PIPE) {                             // (keeps the compiler from moving the recomputation below the wait)
+#pragma unroll
+                for (int r = 0; r < TE; ++r) {
+#pragma unroll
+                    for (int j = 0; j < TE; ++j) asm volatile("" : "+v"(hT[r][j]));
+                    asm volatile("" : "+v"(smid[r]));
+#pragma unroll
+                    for (int j = 0; j < KA; ++j) asm volatile("" : "+v"(aT[r][j]));
+                }
+            }
+            if (late && !soon) {
+                if (wave == 0) {
+                    strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit);
+                    if (tid == 0) {
+                        if (dead) sDead = 1;
+                        lds_poke(&sSeen, dead ? geo.nCX : seen);   // (read at the top of later tiles, too)
+                    }
+                } else {
+                    while (__builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) < geo.nCX - J) __builtin_amdgcn_s_sleep(2);
+                }
+                asm volatile("" ::: "memory");
+                take_row(J);
+            }
+            if (handed && lds_peek(&sDead)) {   // the wait timed out: poison everything downstream
+#pragma unroll
+                for (int j = 0; j < kCkX; ++j) Gd[j] = __builtin_nanf("");
+            }
+            const float gd_old0 = Gd[0];            // G[r0+8][j0]: the corner of the tile on the left
             // ---- reverse sweep, bottom-right to top-left.  K[j] = G[j] - 0.5*a[j]*G[j+1] of the row below: the part of its
             // contribution to g that does not depend on this row.
             float Kd[8];

@@ -153,6 +153,9 @@ __device__ __forceinline__ void st_f32_b(void *base, uint32_t off, int dt, float
 __device__ __forceinline__ int lds_peek(const int *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void lds_poke(int *p, int v) {      // (after everything this thread has written to LDS before)
+    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 // float add to global memory, no value returned (one L2 atomic)
 __device__ __forceinline__ void glb_add(float *p, float v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
