@@ -9,6 +9,7 @@
 // It does what a host binding has to do and nothing else: the reference's TORCH_CHECKs
 // (:188-245, :298-391), allocation of outputs / saved state / scratch, device guard, current-stream
 // lookup, and mapping of a non-zero library status to a c10::Error (Python RuntimeError).
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/extension.h>
@@ -442,6 +443,18 @@ std::vector<at::Tensor> selective_scan_bwd(const at::Tensor &u, const at::Tensor
 at::Tensor rows_contiguous(const at::Tensor &t) { return t.stride(-1) == 1 || t.size(-1) == 1 ? t : t.contiguous(); }
 OptTensor optional_of(const at::Tensor &t) { return t.defined() ? OptTensor(t) : OptTensor(); }
 
+// Held by the functions below in both directions.  Their types are settled before they are called, and the raw pointers they
+// pass on are of those types: no call inside them may be cast.  In the backward autocast is in whatever state backward() was
+// called under (the engine hands it to its threads), which need not be the forward's.
+struct NoAutocast {
+    c10::impl::ExcludeDispatchKeyGuard off{c10::autocast_dispatch_keyset};
+};
+// A tensor whose pointer goes to a kernel as `numel` elements of the type of `like`.
+void check_elements(const at::Tensor &t, const at::Tensor &like, int64_t numel, const char *what) {
+    TORCH_CHECK(t.defined() && t.scalar_type() == like.scalar_type() && t.device() == like.device() && t.is_contiguous() && t.numel() == numel,
+                "selective_nd_scan: ", what, " is not a contiguous ", toString(like.scalar_type()), " tensor of ", numel, " elements on ", like.device());
+}
+
 // The differentiable scan.  The saved state is one buffer [x | x_sd | x_v] that only the backward reads.
 // The block mapping is resolved once, in the forward, and the backward runs the same one: the two kernel families keep
 // different saved-state layouts, so a default changed between a forward and its backward must not reach it.
@@ -451,6 +464,7 @@ struct ScanFn : public torch::autograd::Function<ScanFn> {
                               const OptTensor &A_decay_, const OptTensor &weights_, bool delta_softplus, bool out_float,
                               int64_t directions, bool merge) {
         at::AutoDispatchBelowADInplaceOrView below;
+        NoAutocast no_autocast;
         Options o{delta_softplus, out_float, directions, resolve_schedule(-1), merge};
         OptTensor w;
         const Checked c = check_inputs(u, delta, A, B, C, D_, delta_bias_, A_decay_);
@@ -476,6 +490,7 @@ struct ScanFn : public torch::autograd::Function<ScanFn> {
         return out;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        NoAutocast no_autocast;
         const auto saved = ctx->get_saved_variables();
         const at::Tensor &u = saved[0], &delta = saved[1], &A = saved[2], &B = saved[3], &C = saved[4], &state = saved[9];
         const OptTensor D_ = optional_of(saved[5]), delta_bias_ = optional_of(saved[6]), A_decay_ = optional_of(saved[7]), w = optional_of(saved[8]);
@@ -536,6 +551,7 @@ struct NormFn : public torch::autograd::Function<NormFn> {
     static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &gamma_, const at::Tensor &beta_, double eps,
                               int64_t out_dtype) {
         at::AutoDispatchBelowADInplaceOrView below;
+        NoAutocast no_autocast;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
         const at::Tensor x = x_.contiguous(), gamma = f32c(gamma_), beta = f32c(beta_);
         const int64_t C = x.size(-1), tokens = x.numel() / C;
@@ -548,6 +564,7 @@ struct NormFn : public torch::autograd::Function<NormFn> {
         return y;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        NoAutocast no_autocast;
         const auto saved = ctx->get_saved_variables();
         const at::Tensor &x = saved[0], &gamma = saved[1], &stats = saved[2];
         torch::autograd::variable_list r(5);
@@ -578,6 +595,7 @@ bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) { return M % 2 == 0
 struct LinearFn : public torch::autograd::Function<LinearFn> {
     static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &w_, const OptTensor &b_, int64_t dtype) {
         at::AutoDispatchBelowADInplaceOrView below;
+        NoAutocast no_autocast;
         const auto T = (at::ScalarType)dtype;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
         const at::Tensor x = x_.to(T).contiguous();
@@ -598,6 +616,7 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
         return at::linear(x, w, optional_of(b));
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        NoAutocast no_autocast;
         const auto sv = ctx->get_saved_variables();
         const at::Tensor &x = sv[0], &w = sv[1];
         torch::autograd::variable_list r(4);
@@ -639,6 +658,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
                               const at::Tensor &wx_, const at::Tensor &wdt_, const at::Tensor &dt_bias_, const at::Tensor &A_logs_, const at::Tensor &D_,
                               const OptTensor &mw_, const at::Tensor &gamma_, const at::Tensor &beta_, double eps, bool grad) {
         at::AutoDispatchBelowADInplaceOrView below;
+        NoAutocast no_autocast;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{xz_.device()};
         const snd_stream_t stream = (snd_stream_t)current_stream();
         const at::Tensor xz = xz_.contiguous(), conv_w = f32c(conv_w_), wdt = f32c(wdt_), gamma = f32c(gamma_), beta = f32c(beta_), Dv = f32c(D_);
@@ -653,6 +673,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         check_status(snd_block_params(A_logs.data_ptr<float>(), (int)A.numel(), wx32.data_ptr<float>(), (int)(K * M), (int)Di, s.dtype, A.data_ptr<float>(),
                                       wx.data_ptr(), grad ? wxt.data_ptr() : nullptr, stream), "block");
         const at::Tensor proj = at::bmm(wx.expand({B, K * M, Di}), u.view({B, Di, HW}));                 // [B, K * (R + 2N), HW]
+        check_elements(proj, xz, B * K * M * HW, "the projection");
         at::Tensor delta = at::empty({B, K * Di, H, W}, xz.options());
         check_status(snd_block_dt_fwd(&s, proj.data_ptr(), wdt.data_ptr<float>(), delta.data_ptr(), stream), "block");
         const at::Tensor p5 = proj.view({B, K, M, H, W}), Bs = p5.narrow(2, R, N), Cs = p5.narrow(2, R + N, N);
@@ -685,6 +706,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         return out;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        NoAutocast no_autocast;
         const auto sv = ctx->get_saved_variables();
         torch::autograd::variable_list r(13);
         if (!grads[0].defined()) return r;
@@ -723,6 +745,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         check_status(snd_block_wgrad(dproj.data_ptr(), K * M * HW, 0, u.data_ptr(), Di * HW, 0, (int)B, 1, (int)(K * M), (int)Di, HW, s.dtype, ap + off[2],
                                      stream), "block");
         const at::Tensor du = at::baddbmm(g.du.view({B, Di, HW}), wxt.expand({B, Di, K * M}), dproj);
+        check_elements(du, xz, B * Di * HW, "du");
         check_status(snd_block_conv_bwd(&s, du.data_ptr(), pre.data_ptr(), xz.data_ptr(), conv_w.data_ptr<float>(), dxz.data_ptr(), ap + off[0],
                                         conv_b.has_value() ? ap + off[1] : nullptr, stream), "block");
         const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();

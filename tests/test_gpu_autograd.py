@@ -1,0 +1,84 @@
+"""The autograd functions at their boundary: what the state of autograd and autocast around a call, or around its
+backward, may and may not change."""
+import contextlib
+
+import pytest
+import torch
+import torch.nn as nn
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float((a.detach().double() - b.detach().double()).norm() / b.detach().double().norm().clamp_min(1e-30))
+
+
+def autocast(dtype):
+    return contextlib.nullcontext() if dtype is None else torch.autocast("cuda", dtype=dtype)
+
+
+def block(dev, **kw):
+    import selective_nd_scan as snd
+    torch.manual_seed(12)
+    blk = snd.VSSBlock(24, d_state=3, ssm_ratio=2.0, mlp_ratio=2.0, **kw).to(dev)
+    for p in blk.parameters():
+        p.data.add_(0.02 * torch.randn_like(p))
+    return blk
+
+
+@pytest.mark.parametrize("fwd,bwd", [(None, torch.bfloat16), (None, torch.float16), (torch.bfloat16, torch.float16),
+                                     (torch.float16, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+def test_backward_under_another_autocast(gpu_device, fwd, bwd):
+    """The types of a backward are its forward's, whatever autocast does where backward() is called."""
+    blk = block(gpu_device)
+    if fwd is None:                                  # (torch's own linear layers take autocast's type in their backward)
+        blk = blk.op
+        blk.in_proj, blk.out_proj = nn.Identity(), nn.Identity()
+    x = torch.randn(2, 9, 11, 24 if fwd else 96, device=gpu_device)
+    dy = torch.randn(2, 9, 11, 24 if fwd else 48, device=gpu_device)
+    grads = []
+    for state in (None, bwd):
+        xi = x.clone().requires_grad_()
+        with autocast(fwd):
+            y = blk(xi)
+        with autocast(state):
+            y.backward(dy)
+        grads.append([xi.grad] + [p.grad for p in blk.parameters()])
+        blk.zero_grad(set_to_none=True)
+    # fp32: sums in another order.  16 bits: such a sum that lies at a rounding edge moves by one unit in the last place
+    # (2^-8 in bf16) in a share of the values that is below 1e-2.
+    for a, b in zip(*grads):
+        assert a.dtype == b.dtype and rel(a, b) <= (1e-5 if fwd is None else 1e-3)
+
+
+class Cast(nn.Module):
+    def __init__(self, layer, dtype):
+        super().__init__()
+        self.layer, self.dtype = layer, dtype
+
+    def forward(self, x):
+        return self.layer(x).to(self.dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_in_proj_of_another_type_than_autocast(gpu_device, dtype):
+    """What in_proj returns sets the type of the stages up to out_proj: here not autocast's."""
+    blk = block(gpu_device)
+    x = torch.randn(2, 9, 11, 24, device=gpu_device)
+    dy = torch.randn_like(x)
+
+    def run(forward):
+        xi = x.clone().requires_grad_()
+        forward(xi).backward(dy)
+        r = [xi.grad] + [p.grad for p in blk.parameters()]
+        blk.zero_grad(set_to_none=True)
+        return r
+
+    def cast(xi):
+        with autocast(torch.bfloat16):
+            return blk(xi)
+
+    want = run(blk)                                  # fp32 throughout
+    blk.op.in_proj = Cast(blk.op.in_proj, dtype)
+    for a, b in zip(run(cast), want):
+        assert rel(a, b) <= 2e-2                     # the roundings of the bf16 layers around
