@@ -516,6 +516,9 @@ struct ScanFn : public torch::autograd::Function<ScanFn> {
     }
 };
 
+// Whether a forward-mode tangent is attached (it is where requires_grad() says no, and the raw path would drop it).
+bool has_tangent(const at::Tensor &t) { return t._fw_grad(/*level=*/0).defined(); }
+
 // selective_nd_scan / selective_nd_scan_merged: the differentiable function where a gradient can be asked for, the forward
 // that saves no state where none can.
 at::Tensor scan(const at::Tensor &u_, const at::Tensor &delta_, const at::Tensor &A, const at::Tensor &B_, const at::Tensor &C_,
@@ -523,6 +526,9 @@ at::Tensor scan(const at::Tensor &u_, const at::Tensor &delta_, const at::Tensor
                 int64_t directions, bool merge, const OptTensor &weights_) {
     TORCH_CHECK(u_.dim() == 4 && delta_.dim() == 4 && A.dim() == 2 && B_.dim() == 5 && C_.dim() == 5, "expected u, delta 4-D; A 2-D; B, C 5-D");
     const at::Tensor u = rows_contiguous(u_), delta = rows_contiguous(delta_), B = rows_contiguous(B_), C = rows_contiguous(C_);
+    for (const at::Tensor *t : {&u, &delta, &A, &B, &C}) TORCH_CHECK(!has_tangent(*t), "selective_nd_scan has no forward-mode derivative");
+    for (const OptTensor *t : {&D_, &delta_bias_, &A_decay_, &weights_})
+        TORCH_CHECK(!t->has_value() || !has_tangent(t->value()), "selective_nd_scan has no forward-mode derivative");
     bool grad = false;
     if (at::GradMode::is_enabled()) {
         for (const at::Tensor *t : {&u, &delta, &A, &B, &C}) grad = grad || t->requires_grad();

@@ -82,3 +82,16 @@ def test_in_proj_of_another_type_than_autocast(gpu_device, dtype):
     blk.op.in_proj = Cast(blk.op.in_proj, dtype)
     for a, b in zip(run(cast), want):
         assert rel(a, b) <= 2e-2                     # the roundings of the bf16 layers around
+
+
+@pytest.mark.parametrize("grad", [torch.no_grad, torch.enable_grad])
+def test_forward_mode_of_the_scan_is_refused(gpu_device, grad):
+    import selective_nd_scan as snd
+    import torch.autograd.forward_ad as fwad
+    u, B = torch.randn(1, 8, 6, 6, device=gpu_device), torch.randn(1, 4, 2, 6, 6, device=gpu_device)
+    A = -torch.ones(8, 2, device=gpu_device)
+    with fwad.dual_level():
+        dual = fwad.make_dual(u, torch.randn_like(u))
+        with grad(), pytest.raises(RuntimeError, match="forward-mode"):
+            snd.selective_nd_scan(dual, u, A, B, B)
+        snd.selective_nd_scan(fwad.unpack_dual(dual).primal, u, A, B, B)
