@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <initializer_list>
 #include <vector>
 
 #include "snd_block.h"
@@ -550,6 +551,11 @@ at::Tensor scan(const at::Tensor &u_, const at::Tensor &delta_, const at::Tensor
 // ---------------------------------------------------------------- the passes of a VSS block around its scan
 hipStream_t current_stream() { return at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 at::Tensor f32c(const at::Tensor &t) { return t.to(at::kFloat).contiguous(); }
+// (undefined: an optional tensor that was not given)
+void check_device(const char *what, const at::Tensor &x, std::initializer_list<at::Tensor> others) {
+    TORCH_CHECK(x.is_cuda(), what, ": the tensors must be on the GPU");
+    for (const at::Tensor &t : others) TORCH_CHECK(!t.defined() || t.device() == x.device(), what, ": the tensors must be on one device");
+}
 const float *ptr_or_null(const OptTensor &t) { return t.has_value() ? t.value().data_ptr<float>() : nullptr; }
 
 // LayerNorm over the last axis, its result in `out_dtype` (what the next layer reads under autocast).
@@ -589,6 +595,9 @@ struct NormFn : public torch::autograd::Function<NormFn> {
     }
 };
 at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps, const at::Tensor &like) {
+    TORCH_CHECK(x.dim() >= 1 && gamma.dim() == 1 && beta.dim() == 1 && gamma.size(0) == x.size(-1) && beta.size(0) == x.size(-1),
+                "block_norm: the last axis of x has another size than gamma or beta");
+    check_device("block_norm", x, {gamma, beta});
     return NormFn::apply(x, gamma, beta, eps, (int64_t)like.scalar_type());
 }
 
@@ -648,6 +657,10 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     }
 };
 at::Tensor block_linear(const at::Tensor &x, const at::Tensor &w, const OptTensor &b, const at::Tensor &like) {
+    TORCH_CHECK(x.dim() >= 1 && w.dim() == 2 && w.size(1) == x.size(-1) && (!b.has_value() || (b.value().dim() == 1 && b.value().size(0) == w.size(0))),
+                "block_linear: the shapes of x, weight and bias do not fit");
+    TORCH_CHECK(like.scalar_type() == at::kHalf || like.scalar_type() == at::kBFloat16, "block_linear: the type of `like` must be float16 or bfloat16");
+    check_device("block_linear", x, {w, b.value_or(at::Tensor())});
     return LinearFn::apply(x, w, b, (int64_t)like.scalar_type());
 }
 
@@ -772,15 +785,16 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
 };
 at::Tensor ss2d(const at::Tensor &xz, const at::Tensor &conv_w, const OptTensor &conv_b, const at::Tensor &wx, const at::Tensor &wdt, const at::Tensor &dt_bias,
                 const at::Tensor &A_logs, const at::Tensor &D, const OptTensor &mw, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
-    TORCH_CHECK(xz.is_cuda() && xz.dim() == 4 && xz.size(3) % 2 == 0, "ss2d: xz must be a GPU tensor [batch, rows, cols, 2 * inner]");
+    TORCH_CHECK(xz.dim() == 4 && xz.size(3) % 2 == 0, "ss2d: xz must be [batch, rows, cols, 2 * inner]");
     const int64_t Di = xz.size(3) / 2;
-    TORCH_CHECK(wx.dim() == 3 && wdt.dim() == 3, "ss2d: projections are 3-D");
+    TORCH_CHECK(wx.dim() == 3 && wdt.dim() == 3 && A_logs.dim() == 2, "ss2d: projections are 3-D, A_logs is 2-D");
     const int64_t K = wx.size(0), R = wdt.size(2), N = A_logs.size(1);
     TORCH_CHECK(wx.size(1) == R + 2 * N && wx.size(2) == Di && wdt.size(0) == K && wdt.size(1) == Di && dt_bias.numel() == K * Di && A_logs.size(0) == K * Di &&
-                    D.numel() == K * Di && gamma.numel() == Di && beta.numel() == Di && conv_w.numel() == Di * 9 &&
-                    (!conv_b.has_value() || conv_b.value().numel() == Di),
+                    D.numel() == K * Di && gamma.numel() == Di && beta.numel() == Di && conv_w.sizes() == at::IntArrayRef({Di, 1, 3, 3}) &&
+                    (!conv_b.has_value() || conv_b.value().numel() == Di) && (!mw.has_value() || mw.value().sizes() == at::IntArrayRef({K}) || mw.value().sizes() == at::IntArrayRef({K, 1}) ||
+                     mw.value().sizes() == at::IntArrayRef({K, Di})),
                 "ss2d: parameter shapes do not fit");
-    for (const at::Tensor *t : {&conv_w, &wx, &wdt, &dt_bias, &A_logs, &D, &gamma, &beta}) TORCH_CHECK(t->device() == xz.device(), "ss2d: parameters must be on xz's device");
+    check_device("ss2d", xz, {conv_w, conv_b.value_or(at::Tensor()), wx, wdt, dt_bias, A_logs, D, mw.value_or(at::Tensor()), gamma, beta});
     bool grad = false;
     if (at::GradMode::is_enabled()) {
         for (const at::Tensor *t : {&xz, &conv_w, &wx, &wdt, &dt_bias, &A_logs, &D, &gamma, &beta}) grad = grad || t->requires_grad();

@@ -38,7 +38,7 @@ class TokenNorm(nn.LayerNorm):
     """LayerNorm whose result, under autocast on the GPU, has the type the following linear layer would cast it to."""
 
     def forward(self, x):
-        if not (x.is_cuda and x.dtype in _FLOATS and len(self.normalized_shape) == 1 and self.normalized_shape[0] <= 1024 and self.bias is not None
+        if not (x.is_cuda and x.dtype in _FLOATS and self.normalized_shape == tuple(x.shape[-1:]) and x.shape[-1] <= 1024 and self.bias is not None
                 and x.numel() > 0 and self.weight.is_cuda):
             return super().forward(x)
         return ext().block_norm(x, self.weight, self.bias, self.eps, _autocast_like(x))

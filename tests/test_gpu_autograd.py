@@ -95,3 +95,28 @@ def test_forward_mode_of_the_scan_is_refused(gpu_device, grad):
         with grad(), pytest.raises(RuntimeError, match="forward-mode"):
             snd.selective_nd_scan(dual, u, A, B, B)
         snd.selective_nd_scan(fwad.unpack_dual(dual).primal, u, A, B, B)
+
+
+@pytest.mark.parametrize("C", [8, 16, 32])
+def test_token_norm_refuses_another_last_axis(gpu_device, C):
+    import selective_nd_scan as snd
+    norm = snd.vss_block.TokenNorm(16).to(gpu_device)
+    x = torch.randn(3, 16, C, device=gpu_device)
+    if C == 16:
+        assert norm(x).shape == x.shape
+        return
+    with pytest.raises(RuntimeError, match="normalized_shape"):
+        norm(x)
+
+
+def test_layers_refuse_parameters_elsewhere(gpu_device):
+    import selective_nd_scan as snd
+    from selective_nd_scan.interface import ext
+    x = torch.randn(3, 16, device=gpu_device)
+    w, b = torch.randn(16), torch.randn(16)
+    with pytest.raises(RuntimeError, match="one device"):
+        ext().block_norm(x, w, b.to(gpu_device), 1e-5, x)
+    with pytest.raises(RuntimeError, match="one device"):
+        ext().block_linear(x.bfloat16(), torch.randn(4, 16, device=gpu_device), torch.randn(4), x.bfloat16())
+    with pytest.raises(RuntimeError):
+        snd.vss_block.TokenNorm(16)(x)
