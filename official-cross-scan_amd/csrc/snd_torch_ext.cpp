@@ -12,6 +12,7 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -456,6 +457,21 @@ void check_elements(const at::Tensor &t, const at::Tensor &like, int64_t numel, 
                 "selective_nd_scan: ", what, " is not a contiguous ", toString(like.scalar_type()), " tensor of ", numel, " elements on ", like.device());
 }
 
+// Gradients that come out of kernels have no graph behind them.  Under create_graph they leave through a node that raises
+// when it is differentiated: a second derivative is refused instead of being short of a term.
+torch::autograd::variable_list once_differentiable(torch::autograd::variable_list r, const char *what) {
+    if (!at::GradMode::is_enabled()) return r;
+    torch::autograd::variable_list given;
+    for (const at::Tensor &t : r)
+        if (t.defined()) given.push_back(t.detach().set_requires_grad(true));
+    auto refuse = std::make_shared<torch::autograd::DelayedError>(std::string(what) + " can be differentiated once: its gradients have no derivative", (int64_t)given.size());
+    const torch::autograd::variable_list out = (*refuse)(std::move(given));
+    size_t k = 0;
+    for (at::Tensor &t : r)
+        if (t.defined()) t = out[k++];
+    return r;
+}
+
 // The differentiable scan.  The saved state is one buffer [x | x_sd | x_v] that only the backward reads.
 // The block mapping is resolved once, in the forward, and the backward runs the same one: the two kernel families keep
 // different saved-state layouts, so a default changed between a forward and its backward must not reach it.
@@ -491,6 +507,10 @@ struct ScanFn : public torch::autograd::Function<ScanFn> {
         return out;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        return once_differentiable(gradients(ctx, std::move(grads)), "selective_nd_scan");
+    }
+    static torch::autograd::variable_list gradients(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        at::NoGradGuard no_grad;
         NoAutocast no_autocast;
         const auto saved = ctx->get_saved_variables();
         const at::Tensor &u = saved[0], &delta = saved[1], &A = saved[2], &B = saved[3], &C = saved[4], &state = saved[9];
@@ -558,21 +578,20 @@ void check_device(const char *what, const at::Tensor &x, std::initializer_list<a
 }
 const float *ptr_or_null(const OptTensor &t) { return t.has_value() ? t.value().data_ptr<float>() : nullptr; }
 
-// LayerNorm over the last axis, its result in `out_dtype` (what the next layer reads under autocast).
+// LayerNorm over the last axis of a contiguous x, its result in `out_dtype` (what the next layer reads under autocast); gamma and
+// beta fp32.  Under create_graph its gradients are torch calls on the saved inputs, which can be differentiated again.
 struct NormFn : public torch::autograd::Function<NormFn> {
-    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &gamma_, const at::Tensor &beta_, double eps,
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps,
                               int64_t out_dtype) {
         at::AutoDispatchBelowADInplaceOrView below;
         NoAutocast no_autocast;
-        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
-        const at::Tensor x = x_.contiguous(), gamma = f32c(gamma_), beta = f32c(beta_);
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         const int64_t C = x.size(-1), tokens = x.numel() / C;
         at::Tensor y = at::empty(x.sizes(), x.options().dtype((at::ScalarType)out_dtype)), stats = floats(2 * tokens, x);
         check_status(snd_block_norm_fwd(x.data_ptr(), dtype_code(x.scalar_type()), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, tokens, (int)C,
                                         y.data_ptr(), dtype_code(y.scalar_type()), stats.data_ptr<float>(), (snd_stream_t)current_stream()), "norm");
         ctx->save_for_backward({x, gamma, stats});
-        ctx->saved_data["g"] = (int64_t)gamma_.scalar_type();
-        ctx->saved_data["b"] = (int64_t)beta_.scalar_type();
+        ctx->saved_data["eps"] = eps;
         return y;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
@@ -582,15 +601,23 @@ struct NormFn : public torch::autograd::Function<NormFn> {
         torch::autograd::variable_list r(5);
         if (!grads[0].defined()) return r;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
-        const at::Tensor dy = grads[0].contiguous();
         const int64_t C = x.size(-1), tokens = x.numel() / C;
+        if (at::GradMode::is_enabled()) {
+            const at::Tensor xf = x.to(at::kFloat), d = grads[0].to(at::kFloat), xc = xf - xf.mean(-1, true);
+            const at::Tensor rstd = (xc * xc).mean(-1, true).add(ctx->saved_data["eps"].toDouble()).rsqrt(), xh = xc * rstd, dn = d * gamma;
+            r[0] = (rstd * (dn - dn.mean(-1, true) - xh * (dn * xh).mean(-1, true))).to(x.scalar_type());
+            r[1] = (d * xh).reshape({tokens, C}).sum(0);
+            r[2] = d.reshape({tokens, C}).sum(0);
+            return r;
+        }
+        const at::Tensor dy = grads[0].contiguous();
         at::Tensor dx = at::empty_like(x), acc = at::zeros({2, C}, x.options().dtype(at::kFloat));
         check_status(snd_block_norm_bwd(dy.data_ptr(), dtype_code(dy.scalar_type()), x.data_ptr(), dtype_code(x.scalar_type()), gamma.data_ptr<float>(),
                                         stats.data_ptr<float>(), tokens, (int)C, dx.data_ptr(), acc.data_ptr<float>(), acc.data_ptr<float>() + C,
                                         (snd_stream_t)current_stream()), "norm");
         r[0] = dx;
-        r[1] = acc[0].to((at::ScalarType)ctx->saved_data["g"].toInt());
-        r[2] = acc[1].to((at::ScalarType)ctx->saved_data["b"].toInt());
+        r[1] = acc[0];
+        r[2] = acc[1];
         return r;
     }
 };
@@ -598,7 +625,7 @@ at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Te
     TORCH_CHECK(x.dim() >= 1 && gamma.dim() == 1 && beta.dim() == 1 && gamma.size(0) == x.size(-1) && beta.size(0) == x.size(-1),
                 "block_norm: the last axis of x has another size than gamma or beta");
     check_device("block_norm", x, {gamma, beta});
-    return NormFn::apply(x, gamma, beta, eps, (int64_t)like.scalar_type());
+    return NormFn::apply(x.contiguous(), f32c(gamma), f32c(beta), eps, (int64_t)like.scalar_type());
 }
 
 // A linear layer in the 16-bit type `dtype` (what autocast makes of F.linear) whose weight and bias gradients are summed over
@@ -608,12 +635,11 @@ at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Te
 // library is ahead; few tokens cost either their launches).
 bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) { return M % 2 == 0 && N % 2 == 0 && M * N <= (int64_t)1 << 19; }
 struct LinearFn : public torch::autograd::Function<LinearFn> {
-    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x_, const at::Tensor &w_, const OptTensor &b_, int64_t dtype) {
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x, const at::Tensor &w_, const OptTensor &b_) {
         at::AutoDispatchBelowADInplaceOrView below;
         NoAutocast no_autocast;
-        const auto T = (at::ScalarType)dtype;
-        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x_.device()};
-        const at::Tensor x = x_.to(T).contiguous();
+        const auto T = x.scalar_type();
+        at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         at::Tensor w = w_, b = b_.value_or(at::Tensor());
         if (b.defined() && w.scalar_type() == at::kFloat && b.scalar_type() == at::kFloat && w.is_contiguous() && b.is_contiguous()) {
             w = at::empty(w_.sizes(), x.options());  // both casts in one launch
@@ -625,7 +651,7 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
             if (b.defined()) b = b.to(T);
         }
         ctx->save_for_backward({x, w});
-        ctx->saved_data["x"] = (int64_t)x_.scalar_type();
+        if (!w.is_same(w_)) ctx->saved_data["w_in"] = w_;   // (the copy saved above has no history; used under create_graph alone)
         ctx->saved_data["w"] = (int64_t)w_.scalar_type();
         ctx->saved_data["b"] = b_.has_value() ? (int64_t)b_.value().scalar_type() : (int64_t)-1;
         return at::linear(x, w, optional_of(b));
@@ -633,15 +659,21 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
         NoAutocast no_autocast;
         const auto sv = ctx->get_saved_variables();
-        const at::Tensor &x = sv[0], &w = sv[1];
-        torch::autograd::variable_list r(4);
+        const at::Tensor &x = sv[0];
+        at::Tensor w = sv[1];
+        torch::autograd::variable_list r(3);
         if (!grads[0].defined()) return r;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         const int64_t M = w.size(0), N = w.size(1), tokens = x.numel() / N, btype = ctx->saved_data["b"].toInt();
         const auto wtype = (at::ScalarType)ctx->saved_data["w"].toInt();
+        const bool graph = at::GradMode::is_enabled();      // create_graph: torch calls on the inputs, which can be differentiated again
+        if (graph && ctx->saved_data.count("w_in")) {       // the values of the saved copy, the history of the parameter
+            const at::Tensor now = ctx->saved_data["w_in"].toTensor().to(x.scalar_type());
+            w = w + (now - now.detach());
+        }
         const at::Tensor dy = grads[0].to(x.scalar_type()).contiguous().view({tokens, M}), x2 = x.view({tokens, N});
-        if (ctx->needs_input_grad(0)) r[0] = at::mm(dy, w).view(x.sizes()).to((at::ScalarType)ctx->saved_data["x"].toInt());
-        if (linear_wgrad_pays(tokens, M, N)) {
+        if (ctx->needs_input_grad(0)) r[0] = at::mm(dy, w).view(x.sizes());
+        if (!graph && linear_wgrad_pays(tokens, M, N)) {
             const int64_t nw = (M * N + 15) / 16 * 16;
             at::Tensor acc = at::zeros({nw + M}, x.options().dtype(at::kFloat));
             float *p = acc.data_ptr<float>();
@@ -661,7 +693,7 @@ at::Tensor block_linear(const at::Tensor &x, const at::Tensor &w, const OptTenso
                 "block_linear: the shapes of x, weight and bias do not fit");
     TORCH_CHECK(like.scalar_type() == at::kHalf || like.scalar_type() == at::kBFloat16, "block_linear: the type of `like` must be float16 or bfloat16");
     check_device("block_linear", x, {w, b.value_or(at::Tensor())});
-    return LinearFn::apply(x, w, b, (int64_t)like.scalar_type());
+    return LinearFn::apply(x.to(like.scalar_type()).contiguous(), w, b);
 }
 
 // Everything between in_proj and out_proj of SS2DCrossScan: xz [B, H, W, 2 * inner] -> [B, H, W, inner].
@@ -725,6 +757,10 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         return out;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        return once_differentiable(gradients(ctx, std::move(grads)), "SS2DCrossScan");
+    }
+    static torch::autograd::variable_list gradients(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        at::NoGradGuard no_grad;
         NoAutocast no_autocast;
         const auto sv = ctx->get_saved_variables();
         torch::autograd::variable_list r(13);

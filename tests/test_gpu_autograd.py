@@ -120,3 +120,41 @@ def test_layers_refuse_parameters_elsewhere(gpu_device):
         ext().block_linear(x.bfloat16(), torch.randn(4, 16, device=gpu_device), torch.randn(4), x.bfloat16())
     with pytest.raises(RuntimeError):
         snd.vss_block.TokenNorm(16)(x)
+
+
+@pytest.mark.parametrize("make,dtype", [(lambda v: (v.TokenNorm(24), nn.LayerNorm(24)), None),
+                                        (lambda v: (v.TokenLinear(24, 8), nn.Linear(24, 8)), torch.bfloat16),
+                                        (lambda v: (v.TokenLinear(24, 8, bias=False), nn.Linear(24, 8, bias=False)), torch.float16)])
+def test_second_derivatives_of_layers(gpu_device, make, dtype):
+    """create_graph through a norm or linear layer against torch's own layer in fp32."""
+    import selective_nd_scan as snd
+    torch.manual_seed(13)
+    layer, plain = (m.to(gpu_device) for m in make(snd.vss_block))
+    plain.load_state_dict(layer.state_dict())
+    x, t = torch.randn(7, 24, device=gpu_device), torch.linspace(-1, 1, plain(torch.zeros(1, 24, device=gpu_device)).shape[-1], device=gpu_device)
+    res = []
+    for m in (layer, plain):
+        xi = x.clone().requires_grad_()
+        with autocast(dtype if m is layer else None):
+            y = m(xi).float()
+        params = [xi] + list(m.parameters())
+        first = torch.autograd.grad((y + t).pow(3).sum(), params, create_graph=True)
+        res.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), params)])
+    # 16 bits: y, dy and their products are rounded on the way, three to four roundings of 2^-9 (bf16) in a term
+    for a, b in zip(*res):
+        assert rel(a, b) <= (1e-4 if dtype is None else 2e-2), rel(a, b)
+
+
+def test_second_derivative_through_the_scan_is_refused(gpu_device):
+    """Gradients under create_graph are those without it; differentiating them again raises instead of dropping terms."""
+    import selective_nd_scan as snd
+    blk = block(gpu_device)
+    x = torch.randn(1, 6, 6, 24, device=gpu_device).requires_grad_()
+    u, B = (torch.randn(1, 8, 6, 6, device=gpu_device).requires_grad_(), torch.randn(1, 4, 2, 6, 6, device=gpu_device))
+    A = -torch.ones(8, 2, device=gpu_device)
+    for leaf, f in ((x, lambda: blk(x)), (u, lambda: snd.selective_nd_scan(u, u, A, B, B, delta_softplus=True))):
+        want, = torch.autograd.grad(f().square().sum(), leaf)
+        g, = torch.autograd.grad(f().square().sum(), leaf, create_graph=True)
+        assert rel(g, want) <= 1e-5
+        with pytest.raises(RuntimeError, match="differentiated once"):
+            g.square().sum().backward()
