@@ -14,8 +14,8 @@ Because the scan origins are handled inside the kernels, every tensor stays in i
 orientation: the projections are pointwise, so no flipped (or even repeated) copy of the feature
 map is ever built - the four direction groups read the same u.
 On the GPU everything between the two outer linear layers runs in the extension (snd_block.hip: convolution + SiLU, the
-step-size projection, output norm + gate, weight gradients; the wide products are library GEMMs), forward and backward;
-elsewhere, and with another `scan_fn`, it is plain PyTorch.
+step-size projection, output norm + gate, weight gradients; the wide products are library GEMMs), forward and backward.
+Elsewhere, with another `scan_fn`, and where a stage was replaced, overridden or hooked, it is plain PyTorch.
 """
 import math
 
@@ -32,6 +32,13 @@ _FLOATS = (torch.float32, torch.bfloat16, torch.float16)
 def _autocast_like(x):
     """An empty tensor of the type a layer would compute in: autocast's, or x's own."""
     return x.new_empty(0, dtype=torch.get_autocast_dtype("cuda")) if torch.is_autocast_enabled("cuda") else x
+
+
+def _bare(module, cls):
+    """Whether calling `module` is cls.forward and nothing else: no subclass, replaced forward or hook that a kernel in its place would pass by."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_pre_hooks or module._forward_hooks or module._backward_pre_hooks or module._backward_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
 
 
 class TokenNorm(nn.LayerNorm):
@@ -92,14 +99,22 @@ class SS2DCrossScan(nn.Module):
         return (x, delta.contiguous(), A, Bs.contiguous(), Cs.contiguous(), self.Ds.float(),
                 self.dt_projs_bias.float().reshape(-1))
 
+    def _fused(self, xz):
+        """Whether the extension may stand in for what follows in forward(): every stage is still the one the constructor made."""
+        conv, norm, Di = self.conv2d, self.out_norm, self.d_inner
+        return (self.scan_fn is None and getattr(self.scan_inputs, "__func__", None) is SS2DCrossScan.scan_inputs
+                and _bare(conv, nn.Conv2d) and _bare(norm, nn.LayerNorm)
+                and (conv.kernel_size, conv.stride, conv.padding, conv.dilation, conv.padding_mode) == ((3, 3), (1, 1), (1, 1), (1, 1), "zeros")
+                and conv.in_channels == conv.out_channels == conv.groups == Di
+                and norm.normalized_shape == (Di,) and norm.weight is not None and norm.bias is not None
+                and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16 and conv.weight.is_cuda)
+
     def forward(self, x):
         """x [B, H, W, d_model] -> [B, H, W, d_model]."""
         xz = self.in_proj(x)
-        conv = self.conv2d
-        if (self.scan_fn is None and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16
-                and conv.kernel_size == (3, 3) and conv.weight.is_cuda):
-            return self.out_proj(ext().ss2d(xz, conv.weight, conv.bias, self.x_proj_weight, self.dt_projs_weight, self.dt_projs_bias, self.A_logs,
-                                            self.Ds, self.merge_weights, self.out_norm.weight, self.out_norm.bias, self.out_norm.eps))
+        if self._fused(xz):
+            return self.out_proj(ext().ss2d(xz, self.conv2d.weight, self.conv2d.bias, self.x_proj_weight, self.dt_projs_weight, self.dt_projs_bias,
+                                            self.A_logs, self.Ds, self.merge_weights, self.out_norm.weight, self.out_norm.bias, self.out_norm.eps))
         x, z = xz.chunk(2, dim=-1)
         x = F.silu(self.conv2d(x.permute(0, 3, 1, 2).contiguous()))
         u, delta, A, Bs, Cs, Ds, dt_bias = self.scan_inputs(x)
