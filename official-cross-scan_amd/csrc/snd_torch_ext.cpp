@@ -9,9 +9,11 @@
 // It does what a host binding has to do and nothing else: the reference's TORCH_CHECKs
 // (:188-245, :298-391), allocation of outputs / saved state / scratch, device guard, current-stream
 // lookup, and mapping of a non-zero library status to a c10::Error (Python RuntimeError).
+#include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
@@ -696,6 +698,24 @@ at::Tensor block_linear(const at::Tensor &x, const at::Tensor &w, const OptTenso
     return LinearFn::apply(x.to(like.scalar_type()).contiguous(), w, b);
 }
 
+// Whether kernels may stand in for torch layers on these tensors (an optional one that was not given is None): they lie on one
+// GPU and are ordinary tensors (a DTensor, FakeTensor or other subclass has no memory of its own to point to), and nothing around
+// the call has to see the layers' own calls - tracing, a function transform, a dispatch mode, a forward-mode tangent.
+bool plain(const std::vector<OptTensor> &ts) {
+    if (at::tracer::impl::is_dispatch_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return false;
+    const at::Tensor *first = nullptr;
+    for (const OptTensor &o : ts) {
+        if (!o.has_value()) continue;
+        const at::Tensor &t = o.value();
+        if (!t.is_cuda() || t.layout() != at::kStrided || t.key_set().has(c10::DispatchKey::Python) || has_tangent(t)) return false;
+        if (first && t.device() != first->device()) return false;
+        first = &t;
+    }
+    return true;
+}
+
 // Everything between in_proj and out_proj of SS2DCrossScan: xz [B, H, W, 2 * inner] -> [B, H, W, inner].
 struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
     static snd_block_shape shape_of(const at::Tensor &xz, const at::Tensor &wdt, const at::Tensor &A) {
@@ -861,6 +881,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("A_decay"), py::arg("directions"), py::arg("merge"), py::arg("merge_weights"));
     m.def("block_norm", &block_norm, "LayerNorm over the last axis, in the type of `like`", py::arg("x"), py::arg("gamma"), py::arg("beta"), py::arg("eps"), py::arg("like"));
     m.def("block_linear", &block_linear, "A linear layer in the 16-bit type of `like`", py::arg("x"), py::arg("weight"), py::arg("bias"), py::arg("like"));
+    m.def("plain", &plain, "Whether kernels may stand in for torch layers on these tensors", py::arg("tensors"));
     m.def("ss2d", &ss2d, "SS2DCrossScan between its in and out projections", py::arg("xz"), py::arg("conv_w"), py::arg("conv_b"), py::arg("x_proj"),
           py::arg("dt_proj"), py::arg("dt_bias"), py::arg("A_logs"), py::arg("D"), py::arg("merge_weights"), py::arg("gamma"), py::arg("beta"), py::arg("eps"));
     m.def("set_schedule", [](int mode) {

@@ -15,7 +15,8 @@ orientation: the projections are pointwise, so no flipped (or even repeated) cop
 map is ever built - the four direction groups read the same u.
 On the GPU everything between the two outer linear layers runs in the extension (snd_block.hip: convolution + SiLU, the
 step-size projection, output norm + gate, weight gradients; the wide products are library GEMMs), forward and backward.
-Elsewhere, with another `scan_fn`, and where a stage was replaced, overridden or hooked, it is plain PyTorch.
+Elsewhere, with another `scan_fn`, where a stage was replaced, overridden or hooked, and under tracing, function transforms,
+dispatch modes and with tensor subclasses, it is plain PyTorch.
 """
 import math
 
@@ -34,6 +35,18 @@ def _autocast_like(x):
     return x.new_empty(0, dtype=torch.get_autocast_dtype("cuda")) if torch.is_autocast_enabled("cuda") else x
 
 
+def _plain(*tensors):
+    """Whether kernels of the extension may stand in for torch layers on these tensors (None: not given)."""
+    return (not torch.compiler.is_compiling() and all(t is None or type(t) in (torch.Tensor, nn.Parameter) for t in tensors)
+            and ext().plain(tensors))
+
+
+def _layer_types(like, *params):
+    """Whether a torch layer would take these parameters: any floating type under autocast, else that of what it reads."""
+    ok = _FLOATS if torch.is_autocast_enabled("cuda") else (like,)
+    return all(p is None or p.dtype in ok for p in params)
+
+
 def _bare(module, cls):
     """Whether calling `module` is cls.forward and nothing else: no subclass, replaced forward or hook that a kernel in its place would pass by."""
     return (type(module) is cls and "forward" not in module.__dict__
@@ -45,8 +58,8 @@ class TokenNorm(nn.LayerNorm):
     """LayerNorm whose result, under autocast on the GPU, has the type the following linear layer would cast it to."""
 
     def forward(self, x):
-        if not (x.is_cuda and x.dtype in _FLOATS and self.normalized_shape == tuple(x.shape[-1:]) and x.shape[-1] <= 1024 and self.bias is not None
-                and x.numel() > 0 and self.weight.is_cuda):
+        if not (x.is_cuda and x.dtype in _FLOATS and self.normalized_shape == tuple(x.shape[-1:]) and x.shape[-1] <= 1024 and x.numel() > 0
+                and self.bias is not None and _layer_types(x.dtype, self.weight, self.bias) and _plain(x, self.weight, self.bias)):
             return super().forward(x)
         return ext().block_norm(x, self.weight, self.bias, self.eps, _autocast_like(x))
 
@@ -55,9 +68,11 @@ class TokenLinear(nn.Linear):
     """Linear layer whose weight gradient, in a 16-bit type on the GPU, is split over the tokens."""
 
     def forward(self, x):
-        like = _autocast_like(x) if x.is_cuda else x
-        if not (x.is_cuda and like.dtype in _FLOATS[1:] and x.dtype in _FLOATS and x.numel() > 0 and self.weight.is_cuda
-                and (like is not x or self.weight.dtype == x.dtype) and torch.is_grad_enabled()):
+        if not (x.is_cuda and x.dtype in _FLOATS and x.numel() > 0 and torch.is_grad_enabled() and _layer_types(x.dtype, self.weight, self.bias)
+                and _plain(x, self.weight, self.bias)):
+            return super().forward(x)
+        like = _autocast_like(x)
+        if like.dtype not in _FLOATS[1:]:
             return super().forward(x)
         return ext().block_linear(x, self.weight, self.bias, like)
 
@@ -107,7 +122,10 @@ class SS2DCrossScan(nn.Module):
                 and (conv.kernel_size, conv.stride, conv.padding, conv.dilation, conv.padding_mode) == ((3, 3), (1, 1), (1, 1), (1, 1), "zeros")
                 and conv.in_channels == conv.out_channels == conv.groups == Di
                 and norm.normalized_shape == (Di,) and norm.weight is not None and norm.bias is not None
-                and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16 and conv.weight.is_cuda)
+                and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16
+                and _layer_types(xz.dtype, conv.weight, conv.bias) and _layer_types(torch.float32, norm.weight, norm.bias)
+                and _plain(xz, conv.weight, conv.bias, self.x_proj_weight, self.dt_projs_weight, self.dt_projs_bias, self.A_logs, self.Ds,
+                           self.merge_weights, norm.weight, norm.bias))
 
     def forward(self, x):
         """x [B, H, W, d_model] -> [B, H, W, d_model]."""

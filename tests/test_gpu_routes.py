@@ -100,3 +100,72 @@ def test_untouched_block_runs_in_the_extension(gpu_device):
     assert any("Ss2dFn" in n for n in names(blk))
     P.register_parametrization(blk.op.conv2d, "weight", nn.Identity())
     assert not any("Ss2dFn" in n for n in names(blk))
+
+
+def layers(dev):
+    """A norm and a linear layer of the block, each beside torch's own with the same parameters."""
+    import selective_nd_scan as snd
+    torch.manual_seed(14)
+    for layer, plain in ((snd.vss_block.TokenNorm(24), nn.LayerNorm(24)), (snd.vss_block.TokenLinear(24, 8), nn.Linear(24, 8))):
+        for p in layer.parameters():
+            p.data.add_(0.1 * torch.randn_like(p))
+        plain.load_state_dict(layer.state_dict())
+        yield layer.to(dev, torch.bfloat16), plain.to(dev, torch.bfloat16)
+
+
+def test_layers_in_forward_mode_and_transforms(gpu_device):
+    import torch.autograd.forward_ad as fwad
+    x, t = (torch.randn(3, 5, 24, device=gpu_device, dtype=torch.bfloat16) for _ in range(2))
+    for layer, plain in layers(gpu_device):
+        with fwad.dual_level():
+            got, want = (fwad.unpack_dual(m(fwad.make_dual(x, t))).tangent for m in (layer, plain))
+        assert torch.equal(got, want)
+        assert torch.equal(torch.func.vmap(layer)(x), torch.func.vmap(plain)(x))
+        got, want = (torch.func.grad(lambda v: m(v).float().square().sum())(x) for m in (layer, plain))
+        assert torch.equal(got, want)
+
+
+def test_layers_are_seen_by_modes_tracing_and_compilers(gpu_device):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Logged(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    x = torch.randn(5, 24, device=gpu_device, dtype=torch.bfloat16)
+    for layer, name in zip((l for l, _ in layers(gpu_device)), ("layer_norm", "linear")):
+        seen = []
+        with Log():
+            want = layer(x)
+        assert any(n in s for s in seen for n in ("layer_norm", "addmm"))
+        seen = []
+        layer(x.as_subclass(Logged))
+        assert name in seen
+        traced = torch.jit.trace(layer, (x,), check_trace=False)
+        assert name in str(traced.inlined_graph)
+        assert rel(torch.compile(layer, backend="eager", fullgraph=True)(x), want) <= 1e-2
+
+
+def test_compiled_block(gpu_device):
+    blk = block(gpu_device)
+    both(torch.compile(blk, backend="eager"), blk, torch.randn(2, 9, 7, 24, device=gpu_device))
+
+
+def test_parameters_that_torch_refuses_stay_refused(gpu_device):
+    import selective_nd_scan as snd
+    x = torch.randn(5, 24, device=gpu_device)
+    with pytest.raises(RuntimeError):
+        snd.vss_block.TokenNorm(24).to(gpu_device, torch.float16)(x)
+    with pytest.raises(RuntimeError):
+        snd.vss_block.TokenLinear(24, 8).to(gpu_device, torch.float16)(x)
+    op = block(gpu_device).op
+    op.out_norm.to(torch.float16)
+    with pytest.raises(RuntimeError):
+        op(x.view(1, 1, 5, 24))
