@@ -19,7 +19,32 @@ With directions=0 every group is scanned from the top-left corner, as the refere
 (selective_scan_fwd_kernel_oflex.cuh:140).  directions=1 starts group g at corner g % 4 inside the
 kernels (no flipped copies); cross_scan.py builds the four-corner block on top of it.
 """
+import torch
+
 from ._ext import ext
+
+
+class _TracedScan(torch.autograd.Function):
+    """The scan as one operation of a graph that jit.trace records; a call into the extension alone would leave no more of itself
+    there than the allocation of its result."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        ctx.args = [a.detach().requires_grad_(a.requires_grad) if isinstance(a, torch.Tensor) else a for a in args]
+        with torch.enable_grad():
+            ctx.out = ext().scan(*ctx.args)
+        return ctx.out.detach()
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout):
+        leaves = [a for a in ctx.args if isinstance(a, torch.Tensor) and a.requires_grad]
+        grads = iter(torch.autograd.grad(ctx.out, leaves, dout, retain_graph=True, allow_unused=True))
+        return tuple(next(grads) if isinstance(a, torch.Tensor) and a.requires_grad else None for a in ctx.args)
+
+
+def _scan(*args):
+    return _TracedScan.apply(*args) if torch.jit.is_tracing() else ext().scan(*args)
 
 
 def fwd(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True, A_decay=None,
@@ -76,7 +101,7 @@ class SelectiveNdScanFn:
     @staticmethod
     def apply(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True, A_decay=None,
               directions=0):
-        return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
+        return _scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
 
 
 def selective_nd_scan(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, out_float=True,
@@ -84,7 +109,7 @@ def selective_nd_scan(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus
     """Differentiable 2D-CrossScan selective scan (forward and backward run on the HIP kernels).
     directions=1: group g of B/C (and its dim/G channels) is scanned from corner g % 4.
     Where no gradient can be asked for (no_grad, or no input that requires one) the forward saves no state."""
-    return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
+    return _scan(u, delta, A, B, C, D, delta_bias, delta_softplus, out_float, A_decay, directions, False, None)
 
 
 class SelectiveNdScanMergedFn:
@@ -93,7 +118,7 @@ class SelectiveNdScanMergedFn:
 
     @staticmethod
     def apply(u, delta, A, B, C, D, delta_bias, delta_softplus, A_decay, directions, merge_weights):
-        return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)
+        return _scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)
 
 
 def selective_nd_scan_merged(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=False, A_decay=None,
@@ -109,4 +134,4 @@ def selective_nd_scan_merged(u, delta, A, B, C, D=None, delta_bias=None, delta_s
                 raise ValueError("merge_weights must have shape [G], [G, 1] or [G, D/G]")
         elif tuple(merge_weights.shape) not in ((G, 1), (G, A.shape[0] // G)):
             raise ValueError("merge_weights must have shape [G], [G, 1] or [G, D/G]")
-    return ext().scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)
+    return _scan(u, delta, A, B, C, D, delta_bias, delta_softplus, True, A_decay, directions, True, merge_weights)

@@ -158,3 +158,29 @@ def test_second_derivative_through_the_scan_is_refused(gpu_device):
         assert rel(g, want) <= 1e-5
         with pytest.raises(RuntimeError, match="differentiated once"):
             g.square().sum().backward()
+
+
+@pytest.mark.parametrize("merged", [False, True])
+@pytest.mark.parametrize("train", [False, True])
+def test_traced_scan(gpu_device, merged, train):
+    """jit.trace records the scan as one operation, which runs on the inputs of a later call and has its gradient."""
+    import selective_nd_scan as snd
+    g = torch.Generator(device=gpu_device).manual_seed(15)
+    rn = lambda *s: torch.randn(*s, device=gpu_device, generator=g)
+    A = -torch.ones(8, 2, device=gpu_device)
+    w = torch.linspace(0.5, 2, 8, device=gpu_device).view(4, 2)
+
+    def f(u, delta, B):
+        return (snd.cross_scan_2d(u, delta, A, B, B, merge_weights=w) if merged else snd.selective_nd_scan(u, delta, A, B, B, delta_softplus=True)) + 1
+
+    def inputs(Bt):
+        return [t.requires_grad_(train) for t in (rn(Bt, 2 if merged else 8, 6, 7), rn(Bt, 8, 6, 7), rn(Bt, 4, 2, 6, 7))]
+
+    traced = torch.jit.trace(f, inputs(1), check_trace=False)
+    x = inputs(2)
+    got, want = traced(*x), f(*x)
+    assert torch.equal(got, want)
+    if train:
+        dy = rn(*want.shape)
+        for a, b in zip(torch.autograd.grad(got, x, dy), torch.autograd.grad(want, x, dy)):
+            assert rel(a, b) <= 1e-5
