@@ -169,3 +169,14 @@ def test_parameters_that_torch_refuses_stay_refused(gpu_device):
     op.out_norm.to(torch.float16)
     with pytest.raises(RuntimeError):
         op(x.view(1, 1, 5, 24))
+
+
+def test_many_images(gpu_device):
+    """More (image, direction) pairs than a grid of the block's passes has rows."""
+    blk = block(gpu_device, width=8, states=1, mlp=0.0)
+    x = torch.randn(16384, 1, 1, 8, device=gpu_device)
+    y, first = blk(x), blk(x[:16383])
+    assert rel(y[:16383], first) <= 2e-5
+    # (the gradient of a parameter behind the convolution: torch's own 3x3 backward is slow to set up at this size)
+    g, last = (torch.autograd.grad(v.square().sum(), blk.op.A_logs)[0] for v in (y, blk(x[16383:])))
+    assert rel(g, torch.autograd.grad(first.square().sum(), blk.op.A_logs)[0] + last) <= 1e-4
