@@ -581,7 +581,8 @@ void check_device(const char *what, const at::Tensor &x, std::initializer_list<a
 const float *ptr_or_null(const OptTensor &t) { return t.has_value() ? t.value().data_ptr<float>() : nullptr; }
 
 // LayerNorm over the last axis of a contiguous x, its result in `out_dtype` (what the next layer reads under autocast); gamma and
-// beta fp32.  Under create_graph its gradients are torch calls on the saved inputs, which can be differentiated again.
+// beta fp32.  Its gradients are torch calls on the saved inputs under create_graph, where they are differentiated again, and where
+// deterministic algorithms are asked for: the kernel adds up dgamma and dbeta with atomics.
 struct NormFn : public torch::autograd::Function<NormFn> {
     static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps,
                               int64_t out_dtype) {
@@ -604,7 +605,7 @@ struct NormFn : public torch::autograd::Function<NormFn> {
         if (!grads[0].defined()) return r;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         const int64_t C = x.size(-1), tokens = x.numel() / C;
-        if (at::GradMode::is_enabled()) {
+        if (at::GradMode::is_enabled() || at::globalContext().deterministicAlgorithms()) {
             const at::Tensor xf = x.to(at::kFloat), d = grads[0].to(at::kFloat), xc = xf - xf.mean(-1, true);
             const at::Tensor rstd = (xc * xc).mean(-1, true).add(ctx->saved_data["eps"].toDouble()).rsqrt(), xh = xc * rstd, dn = d * gamma;
             r[0] = (rstd * (dn - dn.mean(-1, true) - xh * (dn * xh).mean(-1, true))).to(x.scalar_type());
@@ -675,17 +676,19 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
         }
         const at::Tensor dy = grads[0].to(x.scalar_type()).contiguous().view({tokens, M}), x2 = x.view({tokens, N});
         if (ctx->needs_input_grad(0)) r[0] = at::mm(dy, w).view(x.sizes());
-        if (!graph && linear_wgrad_pays(tokens, M, N)) {
-            const int64_t nw = (M * N + 15) / 16 * 16;
+        // (edges: x, weight and, where there is one, bias)
+        const bool dw = ctx->needs_input_grad(1), db = btype >= 0 && ctx->needs_input_grad(2);
+        if (dw && !graph && !at::globalContext().deterministicAlgorithms() && linear_wgrad_pays(tokens, M, N)) {
+            const int64_t nw = (M * N + 15) / 16 * 16;     // (the kernel adds up with atomics)
             at::Tensor acc = at::zeros({nw + M}, x.options().dtype(at::kFloat));
             float *p = acc.data_ptr<float>();
-            check_status(snd_block_linear_wgrad(dy.data_ptr(), x2.data_ptr(), tokens, (int)M, (int)N, dtype_code(x.scalar_type()), p, btype >= 0 ? p + nw : nullptr,
+            check_status(snd_block_linear_wgrad(dy.data_ptr(), x2.data_ptr(), tokens, (int)M, (int)N, dtype_code(x.scalar_type()), p, db ? p + nw : nullptr,
                                                 (snd_stream_t)current_stream()), "linear");
             r[1] = acc.narrow(0, 0, M * N).view({M, N}).to(wtype);
-            if (btype >= 0) r[2] = acc.narrow(0, nw, M).to((at::ScalarType)btype);
+            if (db) r[2] = acc.narrow(0, nw, M).to((at::ScalarType)btype);
         } else {
-            r[1] = at::mm(dy.t(), x2).to(wtype);
-            if (btype >= 0) r[2] = dy.sum(0).to((at::ScalarType)btype);
+            if (dw) r[1] = at::mm(dy.t(), x2).to(wtype);
+            if (db) r[2] = dy.sum(0).to((at::ScalarType)btype);
         }
         return r;
     }

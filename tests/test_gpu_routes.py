@@ -82,24 +82,24 @@ def test_weight_pre_hook_of_the_convolution_runs(gpu_device):
     both(blk, torch_route(blk), torch.randn(2, 9, 7, 24, device=gpu_device))
 
 
+def names(y):
+    """The names of the autograd nodes behind y."""
+    seen, todo = set(), [y.grad_fn]
+    while todo:
+        f = todo.pop()
+        if f is not None and f not in seen:
+            seen.add(f)
+            todo += [g for g, _ in f.next_functions]
+    return {f.name() for f in seen}
+
+
 def test_untouched_block_runs_in_the_extension(gpu_device):
     import torch.nn.utils.parametrize as P
     x = torch.randn(2, 9, 7, 24, device=gpu_device)
-
-    def names(blk):
-        y, seen, todo = blk(x), set(), []
-        todo.append(y.grad_fn)
-        while todo:
-            f = todo.pop()
-            if f is not None and f not in seen:
-                seen.add(f)
-                todo += [g for g, _ in f.next_functions]
-        return {f.name() for f in seen}
-
     blk = block(gpu_device)
-    assert any("Ss2dFn" in n for n in names(blk))
+    assert any("Ss2dFn" in n for n in names(blk(x)))
     P.register_parametrization(blk.op.conv2d, "weight", nn.Identity())
-    assert not any("Ss2dFn" in n for n in names(blk))
+    assert not any("Ss2dFn" in n for n in names(blk(x)))
 
 
 def layers(dev):
@@ -180,3 +180,45 @@ def test_many_images(gpu_device):
     # (the gradient of a parameter behind the convolution: torch's own 3x3 backward is slow to set up at this size)
     g, last = (torch.autograd.grad(v.square().sum(), blk.op.A_logs)[0] for v in (y, blk(x[16383:])))
     assert rel(g, torch.autograd.grad(first.square().sum(), blk.op.A_logs)[0] + last) <= 1e-4
+
+
+def test_deterministic_algorithms(gpu_device):
+    """Bit for bit the same parameter gradients from run to run, in the layers and in a block around its scan."""
+    import selective_nd_scan as snd
+    lin, norm = snd.vss_block.TokenLinear(96, 384).to(gpu_device), snd.vss_block.TokenNorm(96).to(gpu_device)
+    x, dy = torch.randn(8000, 96, device=gpu_device), torch.randn(8000, 384, device=gpu_device, dtype=torch.bfloat16)
+    blk = block(gpu_device)
+    torch.use_deterministic_algorithms(True)
+    try:
+        def once():
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = lin(norm(x))
+            return torch.autograd.grad(y, list(lin.parameters()) + list(norm.parameters()), dy)
+        first = once()
+        for _ in range(5):
+            assert all(torch.equal(a, b) for a, b in zip(first, once()))
+        assert not any("Ss2dFn" in n for n in names(blk(x.view(10, 20, 40, 96)[..., :24].contiguous())))
+    finally:
+        torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("tokens,M,N", [(300, 64, 32), (300, 33, 32), (40, 1024, 1026)])
+@pytest.mark.parametrize("frozen", [(), ("weight",), ("bias",), ("weight", "bias")])
+def test_frozen_parameters_of_a_linear_layer(gpu_device, tokens, M, N, frozen):
+    """Both sides of the rule for the weight gradient; what is frozen has no gradient, the rest those of torch's layer."""
+    import selective_nd_scan as snd
+    torch.manual_seed(16)
+    layer = snd.vss_block.TokenLinear(N, M).to(gpu_device, torch.bfloat16)
+    plain = nn.Linear(N, M).to(gpu_device, torch.float32)
+    plain.load_state_dict(layer.state_dict())
+    x, dy = torch.randn(tokens, N, device=gpu_device), torch.randn(tokens, M, device=gpu_device)
+    for m in (layer, plain):
+        for n in frozen:
+            getattr(m, n).requires_grad_(False)
+    xs = [x.bfloat16().requires_grad_(), x.bfloat16().float().requires_grad_()]
+    layer(xs[0]).backward(dy.bfloat16())
+    plain(xs[1]).backward(dy.bfloat16().float())
+    assert rel(xs[0].grad, xs[1].grad) <= 5e-3          # (results in bf16: half an ulp is 2^-9)
+    for n in ("weight", "bias"):
+        a, b = getattr(layer, n).grad, getattr(plain, n).grad
+        assert (a is None) == (n in frozen) and (a is None or rel(a, b) <= 5e-3)
