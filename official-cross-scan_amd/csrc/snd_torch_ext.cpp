@@ -453,10 +453,11 @@ OptTensor optional_of(const at::Tensor &t) { return t.defined() ? OptTensor(t) :
 struct NoAutocast {
     c10::impl::ExcludeDispatchKeyGuard off{c10::autocast_dispatch_keyset};
 };
-// A tensor whose pointer goes to a kernel as `numel` elements of the type of `like`.
-void check_elements(const at::Tensor &t, const at::Tensor &like, int64_t numel, const char *what) {
-    TORCH_CHECK(t.defined() && t.scalar_type() == like.scalar_type() && t.device() == like.device() && t.is_contiguous() && t.numel() == numel,
-                "selective_nd_scan: ", what, " is not a contiguous ", toString(like.scalar_type()), " tensor of ", numel, " elements on ", like.device());
+// A tensor whose pointer goes to a kernel as `numel` elements of `type`: the result of a library call, or one saved for the
+// backward (saved-tensor hooks may hand back another than was saved).
+void check_elements(const at::Tensor &t, at::ScalarType type, const at::Device &device, int64_t numel, const char *what) {
+    TORCH_CHECK(t.defined() && t.scalar_type() == type && t.device() == device && t.is_contiguous() && t.numel() == numel,
+                "selective_nd_scan: ", what, " is not a contiguous ", toString(type), " tensor of ", numel, " elements on ", device);
 }
 
 // Gradients that come out of kernels have no graph behind them.  Under create_graph they leave through a node that raises
@@ -525,7 +526,9 @@ struct ScanFn : public torch::autograd::Function<ScanFn> {
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{u.device()};
         const at::Tensor dout = rows_contiguous(grads[0]);
         check_dout(c, u, dout, o.merge);
+        check_merge(c, o.merge, w, u);
         const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        check_elements(state, at::kFloat, u.device(), 2 * nx + c.plan.x_v_elems, "the saved state");
         const float *st = state.data_ptr<float>();
         int64_t wn = 0;
         if (w.has_value()) {
@@ -605,6 +608,9 @@ struct NormFn : public torch::autograd::Function<NormFn> {
         if (!grads[0].defined()) return r;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         const int64_t C = x.size(-1), tokens = x.numel() / C;
+        check_elements(x, x.scalar_type(), grads[0].device(), grads[0].numel(), "x");
+        check_elements(gamma, at::kFloat, x.device(), C, "gamma");
+        check_elements(stats, at::kFloat, x.device(), 2 * tokens, "the statistics");
         if (at::GradMode::is_enabled() || at::globalContext().deterministicAlgorithms()) {
             const at::Tensor xf = x.to(at::kFloat), d = grads[0].to(at::kFloat), xc = xf - xf.mean(-1, true);
             const at::Tensor rstd = (xc * xc).mean(-1, true).add(ctx->saved_data["eps"].toDouble()).rsqrt(), xh = xc * rstd, dn = d * gamma;
@@ -668,6 +674,7 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
         if (!grads[0].defined()) return r;
         at::hip::HIPGuardMasqueradingAsCUDA device_guard{x.device()};
         const int64_t M = w.size(0), N = w.size(1), tokens = x.numel() / N, btype = ctx->saved_data["b"].toInt();
+        check_elements(x, w.scalar_type(), w.device(), tokens * N, "x");
         const auto wtype = (at::ScalarType)ctx->saved_data["w"].toInt();
         const bool graph = at::GradMode::is_enabled();      // create_graph: torch calls on the inputs, which can be differentiated again
         if (graph && ctx->saved_data.count("w_in")) {       // the values of the saved copy, the history of the parameter
@@ -747,7 +754,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         check_status(snd_block_params(A_logs.data_ptr<float>(), (int)A.numel(), wx32.data_ptr<float>(), (int)(K * M), (int)Di, s.dtype, A.data_ptr<float>(),
                                       wx.data_ptr(), grad ? wxt.data_ptr() : nullptr, stream), "block");
         const at::Tensor proj = at::bmm(wx.expand({B, K * M, Di}), u.view({B, Di, HW}));                 // [B, K * (R + 2N), HW]
-        check_elements(proj, xz, B * K * M * HW, "the projection");
+        check_elements(proj, xz.scalar_type(), xz.device(), B * K * M * HW, "the projection");
         at::Tensor delta = at::empty({B, K * Di, H, W}, xz.options());
         check_status(snd_block_dt_fwd(&s, proj.data_ptr(), wdt.data_ptr<float>(), delta.data_ptr(), stream), "block");
         const at::Tensor p5 = proj.view({B, K, M, H, W}), Bs = p5.narrow(2, R, N), Cs = p5.narrow(2, R + N, N);
@@ -796,6 +803,13 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         const snd_block_shape s = shape_of(xz, wdt, A);
         const int64_t B = s.batch, H = s.nrows, W = s.ncols, Di = s.inner, K = s.n_groups, N = s.dstate, R = s.rank, M = R + 2 * N, HW = H * W;
         const at::Tensor dout = grads[0].to(xz.scalar_type()).contiguous();
+        const auto T = xz.scalar_type();
+        const struct { const at::Tensor *t; at::ScalarType type; int64_t numel; const char *what; } saved[] = {
+            {&dout, T, B * HW * Di, "the gradient"}, {&xz, T, B * HW * 2 * Di, "xz"}, {&wxt, T, Di * K * M, "the projection's weight"}, {&u, T, B * Di * HW, "u"},
+            {&pre, T, B * Di * HW, "the convolution"}, {&proj, T, B * K * M * HW, "the projection"}, {&delta, T, B * K * Di * HW, "delta"},
+            {&y, at::kFloat, B * Di * HW, "y"}, {&stats, at::kFloat, 2 * B * HW, "the statistics"}, {&conv_w, at::kFloat, Di * 9, "the convolution's weight"},
+            {&wdt, at::kFloat, K * Di * R, "the step sizes' weight"}, {&gamma, at::kFloat, Di, "gamma"}, {&beta, at::kFloat, Di, "beta"}};
+        for (const auto &v : saved) check_elements(*v.t, v.type, grads[0].device(), v.numel, v.what);
         // the accumulated parameter gradients: conv weight and bias, the two projections, gamma, beta
         const int64_t sizes[] = {Di * 9, Di, K * M * Di, K * Di * R, Di, Di};
         int64_t off[7] = {0};
@@ -808,7 +822,9 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         const at::Tensor p5 = proj.view({B, K, M, H, W}), Bs = p5.narrow(2, R, N), Cs = p5.narrow(2, R + N, N);
         Options o{true, true, SND_DIR_CORNERS, (int)ctx->saved_data["sched"].toInt(), true};
         const Checked c = check_inputs(u, delta, A, Bs, Cs, Dv, dt_bias, OptTensor());
+        check_merge(c, true, w, u);
         const int64_t nx = (c.plan.x_elems + 63) / 64 * 64;
+        check_elements(state, at::kFloat, u.device(), 2 * nx + c.plan.x_v_elems, "the saved state");
         const float *st = state.data_ptr<float>();
         int64_t wn = 0;
         if (w.has_value()) {
@@ -823,7 +839,7 @@ struct Ss2dFn : public torch::autograd::Function<Ss2dFn> {
         check_status(snd_block_wgrad(dproj.data_ptr(), K * M * HW, 0, u.data_ptr(), Di * HW, 0, (int)B, 1, (int)(K * M), (int)Di, HW, s.dtype, ap + off[2],
                                      stream), "block");
         const at::Tensor du = at::baddbmm(g.du.view({B, Di, HW}), wxt.expand({B, Di, K * M}), dproj);
-        check_elements(du, xz, B * Di * HW, "du");
+        check_elements(du, xz.scalar_type(), xz.device(), B * Di * HW, "du");
         check_status(snd_block_conv_bwd(&s, du.data_ptr(), pre.data_ptr(), xz.data_ptr(), conv_w.data_ptr<float>(), dxz.data_ptr(), ap + off[0],
                                         conv_b.has_value() ? ap + off[1] : nullptr, stream), "block");
         const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();

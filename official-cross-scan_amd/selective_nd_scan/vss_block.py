@@ -122,7 +122,7 @@ class SS2DCrossScan(nn.Module):
                 and _bare(conv, nn.Conv2d) and _bare(norm, nn.LayerNorm)
                 and (conv.kernel_size, conv.stride, conv.padding, conv.dilation, conv.padding_mode) == ((3, 3), (1, 1), (1, 1), (1, 1), "zeros")
                 and conv.in_channels == conv.out_channels == conv.groups == Di
-                and norm.normalized_shape == (Di,) and norm.weight is not None and norm.bias is not None
+                and self.dt_projs_bias.shape == (self.K, Di) and norm.normalized_shape == (Di,) and norm.weight is not None and norm.bias is not None
                 and xz.is_cuda and xz.dtype in _FLOATS and xz.numel() > 0 and self.dt_rank <= 64 and self.d_state <= 16
                 and xz.shape[0] * self.K < 65536     # (image, direction) pairs: rows of a grid
                 and _layer_types(xz.dtype, conv.weight, conv.bias) and _layer_types(torch.float32, norm.weight, norm.bias)

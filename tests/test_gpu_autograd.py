@@ -184,3 +184,38 @@ def test_traced_scan(gpu_device, merged, train):
         dy = rn(*want.shape)
         for a, b in zip(torch.autograd.grad(got, x, dy), torch.autograd.grad(want, x, dy)):
             assert rel(a, b) <= 1e-5
+
+
+def saved_through(pack, unpack, f, leaves, dy):
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        y = f()
+    return torch.autograd.grad(y, leaves, dy.to(y.dtype))
+
+
+def hooked_cases(dev):
+    """(function, leaves, gradient of the result): the scan, a block and its layers."""
+    import selective_nd_scan as snd
+    torch.manual_seed(17)
+    rn = lambda *s: torch.randn(*s, device=dev)
+    u, w, B, A = rn(1, 2, 9, 10).requires_grad_(), rn(4, 2).requires_grad_(), rn(1, 4, 6, 9, 10).requires_grad_(), -torch.rand(8, 6, device=dev) - 0.1
+    delta = rn(1, 8, 9, 10)
+    yield lambda: snd.cross_scan_2d(u, delta, A, B, B, None, None, True, w), [u, w, B], rn(1, 2, 9, 10)
+    op = block(dev).op
+    op.in_proj, op.out_proj = nn.Identity(), nn.Identity()
+    x = rn(1, 9, 10, 96).requires_grad_()
+    yield lambda: op(x), [x] + list(op.parameters()), rn(1, 9, 10, 48)
+    t = rn(30, 24).requires_grad_()
+    norm, lin = snd.vss_block.TokenNorm(24).to(dev), snd.vss_block.TokenLinear(24, 8).to(dev, torch.bfloat16)
+    yield lambda: norm(t), [t] + list(norm.parameters()), rn(30, 24)
+    yield lambda: lin(t.bfloat16()), [t] + list(lin.parameters()), rn(30, 8)
+
+
+def test_saved_tensor_hooks(gpu_device):
+    """Tensors saved to the host and brought back give the same gradients; other tensors than were saved are refused."""
+    for f, leaves, dy in hooked_cases(gpu_device):
+        want = torch.autograd.grad(f(), leaves, dy.to(f().dtype))
+        for a, b in zip(saved_through(lambda t: t.cpu(), lambda t: t.to(gpu_device), f, leaves, dy), want):
+            assert rel(a, b) <= 1e-5
+        for other in (lambda t: t.cpu(), lambda t: t.double(), lambda t: t.flatten()[: max(1, t.numel() // 2)]):
+            with pytest.raises((RuntimeError, IndexError)):
+                saved_through(lambda t: t, other, f, leaves, dy)
