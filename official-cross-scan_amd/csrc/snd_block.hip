@@ -16,9 +16,9 @@
 namespace snd {
 namespace {
 
-__device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
+__device__ __forceinline__ float silu(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float dsilu(float x) {
-    const float s = 1.f / (1.f + __expf(-x));
+    const float s = 1.f / (1.f + expf(-x));
     return s * fmaf(x, 1.f - s, 1.f);
 }
 // The value as a tensor of type T holds it.  Parameters and intermediate results are rounded where the chain of torch layers
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *
 template <typename T>
 __global__ __launch_bounds__(256) void params_kernel(const float *A_logs, int nA, const float *wx, int rows, int cols, float *A, T *w, T *wt) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < nA) A[i] = -__expf(A_logs[i]);
+    if (i < nA) A[i] = -expf(A_logs[i]);
     if (i < rows * cols) {
         stg(w, i, wx[i]);
         if (wt) {                                   // (reads spaced by a row: a few ten thousand elements, all in the L2)
