@@ -16,24 +16,27 @@ struct Job {
     void *out;
     int64_t units, per;                             // work items of the job, and items per (outer) row
     int64_t M, bytes;
-    int32_t R, kind, in_dtype, out_dtype, vec, first;   // first: the job's first block
+    int32_t R, kind, in_dtype, out_dtype, vec, split, first;    // first: the job's first block
 };
 struct Jobs { Job j[kMaxJobs]; int n; };
 
-template <typename T, int V> __device__ __forceinline__ void ld_vec(const T *p, float (&o)[V]) {
-    if constexpr (V == 1) {
-        o[0] = ldg(p, 0);
-    } else {
+// V neighbouring values as they are loaded
+template <typename T, int V> struct Held;
+template <typename T> struct Held<T, 1> {
+    float v;
+    __device__ __forceinline__ void load(const T *p) { v = ldg(p, 0); }
+    __device__ __forceinline__ void add(float (&acc)[1]) const { acc[0] += v; }
+};
+template <typename T> struct Held<T, 4> {
+    Raw4<T> q;
+    __device__ __forceinline__ void load(const T *p) { ldraw4_b(q, p, 0); }
+    __device__ __forceinline__ void add(float (&acc)[4]) const {
+        float t[4];
+        raw4_to_f32(q, t);
 #pragma unroll
-        for (int k = 0; k < V; k += 4) {
-            Raw4<T> q;
-            ldraw4_b(q, p, k * (uint32_t)sizeof(T));
-            float t[4];
-            raw4_to_f32(q, t);
-            o[k] = t[0]; o[k + 1] = t[1]; o[k + 2] = t[2]; o[k + 3] = t[3];
-        }
+        for (int k = 0; k < 4; ++k) acc[k] += t[k];
     }
-}
+};
 template <typename T, int V> __device__ __forceinline__ void st_vec(T *p, const float (&v)[V]) {
     if constexpr (V == 1) {
         stg(p, 0, v[0]);
@@ -45,23 +48,61 @@ template <typename T, int V> __device__ __forceinline__ void st_vec(T *p, const 
         }
     }
 }
-// out[o*M + i] = sum over r < R of in[(o*R + r)*M + i], added up in fp32
-template <typename TI, typename TO, int V> __device__ __forceinline__ void sum_rows(const Job &j, int64_t unit) {
-    const int64_t o = j.units >> 32 ? unit / j.per : (uint32_t)unit / (uint32_t)j.per, i = (unit - o * j.per) * V;
-    const TI *src = (const TI *)j.in + (o * j.R * j.M + i);
-    float acc[V] = {};
-    for (int r = 0; r < j.R; ++r) {
-        float v[V];
-        ld_vec<TI, V>(src + r * j.M, v);
+// out[o*M + i] = sum over r < R of in[(o*R + r)*M + i], added up in fp32.  A thread requests its rows eight (fp32: four) at a
+// time: one after the other they cost a load latency each.
+template <typename TI, int V> __device__ __forceinline__ void add_rows(const TI *src, int64_t M, int r, int r1, float (&acc)[V]) {
+    constexpr int ROWS = sizeof(TI) == 2 ? 8 : 4;   // (kept as they are loaded: 16 registers, so that waves stay at eight per SIMD)
+    for (; r + ROWS <= r1; r += ROWS) {
+        Held<TI, V> h[ROWS];
 #pragma unroll
-        for (int k = 0; k < V; ++k) acc[k] += v[k];
+        for (int q = 0; q < ROWS; ++q) h[q].load(src + (r + q) * M);
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q) h[q].add(acc);
     }
-    st_vec<TO, V>((TO *)j.out + (o * j.M + i), acc);
+#pragma unroll 1
+    for (; r < r1; ++r) {
+        Held<TI, V> h;
+        h.load(src + r * M);
+        h.add(acc);
+    }
 }
-template <typename TI, typename TO> __device__ __forceinline__ void sum_rows_v(const Job &j, int64_t unit) {
-    if (j.vec) sum_rows<TI, TO, 4>(j, unit);
-    else sum_rows<TI, TO, 1>(j, unit);
+// A thread takes a unit (V columns) with all its rows; split: a block takes kUnits units, with their rows dealt to kThreads /
+// kUnits slices that are added up in LDS (runs of 128 bytes for 16-bit values).
+constexpr int kUnits = 16, kSlices = kThreads / kUnits;
+template <typename TI, typename TO, int V> __device__ __forceinline__ void sum_rows(const Job &j, uint32_t blk, float *part) {
+    const int lane = threadIdx.x % kUnits, slice = threadIdx.x / kUnits;
+    const int64_t unit = j.split ? (int64_t)blk * kUnits + lane : (int64_t)blk * kThreads + threadIdx.x, uc = min(unit, j.units - 1);
+    const int64_t o = j.units >> 32 ? uc / j.per : (uint32_t)uc / (uint32_t)j.per, i = (uc - o * j.per) * V;
+    const TI *src = (const TI *)j.in + (o * j.R * j.M + i);
+    TO *dst = (TO *)j.out + (o * j.M + i);
+    float acc[V] = {};
+    if (!j.split) {
+        if (unit >= j.units) return;
+        add_rows<TI, V>(src, j.M, 0, j.R, acc);
+        st_vec<TO, V>(dst, acc);
+        return;
+    }
+    const int n = (j.R + kSlices - 1) / kSlices;
+    add_rows<TI, V>(src, j.M, min(slice * n, j.R), min((slice + 1) * n, j.R), acc);
+#pragma unroll
+    for (int k = 0; k < V; ++k) part[(slice * kUnits + lane) * V + k] = acc[k];
+    __syncthreads();
+    if (slice != 0 || unit >= j.units) return;
+#pragma unroll 5
+    for (int q = 1; q < kSlices; ++q)
+#pragma unroll
+        for (int k = 0; k < V; ++k) acc[k] += part[(q * kUnits + lane) * V + k];
+    st_vec<TO, V>(dst, acc);
 }
+template <typename TI, typename TO> __device__ __forceinline__ void sum_rows_v(const Job &j, uint32_t blk, float *part) {
+    if (j.vec) sum_rows<TI, TO, 4>(j, blk, part);
+    else sum_rows<TI, TO, 1>(j, blk, part);
+}
+// Where the split pays: rows enough for the slices, and units for fewer than two blocks per CU, too few to hide the latency of a
+// thread's walk.  A whole training call with one delta for all channels, one state, bf16, rows one at a time / eight at a
+// time / split, us: 64 x 3072 x 7x7 (3072 rows of 784 units) 940 / 254 / 120, 8 x 768 x 28x28 276 / 94 / 58, 64 x 384 x 56x56
+// (50176 units) 699 / 576 / 566; with a delta per group (96 rows of 200704 units) 583 / 570 / 577.
+bool split_rows(int64_t units, int rows) { return rows >= 2 * kSlices && units < (int64_t)1 << 17; }
 // Magnitude below which a merge weight enters the backward as this value (see snd_job)
 __device__ __forceinline__ float floor_weight(float w) { return fabsf(w) < SND_MERGE_WEIGHT_FLOOR ? SND_MERGE_WEIGHT_FLOOR : w; }
 
@@ -91,21 +132,23 @@ __global__ __launch_bounds__(kThreads) void jobs_kernel(const Jobs a) {
         if (threadIdx.x == 0) ((float *)j.out)[blk] = (part[0] + part[1]) + (part[2] + part[3]);
         return;
     }
+    if (j.kind == SND_JOB_SUM) {
+        __shared__ float part[kThreads * 4];
+        if (j.in_dtype == SND_F32) {
+            if (j.out_dtype == SND_F32) sum_rows_v<float, float>(j, blk, part);
+            else if (j.out_dtype == SND_BF16) sum_rows_v<float, bf16_t>(j, blk, part);
+            else sum_rows_v<float, f16_t>(j, blk, part);
+        } else if (j.in_dtype == SND_BF16) {
+            sum_rows_v<bf16_t, bf16_t>(j, blk, part);
+        } else {
+            sum_rows_v<f16_t, f16_t>(j, blk, part);
+        }
+        return;
+    }
     const int64_t unit = (int64_t)blk * kThreads + threadIdx.x;
     if (unit >= j.units) return;
-    if (j.kind == SND_JOB_WEIGHT) {
-        ((float *)j.out)[unit] = ((const float *)j.in)[unit] / floor_weight(((const float *)j.in2)[unit]);
-    } else if (j.kind == SND_JOB_WEIGHT_FLOOR) {
-        ((float *)j.out)[unit] = floor_weight(((const float *)j.in)[unit]);
-    } else if (j.in_dtype == SND_F32) {
-        if (j.out_dtype == SND_F32) sum_rows_v<float, float>(j, unit);
-        else if (j.out_dtype == SND_BF16) sum_rows_v<float, bf16_t>(j, unit);
-        else sum_rows_v<float, f16_t>(j, unit);
-    } else if (j.in_dtype == SND_BF16) {
-        sum_rows_v<bf16_t, bf16_t>(j, unit);
-    } else {
-        sum_rows_v<f16_t, f16_t>(j, unit);
-    }
+    if (j.kind == SND_JOB_WEIGHT) ((float *)j.out)[unit] = ((const float *)j.in)[unit] / floor_weight(((const float *)j.in2)[unit]);
+    else ((float *)j.out)[unit] = floor_weight(((const float *)j.in)[unit]);
 }
 
 }  // namespace
@@ -145,7 +188,9 @@ extern "C" int snd_run_jobs(const snd_job *jobs, int n, snd_stream_t stream) {
                 const int64_t units = total / (j.vec ? 4 : 1);
                 j.units = units;
                 j.per = q.cols / (j.vec ? 4 : 1);
-                nb = (units + snd::kThreads - 1) / snd::kThreads;
+                j.split = q.kind == SND_JOB_SUM && snd::split_rows(units, q.rows);
+                const int per_block = j.split ? snd::kUnits : snd::kThreads;
+                nb = (units + per_block - 1) / per_block;
             }
         }
         blocks += nb;

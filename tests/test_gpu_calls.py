@@ -37,6 +37,29 @@ def test_jobs_clear_and_sum(gpu_device, src, dst, outer, rows, cols):
     assert torch.equal(out, want.to(dst))
 
 
+@pytest.mark.parametrize("src,dst,outer,rows,cols", [
+    (torch.float32, torch.float32, 1, 31, 20), (torch.float32, torch.float32, 1, 32, 20),       # either side of the split
+    (torch.float32, torch.float32, 3, 33, 1),                                                   # a slice of one row, the last ones of none
+    (torch.float32, torch.bfloat16, 2, 129, 15 * 4), (torch.bfloat16, torch.bfloat16, 2, 100, 17 * 4),
+    (torch.float16, torch.float16, 5, 3072, 49), (torch.bfloat16, torch.bfloat16, 1, 40, ((1 << 17) - 1) * 4),
+    (torch.bfloat16, torch.bfloat16, 1, 40, (1 << 17) * 4), (torch.float32, torch.float16, 1, 8, 1000), (torch.float32, torch.float32, 2, 23, 7),
+])
+def test_jobs_sum_of_many_rows(gpu_device, src, dst, outer, rows, cols):
+    """Rows eight at a time, and dealt to the slices of a block, against float64."""
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    a = torch.randn(outer, rows, cols, device=gpu_device, generator=g).to(src)
+    out = torch.full((outer * cols + 8,), 7.0, device=gpu_device, dtype=dst)
+    dt = {torch.float32: capi.SND_F32, torch.float16: capi.SND_F16, torch.bfloat16: capi.SND_BF16}
+    capi.check(capi.lib().snd_run_jobs((capi.Job * 1)(capi.Job(a.data_ptr(), None, out.data_ptr(), outer, cols, rows, capi.JOB_SUM, dt[src], dt[dst])), 1,
+                                       torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert (out[-8:] == 7).all()
+    want = a.double().sum(1)
+    # `rows` additions of half a unit in the last place of fp32 each, and the rounding of the result
+    bound = rows * 2.0 ** -24 * a.double().abs().sum(1) + want.abs() * {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dst]
+    assert ((out[:-8].view(outer, cols).double() - want).abs() <= bound + 1e-7).all()
+
+
 @pytest.mark.parametrize("G,rg", [(4, 1), (4, 300), (8, 64)])
 def test_jobs_merge_weights(gpu_device, G, rg):
     g = torch.Generator(device=gpu_device).manual_seed(2)
