@@ -637,12 +637,21 @@ at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Te
     return NormFn::apply(x.contiguous(), f32c(gamma), f32c(beta), eps, (int64_t)like.scalar_type());
 }
 
-// A linear layer in the 16-bit type `dtype` (what autocast makes of F.linear) whose weight and bias gradients are summed over
-// the tokens by the extension's kernel where the library's product would leave most of the chip idle (linear_wgrad_pays).
-// The line lies where the library's product has blocks for half the CUs by itself: weight and bias gradient of 25088 tokens,
-// kernel of the extension / library, us: 384 x 96 20 / 119, 768 x 192 40 / 160, 1536 x 384 147 / 175 (12544 x 3072 x 768: the
-// library is ahead; few tokens cost either their launches).
-bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) { return M % 2 == 0 && N % 2 == 0 && M * N <= (int64_t)1 << 19; }
+// A linear layer in the 16-bit type of x (what autocast makes of F.linear) whose weight and bias gradients are summed over the
+// tokens by the extension's kernel where linear_wgrad_pays says so: the library's product has a block per tile of the result and
+// walks all tokens in each, the kernel splits the tokens over the grid and pays with atomics.
+// Kernel / library (product, sum over the tokens, casts), bf16, us, by tokens:
+//     M x N           784        3136       12544        32768       100352       401408
+//     768 x 384     14 / 38    20 / 48    44 /  96     96 / 183    270 / 370   1121 / 1098
+//     1024 x 512    14 / 37    27 / 48    67 / 105    158 / 202    488 / 475   1964 / 1433
+//     1536 x 384    14 / 39    28 / 53    75 / 101    180 / 207    563 / 530   2245 / 1652
+//     1024 x 768    19 / 37    33 / 49    89 / 101    218 / 228    689 / 574   2771 / 1506
+//     1024 x 1024   19 / 37    37 / 49   114 / 107    290 / 232    932 / 578   3726 / 1622
+// Up to 2^19 elements it is the kernel at any number of tokens, the last columns too: its sums are fp32, the library's result
+// is rounded to 16 bits.
+bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) {
+    return M % 2 == 0 && N % 2 == 0 && (M * N <= (int64_t)1 << 19 || (M * N <= (int64_t)3 << 18 && tokens <= 1 << 15));
+}
 struct LinearFn : public torch::autograd::Function<LinearFn> {
     static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x, const at::Tensor &w_, const OptTensor &b_) {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -222,3 +222,16 @@ def test_frozen_parameters_of_a_linear_layer(gpu_device, tokens, M, N, frozen):
     for n in ("weight", "bias"):
         a, b = getattr(layer, n).grad, getattr(plain, n).grad
         assert (a is None) == (n in frozen) and (a is None or rel(a, b) <= 5e-3)
+
+
+@pytest.mark.parametrize("tokens,M,N,kernel", [(32769, 1024, 512, True), (32768, 1026, 512, True), (32769, 1026, 512, False), (65, 1024, 768, True),
+                                               (65, 1024, 770, False), (65, 31, 34, False)])
+def test_rule_for_linear_weight_gradients(gpu_device, tokens, M, N, kernel):
+    """The kernel's sums are fp32 (1e-5 by their order), the library's result is rounded to bf16 (2^-9 at most, 1e-3 on average)."""
+    from selective_nd_scan.interface import ext
+    torch.manual_seed(18)
+    x, dy = (torch.randn(tokens, n, device=gpu_device, dtype=torch.bfloat16) for n in (N, M))
+    w, b = torch.randn(M, N, device=gpu_device).requires_grad_(), torch.randn(M, device=gpu_device).requires_grad_()
+    dw, db = torch.autograd.grad(ext().block_linear(x, w, b, x), (w, b), dy)
+    for got, want in ((dw, dy.double().t() @ x.double()), (db, dy.double().sum(0))):
+        assert rel(got, want) <= (1e-5 if kernel else 4e-3) and (kernel or rel(got, want) >= 1e-4)
