@@ -3,9 +3,9 @@
 // read once from it (halos and second passes come from the L2) and written once, in the layout its reader wants - tokens by
 // channels for the linear layers, channels by pixels for the scan - with the transposition done in LDS on the way.
 // Measured on a block of width 96 (inner 192, rank 6) at 8 x 56 x 56, bf16, us forward / backward, against the torch layers
-// they replace: convolution + SiLU 90 / 420 -> 31 / 63 (layout copies, im2col per image for the weight), projections 100 / 400
-// -> 30 / 90 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 32 / 58,
-// token norm 33 / 70 -> 9 / 26 each, weight gradient of a linear layer 93 + 20 -> 20; the block's training step 2940 -> 1616.
+// they replace: convolution + SiLU 90 / 420 -> 33 / 64 (layout copies, im2col per image for the weight), projections 100 / 400
+// -> 35 / 95 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 22 / 46,
+// token norm 33 / 70 -> 6 / 13 each, weight gradient of a linear layer 93 + 20 -> 20; the block's training step 2940 -> 1500.
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>

@@ -606,9 +606,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // The sweep runs at a raised wave priority, everything else (loads, commit to LDS, per-pixel epilogue) at the
             // default: the two waves a SIMD holds belong to two blocks, and with equal priority they drift into the same
             // phase and stall together; with the wave that is in its dependent arithmetic chain preferred, the other's
-            // memory phases fall into its gaps.  Measured (same box, backward ms): c1 1.332 -> 1.280, c2 0.339 -> 0.331,
-            // c3 1.199 -> 1.181, c4 2.765 -> 2.664; priorities 1, 2, 3 alike, the reverse assignment half as much, a fixed
-            // priority per block nothing.
+            // memory phases fall into its gaps.  Measured before the tile was swept whole (backward ms): 64 x 192 x 56x56 fp32
+            // 1.332 -> 1.280, 64 x 768 x 14x14 bf16 0.339 -> 0.331, 2 x 192 x 200x336 1.199 -> 1.181, 256 channels of 512x512
+            // 2.765 -> 2.664; priorities 1, 2, 3 alike, the reverse assignment half as much, a fixed priority per block nothing.
             __builtin_amdgcn_s_setprio(3);
 
             if (TS) {

@@ -1,4 +1,4 @@
-// Thin PyTorch-ROCm extension over the C ABI in include/snd_scan.h.
+// PyTorch-ROCm extension over the C ABI in include/snd_scan.h.
 //
 // Exports the reference's operator pair with the reference's argument and return lists
 // (kernels/selective_nd_scan/src/cusoflex/selective_scan_oflex.cpp:179-187,282 and :286-297,432-438,
@@ -6,9 +6,11 @@
 //     fwd(u, delta, A, B, C, D?, delta_bias?, delta_softplus, out_float, A_decay?) -> [out, x, x_v, x_sd]
 //     bwd(u, delta, A, B, C, D?, delta_bias?, dout, x?, x_v?, delta_softplus, A_decay?, x_sd?)
 //         -> [du, ddelta, dA, dB, dC, dD, ddelta_bias, dA_decay]
-// It does what a host binding has to do and nothing else: the reference's TORCH_CHECKs
-// (:188-245, :298-391), allocation of outputs / saved state / scratch, device guard, current-stream
-// lookup, and mapping of a non-zero library status to a c10::Error (Python RuntimeError).
+// which does what a host binding has to do: the reference's TORCH_CHECKs (:188-245, :298-391), allocation of outputs / saved
+// state / scratch, device guard, current-stream lookup, and mapping of a non-zero library status to a c10::Error (Python
+// RuntimeError).  On top of it stand the differentiable scan and, over snd_block.h, the norm and linear layers of a block and
+// everything between its projections, as native autograd functions: what they share is said at NoAutocast, check_elements
+// and once_differentiable.
 #include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>

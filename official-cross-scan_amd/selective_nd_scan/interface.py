@@ -125,8 +125,9 @@ def selective_nd_scan_merged(u, delta, A, B, C, D=None, delta_bias=None, delta_s
                              directions=1, merge_weights=None):
     """selective_nd_scan followed by the merge of the G group results of every feature, in one kernel call:
     returns [B, D/G, H, W] fp32 = sum_g merge_weights[g, i] * out[:, g*(D/G) + i].  merge_weights: None (plain
-    sum), [G], [G, 1] or [G, D/G]; differentiable.  The sum is accumulated with float atomics, so its last bits
-    depend on the order the groups arrive in."""
+    sum), [G], [G, 1] or [G, D/G]; differentiable.  The four corners of planes of up to 64 columns are added up inside a
+    block with 1-4 states, where their sums fit in its LDS; everywhere else the sum is accumulated with float atomics.
+    In either case its last bits depend on the order the groups arrive in."""
     if merge_weights is not None:
         G = B.shape[1]
         if merge_weights.dim() == 1:
