@@ -50,21 +50,26 @@ template <typename T, int V> __device__ __forceinline__ void st_vec(T *p, const 
 }
 // out[o*M + i] = sum over r < R of in[(o*R + r)*M + i], added up in fp32.  A thread requests its rows eight (fp32: four) at a
 // time: one after the other they cost a load latency each.
-template <typename TI, int V> __device__ __forceinline__ void add_rows(const TI *src, int64_t M, int r, int r1, float (&acc)[V]) {
-    constexpr int ROWS = sizeof(TI) == 2 ? 8 : 4;   // (kept as they are loaded: 16 registers, so that waves stay at eight per SIMD)
-    for (; r + ROWS <= r1; r += ROWS) {
-        Held<TI, V> h[ROWS];
+template <int ROWS, typename TI, int V> __device__ __forceinline__ void add_batch(const TI *&src, int64_t M, float (&acc)[V]) {
+    Held<TI, V> h[ROWS];                            // (kept as they are loaded: 16 registers, so that waves stay at eight per SIMD)
 #pragma unroll
-        for (int q = 0; q < ROWS; ++q) h[q].load(src + (r + q) * M);
+    for (int q = 0; q < ROWS; ++q) h[q].load(src + q * M);
 #pragma unroll
-        for (int q = 0; q < ROWS; ++q) h[q].add(acc);
+    for (int q = 0; q < ROWS; ++q) h[q].add(acc);
+    src += ROWS * M;
+}
+template <typename TI, int V> __device__ __forceinline__ void add_rows(const TI *src, int64_t M, int rows, float (&acc)[V]) {
+    constexpr int ROWS = sizeof(TI) == 2 ? 8 : 4;
+    for (; rows >= ROWS; rows -= ROWS) add_batch<ROWS, TI, V>(src, M, acc);
+    if (ROWS > 4 && rows >= 4) {
+        add_batch<4, TI, V>(src, M, acc);
+        rows -= 4;
     }
-#pragma unroll 1
-    for (; r < r1; ++r) {
-        Held<TI, V> h;
-        h.load(src + r * M);
-        h.add(acc);
+    if (rows >= 2) {
+        add_batch<2, TI, V>(src, M, acc);
+        rows -= 2;
     }
+    if (rows > 0) add_batch<1, TI, V>(src, M, acc);
 }
 // A thread takes a unit (V columns) with all its rows; split: a block takes kUnits units, with their rows dealt to kThreads /
 // kUnits slices that are added up in LDS (runs of 128 bytes for 16-bit values).
@@ -78,12 +83,13 @@ template <typename TI, typename TO, int V> __device__ __forceinline__ void sum_r
     float acc[V] = {};
     if (!j.split) {
         if (unit >= j.units) return;
-        add_rows<TI, V>(src, j.M, 0, j.R, acc);
+        add_rows<TI, V>(src, j.M, j.R, acc);
         st_vec<TO, V>(dst, acc);
         return;
     }
     const int n = (j.R + kSlices - 1) / kSlices;
-    add_rows<TI, V>(src, j.M, min(slice * n, j.R), min((slice + 1) * n, j.R), acc);
+    const int r0 = min(slice * n, j.R);
+    add_rows<TI, V>(src + r0 * j.M, j.M, min(n, j.R - r0), acc);
 #pragma unroll
     for (int k = 0; k < V; ++k) part[(slice * kUnits + lane) * V + k] = acc[k];
     __syncthreads();
