@@ -117,7 +117,8 @@ class SS2DCrossScan(nn.Module):
     def _fused(self, xz):
         """Whether the extension may stand in for what follows in forward(): every stage is still the one the constructor made."""
         conv, norm, Di = self.conv2d, self.out_norm, self.d_inner
-        return (self.scan_fn is None and not torch.are_deterministic_algorithms_enabled()    # (its parameter gradients are added up with atomics)
+        return (self.scan_fn is None and not torch.compiler.is_compiling()
+                and not torch.are_deterministic_algorithms_enabled()                 # (its parameter gradients are added up with atomics)
                 and getattr(self.scan_inputs, "__func__", None) is SS2DCrossScan.scan_inputs
                 and _bare(conv, nn.Conv2d) and _bare(norm, nn.LayerNorm)
                 and (conv.kernel_size, conv.stride, conv.padding, conv.dilation, conv.padding_mode) == ((3, 3), (1, 1), (1, 1), (1, 1), "zeros")

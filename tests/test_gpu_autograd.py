@@ -219,3 +219,13 @@ def test_saved_tensor_hooks(gpu_device):
         for other in (lambda t: t.cpu(), lambda t: t.double(), lambda t: t.flatten()[: max(1, t.numel() // 2)]):
             with pytest.raises((RuntimeError, IndexError)):
                 saved_through(lambda t: t, other, f, leaves, dy)
+
+
+@pytest.mark.parametrize("transform", [lambda f, u: torch.func.grad(lambda v: f(v).sum())(u), lambda f, u: torch.func.vmap(f)(u[None]),
+                                       lambda f, u: torch.func.jvp(f, (u,), (torch.ones_like(u),))])
+def test_function_transforms_of_the_scan_are_refused(gpu_device, transform):
+    import selective_nd_scan as snd
+    u, B = torch.randn(1, 8, 6, 6, device=gpu_device), torch.randn(1, 4, 2, 6, 6, device=gpu_device)
+    A = -torch.ones(8, 2, device=gpu_device)
+    with pytest.raises(RuntimeError):
+        transform(lambda v: snd.selective_nd_scan(v, u, A, B, B), u)
