@@ -55,13 +55,21 @@ def _bare(module, cls):
 
 
 class TokenNorm(nn.LayerNorm):
-    """LayerNorm whose result, under autocast on the GPU, has the type the following linear layer would cast it to."""
+    """LayerNorm.  narrow: under autocast on the GPU its result has autocast's type instead of float32, for a reader that casts it to that."""
 
-    def forward(self, x):
+    def forward(self, x, narrow=False):
         if not (x.is_cuda and x.dtype in _FLOATS and self.normalized_shape == tuple(x.shape[-1:]) and x.shape[-1] <= 1024 and x.numel() > 0
                 and self.bias is not None and _layer_types(x.dtype, self.weight, self.bias) and _plain(x, self.weight, self.bias)):
             return super().forward(x)
-        return ext().block_norm(x, self.weight, self.bias, self.eps, _autocast_like(x))
+        like = _autocast_like(x) if narrow else x.new_empty(0, dtype=torch.float32) if torch.is_autocast_enabled("cuda") else x
+        return ext().block_norm(x, self.weight, self.bias, self.eps, like)
+
+
+def _normed(norm, x, *readers):
+    """norm(x); narrow if the modules that take its result on its way, `readers`, are the constructor's and end in a linear layer."""
+    if torch.is_autocast_enabled("cuda") and _bare(norm, TokenNorm) and all(_bare(m, cls) for m, cls in readers):
+        return norm(x, True)
+    return norm(x)
 
 
 class TokenLinear(nn.Linear):
@@ -162,7 +170,9 @@ class VSSBlock(nn.Module):
             self.mlp = nn.Sequential(TokenLinear(d_model, hidden), nn.GELU(), TokenLinear(hidden, d_model))
 
     def forward(self, x):
-        x = x + self.op(self.norm(x))
-        if self.mlp is not None:
-            x = x + self.mlp(self.norm2(x))
+        op, mlp = self.op, self.mlp
+        x = x + op(_normed(self.norm, x, (op, SS2DCrossScan), (getattr(op, "in_proj", None), TokenLinear)))
+        if mlp is not None:
+            first = mlp[0] if type(mlp) is nn.Sequential and len(mlp) > 0 else None
+            x = x + mlp(_normed(self.norm2, x, (mlp, nn.Sequential), (first, TokenLinear)))
         return x

@@ -235,3 +235,38 @@ def test_rule_for_linear_weight_gradients(gpu_device, tokens, M, N, kernel):
     dw, db = torch.autograd.grad(ext().block_linear(x, w, b, x), (w, b), dy)
     for got, want in ((dw, dy.double().t() @ x.double()), (db, dy.double().sum(0))):
         assert rel(got, want) <= (1e-5 if kernel else 4e-3) and (kernel or rel(got, want) >= 1e-4)
+
+
+def test_norms_are_float32_where_somebody_else_reads_them(gpu_device):
+    """Under autocast a norm's result is rounded to 16 bits only for a linear layer that would do so itself."""
+    import selective_nd_scan as snd
+    x = torch.randn(2, 9, 7, 24, device=gpu_device)
+
+    def run(blk):
+        seen = {}
+        for n, m in (("op", blk.op), ("mlp", blk.mlp)):
+            m.register_forward_pre_hook(lambda mod, i, n=n: seen.update({n: i[0].dtype}))
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = blk(x)
+        return y, seen
+
+    blk = block(gpu_device)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert blk.norm(x).dtype == torch.float32 and blk.norm(x, True).dtype == torch.bfloat16
+        plain = blk(x)
+    y, seen = run(blk)
+    assert seen == dict(op=torch.float32, mlp=torch.float32) and torch.equal(y, plain)
+    blk = block(gpu_device)
+    inner = blk.op.in_proj
+    got = []
+
+    class Wide(nn.Module):                           # a projection that keeps to float32
+        def forward(self, v):
+            got.append(v.dtype)
+            with torch.autocast("cuda", enabled=False):
+                return inner(v.float())
+
+    blk.op.in_proj = Wide()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        blk(x)
+    assert got == [torch.float32]
