@@ -35,6 +35,13 @@
 
 namespace snd {
 
+// Pitch of the arrays that only the staging and the epilogue touch: with 16 states the 8x8 tiles leave LDS for no padding.
+constexpr int bwd_pcs(int NP, int TE) { return kTile + (NP == 16 && TE == 8 ? 0 : NP < 8 ? NP : 8); }
+// Exchange the upper 32 lanes of a with the lower 32 of b.
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+
 // Sum two sets of four values over the four 16-lane rows of a wave (its four channels when a row
 // holds the 16 states of one channel): a reduce-scatter, row q of the wave ends with the totals of
 // b[q] (in b0) and c[q] (in c0).  v_permlane32_swap exchanges the upper 32 lanes of its first
@@ -61,6 +68,36 @@ __device__ __forceinline__ void rows_scatter4x2(float &b0, float &b1, float &b2,
                  "v_add_f32 %4, %4, %5\n\t"
                  : "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3), "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3));
 }
+// The two reductions of a half row in one block, for the 16-lane layout: group_scatter8 over q0..q3, p0..p3 (sums over the
+// channel's 16 states) and rows_scatter4x2 over b0..b3, c0..c3 (sums over the wave's four channels).  The steps of one fill the
+// slots that the other would spend on s_nops (a wave issues an s_nop as slowly as a multiply-add); both distances named above
+// hold for every operand.
+__device__ __forceinline__ void sweep_reduce16(float &q0, float &q1, float &q2, float &q3, float &p0, float &p1, float &p2, float &p3,
+                                               float &b0, float &b1, float &b2, float &b3, float &c0, float &c1, float &c2, float &c3) {
+    asm volatile("s_nop 1\n\t"
+                 SND_DPPA("%0", "%0", "row_ror:8", "0x3") SND_DPPA("%1", "%1", "row_ror:8", "0x3")
+                 SND_DPPA("%2", "%2", "row_ror:8", "0x3") SND_DPPA("%3", "%3", "row_ror:8", "0x3")
+                 SND_DPPA("%0", "%4", "row_ror:8", "0xc") SND_DPPA("%1", "%5", "row_ror:8", "0xc")
+                 SND_DPPA("%2", "%6", "row_ror:8", "0xc") SND_DPPA("%3", "%7", "row_ror:8", "0xc")
+                 "v_permlane32_swap_b32 %8, %10\n\t"
+                 "v_permlane32_swap_b32 %9, %11\n\t"
+                 "v_permlane32_swap_b32 %12, %14\n\t"
+                 "v_permlane32_swap_b32 %13, %15\n\t"
+                 SND_DPPA("%0", "%0", "row_shl:4", "0x5") SND_DPPA("%1", "%1", "row_shl:4", "0x5")
+                 SND_DPPA("%0", "%2", "row_shr:4", "0xa") SND_DPPA("%1", "%3", "row_shr:4", "0xa")
+                 "v_add_f32 %8, %8, %10\n\t"
+                 "v_add_f32 %9, %9, %11\n\t"
+                 "v_add_f32 %12, %12, %14\n\t"
+                 "v_add_f32 %13, %13, %15\n\t"
+                 SND_DPPA("%0", "%0", "quad_perm:[1,0,3,2]", "0xf") SND_DPPA("%1", "%1", "quad_perm:[1,0,3,2]", "0xf")
+                 "v_permlane16_swap_b32 %8, %9\n\t"
+                 "v_permlane16_swap_b32 %12, %13\n\t"
+                 SND_DPPA("%0", "%0", "quad_perm:[2,3,0,1]", "0xf") SND_DPPA("%1", "%1", "quad_perm:[2,3,0,1]", "0xf")
+                 "v_add_f32 %8, %8, %9\n\t"
+                 "v_add_f32 %12, %12, %13\n\t"
+                 : "+v"(q0), "+v"(q1), "+v"(q2), "+v"(q3), "+v"(p0), "+v"(p1), "+v"(p2), "+v"(p3), "+v"(b0), "+v"(b1), "+v"(b2),
+                   "+v"(b3), "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3));
+}
 // VEC: the tile's inputs are staged, and du / ddelta stored, four columns at a time with one 16-byte (fp32) or
 // 8-byte (16-bit) access per thread and tensor instead of one access per element - a quarter of the memory
 // instructions and of their address arithmetic.  Needs 8x8 tiles, a width that is a multiple of four and tensors
@@ -82,7 +119,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // consecutive banks.  NSD: the dB/dC partial sums, which the 16-lane row q of a wave writes at element q of
     // a state's tile row, so states must start 2 (16 states) or 4 banks apart.
     constexpr int PCH = kTile + (NP == 16 ? 8 : 4);
-    constexpr int PCS = kTile + (NP < 8 ? NP : 8);
+    constexpr int PCS = bwd_pcs(NP, TE);
     constexpr int NSD = NP == 16 ? kTile + 2 : kTile + 4;
     constexpr int NBC = 4;
     constexpr int NPX = kTile / NP;
@@ -110,11 +147,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     float *sSg = sDo + CB * PCH;                    // [CB][PCS] d softplus / d raw
     float *sP = sSg + CB * PCS + 4;                 // sum_n A*da*a (4 banks off sQ: a wave writes both in one instruction)
     float *sHold = sP + CB * PCH;                   // dB, dC sums of a pair's right tile, [2][NP][kTile]
-    // (TS) sum over a wave's channels of dout * delta' * u / 4, [WPB][kTile], and sum over the states of B*C / 4, [kTile]: where
-    // sHold is, which 7x7 tiles have no use for
-    constexpr bool TS = TE == 7;
-    float *sT = sHold, *sS = sT + WPB * kTile;
-    float *sRed = sHold + 2 * NP * kTile;           // [WPB]
+    // sum over a wave's channels of dout * delta' * u / 4, [WPB][kTile], and sum over the states of B*C / 4, [kTile] (7x7 tiles
+    // have no use for sHold)
+    float *sT = TE == 7 ? sHold : sHold + 2 * NP * kTile, *sS = sT + WPB * kTile;
+    float *sRed = sS + kTile;                       // [WPB]
 
     const snd_fwd_params &f = p.f;
     const snd_shape &sh = f.shape;
@@ -230,9 +266,11 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     float *mydB = sdB + wave * NP * NSD + n * NSD;
     float *mydC = sdC + wave * NP * NSD + n * NSD;
     const int qrow = (tid & 63) >> 4;               // 16-lane row of this lane inside its wave
+    float *myQP = ((n & 8) ? sP : sQ) + cl * PCH + ((n >> 1) & 2);   // (16 lanes) where this lane's quad leaves its sums over the states
 
-    // ---- register staging of one tile's raw inputs (loaded at the start of the tile, then committed to LDS)
-    float qb[VEC ? 1 : NBC], qc[VEC ? 1 : NBC], qdl[VEC ? 1 : NPX], qu[VEC ? 1 : NPX], qdo[VEC ? 1 : NPX], qh[VEC ? 1 : NHK];
+    // ---- register staging of one tile's inputs: loaded in the second half of the sweep of the tile before, as they are, masked
+    // and converted where they are committed to LDS
+    uint32_t qb[VEC ? 1 : NBC], qc[VEC ? 1 : NBC], qdl[VEC ? 1 : NPX], qu[VEC ? 1 : NPX], qdo[VEC ? 1 : NPX], qh[VEC ? 1 : NHK];
     Raw4<T> vb, vc, vdl[VEC ? NCH : 1], vu[VEC ? NCH : 1];     // (VEC) one chunk of B and C, NCH chunks of delta, u, dout
     uint32_t vdo[VEC ? NCH : 1][4];
     uint32_t vh[VEC ? NHV : 1];
@@ -242,20 +280,28 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
         else if (hidx < 16) { rr = TE; jj = hidx - 8; }
         else { rr = hidx - 16; jj = -1; }
     };
-    auto prefetch = [&](int I, int J) {
+    // (element-wise) cell k of the ring around the tile in the delta' grid, its coordinates relative to the tile
+    auto ring_cell = [&](int hidx, int &rr, int &jj) {
+        if (hidx < TE + 2) { rr = -1; jj = hidx - 1; }
+        else if (hidx < 2 * TE + 4) { rr = TE; jj = hidx - (TE + 3); }
+        else if (hidx < 3 * TE + 4) { rr = hidx - (2 * TE + 4); jj = -1; }
+        else { rr = hidx - (3 * TE + 4); jj = TE; }
+    };
+    // Loads are always in bounds (clamped coordinates); commit() zeroes what lies outside the plane, the tile (7x7 tiles) and the
+    // state / channel ranges.  part 0: B and C, 1: delta and u, 2: dout and the halo of delta.
+    auto load_part = [&](int I, int J, int part) __attribute__((always_inline)) {
         const int r0 = I * TE, j0 = J * TE;
         // The thread's element maps are re-derived here from an opaque copy of the thread id, so that
         // they are a few integer ops per tile instead of dozens of registers kept live across the tile.
         SND_THREAD_MAPS(NP);
         if constexpr (VEC) {
-            // loads are always in bounds (clamped coordinates); commit() zeroes what lies outside the plane.
             // Chunk q of a tile = row q / 2, columns 4 * (q % 2) .. + 3; under a mirrored column order the same four
             // memory columns in reverse (the chunk then starts at the memory column of its last scan column).
             auto chunk_off = [&](int q, int hB, int esz) {
                 const int row = min(r0 + (q >> 1), H - 1), col = min(j0 + (q & 1) * 4, W - 4);
                 return (uint32_t)mad24(mrow(row), hB, mcol(col + (fh ? 3 : 0)) * esz);
             };
-            {
+            if (part == 0) {
                 const int sn = min(t_ >> 4, N - 1), q = t_ & 15;
                 ldraw4_b(vb, Bb, (uint32_t)sn * (uint32_t)BsB + chunk_off(q, BhB, ESZ));   // (below 2^32: bwd_vec_ok)
                 ldraw4_b(vc, Cb, (uint32_t)sn * (uint32_t)CsB + chunk_off(q, ChB, ESZ));
@@ -263,65 +309,56 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
             for (int k = 0; k < NCH; ++k) {
                 const int q = n + NP * k;
-                ldraw4_b(vdl[k], db, cDb + chunk_off(q, DhB, ESZ));
-                ldraw4_b(vu[k], ub, cUb + chunk_off(q, UhB, ESZ));
-                const char *src = (const char *)dob + (cDob + chunk_off(q, DohB, esz_do));
-                if (sizeof(T) == 4 || sh_do == 2) {
-                    const uint4 v = *(const uint4 *)src;
-                    vdo[k][0] = v.x; vdo[k][1] = v.y; vdo[k][2] = v.z; vdo[k][3] = v.w;
-                } else {
-                    const uint2 v = *(const uint2 *)src;
-                    vdo[k][0] = v.x; vdo[k][1] = v.y;
+                if (part == 1) {
+                    ldraw4_b(vdl[k], db, cDb + chunk_off(q, DhB, ESZ));
+                    ldraw4_b(vu[k], ub, cUb + chunk_off(q, UhB, ESZ));
+                } else if (part == 2) {
+                    const char *src = (const char *)dob + (cDob + chunk_off(q, DohB, esz_do));
+                    if (sizeof(T) == 4 || sh_do == 2) {
+                        const uint4 v = *(const uint4 *)src;
+                        vdo[k][0] = v.x; vdo[k][1] = v.y; vdo[k][2] = v.z; vdo[k][3] = v.w;
+                    } else {
+                        const uint2 v = *(const uint2 *)src;
+                        vdo[k][0] = v.x; vdo[k][1] = v.y;
+                    }
                 }
             }
 #pragma unroll
-            for (int k = 0; k < NHV; ++k) {
+            for (int k = 0; k < (part == 2 ? NHV : 0); ++k) {
                 int rr, jj;
                 halo_cell(n + NP * k, rr, jj);
                 const int row = min(max(r0 + rr, 0), H - 1), col = min(max(j0 + jj, 0), W - 1);
                 vh[k] = ldraw_b(db, cDb + mad24(mrow(row), DhB, mcol(col) * ESZ));
             }
-            return;
-        }
-        // loads are always in bounds (clamped coordinates); values outside the plane become zero
-        {
-            const int row = r0 + pr, col = j0 + pj;
-            const bool in = pr < TE && pj < TE && row < H && col < W;
-            const int mr = mrow(min(row, H - 1)), mcB = mcol(min(col, W - 1)) * ESZ;
-            const uint32_t ob = mad24(mr, BhB, mcB), oc = mad24(mr, ChB, mcB);
+        } else {
+            if (part == 0) {
+                const int mr = mrow(min(r0 + pr, H - 1)), mcB = mcol(min(j0 + pj, W - 1)) * ESZ;
+                const uint32_t ob = mad24(mr, BhB, mcB), oc = mad24(mr, ChB, mcB);
 #pragma unroll
-            for (int k = 0; k < NBC; ++k) {
-                const int sn = wave_u + WPB * k, sc = min(sn, N - 1);       // scalar: folded into the base
-                const float vb_ = ldg_b((const T *)((const char *)Bb + sc * BsB), ob);
-                const float vc_ = ldg_b((const T *)((const char *)Cb + sc * CsB), oc);
-                qb[k] = (in && sn < N) ? vb_ : 0.f;
-                qc[k] = (in && sn < N) ? vc_ : 0.f;
+                for (int k = 0; k < NBC; ++k) {
+                    const int sc = min(wave_u + WPB * k, N - 1);            // scalar: folded into the base
+                    qb[k] = ldraw_b((const T *)((const char *)Bb + sc * BsB), ob);
+                    qc[k] = ldraw_b((const T *)((const char *)Cb + sc * CsB), oc);
+                }
             }
-        }
 #pragma unroll
-        for (int k = 0; k < NPX; ++k) {
-            const int pp = n + NP * k;
-            const int row = r0 + (pp >> 3), col = j0 + (pp & 7);
-            const bool ok = cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W;
-            const int mr = mrow(min(row, H - 1)), mc = mcol(min(col, W - 1));
-            const float vd = ldg_b(db, cDb + mad24(mr, DhB, mc * ESZ)), vu_ = ldg_b(ub, cUb + mad24(mr, UhB, mc * ESZ));
-            const float vo = ld_f32_b(dob, cDob + mad24(mr, DohB, mc << sh_do), p.dout_dtype);
-            qdl[k] = ok ? vd : 0.f;
-            qu[k] = ok ? vu_ : 0.f;
-            qdo[k] = ok ? vo : 0.f;
-        }
+            for (int k = 0; k < NPX; ++k) {
+                const int pp = n + NP * k;
+                const int mr = mrow(min(r0 + (pp >> 3), H - 1)), mc = mcol(min(j0 + (pp & 7), W - 1));
+                if (part == 1) {
+                    qdl[k] = ldraw_b(db, cDb + mad24(mr, DhB, mc * ESZ));
+                    qu[k] = ldraw_b(ub, cUb + mad24(mr, UhB, mc * ESZ));
+                } else if (part == 2) {
+                    const char *src = (const char *)dob + (cDob + mad24(mr, DohB, mc << sh_do));
+                    qdo[k] = sizeof(T) == 4 || sh_do == 2 ? *(const uint32_t *)src : (uint32_t)*(const uint16_t *)src;
+                }
+            }
 #pragma unroll
-        for (int k = 0; k < NHK; ++k) {   // the ring of halo cells around the tile in the delta' grid
-            const int hidx = n + NP * k;
-            int rr, jj;
-            if (hidx < TE + 2) { rr = 0; jj = hidx; }
-            else if (hidx < 2 * TE + 4) { rr = TE + 1; jj = hidx - (TE + 2); }
-            else if (hidx < 3 * TE + 4) { rr = hidx - (2 * TE + 3); jj = 0; }
-            else { rr = hidx - (3 * TE + 3); jj = TE + 1; }
-            const int row = r0 - 1 + rr, col = j0 - 1 + jj;
-            const bool ok = cvalid && hidx < NHALO && row >= 0 && row < H && col >= 0 && col < W;
-            const float vd = ldg_b(db, cDb + mad24(mrow(min(max(row, 0), H - 1)), DhB, mcol(min(max(col, 0), W - 1)) * ESZ));
-            qh[k] = ok ? vd : 0.f;
+            for (int k = 0; k < (part == 2 ? NHK : 0); ++k) {
+                int rr, jj;
+                ring_cell(n + NP * k, rr, jj);
+                qh[k] = ldraw_b(db, cDb + mad24(mrow(min(max(r0 + rr, 0), H - 1)), DhB, mcol(min(max(j0 + jj, 0), W - 1)) * ESZ));
+            }
         }
     };
     auto commit = [&](int I, int J) {
@@ -385,37 +422,42 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             return;
         }
+        const int r0 = I * TE, j0 = J * TE;
+        {
+            const bool in = pr < TE && pj < TE && r0 + pr < H && j0 + pj < W;
 #pragma unroll
-        for (int k = 0; k < NBC; ++k) {
-            const int sn = wave + WPB * k;
-            sB[sn * NSTR + px] = qb[k];
-            sC[sn * NSTR + px] = qc[k];
+            for (int k = 0; k < NBC; ++k) {
+                const int sn = wave + WPB * k;
+                const bool ok = in && wave_u + WPB * k < N;
+                sB[sn * NSTR + px] = ok ? raw_to_f32((const T *)nullptr, qb[k]) : 0.f;
+                sC[sn * NSTR + px] = ok ? raw_to_f32((const T *)nullptr, qc[k]) : 0.f;
+            }
         }
 #pragma unroll
         for (int k = 0; k < NPX; ++k) {
             const int pp = n + NP * k;
-            const float raw = qdl[k] + bias;
+            const bool ok = cvalid && (pp >> 3) < TE && (pp & 7) < TE && r0 + (pp >> 3) < H && j0 + (pp & 7) < W;
+            const float raw = (ok ? raw_to_f32((const T *)nullptr, qdl[k]) : 0.f) + bias, u_ = ok ? raw_to_f32((const T *)nullptr, qu[k]) : 0.f;
+            const float do_ = sizeof(T) == 4 || sh_do == 2 ? __builtin_bit_cast(float, qdo[k]) : raw_to_f32((const T *)nullptr, qdo[k]);
             float dsp = 1.f;
             const float dl = softplus ? softplus20(raw, dsp) : raw;
             if (TE == 8 || ((pp >> 3) < TE && (pp & 7) < TE))     // slots beyond the tile belong to the halo ring
                 sDl[cl * DLP + ((pp >> 3) + 1) * HG + DLO + (pp & 7)] = dl;
-            sDu[cl * PCH + pp] = dl * qu[k];
-            sU[cl * PCS + pp] = qu[k];
-            sDo[cl * PCH + pp] = wm * qdo[k];
+            sDu[cl * PCH + pp] = dl * u_;
+            sU[cl * PCS + pp] = u_;
+            sDo[cl * PCH + pp] = ok ? wm * do_ : 0.f;
             sSg[cl * PCS + pp] = dsp;
         }
 #pragma unroll
         for (int k = 0; k < NHK; ++k) {
             const int hidx = n + NP * k;
             int rr, jj;
-            if (hidx < TE + 2) { rr = 0; jj = hidx; }
-            else if (hidx < 2 * TE + 4) { rr = TE + 1; jj = hidx - (TE + 2); }
-            else if (hidx < 3 * TE + 4) { rr = hidx - (2 * TE + 3); jj = 0; }
-            else { rr = hidx - (3 * TE + 3); jj = TE + 1; }
-            const float raw = qh[k] + bias;
+            ring_cell(hidx, rr, jj);
+            const bool ok = cvalid && hidx < NHALO && r0 + rr >= 0 && r0 + rr < H && j0 + jj >= 0 && j0 + jj < W;
+            const float raw = (ok ? raw_to_f32((const T *)nullptr, qh[k]) : 0.f) + bias;
             float dsp;
-            if (hidx < NHALO && DLO - 1 + jj < HG)      // (the column right of an 8-column tile is never read)
-                sDl[cl * DLP + rr * HG + DLO - 1 + jj] = softplus ? softplus20(raw, dsp) : raw;
+            if (hidx < NHALO && DLO + jj < HG)          // (the column right of an 8-column tile is never read)
+                sDl[cl * DLP + (rr + 1) * HG + DLO + jj] = softplus ? softplus20(raw, dsp) : raw;
         }
     };
 #define DL(r, j) myDl[((r) + 1) * HG + DLO + (j)]
@@ -435,44 +477,39 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // beside dD, at no cost in the sweep.
     float dw_acc = 0.f;
 
-    // dB, dC of a tile leave the block (summed over its channels) one tile late, from the partial sums that stay
-    // in LDS until the next sweep: between the requests for the next tile's inputs and the wait for them, so that the
-    // LDS reads and the address arithmetic of the flush fall under the latency of those loads (B=64, D=192, 56x56:
-    // 1.290 -> 1.258 ms against the flush behind the wait; with the
-    // sums in front of the wait and the atomics behind it the eight values kept across the wait are spilled and
-    // nothing more is gained, and the per-pixel epilogue moved to the same place gains nothing either).
-    // (TS) The terms in dout*C/4 and bu/4 are left out of the sweep: summed over channels (states) they are products of B or C
+    // dB, dC of a tile leave the block (summed over its channels) one tile late, from the partial sums that stay in LDS until the
+    // next sweep, ahead of the commit of the next tile's inputs.  (A state at a time between the rows of the recomputation, where
+    // arithmetic could cover it, it needs a block barrier in front of the sweep: 64 x 192 x 56x56 1.10 ms either way, 2 x 192 x 200x336
+    // 0.945 -> 0.960, 32 x 768 x 28x28 bf16 0.584 -> 0.606.)
+    // The terms in dout*C/4 and bu/4 are left out of the sweep: summed over channels (states) they are products of B or C
     // with per-pixel sums that all states (channels) share,
     //     dB: C * T,  dC: B * T,  T = sum_c dout*delta'*u / 4        sum_n dbu*B: dout * S,  S = sum_n B*C / 4
-    // That and s - bu = a * s[left] take four instructions per cell out of the sweep.  Only where the eight registers B and C of
-    // the flushed tile take until then are free: 7x7 tiles (64 x 768 x 14x14 bf16 312 -> 303 us, 32 x 768 x 28x28 609 -> 600);
-    // 8x8 tiles spill 12 to 14 registers and lose 4 %.  (All schedules alike, so that their results agree bit for bit; in a
-    // pipeline of two strips the sums in front of the sweep cost as much as it saves: 2 x 384 x 14x14 33.9 -> 34.4 us.)
-    float pB[TS ? NBC : 1], pC[TS ? NBC : 1];       // this thread's B, C of that tile
+    // That and s - bu = a * s[left] take four instructions per cell out of the sweep.
+    // (All schedules alike, so that their results agree bit for bit.)
+    float pB[NBC], pC[NBC];                         // this thread's B, C of that tile
     int pI = -1, pJ = 0;                            // the tile whose partial sums are still in LDS
-    auto flush_bc = [&](int I_, int J_) __attribute__((always_inline)) {
+    // Two neighbouring 8x8 tiles leave together: the right one's sums are held in LDS and joined to the left one's, so that an
+    // instruction adds 4 rows x 16 columns instead of 8 rows x 8.  An atomic costs its CU 12 ns per 64-byte line it
+    // touches, however few of the line's words it adds to (2 x 192 x 200x336: 1.09 -> 1.07 ms, 256 channels of 512x512:
+    // 2.56 -> 2.51 ms; rows that are no multiple of 64 bytes gain nothing, 7x7 tiles lose 2 % and keep the plain form).
+    // Lanes outside the plane get an offset that the buffer's range check drops: no branch around an atomic.
+    auto flush_bc = [&]() __attribute__((always_inline)) {
         SND_THREAD_MAPS(NP);
-        // Two neighbouring 8x8 tiles leave together: the right one's sums are held in LDS and joined to the left one's, so that an
-        // instruction adds 4 rows x 16 columns instead of 8 rows x 8.  An atomic costs its CU 12 ns per 64-byte line it
-        // touches, however few of the line's words it adds to (2 x 192 x 200x336: 1.09 -> 1.07 ms, 256 channels of 512x512:
-        // 2.56 -> 2.51 ms; rows that are no multiple of 64 bytes gain nothing, 7x7 tiles lose 2 % and keep the plain form).
-        const bool holds = TE == 8 && (J_ & 1) && J_ > J_lo, joins = TE == 8 && !(J_ & 1) && J_ < J_hi;
-        const int row = I_ * TE + pr, col = J_ * TE + pj;
-        const bool in = pr < TE && pj < TE && row < H && col < W;
-        const uint32_t o = mad24(mrow(row), W4, mcol(col) * 4);
-        // (joined) lane l: row l / 16 (+ 4), column l % 16 of the pair
-        const int jc = px & 7, jr = px >> 4;
-        const bool right = px & 8;
-        const int jcol = (J_ + (right ? 1 : 0)) * TE + jc;
+        const bool holds = TE == 8 && (pJ & 1) && pJ > J_lo, joins = TE == 8 && !(pJ & 1) && pJ < J_hi;
+        // plain: lane l adds row l / 8, column l % 8; joined: row (l / 8) % 4 (+ 4), column l % 8 of the left (lanes 0-31) or right tile
+        const int row = pI * TE + (joins ? pr & 3 : pr), col = (pJ + (joins ? px >> 5 : 0)) * TE + pj;
+        const bool in = pr < TE && pj < TE && col < W;
+        const int cB = mcol(col) * 4;
+        const uint32_t o0 = in && row < H ? (uint32_t)mad24(mrow(row), W4, cB) : kBufOOB;
+        const uint32_t o4 = in && row + 4 < H ? (uint32_t)mad24(mrow(row + 4), W4, cB) : kBufOOB;
         float tsum = 0.f;
-        if (TS) {
 #pragma unroll
-            for (int w = 0; w < WPB; ++w) tsum += sT[w * kTile + px];
-        }
+        for (int w = 0; w < WPB; ++w) tsum += sT[w * kTile + px];
 #pragma unroll
         for (int k = 0; k < NBC; ++k) {
-            const int sn = wave_u + WPB * k;                        // scalar: folded into the base
-            float tb = TS ? pC[TS ? k : 0] * tsum : 0.f, tc = TS ? pB[TS ? k : 0] * tsum : 0.f;
+            int sn = wave_u + WPB * k;              // scalar: folded into the base
+            asm volatile("" : "+s"(sn));            // (not eight descriptors kept across the tile loop)
+            float tb = pC[k] * tsum, tc = pB[k] * tsum;
 #pragma unroll
             for (int w = 0; w < NPART; ++w) {
                 tb += sdB[w * PART + sn * NSD + px];
@@ -481,26 +518,50 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             if (holds) {
                 sHold[sn * kTile + px] = tb;
                 sHold[(NP + sn) * kTile + px] = tc;
-            } else if (joins) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int src = (4 * h + jr) * kCkX + jc, jrow = I_ * TE + 4 * h + jr;
-                    float vb = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src * 4, __builtin_bit_cast(int, tb)));
-                    float vc = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src * 4, __builtin_bit_cast(int, tc)));
-                    const float hb = sHold[sn * kTile + src], hc_ = sHold[(NP + sn) * kTile + src];
-                    if (right) { vb = hb; vc = hc_; }
-                    if (4 * h + jr < TE && jc < TE && jrow < H && jcol < W && sn < N) {
-                        const uint32_t jo = mad24(mrow(jrow), W4, mcol(jcol) * 4);
-                        glb_add((float *)((char *)dBg + sn * HW4 + jo), vb);
-                        glb_add((float *)((char *)dCg + sn * HW4 + jo), vc);
-                    }
+            } else if (sn < N) {
+                const __amdgpu_buffer_rsrc_t rB = buf_rsrc((char *)dBg + sn * HW4), rC = buf_rsrc((char *)dCg + sn * HW4);
+                if (joins) {
+                    // left tile: tb, right tile: what is held.  The swap exchanges the upper half of the first (rows 4-7 of the
+                    // left tile) with the lower half of the second (rows 0-3 of the right one): rows 0-3 of both, rows 4-7 of both.
+                    float hb = sHold[sn * kTile + px], hc_ = sHold[(NP + sn) * kTile + px];
+                    swap_halves(tb, hb);
+                    swap_halves(tc, hc_);
+                    buf_add_f32(rB, o0, 0, tb);
+                    buf_add_f32(rB, o4, 0, hb);
+                    buf_add_f32(rC, o0, 0, tc);
+                    buf_add_f32(rC, o4, 0, hc_);
+                } else {
+                    buf_add_f32(rB, o0, 0, tb);
+                    buf_add_f32(rC, o0, 0, tc);
                 }
-            } else if (in && sn < N) {
-                glb_add((float *)((char *)dBg + sn * HW4 + o), tb);
-                glb_add((float *)((char *)dCg + sn * HW4 + o), tc);
             }
         }
     };
+    // ---- checkpoints of a tile (h of the row above, h and s of the column to the left), loaded like its inputs in the sweep of the
+    // tile before it; clamped to the plane, zeroed where they are needed
+    float hu[kCkX], hlft[kRows], slft[kRows], hc = 0.f;
+    auto load_row_ckpt = [&](int I, int J) __attribute__((always_inline)) {
+        const char *src = xv + ((int64_t)max(I - 1, 0) * geo.nCX + J) * DN8 * 4;
+        const float4 v0 = ck4(src, 0), v1 = ck4(src, DN4);
+        hu[0] = v0.x; hu[1] = v0.y; hu[2] = v0.z; hu[3] = v0.w;
+        hu[4] = v1.x; hu[5] = v1.y; hu[6] = v1.z; hu[7] = v1.w;
+        // last column of the tile on the left
+        hc = *(const float *)(src + (J > 0 ? (((TE - 1) >> 2) * DN4 + ((TE - 1) & 3) - DN8) * 4 : 0) + laneB);
+    };
+    auto load_col_ckpt = [&](int I, int J) __attribute__((always_inline)) {
+        const int64_t t_ = ((int64_t)max(J - 1, 0) * geo.nCY + I) * DN8 * 4;
+        const float4 h0 = ck4(xh + t_, 0), h1 = ck4(xh + t_, DN4);
+        const float4 s0 = ck4(xs + t_, 0), s1 = ck4(xs + t_, DN4);
+        hlft[0] = h0.x; hlft[1] = h0.y; hlft[2] = h0.z; hlft[3] = h0.w;
+        hlft[4] = h1.x; hlft[5] = h1.y; hlft[6] = h1.z; hlft[7] = h1.w;
+        slft[0] = s0.x; slft[1] = s0.y; slft[2] = s0.z; slft[3] = s0.w;
+        slft[4] = s1.x; slft[5] = s1.y; slft[6] = s1.z; slft[7] = s1.w;
+    };
+    load_part(I_hi, J_hi, 0);
+    load_part(I_hi, J_hi, 1);
+    load_part(I_hi, J_hi, 2);
+    load_row_ckpt(I_hi, J_hi);
+    load_col_ckpt(I_hi, J_hi);
     for (int I = I_hi; I >= I_lo; --I) {
         const int r0 = I * TE;
         float GR[kRows], SR[kRows];                 // G, G + Gs at the column right of the tile
@@ -536,34 +597,21 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
         for (int J = SEG ? J_hi : geo.nCX - 1; J >= (SEG ? J_lo : 0); --J) {
             const int j0 = J * TE;
-            // ---- checkpoints and carried adjoints of this tile: requested first, so that they arrive
-            // under the staging below instead of being waited for after the barrier
-            float hu[kCkX], hlft[kRows], slft[kRows], hc = 0.f;   // h row above, h/s column to the left
-            float Gd[kCkX];                                        // G of the row below
-            if (I > 0) {
-                const char *src = xv + ((int64_t)(I - 1) * geo.nCX + J) * DN8 * 4;
-                const float4 v0 = ck4(src, 0), v1 = ck4(src, DN4);
-                hu[0] = v0.x; hu[1] = v0.y; hu[2] = v0.z; hu[3] = v0.w;
-                hu[4] = v1.x; hu[5] = v1.y; hu[6] = v1.z; hu[7] = v1.w;
-                if (J > 0)                          // last column of the tile on the left
-                    hc = *(const float *)(src + (((TE - 1) >> 2) * DN4 + ((TE - 1) & 3) - DN8) * 4 + laneB);
-            } else {
+            // the next tile (the block's last: loads that nobody reads, of a tile that exists)
+            int In = I, Jn = J - 1;
+            if (Jn < (SEG ? J_lo : 0)) { In = I - 1; Jn = J_hi; }
+            if (In < I_lo) { In = I; Jn = J; }
+            if (I == 0) {
 #pragma unroll
                 for (int j = 0; j < kCkX; ++j) hu[j] = 0.f;
+                hc = 0.f;
             }
-            if (J > 0) {
-                const char *sh_ = xh + ((int64_t)(J - 1) * geo.nCY + I) * DN8 * 4;
-                const char *ss_ = xs + ((int64_t)(J - 1) * geo.nCY + I) * DN8 * 4;
-                const float4 h0 = ck4(sh_, 0), h1 = ck4(sh_, DN4);
-                const float4 s0 = ck4(ss_, 0), s1 = ck4(ss_, DN4);
-                hlft[0] = h0.x; hlft[1] = h0.y; hlft[2] = h0.z; hlft[3] = h0.w;
-                hlft[4] = h1.x; hlft[5] = h1.y; hlft[6] = h1.z; hlft[7] = h1.w;
-                slft[0] = s0.x; slft[1] = s0.y; slft[2] = s0.z; slft[3] = s0.w;
-                slft[4] = s1.x; slft[5] = s1.y; slft[6] = s1.z; slft[7] = s1.w;
-            } else {
+            if (J == 0) {
 #pragma unroll
                 for (int r = 0; r < kRows; ++r) { hlft[r] = 0.f; slft[r] = 0.f; }
+                hc = 0.f;
             }
+            float Gd[kCkX];                                        // G of the row below
             // the adjoint row of the strip below: written by this block, or - first strip of a
             // pipelined band - by another block.  It is requested here if it is known to be there (own
             // rows; rows whose hand-over an earlier poll has already seen), else after the wait below.
@@ -571,32 +619,24 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             auto take_row = [&](int J_) __attribute__((always_inline)) {   // (pipelined schedules: through coherent words)
                 if (I + 1 < geo.nCY && lvalid) {
                     const char *src = gdown + (int64_t)J_ * DN8 * 4;
+                    if (PIPE) {
 #pragma unroll
-                    for (int k = 0; k < kCkX; k += 2) ld2_coherent((const float *)(src + (k >> 1) * DN2 * 4 + laneG), Gd[k], Gd[k + 1]);
+                        for (int k = 0; k < kCkX; k += 2) ld2_coherent((const float *)(src + (k >> 1) * DN2 * 4 + laneG), Gd[k], Gd[k + 1]);
+                    } else {
+                        const float4 v0 = *(const float4 *)(src + laneG), v1 = *(const float4 *)(src + DN4 * 4 + laneG);
+                        Gd[0] = v0.x; Gd[1] = v0.y; Gd[2] = v0.z; Gd[3] = v0.w;
+                        Gd[4] = v1.x; Gd[5] = v1.y; Gd[6] = v1.z; Gd[7] = v1.w;
+                    }
                 } else {
 #pragma unroll
                     for (int j = 0; j < kCkX; ++j) Gd[j] = 0.f;
                 }
             };
             const bool late = handed && __builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) < geo.nCX - J;
-            if (!late) {
-                if (PIPE) take_row(J);
-                else if (I + 1 < geo.nCY && lvalid) {
-                    const char *src = gdown + (int64_t)J * DN8 * 4;
-                    const float4 v0 = *(const float4 *)(src + laneG), v1 = *(const float4 *)(src + DN4 * 4 + laneG);
-                    Gd[0] = v0.x; Gd[1] = v0.y; Gd[2] = v0.z; Gd[3] = v0.w;
-                    Gd[4] = v1.x; Gd[5] = v1.y; Gd[6] = v1.z; Gd[7] = v1.w;
-                } else {
-#pragma unroll
-                    for (int j = 0; j < kCkX; ++j) Gd[j] = 0.f;
-                }
-            }
             int peek = 0;                           // wave 0: the count as it is now, there when the staged inputs are
             if (late && wave == 0) peek = __hip_atomic_load(progress + I + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            prefetch(I, J);                         // no loads in flight across the register-hungry sweep
-            if (pI >= 0) flush_bc(pI, pJ);          // the previous tile's dB, dC, under the latency of the loads just requested
+            if (pI >= 0) flush_bc();                // the tile before this one
             commit(I, J);
-            pI = I; pJ = J;
             if (late && wave == 0) {
                 seen = __builtin_amdgcn_readfirstlane(peek);
                 if (tid == 0) lds_poke(&sSeen, dead ? geo.nCX : seen);
@@ -611,7 +651,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // 2.765 -> 2.664; priorities 1, 2, 3 alike, the reverse assignment half as much, a fixed priority per block nothing.
             __builtin_amdgcn_s_setprio(3);
 
-            if (TS) {
+            {
                 // T of this wave's channels (only this wave touches their delta' * u, whose place the sweep reuses), and S:
                 // the pixels dealt over the waves, the states over the lanes of a pixel
                 const int lane = tid & 63;
@@ -631,8 +671,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             float hT[TE][TE], smid[TE];
             // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
             // the tile loop (a spilled register is two vector memory instructions per tile, 2 to 4 % of the kernel); the column
-            // segments' bookkeeping leaves room for two.  In the pipelined schedules the row below is loaded late in this pass or
-            // behind it, which is where the registers for five come from.
+            // segments' bookkeeping leaves room for two.
             constexpr int KA = TE == 7 ? 4 : SEG ? 2 : 5;
             float aT[KA ? TE : 1][KA ? KA : 1];
             {
@@ -645,21 +684,31 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         if (c0 + j < TE) { aprev[c0 + j] = EXPA(dlr[j]); hprev[c0 + j] = hu[c0 + j]; }
                 }
                 float diag0 = hc;
+                // (a half row's operands are requested ahead of the arithmetic of the half row before it)
+                float4 nD = *(const float4 *)(myDl + HG + DLO), nB = *(const float4 *)myB, nU = *(const float4 *)myDu;
+                float nl = DL(0, -1);
 #pragma unroll
                 for (int r = 0; r < TE; ++r) {
-                    if (PIPE && r == 4 && soon) take_row(J);    // it arrives under the rest of the recomputation
-                    float al = AEXP(r, -1), left = hlft[r], sl = slft[r], diag = diag0;
+                    if (r == 4 && (!late || soon)) take_row(J);    // it arrives under the rest of the recomputation
+                    float al = EXPA(nl), left = hlft[r], sl = slft[r], diag = diag0;
                     diag0 = hlft[r];
 #pragma unroll
                     for (int c0 = 0; c0 < 8; c0 += 4) {
-                        dl_row4(r, c0, dlr);
-                        const float4 b4 = *(const float4 *)(myB + r * kCkX + c0), u4 = *(const float4 *)(myDu + r * kCkX + c0);
-                        const float aB[4] = {b4.x, b4.y, b4.z, b4.w}, aU[4] = {u4.x, u4.y, u4.z, u4.w};
+                        const float aD[4] = {nD.x, nD.y, nD.z, nD.w}, aB[4] = {nB.x, nB.y, nB.z, nB.w}, aU[4] = {nU.x, nU.y, nU.z, nU.w};
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (c0 == 0 || r + 1 < TE) {
+                            const int nr = c0 == 0 ? r : r + 1, nc = 4 - c0;
+                            nD = *(const float4 *)(myDl + (nr + 1) * HG + DLO + nc);
+                            nB = *(const float4 *)(myB + nr * kCkX + nc);
+                            nU = *(const float4 *)(myDu + nr * kCkX + nc);
+                            if (c0) nl = DL(nr, -1);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const int c_ = c0 + j;
                             if (c_ >= TE) continue;
-                            const float a = EXPA(dlr[j]);
+                            const float a = EXPA(aD[j]);
                             const float bu = aB[j] * aU[j];
                             const float up = hprev[c_];
                             const float X = fmaf(-0.5f * (aprev[c_] + al), diag, up);
@@ -672,35 +721,33 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         }
                     }
                     smid[r] = sl;
+                    // (computed here: left alone the compiler moves arithmetic that only the sweep reads behind the branches between,
+                    // and holds its operands, twice the registers, until then)
+                    asm volatile("" : "+v"(smid[r]));
+#pragma unroll
+                    for (int j = 0; j < TE; ++j) {
+                        asm volatile("" : "+v"(hT[r][j]));
+                        hprev[j] = hT[r][j];
+                        if (j < KA) {
+                            asm volatile("" : "+v"(aT[r][j]));
+                            aprev[j] = aT[r][j];
+                        }
+                    }
                 }
             }
             // strip pipeline: the strip below must have handed over tile J - wanted here, behind the recomputation, and no sooner.
             // One wave polls the count in memory (more pollers only slow it down), the others the word it leaves in LDS.
             // Waiting ahead of the recomputation cost 1.5-7 % of the pipelined backwards: 1 x 256 x 512^2 bf16, 16 states
             // 2396 -> 2328 us; 2 x 192 x 200x336 fp32 1063 -> 1040; 3 x 152 x 61x83 fp16, 8 states 225 -> 209 (unpipelined: same).
-            if (PIPE) {                             // (keeps the compiler from moving the recomputation below the wait)
-#pragma unroll
-                for (int r = 0; r < TE; ++r) {
-#pragma unroll
-                    for (int j = 0; j < TE; ++j) asm volatile("" : "+v"(hT[r][j]));
-                    asm volatile("" : "+v"(smid[r]));
-#pragma unroll
-                    for (int j = 0; j < KA; ++j) asm volatile("" : "+v"(aT[r][j]));
+            if (late && !soon && wave == 0) {
+                strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit);
+                if (tid == 0) {
+                    if (dead) sDead = 1;
+                    lds_poke(&sSeen, dead ? geo.nCX : seen);   // (read at the top of later tiles, too)
                 }
             }
-            if (late && !soon) {
-                if (wave == 0) {
-                    strip_wait(progress + I + 1, geo.nCX - J, seen, sync, dead, geo.spinLimit);
-                    if (tid == 0) {
-                        if (dead) sDead = 1;
-                        lds_poke(&sSeen, dead ? geo.nCX : seen);   // (read at the top of later tiles, too)
-                    }
-                } else {
-                    while (__builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) < geo.nCX - J) __builtin_amdgcn_s_sleep(2);
-                }
-                asm volatile("" ::: "memory");
-                take_row(J);
-            }
+            if (PIPE) __syncthreads();              // the row below is there
+            if (late && !soon) take_row(J);
             if (handed && lds_peek(&sDead)) {   // the wait timed out: poison everything downstream
 #pragma unroll
                 for (int j = 0; j < kCkX; ++j) Gd[j] = __builtin_nanf("");
@@ -721,31 +768,35 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 }
             }
             float Gd8 = GRc;                        // G[r+1][j0+TE]
+            // a half row's operands are requested ahead of the reductions of the half row before it, under which they arrive
+            float4 nD4, nB4, nU4, nC4, nO4;
+            auto half_row = [&](int r, int C0) __attribute__((always_inline)) {
+                nD4 = *(const float4 *)(myDl + (r + 1) * HG + DLO + C0); nB4 = *(const float4 *)(myB + r * kCkX + C0);
+                nU4 = *(const float4 *)(myDu + r * kCkX + C0); nC4 = *(const float4 *)(myC + r * kCkX + C0);
+                nO4 = *(const float4 *)(myDo + r * kCkX + C0);
+            };
+            half_row(TE - 1, 4);
 #pragma unroll
             for (int r = TE - 1; r >= 0; --r) {
+                // the next tile's loads, between the rows of the second half, where the registers of the rows swept are free
+                if (r == 3) load_part(In, Jn, 0);
+                if (r == 2) load_part(In, Jn, 1);
+                if (r == 1) load_part(In, Jn, 2);
                 float Gr = GR[r], Sr = SR[r], Gdiag = Gd8, tr = tR[r];
 #pragma unroll
                 for (int C0 = 4; C0 >= 0; C0 -= 4) {
                     __builtin_amdgcn_sched_barrier(0);
                     const int HW = C0 == 0 ? 4 : TE - 4;        // columns of this half inside the tile
-                    const float4 nD4 = *(const float4 *)(myDl + (r + 1) * HG + DLO + C0), nB4 = *(const float4 *)(myB + r * kCkX + C0);
-                    const float4 nU4 = *(const float4 *)(myDu + r * kCkX + C0), nC4 = *(const float4 *)(myC + r * kCkX + C0);
-                    const float4 nO4 = *(const float4 *)(myDo + r * kCkX + C0);
                     const float dlr[4] = {nD4.x, nD4.y, nD4.z, nD4.w}, aB[4] = {nB4.x, nB4.y, nB4.z, nB4.w}, aC[4] = {nC4.x, nC4.y, nC4.z, nC4.w};
                     const float aU[4] = {nU4.x, nU4.y, nU4.z, nU4.w}, aO[4] = {nO4.x, nO4.y, nO4.z, nO4.w};
-                    float arow[4], s[4], buv[4] = {}, sbv[4] = {};
+                    float arow[4], s[4], sbv[4] = {};
                     float sp = C0 ? smid[r] : slft[r];
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (j < HW) {
                             arow[j] = C0 + j < KA ? aT[KA ? r : 0][C0 + j < KA ? C0 + j : 0] : EXPA(dlr[j]);
-                            if (TS) {
-                                sbv[j] = arow[j] * sp;             // s - bu
-                                sp = fmaf(aB[j], aU[j], sbv[j]);
-                            } else {
-                                buv[j] = aB[j] * aU[j];
-                                sp = fmaf(arow[j], sp, buv[j]);
-                            }
+                            sbv[j] = arow[j] * sp;                 // s - bu
+                            sp = fmaf(aB[j], aU[j], sbv[j]);
                             s[j] = sp;
                         }
                     float q[4] = {}, pp_[4] = {}, vB[4] = {}, vC[4] = {}, dsum[4] = {};
@@ -753,18 +804,16 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     for (int j = 3; j >= 0; --j) {
                         if (j >= HW) continue;
                         const int cj = C0 + j;
-                        const float dov = aO[j], duv = aU[j], bu = buv[j], a = arow[j];
-                        const float dyC = TS ? 0.f : dov * aC[j];
+                        const float dov = aO[j], duv = aU[j], a = arow[j];
                         const float w = fmaf(tr, Gdiag, Kd[cj]);
-                        const float g_ = TS ? fmaf(dov, aC[j], w + Gr) : (w + Gr) + dyC, gg = w + Sr;   // g, and g + gs (dyC cancels)
-                        const float dbu = TS ? gg : fmaf(0.25f, dyC, gg);
+                        const float g_ = fmaf(dov, aC[j], w + Gr), gg = w + Sr;   // g, and g + gs (dout*C cancels)
                         const float h_l = cj == 0 ? hlft[r] : hT[r][cj - 1 < 0 ? 0 : cj - 1];
                         const float h_u = r == 0 ? hu[cj] : hT[r - 1 < 0 ? 0 : r - 1][cj];
                         // g(h - bu) + gs(s - bu) = g(h - s) + (g + gs)(s - bu)
-                        const float hs = hT[r][cj] - s[j], sb = TS ? sbv[j] : s[j] - bu;
+                        const float hs = hT[r][cj] - s[j];
                         const float cross = fmaf(Gd[cj], h_l, Gr * h_u);
                         const float t = -0.5f * a;
-                        const float da = fmaf(t, cross, fmaf(g_, hs, gg * sb));
+                        const float da = fmaf(t, cross, fmaf(g_, hs, gg * sbv[j]));
                         dA_acc = fmaf(dlr[j], da, dA_acc);
                         dsum[j] = da;
                         const float Gn = a * g_;
@@ -774,21 +823,28 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         Gr = Gn;
                         Sr = a * gg;
                         tr = t;
-                        q[j] = dbu * aB[j];                        // per-pixel terms, summed over states below
+                        q[j] = gg * aB[j];                         // per-pixel terms, summed over states below
                         pp_[j] = A2 * da;
-                        const float z = TS ? hs : fmaf(0.25f, bu, hs);
-                        vB[j] = dbu * duv;                         // dB, dC contributions
-                        vC[j] = dov * z;
+                        vB[j] = gg * duv;                          // dB, dC contributions
+                        vC[j] = dov * hs;
                     }
-                    if (want_decay) dec_acc += (dsum[0] + dsum[1]) + (dsum[2] + dsum[3]);
+                    if (want_decay) {
+                        dec_acc += (dsum[0] + dsum[1]) + (dsum[2] + dsum[3]);
+                        asm volatile("" : "+v"(dec_acc));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (C0) half_row(r, 0);
+                    else if (r > 0) half_row(r - 1, 4);
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" : "+v"(dA_acc));    // (added up here: left alone the compiler keeps the terms of the whole tile for its end)
                     if (NP == 16) {
                         // sums over the channel's 16 states: quads 0,1 of the lane group end with
-                        // q[0..1], q[2..3], quads 2,3 with pp_[0..1], pp_[2..3]
-                        group_scatter8(q[0], q[1], q[2], q[3], pp_[0], pp_[1], pp_[2], pp_[3]);
-                        if ((n & 3) == 0) {
-                            float *dst = ((n & 8) ? sP : sQ) + cl * PCH + r * kCkX + C0 + ((n >> 1) & 2);
-                            *(float2 *)dst = make_float2(q[0], q[1]);
-                        }
+                        // q[0..1], q[2..3], quads 2,3 with pp_[0..1], pp_[2..3] (a quad's four lanes write the same words);
+                        // over the wave's channels: the 16-lane row q ends with column C0+q
+                        sweep_reduce16(q[0], q[1], q[2], q[3], pp_[0], pp_[1], pp_[2], pp_[3], vB[0], vB[1], vB[2], vB[3], vC[0], vC[1], vC[2], vC[3]);
+                        *(float2 *)(myQP + r * kCkX + C0) = make_float2(q[0], q[1]);
+                        mydB[r * kCkX + C0 + qrow] = vB[0];
+                        mydC[r * kCkX + C0 + qrow] = vC[0];
                     } else {
                         group_sum4<NP>(q[0], q[1], q[2], q[3]);
                         group_sum4<NP>(pp_[0], pp_[1], pp_[2], pp_[3]);
@@ -796,8 +852,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                             *(float4 *)(sQ + cl * PCH + r * kCkX + C0) = make_float4(q[0], q[1], q[2], q[3]);
                             *(float4 *)(sP + cl * PCH + r * kCkX + C0) = make_float4(pp_[0], pp_[1], pp_[2], pp_[3]);
                         }
-                    }
-                    {
                         // sum over the wave's channels: lane bits 4-5 by a swap reduce-scatter (the
                         // 16-lane row q ends with column C0+q), bits 3 and 2 (8- and 4-lane layouts) by row rotates
                         rows_scatter4x2(vB[0], vB[1], vB[2], vB[3], vC[0], vC[1], vC[2], vC[3]);
@@ -816,6 +870,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 tR[r] = tr;
             }
             GRc = gd_old0;
+            load_row_ckpt(In, Jn);
+            load_col_ckpt(In, Jn);
             const bool hands_over = PIPE && I == I_lo && I > 0;   // top strip of a band: another block takes the row
             if (I > 0 && lvalid) {                  // adjoint row for the strip above
                 char *dst = gdown + (int64_t)J * DN8 * 4;
@@ -832,13 +888,12 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __syncthreads();
             if (hands_over) strip_signal(progress + I);   // tile J is handed over to the strip above
 
-            if (TS) {
 #pragma unroll
-                for (int k = 0; k < NBC; ++k) {     // (another wave may stage the next tile's B, C by the time the flush needs these)
-                    pB[TS ? k : 0] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
-                    pC[TS ? k : 0] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
-                }
+            for (int k = 0; k < NBC; ++k) {         // (another wave may stage the next tile's B, C by the time the flush needs these)
+                pB[k] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
+                pC[k] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
             }
+            pI = I; pJ = J;
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
             {
             SND_THREAD_MAPS(NP);
@@ -851,7 +906,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     const float4 l4 = *(const float4 *)(sDl + cl * DLP + ((q >> 1) + 1) * HG + DLO + (q & 1) * 4);
                     const float4 u4 = *(const float4 *)(sU + cl * PCS + q * 4), o4 = *(const float4 *)(sDo + cl * PCH + q * 4);
                     const float4 g4 = *(const float4 *)(sSg + cl * PCS + q * 4);
-                    const float aq[4] = {q4.x, q4.y, q4.z, q4.w}, ap[4] = {p4.x, p4.y, p4.z, p4.w}, al[4] = {l4.x, l4.y, l4.z, l4.w};
+                    const float4 ss = *(const float4 *)(sS + q * 4);
+                    const float aq[4] = {fmaf(o4.x, ss.x, q4.x), fmaf(o4.y, ss.y, q4.y), fmaf(o4.z, ss.z, q4.z), fmaf(o4.w, ss.w, q4.w)}, ap[4] = {p4.x, p4.y, p4.z, p4.w}, al[4] = {l4.x, l4.y, l4.z, l4.w};
                     const float au[4] = {u4.x, u4.y, u4.z, u4.w}, ao[4] = {o4.x, o4.y, o4.z, o4.w}, ag[4] = {g4.x, g4.y, g4.z, g4.w};
                     float duv[4], ddl[4];
 #pragma unroll
@@ -884,7 +940,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 const float pv = sP[cl * PCH + pp];
                 const float dl = sDl[cl * DLP + ((pp >> 3) + 1) * HG + DLO + (pp & 7)];
                 const float uv = sU[cl * PCS + pp], dov = sDo[cl * PCH + pp], sg = sSg[cl * PCS + pp];
-                const float qv = TS ? fmaf(dov, sS[pp], sQ[cl * PCH + pp]) : sQ[cl * PCH + pp];
+                const float qv = fmaf(dov, sS[pp], sQ[cl * PCH + pp]);
                 const float duv = fmaf(Dv, dov, dl * qv);
                 const float ddl = fmaf(kLn2, pv, uv * qv) * sg;
                 if (cvalid && (pp >> 3) < TE && (pp & 7) < TE && row < H && col < W) {
@@ -915,7 +971,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             strip_signal(segdone + I);
         }
     }
-    if (pI >= 0) flush_bc(pI, pJ);
+    if (pI >= 0) flush_bc();
 #undef DL
 #undef AEXP
 #undef EXPA
@@ -948,15 +1004,17 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 }
 
 // Dynamic LDS of one backward block (more than the 64 KB a kernel gets without asking).
-template <int NP> constexpr size_t bwd_lds_bytes() {
-    constexpr int PCH = kTile + (NP == 16 ? 8 : 4), PCS = kTile + (NP < 8 ? NP : 8), NSD = NP == 16 ? kTile + 2 : kTile + 4;
-    return sizeof(float) * (2 * NP * (kTile + 4) + 2 * (NP / 4) * NP * NSD + 16 * 120 + 16 * (3 * PCH + 2 * PCS) + 4 + 2 * NP * kTile + NP / 4);
+template <int NP, int TE> constexpr size_t bwd_lds_bytes() {
+    constexpr int PCH = kTile + (NP == 16 ? 8 : 4), PCS = bwd_pcs(NP, TE), NSD = NP == 16 ? kTile + 2 : kTile + 4;
+    constexpr int sums = (NP / 4 + 1) * kTile, hold = 2 * NP * kTile;
+    return sizeof(float) * (2 * NP * (kTile + 4) + 2 * (NP / 4) * NP * NSD + 16 * 120 + 16 * (3 * PCH + 2 * PCS) + 4 +
+                            (TE == 7 ? (hold > sums ? hold : sums) : hold + sums) + NP / 4);
 }
 // Raise the dynamic LDS limit of every backward instantiation of one input dtype on the current device.
 // hipFuncSetAttribute is not stream-ordered and must not run under a stream capture, which is why it is
 // done once per device at set-up and not inside the launch path.
 template <typename T, int NP, int TE, bool VEC> static bool configure_bwd_one() {
-    const int lds = (int)bwd_lds_bytes<NP>();
+    const int lds = (int)bwd_lds_bytes<NP, TE>();
     if (NP == 16 && hipFuncSetAttribute((const void *)bwd_kernel<T, NP, true, TE, VEC, NP == 16>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return false;
     return hipFuncSetAttribute((const void *)bwd_kernel<T, NP, true, TE, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess &&
@@ -1001,7 +1059,7 @@ static int launch_bwd_te(const snd_bwd_params &p, const Geo &geo, hipStream_t st
     const int rg = sh.dim / sh.n_groups;
     const int nChunks = (rg + 15) / 16;
     const int64_t nPC = (int64_t)sh.batch * sh.n_groups * nChunks;
-    constexpr size_t lds = bwd_lds_bytes<NP>();
+    constexpr size_t lds = bwd_lds_bytes<NP, TE>();
     const int bands = bwd_band_count(p.f.schedule, (int64_t)sh.batch * sh.n_groups, nChunks, geo.nCY, p.workspace, sh.dstate, geo.nCX);   // 0: one block per plane chunk
     const bool pipe = bands > 0;
     // the dynamic LDS limit of these kernels is raised by snd_init() / on the first launch on a device
