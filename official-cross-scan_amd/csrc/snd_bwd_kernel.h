@@ -872,6 +872,11 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             GRc = gd_old0;
             load_row_ckpt(In, Jn);
             load_col_ckpt(In, Jn);
+#pragma unroll
+            for (int k = 0; k < NBC; ++k) {         // (ahead of the barrier: behind it another wave may stage the next tile's B and C)
+                pB[k] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
+                pC[k] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
+            }
             const bool hands_over = PIPE && I == I_lo && I > 0;   // top strip of a band: another block takes the row
             if (I > 0 && lvalid) {                  // adjoint row for the strip above
                 char *dst = gdown + (int64_t)J * DN8 * 4;
@@ -888,11 +893,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __syncthreads();
             if (hands_over) strip_signal(progress + I);   // tile J is handed over to the strip above
 
-#pragma unroll
-            for (int k = 0; k < NBC; ++k) {         // (another wave may stage the next tile's B, C by the time the flush needs these)
-                pB[k] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
-                pC[k] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
-            }
             pI = I; pJ = J;
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
             {
