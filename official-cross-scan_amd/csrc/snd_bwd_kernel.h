@@ -689,7 +689,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 float nl = DL(0, -1);
 #pragma unroll
                 for (int r = 0; r < TE; ++r) {
-                    if (r == 4 && (!late || soon)) take_row(J);    // it arrives under the rest of the recomputation
+                    if (r == 2 && (!late || soon)) take_row(J);    // it arrives under the rest of the recomputation
                     float al = EXPA(nl), left = hlft[r], sl = slft[r], diag = diag0;
                     diag0 = hlft[r];
 #pragma unroll
@@ -779,9 +779,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
             for (int r = TE - 1; r >= 0; --r) {
                 // the next tile's loads, between the rows of the second half, where the registers of the rows swept are free
-                if (r == 3) load_part(In, Jn, 0);
-                if (r == 2) load_part(In, Jn, 1);
-                if (r == 1) load_part(In, Jn, 2);
+                if (r == 4) load_part(In, Jn, 0);
+                if (r == 3) load_part(In, Jn, 1);
+                if (r == 2) load_part(In, Jn, 2);
                 float Gr = GR[r], Sr = SR[r], Gdiag = Gd8, tr = tR[r];
 #pragma unroll
                 for (int C0 = 4; C0 >= 0; C0 -= 4) {
@@ -870,8 +870,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 tR[r] = tr;
             }
             GRc = gd_old0;
-            load_row_ckpt(In, Jn);
-            load_col_ckpt(In, Jn);
 #pragma unroll
             for (int k = 0; k < NBC; ++k) {         // (ahead of the barrier: behind it another wave may stage the next tile's B and C)
                 pB[k] = sB[(wave_u + WPB * k) * NSTR + (tid & 63)];
@@ -892,6 +890,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             if (hands_over) strip_stores_done();
             __syncthreads();
             if (hands_over) strip_signal(progress + I);   // tile J is handed over to the strip above
+            // (not ahead of the hand-over: its wait for the row's stores would cover them)
+            load_row_ckpt(In, Jn);
+            load_col_ckpt(In, Jn);
 
             pI = I; pJ = J;
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
