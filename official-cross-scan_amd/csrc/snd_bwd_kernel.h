@@ -643,14 +643,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             __syncthreads();
             const bool soon = late && __builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) >= geo.nCX - J;
-            // The sweep runs at a raised wave priority, everything else (loads, commit to LDS, per-pixel epilogue) at the
-            // default: the two waves a SIMD holds belong to two blocks, and with equal priority they drift into the same
-            // phase and stall together; with the wave that is in its dependent arithmetic chain preferred, the other's
-            // memory phases fall into its gaps.  Measured before the tile was swept whole (backward ms): 64 x 192 x 56x56 fp32
-            // 1.332 -> 1.280, 64 x 768 x 14x14 bf16 0.339 -> 0.331, 2 x 192 x 200x336 1.199 -> 1.181, 256 channels of 512x512
-            // 2.765 -> 2.664; priorities 1, 2, 3 alike, the reverse assignment half as much, a fixed priority per block nothing.
-            __builtin_amdgcn_s_setprio(3);
-
             {
                 // T of this wave's channels (only this wave touches their delta' * u, whose place the sweep reuses), and S:
                 // the pixels dealt over the waves, the states over the lanes of a pixel
@@ -767,6 +759,13 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         if (c0 + j < TE) Kd[c0 + j] = fmaf(-0.5f * EXPA(dlr[j]), c0 + j + 1 < TE ? Gd[c0 + j + 1 < 8 ? c0 + j + 1 : 7] : GRc, Gd[c0 + j]);
                 }
             }
+            // The sweep runs at a raised wave priority, everything else (loads, commit to LDS, recomputation, per-pixel epilogue)
+            // at the default: the two waves a SIMD holds belong to two blocks, and with equal priority they drift into the same
+            // phase and stall together; with the wave that is in its long arithmetic preferred, the other's phases fall into its
+            // gaps.  Backward in us, raised from the recomputation on / raised for the sweep alone: 64 x 192 x
+            // 56x56 fp32 1064 / 1057, 1 x 256 x 512^2 bf16 2072 / 1998, 32 x 768 x 28x28 bf16 575 / 551, 64 x 768 x
+            // 14x14 291 / 286, 2 x 192 x 200x336 916 / 915.  Middle levels for the recomputation or the memory phases: alike.
+            __builtin_amdgcn_s_setprio(3);
             float Gd8 = GRc;                        // G[r+1][j0+TE]
             // a half row's operands are requested ahead of the reductions of the half row before it, under which they arrive
             float4 nD4, nB4, nU4, nC4, nO4;
