@@ -191,15 +191,15 @@ __device__ __forceinline__ float4 ld4_stream(const float *src) {
 // ---------------------------------------------------------------- math
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// softplus with the reference's threshold (fwd.cuh:223): log1p(e) = log(1+e) * e / ((1+e) - 1)
-// keeps full relative accuracy for the tiny e = exp(x) that small time steps produce, using the
-// hardware exp2/log2/rcp (about 1 ulp each).  Also returns the derivative sigmoid(x) (bwd.cuh:792).
+// softplus with the reference's threshold (fwd.cuh:223): log1p(e) = log(w) + (e - (w - 1)) / w with w = 1 + e rounded, which
+// keeps full relative accuracy for the tiny e = exp(x) that small time steps produce, using the hardware exp2/log2/rcp
+// (about 1 ulp each).  Also returns the derivative sigmoid(x) (bwd.cuh:792), from the same reciprocal.  Error against 64 bits
+// for x of -8 to 20 at most 6.6e-7 of the value (log(w) * e / (w - 1), three instructions and a second reciprocal more: 7.1e-7).
 __device__ __forceinline__ float softplus20(float x, float &dsp) {
     const float e = fast_exp2(x * kLog2e);
     const float w = 1.f + e;
-    const float d = w - 1.f;
     const float rw = __builtin_amdgcn_rcpf(w);
-    float sp = (d == 0.f) ? e : __builtin_amdgcn_logf(w) * kLn2 * (e * __builtin_amdgcn_rcpf(d));
+    float sp = fmaf(e - (w - 1.f), rw, __builtin_amdgcn_logf(w) * kLn2);
     dsp = e * rw;
     if (x > 20.f) { sp = x; dsp = 1.f; }
     return sp;
