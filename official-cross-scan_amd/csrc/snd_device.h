@@ -542,7 +542,7 @@ struct WaveGeo {
     int extL, extR;                // whether a column group lies to the left / right of this launch's
     float *colh, *cols;            // (wide planes, forward) where column groups hand over h, a and s: the saved state
                                    // x, x_sd themselves, or a workspace of the same layout when no state is saved
-    float *bcol;                   // (wide planes, backward) G, Gs, a at the first column of every column group;
+    float *bcol;                   // (wide planes, backward) G, G + Gs, -a/2 at the first column of every column group;
                                    // (split planes, backward) the same as tagged words, see wave_bwd_split()
     int *sync;                     // (split planes) the workspace's sync words (error word) and the bound of a wait
     int spinLimit;
@@ -826,6 +826,18 @@ template <int PK> __device__ __forceinline__ float from_prev_lane_pk(float v, fl
     const float t = from_prev_lane(v, edge);
     return first ? edge : t;
 }
+// The same where nothing enters the plane (a plane one segment wide): the first / last lane gets zero, and the compiler can
+// fold the move into the instruction that reads it.
+template <int PK> __device__ __forceinline__ float from_prev_lane_one(float v, bool first) {
+    if (PK == 4 || PK == 8) return dpp_mov<0x111>(v);                  // row_shr:1
+    const float t = dpp_mov<0x138>(v);                                 // wave_shr:1
+    return PK == 2 && first ? 0.f : t;
+}
+template <int PK> __device__ __forceinline__ float from_next_lane_one(float v, bool last) {
+    if (PK == 4 || PK == 8) return dpp_mov<0x101>(v);                  // row_shl:1
+    const float t = dpp_mov<0x130>(v);                                 // wave_shl:1
+    return PK == 2 && last ? 0.f : t;
+}
 // v of the lane above inside the lane's plane; the plane's last lane (`last`) keeps `edge`.
 template <int PK> __device__ __forceinline__ float from_next_lane_pk(float v, float edge, bool last) {
     if (PK == 1) return from_next_lane(v, edge);
@@ -839,7 +851,8 @@ template <int PK> __device__ __forceinline__ float from_next_lane_pk(float v, fl
 // lanes, lanes ascending in the direction of the recurrence, cy / cs entering the first column of lane 0.
 // The CPL maps of a lane are composed first, one scan runs over the lanes, and the lane's columns are filled
 // in from the value entering the lane.  Returns the solutions per column (the lane's last: oy[CPL-1]).
-template <int CPL, int PK = 1>
+// ONE: nothing enters lane 0 (cy, cs are not read): the scan's sums are the solutions.
+template <int CPL, int PK = 1, bool ONE = false>
 __device__ __forceinline__ void wave_row_solve(const float (&a)[CPL], const float (&y)[CPL], const float (&sv)[CPL], float cy,
                                                float cs, float (&oy)[CPL], float (&os)[CPL]) {
     static_assert(PK == 1 || CPL == 1, "packed planes: one column per lane");
@@ -851,6 +864,11 @@ __device__ __forceinline__ void wave_row_solve(const float (&a)[CPL], const floa
         Ap *= a[k];
     }
     wave_scan3_pk<PK>(Y, S, Ap);
+    if (ONE && CPL == 1) {
+        oy[0] = Y;
+        os[0] = S;
+        return;
+    }
     const float ey = fmaf(Ap, cy, Y), es = fmaf(Ap, cs, S);      // at the lane's last column
     if (CPL > 1) {
         float ty = from_prev_lane(ey, cy), ts = from_prev_lane(es, cs);   // entering the lane

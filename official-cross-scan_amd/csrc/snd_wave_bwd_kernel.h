@@ -19,7 +19,7 @@
 // a register crossbar move, no LDS memory).
 // A wave handles its segment band by band (R rows), bottom band first: recompute h, s of the band's rows
 // from the forward's checkpoints (row above the band from x_v, what entered the segment on every row from
-// x / x_sd: no wave waits for another here), then sweep the band's rows bottom-up.  The sweep needs G, Gs, a
+// x / x_sd: no wave waits for another here), then sweep the band's rows bottom-up.  The sweep needs G, P = G + Gs, a
 // of the segment on the right at its first column: wave w runs one band behind wave w+1 and finds them in
 // LDS (one block barrier per band, no polling).  dB, dC leave as one global atomic per element and channel
 // (a wave-wide instruction covers 256 consecutive bytes), du / ddelta as whole row segments.
@@ -52,20 +52,26 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // XW: the most waves a block may have, 8 or (two channels of five to eight segments) 16.
 //
 // EXT: the launch works on one column group of a wide plane (wave_wide() in snd_device.h), segments seg0 .. seg0+nseg-1;
-// the groups are launched right to left.  The group's last wave takes G, Gs, a of the column on its right from global
+// the groups are launched right to left.  The group's last wave takes G, P, -a/2 of the column on its right from global
 // memory (with the band's loads, three values per state and row spread over the lanes of one register), where the
 // first wave of the group on the right left them, and puts them into the LDS slot a neighbouring wave would have filled.
 //
 // SPL (with EXT): a split plane (wave_bwd_split() in snd_device.h): the block works on one half of the segments of two
 // channels, the two halves of a channel pair are blocks of the same launch, and the hand-over goes through tagged
 // words that the left half's edge wave checks.
-template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false>
+// ONE: the plane is one segment wide (always so with packed planes): nothing enters a row, so the scan's sums are the solutions,
+// neighbours beyond the plane are zeros, and nothing is handed over or waited for.  Bound by its vector instructions (167 a row
+// of 64 cells, four waves per SIMD).  Together with the softplus taken out of its branch and P swept instead of Gs, 137 a row (us):
+// 64 x 384 x 56x56 bf16, one state 381 -> 336, two 632 -> 542; 8 x 384 x 56x56, four 174 -> 140; 8 x 96 x 56x56 fp32, three
+// 99 -> 68; packed, 32 x 768 x 28x28 92 -> 86; several segments (no ONE) 64 x 96 x 112x112 411 -> 408.
+template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1)>
 __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
     static_assert(!EXT || (CHB == (SPL ? 2 : 1) && PK == 1 && CPL == 1 && (!EVEN || SPL)), "column groups: one channel per block, one column per lane");
     static_assert(!SPL || EXT, "a split plane hands over like a column group");
     static_assert(CHB == 1 || CPL == 1, "shared atomics: one column per lane");
     static_assert(PK == 1 || (CHB > 1 && !EVEN), "packed planes share their atomics");
+    static_assert(ONE ? CPL == 1 && !EXT : PK == 1, "one segment: one column per lane; packed planes are one segment wide");
     constexpr int S = 64 / PK;                       // lanes per plane
     constexpr int kItems = R * NS * 2;               // dB and dC rows of a band
     static_assert(kItems % CHB == 0, "the waves of a segment take equal shares of a band's dB / dC rows");
@@ -78,17 +84,17 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     // load a band's inputs one band ahead (with three or four states it measured 20 % slower, and with two columns per
     // lane the registers are needed elsewhere)
     constexpr bool PF = NS <= 2 && CPL == 1;
-    // what a wave leaves for the wave on its left: {G, Gs, a, -} at its first column, per band parity, row and
+    // what a wave leaves for the wave on its left: {G, P, -a/2, -} at its first column, per band parity, row and
     // state.  Wave w writes slot w and reads slot w+1; the slot after the last wave stays zero.
-    __shared__ float4 sHO[2][CHB][kMaxSeg + 1][R][NS];
+    __shared__ float4 sHO[ONE ? 1 : 2][ONE ? 1 : CHB][ONE ? 1 : kMaxSeg + 1][ONE ? 1 : R][NS];
 
     const snd_fwd_params &f = p.f;
     const snd_shape &sh = f.shape;
     const int H = sh.nrows, W = sh.ncols, N = sh.dstate, Dm = sh.dim, G = sh.n_groups;
     const int rg = wg.rg, rd = wg.rd;
-    const int nseg = wg.nseg;
+    const int nseg = ONE ? 1 : wg.nseg;
     const int lane = threadIdx.x & 63, wi = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int kc = CHB > 1 ? wi / nseg : 0, w = PK > 1 ? 0 : wi - kc * nseg;     // channel of the block, segment of the channel
+    const int kc = CHB > 1 ? (ONE ? wi : wi / nseg) : 0, w = ONE ? 0 : wi - kc * nseg;     // channel of the block, segment of the channel
     const int sl = PK > 1 ? lane % S : lane;         // the lane inside its plane
     int pair, chunk, half = 0;
     if (SPL) {
@@ -153,8 +159,8 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     const int c = g * rg + chunk, cd = rd == 1 ? c : c / rd;   // channel of u, of delta
     // channel offsets: in the scalar base pointers, or (packed) in the lanes' offsets
     const int cB = PK > 1 ? 0 : c, chB = PK > 1 ? 0 : chunk, cL = PK > 1 ? c : 0, chL = PK > 1 ? chunk : 0;
-    const bool multi = nseg > 1;
-    if (threadIdx.x < 2 * R * NS)
+    const bool multi = !ONE && nseg > 1;
+    if (!ONE && threadIdx.x < 2 * R * NS)
 #pragma unroll
         for (int q = 0; q < CHB; ++q) sHO[threadIdx.x / (R * NS)][q][nseg][threadIdx.x % (R * NS) / NS][threadIdx.x % NS] = make_float4(0.f, 0.f, 0.f, 0.f);
 
@@ -223,7 +229,7 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     const float *xv = f.x_v + plane0 * wave_xv_plane(wg) + jn0;
     const float *xh = f.x + plane0 * wave_x_plane(wg) + (int64_t)sg * 2 * wg.Hp;
     const float *xs = f.x_sd + plane0 * wave_x_plane(wg) + (int64_t)sg * 2 * wg.Hp;
-    // (column groups) lane (q*NS + n)*R + r fetches G (q = 0), Gs (1), a (2) of the group on the right: row r of a band, state n
+    // (column groups) lane (q*NS + n)*R + r fetches G (q = 0), P (1), -a/2 (2) of the group on the right: row r of a band, state n
     constexpr int kExtLanes = 3 * NS * R;
     const int el = lane < kExtLanes ? lane : 0, eq = el / (NS * R), er = el % R, gq = EXT ? wg.seg0 / kMaxSeg : 0;
     const float *ebase = EXT ? wg.bcol + (plane0 + (el / R) % NS) * wave_bcol_plane(wg)
@@ -302,14 +308,14 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
         if (CPL == 2 && !fh) { const float t = v[0]; v[0] = v[CPL - 1]; v[CPL - 1] = t; }
     };
 
-    float Gd[NS][CPL], ad[NS][CPL], GdEdge[NS];     // G, a of the row below at this lane's columns; G[i+1, S*(w+1)]
+    float Gd[NS][CPL], td[NS][CPL], GdEdge[NS];     // G, -a/2 of the row below at this lane's columns; G[i+1, S*(w+1)]
     float dA_acc[NS];
     float dec_acc = 0.f, dD_acc = 0.f, dbias_acc = 0.f, dw_acc = 0.f;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
         GdEdge[n] = 0.f; dA_acc[n] = 0.f;
 #pragma unroll
-        for (int k = 0; k < CPL; ++k) { Gd[n][k] = 0.f; ad[n][k] = 0.f; }
+        for (int k = 0; k < CPL; ++k) { Gd[n][k] = 0.f; td[n][k] = 0.f; }
     }
     int step = nseg - 1 - w;                         // the waves on the right go first
     const bool hands_over = multi && w > 0;
@@ -334,12 +340,13 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
 #pragma unroll
             for (int t = 0; t < CPL; ++t) {
                 const float raw = dtop[t] + bias;
-                float sg;
-                dtop[t] = softplus ? softplus20(raw, sg) : raw;
+                float sg, sp = softplus20(raw, sg);
+                asm volatile("" : "+v"(sp));
+                dtop[t] = softplus ? sp : raw;
             }
 #pragma unroll
             for (int n = 0; n < NS; ++n) {
-                hdiag[n] = bcast(cur.ch[n], 0);
+                hdiag[n] = ONE ? 0.f : bcast(cur.ch[n], 0);
 #pragma unroll
                 for (int k = 0; k < CPL; ++k) {
                     hp[n][k] = cur.h0[n][k];
@@ -359,10 +366,13 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                 unpack(cur.d[r], dl[r]);
 #pragma unroll
                 for (int t = 0; t < CPL; ++t) {
+                    // (always evaluated, then selected: a branch around each would keep the chains from filling each
+                    // other's latencies)
                     const float raw = dl[r][t] + bias;
-                    float sg = 1.f;
-                    dl[r][t] = softplus ? softplus20(raw, sg) : raw;
-                    dsp[r][t] = sg;
+                    float sg, sp = softplus20(raw, sg);
+                    asm volatile("" : "+v"(sp), "+v"(sg));
+                    dl[r][t] = softplus ? sp : raw;
+                    dsp[r][t] = softplus ? sg : 1.f;
                 }
             }
 #pragma unroll
@@ -389,7 +399,7 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
 #pragma unroll
                     for (int n = 0; n < NS; ++n) {
                         // (rows past the plane's last have no column checkpoint: zeros, so that what is computed there is finite)
-                        const bool rin = EVEN || i0 + r < H;
+                        const bool rin = !ONE && (EVEN || i0 + r < H);
                         const float hin = rin ? bcast(cur.ch[n], r + 1) : 0.f, sin_ = rin ? bcast(cur.cs[n], r + 1) : 0.f, ain = rin ? bcast(cur.ca[n], r + 1) : 0.f;
                         float a[CPL], bu[CPL], y[CPL], h[CPL], s[CPL];
 #pragma unroll
@@ -398,15 +408,15 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                             bu[k] = bn_[r][n][k] * dlun[k];
                             if (PK == 8) { a[k] = bar ? 0.f : a[k]; bu[k] = bar ? 0.f : bu[k]; }   // the barrier lane's map is (0, 0)
                         }
-                        const float a_l = from_prev_lane_pk<PK>(a[CPL - 1], ain, sl == 0);                 // a[i, j-1] of the lane's first column
-                        const float h_d = from_prev_lane_pk<PK>(hp[n][CPL - 1], hdiag[n], sl == 0);        // h[i-1, j-1]
+                        const float a_l = ONE ? from_prev_lane_one<PK>(a[CPL - 1], sl == 0) : from_prev_lane_pk<PK>(a[CPL - 1], ain, sl == 0);   // a[i, j-1] of the lane's first column
+                        const float h_d = ONE ? from_prev_lane_one<PK>(hp[n][CPL - 1], sl == 0) : from_prev_lane_pk<PK>(hp[n][CPL - 1], hdiag[n], sl == 0);   // h[i-1, j-1]
 #pragma unroll
                         for (int k = 0; k < CPL; ++k) {
                             const float al = k == 0 ? a_l : a[k > 0 ? k - 1 : 0], hd = k == 0 ? h_d : hp[n][k > 0 ? k - 1 : 0];
                             const float X = fmaf(-0.5f * (ap[n][k] + al), hd, hp[n][k]);
                             y[k] = fmaf(a[k], X, bu[k]);
                         }
-                        wave_row_solve<CPL, PK>(a, y, bu, hin, sin_, h, s);
+                        wave_row_solve<CPL, PK, ONE>(a, y, bu, hin, sin_, h, s);
 #pragma unroll
                         for (int k = 0; k < CPL; ++k) {
                             hT[r][n][CPL - 1 - k] = mirror(h[k]);
@@ -453,42 +463,47 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                 }
 #pragma unroll
                 for (int n = 0; n < NS; ++n) {
-                    // what the segment on the right left for this row: G, Gs, a at column S*(w+1)
-                    const float4 in = (PK > 1 && NS <= 2) ? make_float4(0.f, 0.f, 0.f, 0.f) : sHO[(step + 1) & 1][kc][w + 1][r][n];   // (packed planes have no neighbour)
-                    const float hin = (EVEN || i0 + r < H) ? bcast(cur.ch[n], r + 1) : 0.f;   // h[i, S*w-1]
-                    float Bv[CPL], Cv[CPL], a[CPL], bu[CPL], dyC[CPL], z[CPL], ya[CPL], ys[CPL], Gt[CPL], Gst[CPL];
+                    // what the segment on the right left for this row: G, P, -a/2 at column S*(w+1)
+                    const float4 in = ONE ? make_float4(0.f, 0.f, 0.f, 0.f) : sHO[(step + 1) & 1][kc][w + 1][r][n];
+                    const float hin = !ONE && (EVEN || i0 + r < H) ? bcast(cur.ch[n], r + 1) : 0.f;   // h[i, S*w-1]
+                    float Bv[CPL], Cv[CPL], a[CPL], th[CPL], bu[CPL], dyC[CPL], z[CPL], zz[CPL], ya[CPL], ys[CPL], Gt[CPL], Pt[CPL];
                     unpack(cur.b[r][n], Bv);
                     unpack(cur.c[r][n], Cv);
 #pragma unroll
                     for (int t = 0; t < CPL; ++t) {
                         a[t] = aT[r][n][t];
+                        th[t] = -0.5f * a[t];
                         bu[t] = Bv[t] * dlu[t];
                         dyC[t] = dov[t] * Cv[t];
                     }
-                    const float a_r0 = from_prev_lane_pk<PK>(a[CPL - 1], in.z, sl == 0);               // a[i, j+1] of the lane's first column
-                    const float Gdg0 = from_prev_lane_pk<PK>(Gd[n][CPL - 1], GdEdge[n], sl == 0);      // G[i+1, j+1]
+                    const float t_r0 = ONE ? from_prev_lane_one<PK>(th[CPL - 1], sl == 0) : from_prev_lane_pk<PK>(th[CPL - 1], in.z, sl == 0);   // -a[i, j+1]/2 of the lane's first column
+                    const float Gdg0 = ONE ? from_prev_lane_one<PK>(Gd[n][CPL - 1], sl == 0) : from_prev_lane_pk<PK>(Gd[n][CPL - 1], GdEdge[n], sl == 0);   // G[i+1, j+1]
+                    // Swept are G and P = G + Gs, which enters g + gs: dout*C cancels there and is left out,
+                    //     g = G[i,j+1] + zz + dout*C,   g + gs = P[i,j+1] + zz,   zz = G[i+1,j] - 0.5*(a[i,j+1] + a[i+1,j])*G[i+1,j+1]
 #pragma unroll
                     for (int t = 0; t < CPL; ++t) {
-                        const float ar = t == 0 ? a_r0 : a[t > 0 ? t - 1 : 0], gdg = t == 0 ? Gdg0 : Gd[n][t > 0 ? t - 1 : 0];
-                        z[t] = fmaf(-0.5f * (ar + ad[n][t]), gdg, dyC[t] + Gd[n][t]);
+                        const float tr = t == 0 ? t_r0 : th[t > 0 ? t - 1 : 0], gdg = t == 0 ? Gdg0 : Gd[n][t > 0 ? t - 1 : 0];
+                        zz[t] = fmaf(tr + td[n][t], gdg, Gd[n][t]);
+                        z[t] = zz[t] + dyC[t];
                         ya[t] = a[t] * z[t];
-                        ys[t] = -a[t] * dyC[t];
+                        ys[t] = a[t] * zz[t];
                     }
-                    wave_row_solve<CPL, PK>(a, ya, ys, in.x, in.y, Gt, Gst);           // G[i,j], Gs[i,j]
-                    const float Gr0 = from_prev_lane_pk<PK>(Gt[CPL - 1], in.x, sl == 0), Gsr0 = from_prev_lane_pk<PK>(Gst[CPL - 1], in.y, sl == 0);
-                    const float hl_last = from_next_lane_pk<PK>(hT[r][n][0], hin, sl == S - 1);   // h[i, j-1] of the lane's last column
+                    wave_row_solve<CPL, PK, ONE>(a, ya, ys, in.x, in.y, Gt, Pt);           // G[i,j], P[i,j]
+                    const float Gr0 = ONE ? from_prev_lane_one<PK>(Gt[CPL - 1], sl == 0) : from_prev_lane_pk<PK>(Gt[CPL - 1], in.x, sl == 0);
+                    const float Pr0 = ONE ? from_prev_lane_one<PK>(Pt[CPL - 1], sl == 0) : from_prev_lane_pk<PK>(Pt[CPL - 1], in.y, sl == 0);
+                    const float hl_last = ONE ? from_next_lane_one<PK>(hT[r][n][0], sl == S - 1) : from_next_lane_pk<PK>(hT[r][n][0], hin, sl == S - 1);   // h[i, j-1] of the lane's last column
 #pragma unroll
                     for (int t = 0; t < CPL; ++t) {
-                        const float Gr = t == 0 ? Gr0 : Gt[t > 0 ? t - 1 : 0], Gsr = t == 0 ? Gsr0 : Gst[t > 0 ? t - 1 : 0];
-                        float g_ = Gr + z[t], gs = Gsr - dyC[t];
-                        if (PK == 8) { g_ = bar ? 0.f : g_; gs = bar ? 0.f : gs; }         // (what the barrier lane fetched is another plane's)
-                        const float dbu = fmaf(0.25f, dyC[t], g_ + gs);
+                        const float Gr = t == 0 ? Gr0 : Gt[t > 0 ? t - 1 : 0], Pr = t == 0 ? Pr0 : Pt[t > 0 ? t - 1 : 0];
+                        float g_ = Gr + z[t], gg = Pr + zz[t];
+                        if (PK == 8) { g_ = bar ? 0.f : g_; gg = bar ? 0.f : gg; }         // (what the barrier lane fetched is another plane's)
+                        const float dbu = fmaf(0.25f, dyC[t], gg);
                         const float hv = hT[r][n][t], sv = sT[r][n][t];
                         const float h_l = t == CPL - 1 ? hl_last : hT[r][n][t < CPL - 1 ? t + 1 : 0];
                         const float h_u = r > 0 ? hT[r > 0 ? r - 1 : 0][n][t] : hTop[n][t];
                         const float hs = hv - sv, sb = sv - bu[t];
                         const float cross = fmaf(Gd[n][t], h_l, Gr * h_u);
-                        const float da = fmaf(-0.5f * a[t], cross, fmaf(g_, hs, (g_ + gs) * sb));
+                        const float da = fmaf(th[t], cross, fmaf(g_, hs, gg * sb));
                         dA_acc[n] = fmaf(dl[r][t], da, dA_acc[n]);
                         if (want_decay) dec_acc += da;
                         qsum[t] = fmaf(dbu, Bv[t], qsum[t]);
@@ -511,20 +526,20 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                     }
                     GdEdge[n] = in.x;
 #pragma unroll
-                    for (int t = 0; t < CPL; ++t) { Gd[n][t] = Gt[t]; ad[n][t] = a[t]; }
-                    if (hands_over && lane == 63) sHO[step & 1][kc][w][r][n] = make_float4(Gt[CPL - 1], Gst[CPL - 1], a[CPL - 1], 0.f);
+                    for (int t = 0; t < CPL; ++t) { Gd[n][t] = Gt[t]; td[n][t] = th[t]; }
+                    if (hands_over && lane == 63) sHO[step & 1][kc][w][r][n] = make_float4(Gt[CPL - 1], Pt[CPL - 1], th[CPL - 1], 0.f);
                     if (EXT && !SPL && ext_out && lane == 63) {   // for the column group on the left
                         float *d = eout + (int64_t)n * wave_bcol_plane(wg) + i0 + r;
                         d[0] = Gt[CPL - 1];
-                        d[wg.Hp] = Gst[CPL - 1];
-                        d[2 * wg.Hp] = a[CPL - 1];
+                        d[wg.Hp] = Pt[CPL - 1];
+                        d[2 * wg.Hp] = th[CPL - 1];
                     }
                     if (SPL && ext_out && lane == 63) {           // for the left half: tagged with the band
                         float *d = eouttag + (int64_t)n * wave_split_words(wg) + (int64_t)band * (6 * R) + 2 * r;
                         const float tg = __builtin_bit_cast(float, (uint32_t)band + 1u);
                         st2_coherent(d, Gt[CPL - 1], tg);
-                        st2_coherent(d + 2 * R, Gst[CPL - 1], tg);
-                        st2_coherent(d + 4 * R, a[CPL - 1], tg);
+                        st2_coherent(d + 2 * R, Pt[CPL - 1], tg);
+                        st2_coherent(d + 4 * R, th[CPL - 1], tg);
                     }
                 }
                 {
@@ -575,7 +590,7 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     if (PF) load_band(sA, wg.nBands - 1);
     // (nothing in flight on the way into the band loop: its first waits then follow the loop's own path as well)
     if (PF) __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
-    lds_barrier();                                   // the zeroed slot
+    if (!ONE) lds_barrier();                         // the zeroed slot
     if (SPL) lds_barrier();                          // (and what the block's extra wave has fetched for the first band)
     if (multi)
         for (int e = 0; e < (nseg - 1 - w) * (CHB > 1 && kXBuf == 1 ? 2 : 1); ++e) lds_barrier();
@@ -642,7 +657,7 @@ static inline int wave_bwd_share(const snd_shape &sh, const WaveGeo &wg) {
     return wg.nseg * 4 <= kWaveShareWaves ? 4 : 2;
 }
 
-template <typename T, int NS, int CPL, bool VEC, int CHB, int PK, int XW = kMaxSeg>
+template <typename T, int NS, int CPL, bool VEC, int CHB, int PK, int XW = kMaxSeg, bool ONE = (PK > 1)>
 static int launch_wave_bwd_c(const snd_bwd_params &p, const WaveGeo &wg, hipStream_t stream) {
     const snd_shape &sh = p.f.shape;
     const int rg = sh.dim / sh.n_groups;
@@ -653,11 +668,11 @@ static int launch_wave_bwd_c(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     const bool even = NS <= 2 && CPL == 1 && PK == 1 && sh.nrows % R == 0 && sh.ncols % (kSeg * CPL) == 0;
     if (even) {
         constexpr bool E = NS <= 2 && CPL == 1 && PK == 1;
-        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, E, CHB, PK, XW>), grid, block, 0, stream, p, wg);
-        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, E, CHB, PK, XW>), grid, block, 0, stream, p, wg);
+        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, E, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
+        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, E, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
     } else {
-        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, false, CHB, PK, XW>), grid, block, 0, stream, p, wg);
-        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, false, CHB, PK, XW>), grid, block, 0, stream, p, wg);
+        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, false, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
+        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, false, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
     }
     return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
 }
@@ -670,6 +685,7 @@ static int launch_wave_bwd_v(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     if (pk == 8) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 8 : 1>(p, wg, stream);
     if (pk == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 4 : 1>(p, wg, stream);
     if (pk == 2) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 2 : 1>(p, wg, stream);
+    if (share == 4 && wg.nseg == 1) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, 1, kMaxSeg, CPL == 1>(p, wg, stream);
     if (share == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, 1>(p, wg, stream);
     if (share == 2 && wg.nseg > 4) return launch_wave_bwd_c<T, NS, CPL, VEC, (CPL == 1 && NS <= 2) ? 2 : 1, 1, (CPL == 1 && NS <= 2) ? 16 : kMaxSeg>(p, wg, stream);
     if (share == 2) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 2 : 1, 1>(p, wg, stream);
