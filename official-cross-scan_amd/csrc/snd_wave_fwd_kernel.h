@@ -39,6 +39,10 @@ namespace snd {
 // block is kOneWaves independent waves, each with a channel (PK channels) of its own, a quarter of the blocks to hand
 // out (measured against blocks of one wave, bf16, one state: 64 x 1536 x 14x14 0.055 -> 0.049 ms, 64 x 768 x 14x14
 // 0.035 -> 0.031, 64 x 3072 x 7x7 unchanged at 0.051).
+// The scan's sums are the solutions there and a neighbour's value is zero at the plane's edge, which takes 8 instructions
+// per row and state out (four states, 8 x 384 x 56x56 bf16: 62 -> 59 us; two states, 32 x 768 x 28x28 fp32: 62 -> 59).  In fp32 at
+// most four waves to a SIMD, although the registers allow five: bound by memory, and the fifth wave's streams cost more than they
+// hide (64 x 384 x 56x56, one state: 216 -> 204 us, two: 298 -> 289; bf16, one state, loses: 171 -> 178).
 // EXT: the launch works on one column group of a wide plane (wave_wide() in snd_device.h): segments seg0 .. seg0+nseg-1.
 // The group's first wave takes what enters it on every row - h, s, a of the column on its left - from global memory,
 // where the launch of the group on the left put them (a band's values come with the band's loads, three per state and
@@ -57,7 +61,7 @@ namespace snd {
 // 64 x 384 x 56x56, one state, bf16: 288 -> 190 us, 64 x 768 x 28x28 178 -> 87, 64 x 1536 x 7x7 52 -> 28; out needs no
 // clearing before (18 us at the first of these).
 template <typename T, int NS, int CPL, bool VEC, bool SAVE, bool OUT32, int PK, int EU, bool ONE, bool EXT = false, bool EVEN = false, bool FOLD = false>
-__global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__((amdgpu_waves_per_eu(EU))) void wave_fwd_kernel(const snd_fwd_params p, const WaveGeo wg) {
+__global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__((amdgpu_waves_per_eu(EU, ONE && sizeof(T) == 4 ? 4 : 8))) void wave_fwd_kernel(const snd_fwd_params p, const WaveGeo wg) {
     static_assert(ONE || PK == 1, "packed planes are one segment wide");
     static_assert(!FOLD || (ONE && OUT32 && CPL == 1), "merge in LDS: one segment, fp32 out");
     static_assert(!EVEN || (!ONE && PK == 1 && CPL == 1 && !EXT), "whole planes: several segments, one column per lane");
@@ -283,15 +287,15 @@ __global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__(
                         bu[k] = bu[k] * du[k];
                         if (PK == 8) { a[k] = bar ? 0.f : a[k]; bu[k] = bar ? 0.f : bu[k]; }   // the barrier lane's map is (0, 0)
                     }
-                    const float a_l = from_prev_lane_pk<PK>(a[CPL - 1], in.z, sl == 0);                // a[i, j-1] of the lane's first column
-                    const float h_d = from_prev_lane_pk<PK>(hprev[n][CPL - 1], hdiag[n], sl == 0);     // h[i-1, j-1]
+                    const float a_l = ONE ? from_prev_lane_one<PK>(a[CPL - 1], sl == 0) : from_prev_lane_pk<PK>(a[CPL - 1], in.z, sl == 0);   // a[i, j-1] of the lane's first column
+                    const float h_d = ONE ? from_prev_lane_one<PK>(hprev[n][CPL - 1], sl == 0) : from_prev_lane_pk<PK>(hprev[n][CPL - 1], hdiag[n], sl == 0);   // h[i-1, j-1]
 #pragma unroll
                     for (int k = 0; k < CPL; ++k) {
                         const float al = k == 0 ? a_l : a[k > 0 ? k - 1 : 0], hd = k == 0 ? h_d : hprev[n][k > 0 ? k - 1 : 0];
                         const float X = fmaf(-0.5f * (aprev[n][k] + al), hd, hprev[n][k]);
                         y[k] = fmaf(a[k], X, bu[k]);
                     }
-                    wave_row_solve<CPL, PK>(a, y, bu, in.x, in.y, h, s);
+                    wave_row_solve<CPL, PK, ONE>(a, y, bu, in.x, in.y, h, s);
 #pragma unroll
                     for (int k = 0; k < CPL; ++k) {
                         acc[k] = fmaf(cv[k], fmaf(0.25f, bu[k], h[k] - s[k]), acc[k]);
