@@ -84,6 +84,10 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     // load a band's inputs one band ahead (with three or four states it measured 20 % slower, and with two columns per
     // lane the registers are needed elsewhere)
     constexpr bool PF = NS <= 2 && CPL == 1;
+    // The rows' hand-overs behind the band's last row instead of each behind its own: without a branch between the rows the
+    // compiler overlaps one row's sums with the next row's scan.  One state, 256 channels of 512x512 398 -> 383 us, 64 channels of
+    // 600x900 873 -> 831; two states lose by it (bands of two rows; 2 x 192 x 200x336 381 -> 386).
+    constexpr bool HO_LATE = !ONE && NS == 1;
     // what a wave leaves for the wave on its left: {G, P, -a/2, -} at its first column, per band parity, row and
     // state.  Wave w writes slot w and reads slot w+1; the slot after the last wave stays zero.
     __shared__ float4 sHO[ONE ? 1 : 2][ONE ? 1 : CHB][ONE ? 1 : kMaxSeg + 1][ONE ? 1 : R][NS];
@@ -446,6 +450,24 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
         // (from the band's last row up, rows past the plane's last included: their offsets are never used)
         const int mlast = mad24(i0 + R - 1, rs, r0m);
         uint32_t og = mad24(mlast, WB * rs, colG), o4 = mad24(mlast, W4 * rs, col4);   // du / ddelta and dB / dC offsets of the row
+        // what the segment on the left needs of the rows: G, P, -a/2 at this segment's first column
+        float ho[R][NS][3];
+        auto hand_over = [&](int r, int n) __attribute__((always_inline)) {
+            if (hands_over && lane == 63) sHO[step & 1][kc][w][r][n] = make_float4(ho[r][n][0], ho[r][n][1], ho[r][n][2], 0.f);
+            if (EXT && !SPL && ext_out && lane == 63) {   // for the column group on the left
+                float *d = eout + (int64_t)n * wave_bcol_plane(wg) + i0 + r;
+                d[0] = ho[r][n][0];
+                d[wg.Hp] = ho[r][n][1];
+                d[2 * wg.Hp] = ho[r][n][2];
+            }
+            if (SPL && ext_out && lane == 63) {           // for the left half: tagged with the band
+                float *d = eouttag + (int64_t)n * wave_split_words(wg) + (int64_t)band * (6 * R) + 2 * r;
+                const float tg = __builtin_bit_cast(float, (uint32_t)band + 1u);
+                st2_coherent(d, ho[r][n][0], tg);
+                st2_coherent(d + 2 * R, ho[r][n][1], tg);
+                st2_coherent(d + 4 * R, ho[r][n][2], tg);
+            }
+        };
 #pragma unroll
         for (int r = R - 1; r >= 0; --r) {
             {
@@ -527,20 +549,8 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                     GdEdge[n] = in.x;
 #pragma unroll
                     for (int t = 0; t < CPL; ++t) { Gd[n][t] = Gt[t]; td[n][t] = th[t]; }
-                    if (hands_over && lane == 63) sHO[step & 1][kc][w][r][n] = make_float4(Gt[CPL - 1], Pt[CPL - 1], th[CPL - 1], 0.f);
-                    if (EXT && !SPL && ext_out && lane == 63) {   // for the column group on the left
-                        float *d = eout + (int64_t)n * wave_bcol_plane(wg) + i0 + r;
-                        d[0] = Gt[CPL - 1];
-                        d[wg.Hp] = Pt[CPL - 1];
-                        d[2 * wg.Hp] = th[CPL - 1];
-                    }
-                    if (SPL && ext_out && lane == 63) {           // for the left half: tagged with the band
-                        float *d = eouttag + (int64_t)n * wave_split_words(wg) + (int64_t)band * (6 * R) + 2 * r;
-                        const float tg = __builtin_bit_cast(float, (uint32_t)band + 1u);
-                        st2_coherent(d, Gt[CPL - 1], tg);
-                        st2_coherent(d + 2 * R, Pt[CPL - 1], tg);
-                        st2_coherent(d + 4 * R, th[CPL - 1], tg);
-                    }
+                    ho[r][n][0] = Gt[CPL - 1]; ho[r][n][1] = Pt[CPL - 1]; ho[r][n][2] = th[CPL - 1];
+                    if (!HO_LATE) hand_over(r, n);
                 }
                 {
                     float duv[CPL], ddl[CPL];
@@ -564,6 +574,12 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
                 og -= WB;
                 o4 -= W4;
             }
+        }
+        if (HO_LATE) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int n = 0; n < NS; ++n) hand_over(r, n);
         }
         if (CHB > 1) {
             // Wave kc of a segment adds up rows kc, kc + CHB, ... of what the segment's CHB waves left and issues
