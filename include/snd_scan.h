@@ -76,7 +76,10 @@ typedef struct snd_plan {
                                                   (16-byte aligned, uninitialised; one row per plane) */
     int32_t auto_schedule;                     /* what SND_SCHED_AUTO resolves to in the forward for this shape
                                                   (PLANE, STRIPS, BANDS or WAVEFRONT): a caller may skip the fwd
-                                                  workspace for PLANE and WAVEFRONT (see wavefront_workspace) */
+                                                  workspace for PLANE and WAVEFRONT (see wavefront_workspace).  Where it is
+                                                  none of WAVEFRONT's, 5 to 16 states and few planes of at most 64 columns
+                                                  run on a kernel with a wave per state, which needs no workspace and saves
+                                                  the same state */
     int32_t auto_bwd_jobs;                     /* jobs per plane chunk SND_SCHED_AUTO gives the backward: 0 = one
                                                   block per plane chunk (also when auto_schedule is WAVEFRONT: then
                                                   the backward runs WAVEFRONT too and needs no workspace unless

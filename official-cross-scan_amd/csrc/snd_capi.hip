@@ -22,6 +22,9 @@ int launch_bwd_f16(const snd_bwd_params &p, hipStream_t stream);
 int launch_wave_fwd_f32(const snd_fwd_params &p, float *group_ws, hipStream_t stream);
 int launch_wave_fwd_bf16(const snd_fwd_params &p, float *group_ws, hipStream_t stream);
 int launch_wave_fwd_f16(const snd_fwd_params &p, float *group_ws, hipStream_t stream);
+int launch_wave_states_f32(const snd_fwd_params &p, hipStream_t stream);
+int launch_wave_states_bf16(const snd_fwd_params &p, hipStream_t stream);
+int launch_wave_states_f16(const snd_fwd_params &p, hipStream_t stream);
 int launch_wave_bwd_f32(const snd_bwd_params &p, float *group_ws, hipStream_t stream);
 int launch_wave_bwd_bf16(const snd_bwd_params &p, float *group_ws, hipStream_t stream);
 int launch_wave_bwd_f16(const snd_bwd_params &p, float *group_ws, hipStream_t stream);
@@ -202,6 +205,23 @@ int use_wavefront(const snd_shape &s, int schedule) {
     return schedule == SND_SCHED_AUTO && fits && wave_family_pays(s) ? 1 : 0;
 }
 
+// Whether a forward runs on the kernel with a wave per state (5 to 16 states, at most 64 columns).  Both sides in us, fitted to
+// measurements of 1 to 16 images of 64 to 768 channels, 5 to 16 states, 7x7 to 200x48, with and without saved state (one rule, so that
+// out does not depend on whether it is saved): the tile kernels take at least the longest chain of their tiles, however few the
+// planes; the other a row's scan times the rows, longer with more states in a block and, once the waves fill the GPU, with the
+// waves.  Where the two are close (16 states, bf16, tile kernels / wave per state, without | with saved state): 8 x 192 x 28x28
+// 44 / 32 | 47 / 44, taken; 8 x 192 x 56x56 92 / 99, 4 x 768 x 9x60 64 / 55 | 66 / 83, a single tile of 7x7 6.8 / 6.4 | 7.1 / 8.2, stay.
+bool wave_states_pays(const snd_fwd_params &p) {
+    const snd_shape &s = p.shape;
+    const snd::Geo g = snd::make_geo(s.nrows, s.ncols);
+    const int steps = g.nCX + g.nCY - 1;
+    if (p.schedule != SND_SCHED_AUTO || s.dstate < 5 || s.ncols > snd::kSeg || steps == 1) return false;
+    const int rg = s.dim / s.n_groups, pk = snd::wave_states_pack(s.ncols);
+    const double waves = (double)s.batch * s.n_groups * ((rg + pk - 1) / pk) * s.dstate;
+    const double alone = std::max(0.22, 0.10 + 0.0157 * s.dstate);
+    return 1.07 * (2.5 * std::max(1.0, waves / 8192) + s.nrows * std::max(alone, 0.17 + 7e-5 * waves)) <= 2.0 + 4.8 * steps;
+}
+
 // The kernels address inside one batch image with unsigned 32-bit BYTE offsets from a scalar base
 // and form row offsets with 24-bit multiplies: a (count x stride) walk plus rows must stay below
 // 2^32 bytes and a row pitch below 2^23 bytes.
@@ -369,6 +389,13 @@ int snd_fwd(const snd_fwd_params *params, snd_stream_t stream) {
         if (!aligned16(params->workspace)) return SND_ERR_ALIGN;
     } else if (params->schedule == SND_SCHED_STRIPS || params->schedule == SND_SCHED_BANDS) {
         return SND_ERR_WORKSPACE;
+    }
+    if (wave_states_pays(*params)) {
+        switch (params->shape.in_dtype) {
+            case SND_F32: return snd::launch_wave_states_f32(*params, (hipStream_t)stream);
+            case SND_BF16: return snd::launch_wave_states_bf16(*params, (hipStream_t)stream);
+            default: return snd::launch_wave_states_f16(*params, (hipStream_t)stream);
+        }
     }
     switch (params->shape.in_dtype) {
         case SND_F32: return snd::launch_fwd_f32(*params, (hipStream_t)stream);

@@ -586,6 +586,8 @@ __host__ __device__ inline int wave_groups(int nsegAll) { return (nsegAll + kMax
 // wide as a plane's lanes).  With eight planes the first lane of a plane is a barrier lane (wave_scan3_pk) and its
 // columns are in lanes 1..7.
 __host__ __device__ inline int wave_pack(const WaveGeo &g, int W) { return g.cpl == 1 && g.nsegAll == 1 ? (W <= 7 ? 8 : W <= 16 ? 4 : W <= 32 ? 2 : 1) : 1; }
+// planes per wave of the kernel with a wave per state: no barrier lanes, whose product with an infinity would reach the next plane
+__host__ __device__ inline int wave_states_pack(int W) { return W <= 16 ? 4 : W <= 32 ? 2 : 1; }
 __host__ __device__ inline WaveGeo make_wave_geo(int H, int W, int N) {
     WaveGeo g;
     g.cpl = wave_cpl(W, N);

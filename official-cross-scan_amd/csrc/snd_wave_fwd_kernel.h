@@ -519,4 +519,202 @@ int launch_wave_fwd_t(const snd_fwd_params &p, float *group_ws, hipStream_t stre
          : N == 3 ? launch_wave_fwd_v<T, 3, 1, true>(p, wg, stream) : launch_wave_fwd_v<T, 4, 1, true>(p, wg, stream);
 }
 
+// Forward of few planes with 5 to 16 states and at most 64 columns: a wave per state.  The tile kernels walk a plane tile by tile,
+// 49 or 64 cells one after the other by the same lanes, 4 to 5 us a tile whatever the launch; where the planes do not fill the GPU
+// that chain is all the call takes.  Here the N waves of a block hold one state each of the same channel (PK channels) and take a
+// whole row per step (a scan over its columns, as in the kernel above): the chain is a row's scan times the rows.
+// Rows are taken in bands of four and TE - 4, two bands to a strip of tiles.  What the states share is done once: the last waves
+// prepare a row of the next band each (softplus, delta' * u, through LDS), and the states' shares of out meet in LDS, where the first
+// waves add up and store a row each.  Both through two buffers, so that one barrier per band is enough.  One to four planes to a
+// wave, so that none sees another's infinities.
+// SAVE: state is saved as the tile kernels save it, and they run the backward: h of the last row of every strip but the last (x_v
+// [b][I][J][half][c][n][4 cols]), h and s of the last column of every tile that another follows (x, x_sd [b][J][I][half][c][n]
+// [4 rows]: a band's rows are one access), zeros where a tile extends beyond the plane.
+// us, tile kernels -> here, bf16, without | with saved state: 16 states, 1 x 64 x 14x14 18.4 -> 8.4 | 19.1 -> 10.7, 1 x 192 x 56x56
+// 67 -> 24 | 71 -> 30, 2 x 384 x 28x28 38 -> 22 | 40 -> 31; 8 states, 1 x 64 x 28x28 37 -> 9.5 | 38 -> 12.  (softplus and delta' * u
+// in every wave instead of once: 28 without saved state at 1 x 192 x 56x56.)
+template <typename T, bool OUT32, int PK, int TE, bool SAVE>
+__global__ __launch_bounds__(64 * 16) __attribute__((amdgpu_waves_per_eu(8))) void wave_states_kernel(const snd_fwd_params p, const WaveGeo wg, const Geo geo) {
+    constexpr int R = 4;                             // rows of a strip's first band (at least five waves: one for every row's output)
+    constexpr int S = 64 / PK;                       // lanes per plane
+    __shared__ float sAcc[2][16][R][64];             // the states' shares of out
+    __shared__ float2 sDl[2][R][64];                 // delta', delta' * u
+    const snd_shape &sh = p.shape;
+    const int H = sh.nrows, W = sh.ncols, N = sh.dstate, G = sh.n_groups, rg = wg.rg;
+    int pair, chunk;
+    if (!wave_job2(wg, sh.batch * G, pair, chunk)) return;   // (the whole block)
+    const int lane = threadIdx.x & 63, n = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));   // this wave's state
+    const int sl = PK > 1 ? lane % S : lane;         // the lane inside its plane: its scan column
+    chunk = chunk * PK + (PK > 1 ? lane / S : 0);
+    const bool act = PK == 1 || chunk < rg;          // (a plane past the group's last channel repeats it and stores nothing)
+    chunk = min(chunk, rg - 1);
+    int b, g;
+    wave_pair_split(wg, pair, G, b, g);
+    const int c = g * rg + chunk, cd = wg.rd == 1 ? c : c / wg.rd;   // channel of u, of delta
+    const bool fv = p.directions == SND_DIR_CORNERS && (g & 2), fh = p.directions == SND_DIR_CORNERS && (g & 1);
+    const int r0m = fv ? H - 1 : 0, rs = fv ? -1 : 1;
+    const bool jin = sl < W;
+    const int jc = min(sl, W - 1), mc = fh ? W - 1 - jc : jc;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
+        if (SAVE && geo.tag) *(uint32_t *)geo.tag = kTagTile;
+        if (p.workspace) ((int *)p.workspace)[kErrorWord] = 0;   // (as a pipelined launch leaves it: no wait has given up)
+    }
+
+    constexpr int ESZ = (int)sizeof(T);
+    using OutT = typename std::conditional<OUT32, float, T>::type;
+    const bool merge = p.merge != 0;
+    const T *Bb = (const T *)p.B + (int64_t)b * p.B_batch_stride + (int64_t)g * p.B_group_stride + n * p.B_dstate_stride;
+    const T *Cb = (const T *)p.C + (int64_t)b * p.C_batch_stride + (int64_t)g * p.C_group_stride + n * p.C_dstate_stride;
+    const T *ub = (const T *)p.u + (int64_t)b * p.u_batch_stride, *db = (const T *)p.delta + (int64_t)b * p.delta_batch_stride;
+    OutT *outb = (OutT *)p.out + (int64_t)b * p.out_batch_stride;
+    const int UhB = (int)p.u_h_stride * ESZ, DhB = (int)p.delta_h_stride * ESZ, BhB = (int)p.B_h_stride * ESZ, ChB = (int)p.C_h_stride * ESZ,
+              OhB = (int)p.out_h_stride * (int)sizeof(OutT);
+    const uint32_t colB = (uint32_t)mc * ESZ, colU = colB + (uint32_t)(p.u_shared ? chunk : c) * (uint32_t)p.u_d_stride * ESZ,
+                   colD = colB + (uint32_t)cd * (uint32_t)p.delta_d_stride * ESZ,
+                   colO = ((uint32_t)mc + (uint32_t)(merge ? chunk : c) * (uint32_t)p.out_d_stride) * (uint32_t)sizeof(OutT);
+
+    // (always in bounds: lanes beyond the last column read the last, rows beyond the last row the last; every wave the same loads,
+    // whether it prepares and stores a row or not: the waits for them can then be exact)
+    typedef WaveRaw<T, 1, true> Raw;
+    const int orow = n & (R - 1), prow = (N - 1 - n) & (R - 1);        // the row of a band this wave stores, and the one it prepares
+    const bool stores = n < R, prepares = N - 1 - n < R;
+    struct Stage { Raw b[R], c[R], uo, u, d; };      // B, C and the stored row's u of a band; u, delta of the band behind it
+    auto row0 = [&](int band) { return (band >> 1) * TE + (band & 1) * R; };   // a band's first row
+    auto mem_row = [&](int i) { return mad24(min(i, H - 1), rs, r0m); };
+    auto load_row = [&](Stage &q, int band) {
+        const int m = mem_row(row0(band) + prow);
+        wave_ld(q.u, ub, mad24(m, UhB, colU));
+        wave_ld(q.d, db, mad24(m, DhB, colD));
+    };
+    auto load_band = [&](Stage &q, int band) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {                // (a strip's second band: its fourth row, if any, is never used)
+            const int m = mem_row(row0(band) + r);
+            wave_ld(q.b[r], Bb, mad24(m, BhB, colB));
+            wave_ld(q.c[r], Cb, mad24(m, ChB, colB));
+        }
+        wave_ld(q.uo, ub, mad24(mem_row(row0(band) + orow), UhB, colU));
+        load_row(q, band + 1);
+    };
+    Stage sA, sB;
+    load_row(sB, 0);
+    load_band(sA, 0);
+    // (per-channel parameters behind the first band's loads, see above)
+    const float A2 = p.A[(int64_t)c * p.A_d_stride + (int64_t)n * p.A_dstate_stride] * kLog2e;
+    const float ld = p.A_decay ? __log2f(p.A_decay[0]) : 0.f;
+    const float Dv = p.D ? p.D[c] : 0.f, bias = p.delta_bias ? p.delta_bias[cd] : 0.f;
+    const float wm = merge && p.merge_weights ? p.merge_weights[c] : 1.f;
+    const bool softplus = p.delta_softplus != 0;
+
+    // (SAVE) this lane's tile and its column there; where its values of strip 0 go (64-bit, stepped from strip to strip)
+    const int J = sl / TE, tc = sl - J * TE;
+    const bool cols = act && tc == TE - 1 && J < geo.nCX - 1;
+    const int64_t DN4 = (int64_t)sh.dim * N * 4, lane4 = ((int64_t)c * N + n) * 4;
+    const int64_t xcol = ((int64_t)b * geo.nCX + J) * geo.nCY * 2 * DN4 + lane4;
+    float *sx = SAVE ? p.x + xcol : nullptr, *ss = SAVE ? p.x_sd + xcol : nullptr;
+    float *sv = SAVE ? p.x_v + ((int64_t)b * geo.nCY * geo.nCX + J) * 2 * DN4 + (tc >> 2) * DN4 + lane4 + (tc & 3) : nullptr;
+    // the columns of the plane's last tile beyond the plane's lanes, fewer than a tile's: their place from the lane's own
+    const int c2 = sl + S, J2 = c2 / TE, tc2 = c2 - J2 * TE;
+    const int64_t beyond = ((int64_t)(J2 - J) * 2 + (tc2 >> 2) - (tc >> 2)) * DN4 + (tc2 & 3) - (tc & 3);
+    const int nc = geo.nCX * TE;
+
+    auto prepare = [&](const Stage &q, int band) {
+        const float raw = wave_elem(q.d, 0) + bias;
+        float dsp, sp = softplus20(raw, dsp);
+        asm volatile("" : "+v"(sp));                 // (evaluated, then selected, as above)
+        const float dl = softplus ? sp : raw;
+        if (prepares) sDl[band & 1][prow][lane] = make_float2(dl, dl * wave_elem(q.u, 0));
+    };
+    prepare(sB, 0);
+    lds_barrier();
+    float hprev = 0.f, aprev = 0.f;                  // h, a of the row above
+    // RB rows, the first (four) or the second band of strip I
+    auto do_band = [&](auto RB_, Stage &cur, Stage &nxt, int band) {
+        constexpr int RB = decltype(RB_)::value, half = RB == R && TE == 8 ? -1 : RB == R ? 0 : 1;
+        const int odd = half < 0 ? band & 1 : half, i0 = row0(band);
+        load_band(nxt, band + 1);                    // (behind the last band: its last row once more, which nobody uses)
+        float2 dl[RB];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) dl[r] = sDl[odd][r][lane];
+        prepare(cur, band + 1);
+        float hc[R] = {}, sc[R] = {};
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            float a[1], y[1], bu[1], h[1], s_[1];
+            a[0] = fast_exp2(fmaf(dl[r].x, A2, ld));
+            bu[0] = wave_elem(cur.b[r], 0) * dl[r].y;
+            const float al = from_prev_lane_one<PK>(a[0], sl == 0), hd = from_prev_lane_one<PK>(hprev, sl == 0);
+            y[0] = fmaf(a[0], fmaf(-0.5f * (aprev + al), hd, hprev), bu[0]);
+            wave_row_solve<1, PK, true>(a, y, bu, 0.f, 0.f, h, s_);
+            sAcc[odd][n][r][lane] = wave_elem(cur.c[r], 0) * fmaf(0.25f, bu[0], h[0] - s_[0]);
+            hprev = h[0];
+            aprev = a[0];
+            if (SAVE) { hc[r] = i0 + r < H ? h[0] : 0.f; sc[r] = i0 + r < H ? s_[0] : 0.f; }
+        }
+        if (SAVE) {
+            if (cols) {
+                *(float4 *)(sx + odd * DN4) = make_float4(hc[0], hc[1], hc[2], hc[3]);
+                *(float4 *)(ss + odd * DN4) = make_float4(sc[0], sc[1], sc[2], sc[3]);
+            }
+            if (odd) {
+                if ((band >> 1) < geo.nCY - 1 && act) {
+                    if (sl < nc) *sv = jin ? hprev : 0.f;
+                    if (c2 < nc) sv[beyond] = 0.f;
+                }
+                sx += 2 * DN4;
+                ss += 2 * DN4;
+                sv += geo.nCX * 2 * DN4;
+            }
+        }
+        lds_barrier();
+        if (stores && orow < RB && i0 + orow < H) {
+            float t = 0.f;
+            for (int k = 0; k < N; ++k) t += sAcc[odd][k][orow][lane];
+            const float v = fmaf(Dv, wave_elem(cur.uo, 0), t);
+            const uint32_t o = mad24(mem_row(i0 + orow), OhB, colO);
+            if (jin && act) {
+                if (OUT32 && merge) glb_add((float *)((char *)outb + o), wm * v);
+                else stg_b(outb, o, v);
+            }
+        }
+    };
+    for (int I = 0; I < geo.nCY; ++I) {
+        do_band(std::integral_constant<int, R>(), sA, sB, 2 * I);
+        if (I * TE + R < H) {
+            do_band(std::integral_constant<int, TE - R>(), sB, sA, 2 * I + 1);
+        } else if (SAVE && cols) {                   // the last strip ends in its first band
+            *(float4 *)(sx + DN4) = make_float4(0.f, 0.f, 0.f, 0.f);
+            *(float4 *)(ss + DN4) = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+}
+
+template <typename T, int PK, int TE>
+static int launch_wave_states_p(const snd_fwd_params &p, const WaveGeo &wg, const Geo &geo, hipStream_t stream) {
+    constexpr bool F = std::is_same<T, float>::value;
+    const dim3 grid = wave_grid2(p.shape.batch * p.shape.n_groups, (wg.rg + PK - 1) / PK), block(64 * p.shape.dstate);
+    const bool save = p.x != nullptr, out32 = p.out_dtype == SND_F32;
+    if (save && out32) hipLaunchKernelGGL((wave_states_kernel<T, true, PK, TE, true>), grid, block, 0, stream, p, wg, geo);
+    else if (save) hipLaunchKernelGGL((wave_states_kernel<T, F, PK, TE, true>), grid, block, 0, stream, p, wg, geo);
+    else if (out32) hipLaunchKernelGGL((wave_states_kernel<T, true, PK, TE, false>), grid, block, 0, stream, p, wg, geo);
+    else hipLaunchKernelGGL((wave_states_kernel<T, F, PK, TE, false>), grid, block, 0, stream, p, wg, geo);
+    return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
+}
+
+template <typename T>
+int launch_wave_states_t(const snd_fwd_params &p, hipStream_t stream) {
+    const snd_shape &sh = p.shape;
+    if (sh.dstate < 5 || sh.dstate > 16 || sh.ncols > kSeg) return SND_ERR_SHAPE;
+    Geo geo = make_geo(sh.nrows, sh.ncols);
+    geo.tag = state_tag(p.x_sd, sh);
+    WaveGeo wg = make_wave_geo(sh.nrows, sh.ncols, sh.dstate);
+    wave_geo_channels(wg, sh.batch, sh.dim, sh.n_groups, sh.delta_dim);
+    const bool t7 = geo.te == 7;
+    switch (wave_states_pack(sh.ncols)) {
+        case 4: return t7 ? launch_wave_states_p<T, 4, 7>(p, wg, geo, stream) : launch_wave_states_p<T, 4, 8>(p, wg, geo, stream);
+        case 2: return t7 ? launch_wave_states_p<T, 2, 7>(p, wg, geo, stream) : launch_wave_states_p<T, 2, 8>(p, wg, geo, stream);
+        default: return t7 ? launch_wave_states_p<T, 1, 7>(p, wg, geo, stream) : launch_wave_states_p<T, 1, 8>(p, wg, geo, stream);
+    }
+}
+
 }  // namespace snd
