@@ -22,10 +22,13 @@
 // left stays in registers.  dB/dC are reduced over a wave's channels with lane swaps, over the block's waves
 // through LDS, and leave the block once per tile; du/ddelta are reduced over states by DPP and
 // finished once per pixel by the thread that staged it.
-// What the sweep evaluates per cell (26 vector instructions): the part of a lower row's contribution that does not depend on
-// the row above it is formed where the row is swept, K = G - a/2 * G[right], and G + Gs is carried instead of Gs, since
+// What the sweep evaluates per cell (22 vector instructions, and 7 for the sums over states and channels): the part of a lower
+// row's contribution that does not depend on the row above it is formed where the row is swept, K = G - a/2 * G[right]; G + Gs is
+// carried instead of Gs, since
 //     g = dout*C + G[i,j+1] + K[i+1,j] - a[i,j+1]/2 * G[i+1,j+1]       g + gs = (G + Gs)[i,j+1] + K[i+1,j] - a[i,j+1]/2 * G[i+1,j+1]
-// share their tail and dout*C cancels in the second.
+// share their tail and dout*C cancels in the second; s - bu is a * s[left]; and the quarter terms of dB, dC and sum_n dbu*B are
+// left to sums per pixel (flush_bc).  With the rest of a tile about 49 vector instructions per cell: two waves per SIMD issue
+// them in 60 % of the kernel's time (64 x 192 x 56x56), the remainder are waits for operands, barriers and memory.
 // As in the forward, tiles are computed in full on zero-padded staging (dout = B = C = 0 outside
 // the plane makes every adjoint there exactly zero), so the inner loops have no bounds checks.
 #pragma once

@@ -63,7 +63,8 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // neighbours beyond the plane are zeros, and nothing is handed over or waited for.  Bound by its vector instructions (167 a row
 // of 64 cells, four waves per SIMD).  Together with the softplus taken out of its branch and P swept instead of Gs, 137 a row (us):
 // 64 x 384 x 56x56 bf16, one state 381 -> 336, two 632 -> 542; 8 x 384 x 56x56, four 174 -> 140; 8 x 96 x 56x56 fp32, three
-// 99 -> 68; packed, 32 x 768 x 28x28 92 -> 86; several segments (no ONE) 64 x 96 x 112x112 411 -> 408.
+// 99 -> 68; packed, 32 x 768 x 28x28 92 -> 86; several segments (no ONE) 64 x 96 x 112x112 411 -> 408;
+// one channel per block, 1 x 192 x 56x56 bf16, one state 31 -> 26, 1 x 64 x 56x56 fp32, two 51 -> 35.
 template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1)>
 __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
@@ -705,6 +706,7 @@ static int launch_wave_bwd_v(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     if (share == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, 1>(p, wg, stream);
     if (share == 2 && wg.nseg > 4) return launch_wave_bwd_c<T, NS, CPL, VEC, (CPL == 1 && NS <= 2) ? 2 : 1, 1, (CPL == 1 && NS <= 2) ? 16 : kMaxSeg>(p, wg, stream);
     if (share == 2) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 2 : 1, 1>(p, wg, stream);
+    if (wg.nseg == 1) return launch_wave_bwd_c<T, NS, CPL, VEC, 1, 1, kMaxSeg, CPL == 1>(p, wg, stream);
     return launch_wave_bwd_c<T, NS, CPL, VEC, 1, 1>(p, wg, stream);
 }
 
