@@ -108,10 +108,15 @@ __device__ __forceinline__ void sweep_reduce16(float &q0, float &q1, float &q2, 
 // SEG: (pipelined strips only) a job is a column segment of a strip; the carried column state goes from one
 // segment's block to the next through the workspace (strip_segments).  A variant of its own, because the few
 // registers it takes are registers the other variants do not have.
-template <typename T, int NP, bool PIPE, int TE, bool VEC, bool SEG = false>
+// SINGLE: (whole planes) the plane is one tile: no tile follows whose inputs would be requested - the general kernel requests its own
+// again - and nothing enters it, so no checkpoint is read.  64 x 1536 x 7x7 bf16, 16 states 174 -> 147 us, 64 x 768 x 7x7 fp16,
+// 8 states 72 -> 60, 8 x 768 x 7x7 18.6 -> 16.1.  Branches around the requests instead: planes of several tiles lose up to 7 %
+// (32 x 768 x 28x28 548 -> 586).
+template <typename T, int NP, bool PIPE, int TE, bool VEC, bool SEG = false, bool SINGLE = false>
 __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_kernel(const snd_bwd_params p, const Geo geo) {
     static_assert(!VEC || TE == 8, "vector staging needs 8x8 tiles");
     static_assert(!SEG || PIPE, "column segments belong to the strip pipeline");
+    static_assert(!SINGLE || !PIPE, "a plane of one tile has no strips");
     constexpr int WPB = NP / 4;                     // waves per block
     constexpr int CB = 16;                          // channels per block
     constexpr int NSTR = kTile + 4;
@@ -563,8 +568,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     load_part(I_hi, J_hi, 0);
     load_part(I_hi, J_hi, 1);
     load_part(I_hi, J_hi, 2);
-    load_row_ckpt(I_hi, J_hi);
-    load_col_ckpt(I_hi, J_hi);
+    if (!SINGLE) {
+        load_row_ckpt(I_hi, J_hi);
+        load_col_ckpt(I_hi, J_hi);
+    }
     for (int I = I_hi; I >= I_lo; --I) {
         const int r0 = I * TE;
         float GR[kRows], SR[kRows];                 // G, G + Gs at the column right of the tile
@@ -604,12 +611,12 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             int In = I, Jn = J - 1;
             if (Jn < (SEG ? J_lo : 0)) { In = I - 1; Jn = J_hi; }
             if (In < I_lo) { In = I; Jn = J; }
-            if (I == 0) {
+            if (SINGLE || I == 0) {
 #pragma unroll
                 for (int j = 0; j < kCkX; ++j) hu[j] = 0.f;
                 hc = 0.f;
             }
-            if (J == 0) {
+            if (SINGLE || J == 0) {
 #pragma unroll
                 for (int r = 0; r < kRows; ++r) { hlft[r] = 0.f; slft[r] = 0.f; }
                 hc = 0.f;
@@ -620,7 +627,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // rows; rows whose hand-over an earlier poll has already seen), else after the wait below.
             const bool handed = PIPE && I == I_hi && I + 1 < geo.nCY;
             auto take_row = [&](int J_) __attribute__((always_inline)) {   // (pipelined schedules: through coherent words)
-                if (I + 1 < geo.nCY && lvalid) {
+                if (!SINGLE && I + 1 < geo.nCY && lvalid) {
                     const char *src = gdown + (int64_t)J_ * DN8 * 4;
                     if (PIPE) {
 #pragma unroll
@@ -781,9 +788,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
             for (int r = TE - 1; r >= 0; --r) {
                 // the next tile's loads, between the rows of the second half, where the registers of the rows swept are free
-                if (r == 4) load_part(In, Jn, 0);
-                if (r == 3) load_part(In, Jn, 1);
-                if (r == 2) load_part(In, Jn, 2);
+                if (!SINGLE && r == 4) load_part(In, Jn, 0);
+                if (!SINGLE && r == 3) load_part(In, Jn, 1);
+                if (!SINGLE && r == 2) load_part(In, Jn, 2);
                 float Gr = GR[r], Sr = SR[r], Gdiag = Gd8, tr = tR[r];
 #pragma unroll
                 for (int C0 = 4; C0 >= 0; C0 -= 4) {
@@ -878,7 +885,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 pC[k] = sC[(wave_u + WPB * k) * NSTR + (tid & 63)];
             }
             const bool hands_over = PIPE && I == I_lo && I > 0;   // top strip of a band: another block takes the row
-            if (I > 0 && lvalid) {                  // adjoint row for the strip above
+            if (!SINGLE && I > 0 && lvalid) {       // adjoint row for the strip above
                 char *dst = gdown + (int64_t)J * DN8 * 4;
                 if (PIPE) {
 #pragma unroll
@@ -893,8 +900,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             __syncthreads();
             if (hands_over) strip_signal(progress + I);   // tile J is handed over to the strip above
             // (not ahead of the hand-over: its wait for the row's stores would cover them)
-            load_row_ckpt(In, Jn);
-            load_col_ckpt(In, Jn);
+            if (!SINGLE) {
+                load_row_ckpt(In, Jn);
+                load_col_ckpt(In, Jn);
+            }
 
             pI = I; pJ = J;
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
@@ -1020,6 +1029,9 @@ template <typename T, int NP, int TE, bool VEC> static bool configure_bwd_one() 
     const int lds = (int)bwd_lds_bytes<NP, TE>();
     if (NP == 16 && hipFuncSetAttribute((const void *)bwd_kernel<T, NP, true, TE, VEC, NP == 16>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return false;
+    constexpr bool S = TE == 7 || VEC;               // (8x8 tiles element by element: the general kernel)
+    if (S && hipFuncSetAttribute((const void *)bwd_kernel<T, NP, false, TE, VEC, false, S>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        return false;
     return hipFuncSetAttribute((const void *)bwd_kernel<T, NP, true, TE, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess &&
            hipFuncSetAttribute((const void *)bwd_kernel<T, NP, false, TE, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
 }
@@ -1085,7 +1097,11 @@ static int launch_bwd_te(const snd_bwd_params &p, const Geo &geo, hipStream_t st
             hipLaunchKernelGGL((bwd_kernel<T, NP, true, TE, VEC>), dim3((int)(nPC * bands)), dim3(16 * NP), lds, stream, p, gb);
     } else {
         const int grid = xcd_grid(sh.batch * sh.n_groups, nChunks);
-        hipLaunchKernelGGL((bwd_kernel<T, NP, false, TE, VEC>), dim3(grid), dim3(16 * NP), lds, stream, p, geo);
+        constexpr bool S = TE == 7 || VEC;
+        if (S && geo.nCX == 1 && geo.nCY == 1)
+            hipLaunchKernelGGL((bwd_kernel<T, NP, false, TE, VEC, false, S>), dim3(grid), dim3(16 * NP), lds, stream, p, geo);
+        else
+            hipLaunchKernelGGL((bwd_kernel<T, NP, false, TE, VEC>), dim3(grid), dim3(16 * NP), lds, stream, p, geo);
     }
     return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
 }

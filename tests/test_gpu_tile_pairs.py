@@ -1,6 +1,6 @@
 """The tile backward's dB / dC: neighbouring 8x8 tiles of a strip leave together (an odd tile out at either end leaves alone), the
 terms that all states or all channels share are summed per pixel, and each tile's inputs are requested under the tile before it.
-Odd and even numbers of tiles, tiles cut by the plane's edge, vector and element-wise staging, 7x7 tiles, fewer states than lanes,
+Odd and even numbers of tiles, a single one, tiles cut by the plane's edge, vector and element-wise staging, 7x7 tiles, fewer states than lanes,
 against the float64 oracle."""
 import pytest
 import torch
@@ -24,6 +24,11 @@ PAIRS = [
     (2, 64, 14, 14, 16, torch.float32, dict(dirs=capi.DIR_CORNERS)),  # 7x7 tiles
     (1, 64, 16, 72, 16, torch.bfloat16, dict(dirs=capi.DIR_CORNERS)),
     (1, 64, 13, 45, 8, torch.float16, {}),
+    (2, 72, 7, 7, 16, torch.float32, dict(dirs=capi.DIR_CORNERS, decay=0.9)),   # planes of a single tile: 7x7, cut, 8x8
+    (3, 64, 5, 6, 9, torch.bfloat16, {}),
+    (2, 64, 8, 8, 7, torch.float32, dict(dirs=capi.DIR_CORNERS)),
+    (2, 64, 8, 8, 16, torch.bfloat16, {}),
+    (2, 64, 6, 7, 3, torch.float32, {}),
 ]
 
 
