@@ -309,7 +309,7 @@ int snd_make_plan(const snd_shape *shape, snd_plan *plan) {
     if (wave && snd::wave_wide(shape->ncols, shape->dstate)) {
         plan->wavefront_workspace = 1;
         // wide planes under the row-segment kernels: what column groups hand over (behind the sync words, which stay
-        // the tile kernels'): forward without saved state, a stand-in for x and x_sd; backward, G, Gs, a per boundary
+        // the tile kernels'): forward without saved state, a stand-in for x and x_sd; backward, G, G + Gs, -a/2 per boundary
         const snd::WaveGeo wg = snd::make_wave_geo(shape->nrows, shape->ncols, shape->dstate);
         const int64_t off = group_ws_offset(*shape);
         const int64_t fw = off + 2 * planes * snd::wave_x_plane(wg) * (int64_t)sizeof(float), bw = off + planes * snd::wave_bcol_plane(wg) * (int64_t)sizeof(float);

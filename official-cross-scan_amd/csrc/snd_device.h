@@ -416,7 +416,7 @@ __host__ inline int job_queues(int nPairs) { return nPairs >= 16 ? 8 : 1; }
 // the ticket order through a list-scheduling model (unit tile time, `slots` blocks at once; cached per shape):
 // segments are taken where the model gains at least 8 %.  (256 channels of 512 x 512: 159 steps either way.)
 int strip_segments(int64_t nPlaneChunks, int nStrips, int nTilesX, int64_t slots, int nQueues);
-// floats of one strip's carried column state in the workspace (G, Gs, a of eight rows and the corner G per lane of a
+// floats of one strip's carried column state in the workspace (G, G + Gs, -a/2 of eight rows and the corner G per lane of a
 // 256-thread block, as 8-byte words of all lanes one after the other)
 constexpr int kColStateFloats = 13 * 2 * 256;
 // Enqueue a fill kernel that zeroes n int32 words (defined with the C entry points).
@@ -577,7 +577,7 @@ __host__ __device__ inline int wave_cpl(int W, int N) { return (N <= 1 && W > kS
 __host__ __device__ inline bool wave_family_fits(int W, int N) { return N <= 4; }
 // A wide plane: more row segments than a block has waves.  Its segments are taken in column groups of kMaxSeg, left to
 // right in the forward and right to left in the backward, one launch per group (the stream orders them); what crosses a
-// group boundary - h, s, a of the column on its left (forward), G, Gs, a of the column on its right (backward), per row
+// group boundary - h, s, a of the column on its left (forward), G, G + Gs, -a/2 of the column on its right (backward), per row
 // and state - goes through global memory instead of LDS.
 __host__ __device__ inline bool wave_wide(int W, int N) { return (W + kSeg * wave_cpl(W, N) - 1) / (kSeg * wave_cpl(W, N)) > kMaxSeg; }
 __host__ __device__ inline int wave_groups(int nsegAll) { return (nsegAll + kMaxSeg - 1) / kMaxSeg; }
@@ -611,7 +611,7 @@ __host__ __device__ inline WaveGeo make_wave_geo(int H, int W, int N) {
 typedef float wave_f2 __attribute__((ext_vector_type(2)));
 __host__ __device__ inline int64_t wave_x_plane(const WaveGeo &g) { return (int64_t)g.nsegAll * 2 * g.Hp; }
 // (wide planes, backward) the hand-over between column groups, per (batch, channel, state) plane:
-//   bcol [group q][3][Hp]   G, Gs, a at the first column of group q on every row (written by group q, read by group q-1)
+//   bcol [group q][3][Hp]   G, G + Gs, -a/2 at the first column of group q on every row (written by group q, read by group q-1)
 __host__ __device__ inline int64_t wave_bcol_plane(const WaveGeo &g) { return (int64_t)wave_groups(g.nsegAll) * 3 * g.Hp; }
 // Split planes (backward).  Few planes of eight segments with one or two states - 256 planes of 512 x 512 are
 // one block of eight waves per CU - leave no room for two channels in a block, which is what halves the dB / dC

@@ -19,7 +19,7 @@
 // a register crossbar move, no LDS memory).
 // A wave handles its segment band by band (R rows), bottom band first: recompute h, s of the band's rows
 // from the forward's checkpoints (row above the band from x_v, what entered the segment on every row from
-// x / x_sd: no wave waits for another here), then sweep the band's rows bottom-up.  The sweep needs G, P = G + Gs, a
+// x / x_sd: no wave waits for another here), then sweep the band's rows bottom-up.  The sweep needs G, P = G + Gs, -a/2
 // of the segment on the right at its first column: wave w runs one band behind wave w+1 and finds them in
 // LDS (one block barrier per band, no polling).  dB, dC leave as one global atomic per element and channel
 // (a wave-wide instruction covers 256 consecutive bytes), du / ddelta as whole row segments.
