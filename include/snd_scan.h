@@ -75,11 +75,8 @@ typedef struct snd_plan {
     int64_t fwd_workspace_bytes;               /* scratch fwd uses when it splits planes into strips
                                                   (16-byte aligned, uninitialised; one row per plane) */
     int32_t auto_schedule;                     /* what SND_SCHED_AUTO resolves to in the forward for this shape
-                                                  (PLANE, STRIPS, BANDS or WAVEFRONT): a caller may skip the fwd
-                                                  workspace for PLANE and WAVEFRONT (see wavefront_workspace).  Where it is
-                                                  none of WAVEFRONT's, 5 to 16 states and few planes of at most 64 columns
-                                                  run on a kernel with a wave per state, which needs no workspace and saves
-                                                  the same state */
+                                                  (PLANE, STRIPS, BANDS or WAVEFRONT) unless wave_per_state is 1: a caller may
+                                                  skip the fwd workspace for PLANE and WAVEFRONT (see wavefront_workspace) */
     int32_t auto_bwd_jobs;                     /* jobs per plane chunk SND_SCHED_AUTO gives the backward: 0 = one
                                                   block per plane chunk (also when auto_schedule is WAVEFRONT: then
                                                   the backward runs WAVEFRONT too and needs no workspace unless
@@ -103,7 +100,12 @@ typedef struct snd_plan {
                                                   states (at most 256 planes, e.g. 256 of 512x512): bwd cuts each plane
                                                   in two halves that run side by side if it is given its workspace
                                                   (about a fifth faster), and runs whole planes without one */
-    int32_t reserved_;
+    int32_t wave_per_state;                    /* 1 if SND_SCHED_AUTO's forward runs the kernel with a wave per state (few
+                                                  planes of at most 64 columns, 5 to 16 states); auto_schedule is then what
+                                                  the tile kernels would take in its place.  It needs no fwd workspace (nothing
+                                                  is cleared, snd_clear_bytes() is 0) and uses none of x_v where no state is
+                                                  saved; the state it saves is the tile kernels', which run the backward.
+                                                  (Reserved, 0, before version 211.) */
 } snd_plan;
 
 /* How a launch maps work to blocks.  The reference has one fixed mapping (one block per
@@ -148,15 +150,16 @@ typedef struct snd_fwd_params {
                                       required (it also carries h from one row strip to the next);
                                       x and x_sd may both be null = inference only (bwd impossible): x_v is
                                       then scratch, of which the first x_v_elems / n_chunks_y *
-                                      min(4, n_chunks_y) floats are used (none by the row-segment kernels) */
+                                      min(4, n_chunks_y) floats are used (none by the row-segment
+                                      kernels or where snd_plan.wave_per_state is 1) */
     int64_t u_batch_stride, u_d_stride, u_h_stride;
     int64_t delta_batch_stride, delta_d_stride, delta_h_stride;
     int64_t A_d_stride, A_dstate_stride;
     int64_t B_batch_stride, B_group_stride, B_dstate_stride, B_h_stride;
     int64_t C_batch_stride, C_group_stride, C_dstate_stride, C_h_stride;
     int64_t out_batch_stride, out_d_stride, out_h_stride;
-    void *workspace;               /* plan.fwd_workspace_bytes bytes, 16-byte aligned, or null (then the
-                                      PLANE schedule is used).  In snd_bwd_params.f it is ignored. */
+    void *workspace;               /* plan.fwd_workspace_bytes bytes, 16-byte aligned, or null (the tile kernels
+                                      then use the PLANE schedule).  In snd_bwd_params.f it is ignored. */
     int64_t workspace_bytes;
     int32_t schedule;              /* snd_schedule, for fwd and (through snd_bwd_params.f) for bwd */
     int32_t directions;            /* snd_directions, for fwd and (through snd_bwd_params.f) for bwd */

@@ -207,15 +207,14 @@ int use_wavefront(const snd_shape &s, int schedule) {
 
 // Whether a forward runs on the kernel with a wave per state (5 to 16 states, at most 64 columns).  Both sides in us, fitted to
 // measurements of 1 to 16 images of 64 to 768 channels, 5 to 16 states, 7x7 to 200x48, with and without saved state (one rule, so that
-// out does not depend on whether it is saved): the tile kernels take at least the longest chain of their tiles, however few the
-// planes; the other a row's scan times the rows, longer with more states in a block and, once the waves fill the GPU, with the
-// waves.  Where the two are close (16 states, bf16, tile kernels / wave per state, without | with saved state): 8 x 192 x 28x28
+// out does not depend on whether it is saved; from the shape alone, so that the plan, snd_clear_bytes() and the launch agree): the
+// tile kernels take at least the longest chain of their tiles, however few the planes; the other a row's scan times the rows, longer
+// with more states in a block and, once the waves fill the GPU, with the waves.  Where the two are close (16 states, bf16, tile kernels / wave per state, without | with saved state): 8 x 192 x 28x28
 // 44 / 32 | 47 / 44, taken; 8 x 192 x 56x56 92 / 99, 4 x 768 x 9x60 64 / 55 | 66 / 83, a single tile of 7x7 6.8 / 6.4 | 7.1 / 8.2, stay.
-bool wave_states_pays(const snd_fwd_params &p) {
-    const snd_shape &s = p.shape;
+bool wave_states_pays(const snd_shape &s, int schedule) {
     const snd::Geo g = snd::make_geo(s.nrows, s.ncols);
     const int steps = g.nCX + g.nCY - 1;
-    if (p.schedule != SND_SCHED_AUTO || s.dstate < 5 || s.ncols > snd::kSeg || steps == 1) return false;
+    if (schedule != SND_SCHED_AUTO || s.dstate < 5 || s.ncols > snd::kSeg || steps == 1) return false;
     const int rg = s.dim / s.n_groups, pk = snd::wave_states_pack(s.ncols);
     const double waves = (double)s.batch * s.n_groups * ((rg + pk - 1) / pk) * s.dstate;
     const double alone = std::max(0.22, 0.10 + 0.0157 * s.dstate);
@@ -259,7 +258,7 @@ int check_fwd(const snd_fwd_params &p, bool need_state) {
 
 extern "C" {
 
-int snd_version(void) { return 210; }
+int snd_version(void) { return 211; }
 
 const char *snd_status_string(int status) {
     switch (status) {
@@ -305,7 +304,7 @@ int snd_make_plan(const snd_shape *shape, snd_plan *plan) {
     plan->fwd_workspace_bytes = sync_bytes + row_bytes;      // the strip schedule's hand-over row of h
     plan->bwd_workspace_bytes = sync_bytes + row_bytes;      // the adjoint row G = a*g
     plan->wavefront_workspace = 0;
-    plan->reserved_ = 0;
+    plan->wave_per_state = wave_states_pays(*shape, SND_SCHED_AUTO) ? 1 : 0;
     if (wave && snd::wave_wide(shape->ncols, shape->dstate)) {
         plan->wavefront_workspace = 1;
         // wide planes under the row-segment kernels: what column groups hand over (behind the sync words, which stay
@@ -390,7 +389,7 @@ int snd_fwd(const snd_fwd_params *params, snd_stream_t stream) {
     } else if (params->schedule == SND_SCHED_STRIPS || params->schedule == SND_SCHED_BANDS) {
         return SND_ERR_WORKSPACE;
     }
-    if (wave_states_pays(*params)) {
+    if (wave_states_pays(params->shape, params->schedule)) {
         switch (params->shape.in_dtype) {
             case SND_F32: return snd::launch_wave_states_f32(*params, (hipStream_t)stream);
             case SND_BF16: return snd::launch_wave_states_bf16(*params, (hipStream_t)stream);
@@ -467,6 +466,7 @@ int64_t snd_clear_bytes(const snd_shape *shape, int schedule, int backward) {
         if (!backward || snd::wave_wide(s.ncols, s.dstate) || !snd::wave_bwd_split(s.batch, s.dim, s.ncols, s.dstate)) return 0;
         return group_ws_offset(s) + (int64_t)s.batch * s.dim * s.dstate * snd::wave_split_words(snd::make_wave_geo(s.nrows, s.ncols, s.dstate)) * (int64_t)sizeof(float);
     }
+    if (!backward && wave_states_pays(s, schedule)) return 0;      // (a wave per state hands nothing over between blocks)
     const snd::Geo g = snd::make_geo(s.nrows, s.ncols);
     const int64_t pairs = (int64_t)s.batch * s.n_groups;
     const int nChunks = (s.dim / s.n_groups + 15) / 16;

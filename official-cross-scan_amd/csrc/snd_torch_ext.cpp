@@ -229,17 +229,17 @@ at::Tensor launch_fwd(const Checked &c, const at::Tensor &u, const at::Tensor &d
     p.merge_weights = o.merge && merge_weights_.has_value() ? merge_weights_.value().data_ptr<float>() : nullptr;
     // scratch for the pipelined schedules, and for wide planes without saved state (only when it will be used); released to
     // the caching allocator in stream order
-    const bool wave = wavefront(o.sched, c.plan);
-    const bool need_ws = wave ? !x && c.plan.wavefront_workspace : pipelined(o.sched, c.plan.auto_schedule);
+    const bool wave = wavefront(o.sched, c.plan), states = o.sched == SND_SCHED_AUTO && c.plan.wave_per_state;
+    const bool need_ws = wave ? !x && c.plan.wavefront_workspace : !states && pipelined(o.sched, c.plan.auto_schedule);
     at::Tensor ws, scratch;
     if (need_ws) {
         ws = floats((c.plan.fwd_workspace_bytes + 3) / 4, u);
         p.workspace = ws.data_ptr();
         p.workspace_bytes = c.plan.fwd_workspace_bytes;
     }
-    if (!x) {                                       // (the row-segment kernels carry the row in registers and touch none of it)
+    if (!x) {                                       // (where a wave takes whole rows it carries them in registers and touches none of it)
         const int64_t slabs = std::min(4, (int)c.plan.n_chunks_y);
-        scratch = floats(wave ? 4 : c.plan.x_v_elems / c.plan.n_chunks_y * slabs, u);
+        scratch = floats(wave || states ? 4 : c.plan.x_v_elems / c.plan.n_chunks_y * slabs, u);
         x_v = scratch.data_ptr<float>();
     }
     p.x = x; p.x_v = x_v; p.x_sd = x_sd;

@@ -2,6 +2,8 @@
 the tile kernels over what the route accepts - one, two and four planes to a wave and partly filled waves, rows that are no
 multiple of a band, mirrored orders, spaced rows, shared delta, both out types, the fused merge, decay, no softplus, infinities, a
 captured graph - and the tile backward from the state it saves."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -9,6 +11,7 @@ import torch
 import capi
 from oracle import snd_oracle as O
 from oracle_ref import reference
+from selective_nd_scan import selective_nd_scan
 from test_gpu_fwd import relerr
 from test_gpu_wave import NAMES
 
@@ -134,3 +137,24 @@ def test_wave_per_state_in_a_captured_graph(gpu_device):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(f.out, e.out)
+
+
+def test_wave_per_state_is_one_launch(gpu_device):
+    """The public call without gradients: out and nothing beside it is worked on - no workspace, no clearing launch."""
+    _, t = _make(gpu_device, 1, 64, 14, 14, 16, 4, None, torch.float32)
+    args = [t[k] for k in ("u", "delta", "A", "B", "C", "D", "delta_bias")]
+    with torch.no_grad():
+        ref = selective_nd_scan(*args, True)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            out = selective_nd_scan(*args, True)
+    n = C.c_size_t(0)
+    assert capi.lib().hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    assert n.value == 1
+    g.instantiate()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)

@@ -329,6 +329,25 @@ def test_pipeline_error_contract_on_the_host():
     assert "word [1] is an error flag" in header and "snd_workspace_error" in header
 
 
+@pytest.mark.parametrize("shape,states", [
+    ((1, 64, 14, 14, 16), 1), ((2, 384, 14, 14, 16), 1), ((1, 192, 56, 56, 16), 1), ((2, 384, 28, 28, 16), 1), ((1, 64, 28, 28, 8), 1),
+    ((8, 192, 28, 28, 16), 1), ((64, 192, 56, 56, 16), 0), ((1, 64, 7, 7, 16), 0), ((3, 152, 61, 83, 8), 0), ((1, 64, 14, 14, 4), 0),
+])
+def test_plan_names_the_forward_with_a_wave_per_state(shape, states):
+    """The plan says where AUTO's forward runs a wave per state; nothing is to be cleared for it then.  An explicit schedule, and
+    the backward, run the tile kernels and are planned as ever."""
+    sh = capi.Shape(*shape, 4, shape[1], capi.SND_BF16)
+    st, plan = capi.make_plan(sh)
+    assert st == 0 and plan.wave_per_state == states
+    clear = lambda sched, backward: capi.lib().snd_clear_bytes(C.byref(sh), sched, backward)
+    if states:
+        assert clear(capi.SCHED_AUTO, 0) == 0
+        assert clear(capi.SCHED_STRIPS, 0) == clear(capi.SCHED_STRIPS, 1) > 0
+        assert clear(capi.SCHED_AUTO, 1) == (clear(capi.SCHED_STRIPS, 1) if plan.auto_bwd_jobs else 0)
+    else:
+        assert (clear(capi.SCHED_AUTO, 0) > 0) == (plan.auto_schedule in (capi.SCHED_STRIPS, capi.SCHED_BANDS))
+
+
 def test_init_without_a_gpu_is_a_status_not_a_crash():
     torch = pytest.importorskip("torch")
     if torch.cuda.is_available():
