@@ -122,7 +122,12 @@ typedef struct snd_plan {
  *           (what AUTO picks whenever its timing model prefers it).  Planes of more than eight segments
  *           are taken in column groups of eight, one launch per group (snd_plan.wavefront_workspace).  Its saved state has a
  *           layout of its own: fwd and bwd of one call pair must both run WAVEFRONT or both run one of the
- *           three tile schedules above (AUTO decides by shape alone, so AUTO on both sides always agrees). */
+ *           three tile schedules above (AUTO decides by shape alone, so AUTO on both sides always agrees).
+ *           It solves a row by a scan that multiplies the a = exp(delta' * A) * A_decay of neighbouring cells before
+ *           any state meets them, as the reference's block scan does (common.h:100-107).  With a <= 1 (A <= 0, as
+ *           models have it) that is safe; with a > 1 the product over up to 64 cells can overflow where the recurrence
+ *           itself stays finite, and the results behind it in the plane are then inf or NaN.  The tile schedules, and
+ *           the forward of snd_plan.wave_per_state, take such rows cell by cell. */
 typedef enum snd_schedule { SND_SCHED_AUTO = 0, SND_SCHED_PLANE = 1, SND_SCHED_STRIPS = 2, SND_SCHED_BANDS = 3, SND_SCHED_WAVEFRONT = 4 } snd_schedule;
 
 /* Scan origin per group.  The reference scans every group from the top-left corner and leaves the

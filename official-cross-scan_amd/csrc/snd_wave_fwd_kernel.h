@@ -519,6 +519,22 @@ int launch_wave_fwd_t(const snd_fwd_params &p, float *group_ws, hipStream_t stre
          : N == 3 ? launch_wave_fwd_v<T, 3, 1, true>(p, wg, stream) : launch_wave_fwd_v<T, 4, 1, true>(p, wg, stream);
 }
 
+// A row of the kernel below cell by cell, as the tile kernels take it: t_j = a_j*t_{j-1} + y_j, and the same with s_j.  `bad`: the
+// lanes whose scanned value is not finite; planes with such a lane take what is computed here.  After k steps the first k + 1 cells
+// are right.
+template <int PK> __device__ __forceinline__ void wave_row_cells(float a, float y, float sv, uint64_t bad, float &h, float &s) {
+    constexpr int S = 64 / PK;
+    const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), sl = lane % S;
+    float eh = y, es = sv;
+#pragma unroll 1
+    for (int k = 1; k < S; ++k) {
+        const float th = from_prev_lane_one<PK>(eh, sl == 0), ts = from_prev_lane_one<PK>(es, sl == 0);
+        eh = fmaf(a, th, y);
+        es = fmaf(a, ts, sv);
+    }
+    if (PK == 1 || ((bad >> (lane - sl)) & ((1ull << (S & 63)) - 1)) != 0) { h = eh; s = es; }
+}
+
 // Forward of few planes with 5 to 16 states and at most 64 columns: a wave per state.  The tile kernels walk a plane tile by tile,
 // 49 or 64 cells one after the other by the same lanes, 4 to 5 us a tile whatever the launch; where the planes do not fill the GPU
 // that chain is all the call takes.  Here the N waves of a block hold one state each of the same channel (PK channels) and take a
@@ -638,18 +654,51 @@ __global__ __launch_bounds__(64 * 16) __attribute__((amdgpu_waves_per_eu(8))) vo
         for (int r = 0; r < RB; ++r) dl[r] = sDl[odd][r][lane];
         prepare(cur, band + 1);
         float hc[R] = {}, sc[R] = {};
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
+        const float h0 = hprev, a0 = aprev;
+        float sum = 0.f;
+        // (CELLS: a row with a value that is not finite is taken once more, cell by cell)
+        auto row = [&](auto CELLS, int r, float2 d, float bv, float cv) {
             float a[1], y[1], bu[1], h[1], s_[1];
-            a[0] = fast_exp2(fmaf(dl[r].x, A2, ld));
-            bu[0] = wave_elem(cur.b[r], 0) * dl[r].y;
+            a[0] = fast_exp2(fmaf(d.x, A2, ld));
+            bu[0] = bv * d.y;
             const float al = from_prev_lane_one<PK>(a[0], sl == 0), hd = from_prev_lane_one<PK>(hprev, sl == 0);
             y[0] = fmaf(a[0], fmaf(-0.5f * (aprev + al), hd, hprev), bu[0]);
             wave_row_solve<1, PK, true>(a, y, bu, 0.f, 0.f, h, s_);
-            sAcc[odd][n][r][lane] = wave_elem(cur.c[r], 0) * fmaf(0.25f, bu[0], h[0] - s_[0]);
+            float q = fmaf(0.25f, bu[0], h[0] - s_[0]);
+            if (decltype(CELLS)::value) {
+                const uint64_t bad = __builtin_amdgcn_ballot_w64(!(fabsf(q) < __builtin_inff()));
+                if (bad) wave_row_cells<PK>(a[0], y[0], bu[0], bad, h[0], s_[0]);
+                q = fmaf(0.25f, bu[0], h[0] - s_[0]);
+            }
+            sum += q;
+            sAcc[odd][n][r][lane] = cv * q;
             hprev = h[0];
             aprev = a[0];
-            if (SAVE) { hc[r] = i0 + r < H ? h[0] : 0.f; sc[r] = i0 + r < H ? s_[0] : 0.f; }
+            if (SAVE) {
+#pragma unroll
+                for (int k = 0; k < RB; ++k)
+                    if (k == r) { hc[k] = i0 + r < H ? h[0] : 0.f; sc[k] = i0 + r < H ? s_[0] : 0.f; }
+            }
+        };
+#pragma unroll
+        for (int r = 0; r < RB; ++r) row(std::false_type{}, r, dl[r], wave_elem(cur.b[r], 0), wave_elem(cur.c[r], 0));
+        // The scan multiplies the a of neighbouring cells before any state meets them.  For a > 1 (a positive A) that can overflow
+        // where the recurrence does not - inf * a state of zero is NaN - and the band is then taken again (a sum that is not finite
+        // shows it; with a <= 1, as models have it, never).  What it needs is fetched again, so that a band that does without
+        // keeps no registers for it.  2 x 384 x 14x14, 16 states, bf16, without | with saved state: 8.9 | 11.6 us without the test, 9.1 | 12.0
+        // so, 9.4 | 12.6 with a test at every row, between the rows of the chain.
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(sum) < __builtin_inff())) != 0, 0)) {
+            asm volatile("" ::: "memory");
+            hprev = h0;
+            aprev = a0;
+#pragma unroll 1
+            for (int r = 0; r < RB; ++r) {
+                const int m = mem_row(i0 + r);
+                Raw bq, cq;
+                wave_ld(bq, Bb, mad24(m, BhB, colB));
+                wave_ld(cq, Cb, mad24(m, ChB, colB));
+                row(std::true_type{}, r, sDl[odd][r][lane], wave_elem(bq, 0), wave_elem(cq, 0));
+            }
         }
         if (SAVE) {
             if (cols) {

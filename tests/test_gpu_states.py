@@ -120,6 +120,46 @@ def test_wave_per_state_keeps_infinities_to_their_plane(gpu_device, W):
     assert not torch.isfinite(f.out[0, 7, 2:, W // 2:]).all() and torch.equal(f.out[0, 7, :2], clean.out[0, 7, :2])
 
 
+# (run: the cells whose a the scan has multiplied when it first meets the state on their left: 8 lanes of a row of 16, the
+# 16-lane rows of a half wave, the upper half wave)
+@pytest.mark.parametrize("H,W,N,first,run", [(10, 14, 16, 6, 8), (16, 16, 5, 8, 8), (9, 30, 8, 16, 14), (10, 33, 6, 16, 16), (12, 60, 16, 32, 28)])
+@pytest.mark.parametrize("left", [0.0, 1e-30])
+def test_wave_per_state_where_products_of_a_overflow(gpu_device, H, W, N, first, run, left):
+    """a > 1: along a row the a of neighbouring cells multiply to more than a float holds while the states stay in range, as the
+    recurrence has it - nothing on the left (0) or a state so small that the product brings it to about 1e10.  One such channel among
+    ordinary ones, whose results do not change."""
+    Bt, Dm, K, odd = 1, 24, 4, 8
+    d, t = _make(gpu_device, Bt, Dm, H, W, N, K, None, torch.float32)
+    assert capi.make_plan(capi.make_shape(t["u"], t["delta"], t["A"], t["B"]))[1].wave_per_state == 1
+    lam = 92.0 / run
+    t["delta"] = torch.nn.functional.softplus(t["delta"] - 3.0)
+
+    def call(sched):
+        f = capi.FwdCall(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], None, False, True, None, True, sched)
+        for x in (f.x, f.x_v, f.x_sd):
+            x.zero_()
+        f.launch()
+        torch.cuda.synchronize()
+        return f
+    plain = call(capi.SCHED_AUTO).out
+    t["u"][0, odd] = 0.0
+    t["u"][0, odd, H - 2, first - 1] = left
+    t["u"][0, odd, H - 2, W - 2] = 1.0
+    t["delta"][0, odd], t["A"][odd] = lam, 1.0
+    auto, tiles = call(capi.SCHED_AUTO), call(capi.SCHED_PLANE)
+    keep = torch.arange(Dm, device=gpu_device) != odd
+    assert torch.equal(auto.out[:, keep], plain[:, keep])
+    r = {k: t[k].cpu().numpy() for k in ("u", "delta", "A", "B", "C")}
+    ref, _ = reference(r["u"], r["delta"], r["A"], r["B"], r["C"], d["D"], None, d["dout"], False, None, False)
+    # four roundings per cell, and an exponent's rounding: a product's exponent adds up to 92 or so
+    bound = (4 * (H + W) + N + 16 + 2 * 100) * 2.0 ** -24
+    for f in (auto, tiles):
+        assert bool(torch.isfinite(f.out).all())
+        assert relerr(f.out[0, odd].cpu().numpy(), ref[0, odd]) <= bound
+    for x in (auto.x, auto.x_v, auto.x_sd.flatten()[:-1]):   # (the last word of x_sd says which family wrote it)
+        assert bool(torch.isfinite(x).all())
+
+
 def test_wave_per_state_in_a_captured_graph(gpu_device):
     _, t = _make(gpu_device, 1, 64, 14, 14, 16, 4, None, torch.float32)
     args = [t[k] for k in ("u", "delta", "A", "B", "C", "D", "delta_bias")]
