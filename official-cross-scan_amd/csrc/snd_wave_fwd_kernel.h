@@ -40,9 +40,8 @@ namespace snd {
 // out (measured against blocks of one wave, bf16, one state: 64 x 1536 x 14x14 0.055 -> 0.049 ms, 64 x 768 x 14x14
 // 0.035 -> 0.031, 64 x 3072 x 7x7 unchanged at 0.051).
 // The scan's sums are the solutions there and a neighbour's value is zero at the plane's edge, which takes 8 instructions
-// per row and state out (four states, 8 x 384 x 56x56 bf16: 62 -> 59 us; two states, 32 x 768 x 28x28 fp32: 62 -> 59).  In fp32 at
-// most four waves to a SIMD, although the registers allow five: bound by memory, and the fifth wave's streams cost more than they
-// hide (64 x 384 x 56x56, one state: 216 -> 204 us, two: 298 -> 289; bf16, one state, loses: 171 -> 178).
+// per row and state out (four states, 8 x 384 x 56x56 bf16: 62 -> 59 us; two states, 32 x 768 x 28x28 fp32: 62 -> 59).  In fp32 some
+// of these keep to four waves a SIMD although the registers allow five and more (wave_fwd_max_waves): see there.
 // EXT: the launch works on one column group of a wide plane (wave_wide() in snd_device.h): segments seg0 .. seg0+nseg-1.
 // The group's first wave takes what enters it on every row - h, s, a of the column on its left - from global memory,
 // where the launch of the group on the left put them (a band's values come with the band's loads, three per state and
@@ -60,8 +59,17 @@ namespace snd {
 // a barrier per band keeps them in step, and they meet once; who comes to a row first stores, who comes second adds.
 // 64 x 384 x 56x56, one state, bf16: 288 -> 190 us, 64 x 768 x 28x28 178 -> 87, 64 x 1536 x 7x7 52 -> 28; out needs no
 // clearing before (18 us at the first of these).
+//
+// The most waves a SIMD is to hold.  Planes one segment wide in fp32, written plainly, are bound by memory, and a fifth wave's streams
+// cost more than they hide - where a wave's rows are long or its states few.  us, at most four | as many as fit, with saved state:
+// 64 x 384 x 56x56, one to four states 207 | 220, 292 | 301, 383 | 411, 487 | 502; packed planes, one state, 64 x 1536 x 14x14 43.0 |
+// 44.3, 64 x 3072 x 7x7 42.3 | 42.2.  Packed planes of more states gain by the waves (14x14, three states 71.5 | 68.6), and so does the
+// merge in LDS, whose groups wait for each other (one state, 56x56 182 | 166, 28x28 53 | 45, 14x14 60 | 48, 7x7 55 | 48; four states, 14x14
+// 103 | 98); in 16 bits the limit loses (one state, 56x56 171 -> 178).
+constexpr int wave_fwd_max_waves(int esize, int ns, int pk, bool one, bool fold) { return one && !fold && esize == 4 && (pk == 1 || ns == 1) ? 4 : 8; }
+
 template <typename T, int NS, int CPL, bool VEC, bool SAVE, bool OUT32, int PK, int EU, bool ONE, bool EXT = false, bool EVEN = false, bool FOLD = false>
-__global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__((amdgpu_waves_per_eu(EU, ONE && sizeof(T) == 4 ? 4 : 8))) void wave_fwd_kernel(const snd_fwd_params p, const WaveGeo wg) {
+__global__ __launch_bounds__(ONE ? 64 * kOneWaves : 64 * kMaxSeg) __attribute__((amdgpu_waves_per_eu(EU, wave_fwd_max_waves((int)sizeof(T), NS, PK, ONE, FOLD)))) void wave_fwd_kernel(const snd_fwd_params p, const WaveGeo wg) {
     static_assert(ONE || PK == 1, "packed planes are one segment wide");
     static_assert(!FOLD || (ONE && OUT32 && CPL == 1), "merge in LDS: one segment, fp32 out");
     static_assert(!EVEN || (!ONE && PK == 1 && CPL == 1 && !EXT), "whole planes: several segments, one column per lane");
