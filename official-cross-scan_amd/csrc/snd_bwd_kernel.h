@@ -110,7 +110,9 @@ __device__ __forceinline__ void sweep_reduce16(float &q0, float &q1, float &q2, 
 // registers it takes are registers the other variants do not have.
 // SINGLE: (whole planes) the plane is one tile: no tile follows whose inputs would be requested - the general kernel requests its own
 // again - and nothing enters it, so no checkpoint is read.  64 x 1536 x 7x7 bf16, 16 states 174 -> 147 us, 64 x 768 x 7x7 fp16,
-// 8 states 72 -> 60, 8 x 768 x 7x7 18.6 -> 16.1.  Branches around the requests instead: planes of several tiles lose up to 7 %
+// 8 states 72 -> 60, 8 x 768 x 7x7 18.6 -> 16.1.  With four lanes per channel (up to 4 states) on 8x8 tiles it spills 29 registers
+// where the general kernel spills none, and is the faster one all the same but for large fp32 launches: 64 x 3072 x 8x8, four states,
+// bf16 208 -> 200, fp32 205 -> 207; 64 x 3072 x 7x8, two states, bf16 203 -> 192; 4 x 768 x 8x8, four, fp32 16.7 -> 15.9.  Branches around the requests instead: planes of several tiles lose up to 7 %
 // (32 x 768 x 28x28 548 -> 586).
 template <typename T, int NP, bool PIPE, int TE, bool VEC, bool SEG = false, bool SINGLE = false>
 __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_kernel(const snd_bwd_params p, const Geo geo) {

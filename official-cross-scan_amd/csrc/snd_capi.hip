@@ -210,7 +210,8 @@ int use_wavefront(const snd_shape &s, int schedule) {
 // out does not depend on whether it is saved; from the shape alone, so that the plan, snd_clear_bytes() and the launch agree): the
 // tile kernels take at least the longest chain of their tiles, however few the planes; the other a row's scan times the rows, longer
 // with more states in a block and, once the waves fill the GPU, with the waves.  Where the two are close (16 states, bf16, tile kernels / wave per state, without | with saved state): 8 x 192 x 28x28
-// 44 / 32 | 47 / 44, taken; 8 x 192 x 56x56 92 / 99, 4 x 768 x 9x60 64 / 55 | 66 / 83, a single tile of 7x7 6.8 / 6.4 | 7.1 / 8.2, stay.
+// 45 / 34 | 48 / 44, taken; 8 x 192 x 56x56 94 / 107 | 104 / 138, 4 x 768 x 9x60 64 / 57 | 66 / 82, a single tile of 7x7 7.0 / 7.3 |
+// 6.8 / 8.6, stay.
 bool wave_states_pays(const snd_shape &s, int schedule) {
     const snd::Geo g = snd::make_geo(s.nrows, s.ncols);
     const int steps = g.nCX + g.nCY - 1;

@@ -554,8 +554,8 @@ template <int PK> __device__ __forceinline__ void wave_row_cells(float a, float 
 // SAVE: state is saved as the tile kernels save it, and they run the backward: h of the last row of every strip but the last (x_v
 // [b][I][J][half][c][n][4 cols]), h and s of the last column of every tile that another follows (x, x_sd [b][J][I][half][c][n]
 // [4 rows]: a band's rows are one access), zeros where a tile extends beyond the plane.
-// us, tile kernels -> here, bf16, without | with saved state: 16 states, 1 x 64 x 14x14 18.4 -> 8.4 | 19.1 -> 10.7, 1 x 192 x 56x56
-// 67 -> 24 | 71 -> 30, 2 x 384 x 28x28 38 -> 22 | 40 -> 31; 8 states, 1 x 64 x 28x28 37 -> 9.5 | 38 -> 12.  (softplus and delta' * u
+// us, tile kernels -> here, bf16, without | with saved state: 16 states, 1 x 64 x 14x14 18.6 -> 8.9 | 19.2 -> 11.3, 1 x 192 x 56x56
+// 67 -> 25 | 72 -> 31, 2 x 384 x 28x28 38 -> 24 | 40 -> 30; 8 states, 1 x 64 x 28x28 37 -> 9.8 | 38 -> 12.  (softplus and delta' * u
 // in every wave instead of once: 28 without saved state at 1 x 192 x 56x56.)
 template <typename T, bool OUT32, int PK, int TE, bool SAVE>
 __global__ __launch_bounds__(64 * 16) __attribute__((amdgpu_waves_per_eu(8))) void wave_states_kernel(const snd_fwd_params p, const WaveGeo wg, const Geo geo) {

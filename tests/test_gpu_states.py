@@ -20,8 +20,11 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # Bt, Dm, H, W, N, K, Dd, dtype, kw
     (1, 64, 14, 14, 16, 4, None, torch.float32, {}),
-    (2, 24, 1, 1, 5, 4, None, torch.float32, {}),                  # one cell
-    (1, 36, 3, 7, 16, 4, None, torch.float32, dict(corners=True)), # 9 channels per group: the last wave holds one plane of four
+    (2, 24, 1, 1, 5, 4, None, torch.float32, {}),                  # one cell, (below) a plane of one tile: both stay with the tile kernels
+    (1, 36, 3, 7, 16, 4, None, torch.float32, dict(corners=True)),
+    (2, 24, 9, 1, 5, 4, None, torch.float32, {}),                  # one column
+    (1, 24, 1, 9, 5, 4, None, torch.float32, dict(corners=True)),  # one row
+    (1, 36, 15, 7, 16, 4, None, torch.float32, dict(corners=True)),  # 9 channels per group: the last wave holds one plane of four
     (1, 20, 4, 16, 8, 2, 10, torch.bfloat16, dict(corners=True)),  # a full quarter wave, one whole band, delta shared in pairs
     (3, 15, 5, 17, 9, 3, None, torch.float16, {}),                 # two planes to a wave, three groups, one row in the last band
     (1, 28, 9, 32, 12, 4, None, torch.float32, dict(corners=True, decay=0.9)),
@@ -38,6 +41,11 @@ def _make(dev, Bt, Dm, H, W, N, K, Dd, dtype, seed=5):
     for k in ("u", "delta", "B", "C"):
         t[k] = t[k].to(dtype)
     return d, t
+
+
+def _route(f):
+    """Whether the plan says that AUTO's forward of this call is the one with a wave per state."""
+    return f.plan.wave_per_state == 1
 
 
 @pytest.mark.parametrize("Bt,Dm,H,W,N,K,Dd,dtype,kw", CASES)
@@ -59,6 +67,7 @@ def test_wave_per_state_matches_oracle_and_tiles(gpu_device, Bt, Dm, H, W, N, K,
     outs, grads = [], []
     for sched in (capi.SCHED_AUTO, capi.SCHED_PLANE):  # the wave per state, the tile kernels
         f = capi.FwdCall(*args, softplus, kw.get("out_float", True), dec, True, sched, dirs)
+        assert _route(f) == (f.plan.n_chunks_x * f.plan.n_chunks_y > 1)
         f.out.fill_(float("nan"))
         for x in (f.x, f.x_v, f.x_sd):                 # (what a launch does not write must not matter to the backward)
             x.fill_(float("nan"))
@@ -87,7 +96,7 @@ def test_wave_per_state_matches_oracle_and_tiles(gpu_device, Bt, Dm, H, W, N, K,
                 assert relerr(a, r_) <= relerr(w, r_) + bound + (Bt * H * W) ** 0.5 * 2.0 ** -24, nm
 
 
-@pytest.mark.parametrize("H,W,N", [(7, 7, 16), (10, 30, 6), (6, 50, 9)])
+@pytest.mark.parametrize("H,W,N", [(15, 7, 16), (10, 30, 6), (6, 50, 9)])
 def test_wave_per_state_merge(gpu_device, H, W, N):
     """The four corners of one map added up inside the call, against the same without the merge."""
     Bt, Dm, K = 2, 20, 4
@@ -96,6 +105,7 @@ def test_wave_per_state_merge(gpu_device, H, W, N):
     u = t["u"][:, :Dm // K].contiguous()
     args = (u, t["delta"], t["A"], t["B"], t["C"], t["D"], t["delta_bias"])
     m = capi.FwdCall(*args, True, True, None, False, capi.SCHED_AUTO, capi.DIR_CORNERS, True, w)
+    assert _route(m)
     m.launch()
     f = capi.FwdCall(u.repeat(1, K, 1, 1), *args[1:], True, True, None, False, capi.SCHED_PLANE, capi.DIR_CORNERS)
     f.launch()
@@ -105,10 +115,11 @@ def test_wave_per_state_merge(gpu_device, H, W, N):
 
 @pytest.mark.parametrize("W", [7, 16, 30, 64])
 def test_wave_per_state_keeps_infinities_to_their_plane(gpu_device, W):
-    Bt, Dm, H, N, K = 1, 24, 6, 8, 4
+    Bt, Dm, H, N, K = 1, 24, 9, 8, 4
     _, t = _make(gpu_device, Bt, Dm, H, W, N, K, None, torch.float32)
     args = [t[k] for k in ("u", "delta", "A", "B", "C", "D", "delta_bias")]
     clean = capi.FwdCall(*args, True, True, None, False)
+    assert _route(clean)
     clean.launch()
     args[0] = t["u"].clone()
     args[0][0, 7, 2, W // 2] = float("inf")
@@ -130,7 +141,6 @@ def test_wave_per_state_where_products_of_a_overflow(gpu_device, H, W, N, first,
     ordinary ones, whose results do not change."""
     Bt, Dm, K, odd = 1, 24, 4, 8
     d, t = _make(gpu_device, Bt, Dm, H, W, N, K, None, torch.float32)
-    assert capi.make_plan(capi.make_shape(t["u"], t["delta"], t["A"], t["B"]))[1].wave_per_state == 1
     lam = 92.0 / run
     t["delta"] = torch.nn.functional.softplus(t["delta"] - 3.0)
 
@@ -141,7 +151,9 @@ def test_wave_per_state_where_products_of_a_overflow(gpu_device, H, W, N, first,
         f.launch()
         torch.cuda.synchronize()
         return f
-    plain = call(capi.SCHED_AUTO).out
+    plain = call(capi.SCHED_AUTO)
+    assert _route(plain)
+    plain = plain.out
     t["u"][0, odd] = 0.0
     t["u"][0, odd, H - 2, first - 1] = left
     t["u"][0, odd, H - 2, W - 2] = 1.0
@@ -164,6 +176,7 @@ def test_wave_per_state_in_a_captured_graph(gpu_device):
     _, t = _make(gpu_device, 1, 64, 14, 14, 16, 4, None, torch.float32)
     args = [t[k] for k in ("u", "delta", "A", "B", "C", "D", "delta_bias")]
     f = capi.FwdCall(*args, True, True, None, False)
+    assert _route(f)
     f.launch()
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
