@@ -37,6 +37,22 @@ def test_jobs_clear_and_sum(gpu_device, src, dst, outer, rows, cols):
     assert torch.equal(out, want.to(dst))
 
 
+@pytest.mark.parametrize("n", [1, 65536 * 3 + 1])
+def test_rounding_to_bfloat16(gpu_device, n):
+    """To nearest even, bit for bit as torch rounds: ties, subnormal values, the largest ones, infinities; a NaN stays one."""
+    bits = torch.arange(n, device=gpu_device, dtype=torch.int64) * 21845 + (torch.arange(n, device=gpu_device) % 5 - 2) + 0x8000
+    special = torch.tensor([0x00008000, 0x00018000, 0x3f808000, 0x3f818000, 0x7f7fffff, 0x7f7f8000, 0x7f800000, 0x7f800001, 0x7fc00000, 1, 0x007fffff],
+                           device=gpu_device, dtype=torch.int64)
+    bits = torch.cat([bits, special, special + 0x80000000]) & 0xffffffff
+    a = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32)
+    out = torch.empty(a.numel(), device=gpu_device, dtype=torch.bfloat16)
+    job = capi.Job(a.data_ptr(), None, out.data_ptr(), 1, a.numel(), 1, capi.JOB_SUM, capi.SND_F32, capi.SND_BF16)
+    capi.check(capi.lib().snd_run_jobs((capi.Job * 1)(job), 1, torch.cuda.current_stream().cuda_stream))
+    want, nan = a.to(torch.bfloat16), torch.isnan(a)
+    assert torch.equal(torch.isnan(out), nan)
+    assert torch.equal(out.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
 @pytest.mark.parametrize("src,dst,outer,rows,cols", [
     (torch.float32, torch.float32, 1, 31, 20), (torch.float32, torch.float32, 1, 32, 20),       # either side of the split
     (torch.float32, torch.float32, 3, 33, 1),                                                   # a slice of one row, the last ones of none
