@@ -487,34 +487,48 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // beside dD, at no cost in the sweep.
     float dw_acc = 0.f;
 
-    // dB, dC of a tile leave the block (summed over its channels) one tile late, from the partial sums that stay in LDS until the
-    // next sweep, ahead of the commit of the next tile's inputs.  (A state at a time between the rows of the recomputation, where
-    // arithmetic could cover it, it needs a block barrier in front of the sweep: 64 x 192 x 56x56 1.10 ms either way, 2 x 192 x 200x336
-    // 0.945 -> 0.960, 32 x 768 x 28x28 bf16 0.584 -> 0.606.)
+    // dB, dC of a tile leave the block (summed over its channels) behind its sweep, from the waves' partial sums in LDS.  They are
+    // read (flush_read) ahead of the per-pixel epilogue, which covers the reads' latency, and added up and sent behind it; a wave
+    // alone with its arithmetic is what such a wait costs, two waves per SIMD hide little of it.  Read where they are added up, ahead
+    // of the next tile's commit, us: 64 x 192 x 56x56 fp32 1059 -> 1024, 2 x 192 x 200x336 920 -> 880, 1 x 256 x 512^2 bf16 2020 ->
+    // 1960, 8 x 768 x 56x56 bf16 552 -> 532, 12 x 196 x 65x91 660 -> 631.  (The atomics one state at a time between the rows of the
+    // next recomputation: 1.3 to 4 % slower than all at once, with those of held tiles dropped by their offset.)
     // The terms in dout*C/4 and bu/4 are left out of the sweep: summed over channels (states) they are products of B or C
     // with per-pixel sums that all states (channels) share,
     //     dB: C * T,  dC: B * T,  T = sum_c dout*delta'*u / 4        sum_n dbu*B: dout * S,  S = sum_n B*C / 4
     // That and s - bu = a * s[left] take four instructions per cell out of the sweep.
     // (All schedules alike, so that their results agree bit for bit.)
-    float pB[NBC], pC[NBC];                         // this thread's B, C of that tile
-    int pI = -1, pJ = 0;                            // the tile whose partial sums are still in LDS
+    float pB[NBC], pC[NBC];                         // this thread's B, C of the tile
     // Two neighbouring 8x8 tiles leave together: the right one's sums are held in LDS and joined to the left one's, so that an
     // instruction adds 4 rows x 16 columns instead of 8 rows x 8.  An atomic costs its CU 12 ns per 64-byte line it
     // touches, however few of the line's words it adds to (2 x 192 x 200x336: 1.09 -> 1.07 ms, 256 channels of 512x512:
     // 2.56 -> 2.51 ms; rows that are no multiple of 64 bytes gain nothing, 7x7 tiles lose 2 % and keep the plain form).
     // Lanes outside the plane get an offset that the buffer's range check drops: no branch around an atomic.
-    auto flush_bc = [&]() __attribute__((always_inline)) {
+    struct Part { float t[WPB], b[NBC][NPART], c[NBC][NPART]; };
+    auto flush_read = [&](Part &q) __attribute__((always_inline)) {
         SND_THREAD_MAPS(NP);
-        const bool holds = TE == 8 && (pJ & 1) && pJ > J_lo, joins = TE == 8 && !(pJ & 1) && pJ < J_hi;
+#pragma unroll
+        for (int w = 0; w < WPB; ++w) q.t[w] = sT[w * kTile + px];
+#pragma unroll
+        for (int k = 0; k < NBC; ++k)
+#pragma unroll
+            for (int w = 0; w < NPART; ++w) {
+                q.b[k][w] = sdB[w * PART + (wave_u + WPB * k) * NSD + px];
+                q.c[k][w] = sdC[w * PART + (wave_u + WPB * k) * NSD + px];
+            }
+    };
+    auto flush_bc = [&](const Part &q, int I, int J) __attribute__((always_inline)) {
+        SND_THREAD_MAPS(NP);
+        const bool holds = TE == 8 && (J & 1) && J > J_lo, joins = TE == 8 && !(J & 1) && J < J_hi;
         // plain: lane l adds row l / 8, column l % 8; joined: row (l / 8) % 4 (+ 4), column l % 8 of the left (lanes 0-31) or right tile
-        const int row = pI * TE + (joins ? pr & 3 : pr), col = (pJ + (joins ? px >> 5 : 0)) * TE + pj;
+        const int row = I * TE + (joins ? pr & 3 : pr), col = (J + (joins ? px >> 5 : 0)) * TE + pj;
         const bool in = pr < TE && pj < TE && col < W;
         const int cB = mcol(col) * 4;
         const uint32_t o0 = in && row < H ? (uint32_t)mad24(mrow(row), W4, cB) : kBufOOB;
         const uint32_t o4 = in && row + 4 < H ? (uint32_t)mad24(mrow(row + 4), W4, cB) : kBufOOB;
         float tsum = 0.f;
 #pragma unroll
-        for (int w = 0; w < WPB; ++w) tsum += sT[w * kTile + px];
+        for (int w = 0; w < WPB; ++w) tsum += q.t[w];
 #pragma unroll
         for (int k = 0; k < NBC; ++k) {
             int sn = wave_u + WPB * k;              // scalar: folded into the base
@@ -522,8 +536,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             float tb = pC[k] * tsum, tc = pB[k] * tsum;
 #pragma unroll
             for (int w = 0; w < NPART; ++w) {
-                tb += sdB[w * PART + sn * NSD + px];
-                tc += sdC[w * PART + sn * NSD + px];
+                tb += q.b[k][w];
+                tc += q.c[k][w];
             }
             if (holds) {
                 sHold[sn * kTile + px] = tb;
@@ -574,6 +588,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
         load_row_ckpt(I_hi, J_hi);
         load_col_ckpt(I_hi, J_hi);
     }
+    // Nothing in flight on the way into the tile loop: the waits that the compiler derives for the staged inputs then count the loop's own
+    // instructions behind them instead of waiting for all of them (64 x 192 x 56x56 1055 -> 1048 us; planes of one tile 144 -> 136,
+    // 64 x 1536 x 7x7).  Whole planes of several tiles lose by it (64 x 768 x 14x14 282 -> 291).
+    if (PIPE || SINGLE) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     for (int I = I_hi; I >= I_lo; --I) {
         const int r0 = I * TE;
         float GR[kRows], SR[kRows];                 // G, G + Gs at the column right of the tile
@@ -613,16 +631,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             int In = I, Jn = J - 1;
             if (Jn < (SEG ? J_lo : 0)) { In = I - 1; Jn = J_hi; }
             if (In < I_lo) { In = I; Jn = J; }
-            if (SINGLE || I == 0) {
-#pragma unroll
-                for (int j = 0; j < kCkX; ++j) hu[j] = 0.f;
-                hc = 0.f;
-            }
-            if (SINGLE || J == 0) {
-#pragma unroll
-                for (int r = 0; r < kRows; ++r) { hlft[r] = 0.f; slft[r] = 0.f; }
-                hc = 0.f;
-            }
             float Gd[kCkX];                                        // G of the row below
             // the adjoint row of the strip below: written by this block, or - first strip of a
             // pipelined band - by another block.  It is requested here if it is known to be there (own
@@ -647,7 +655,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             const bool late = handed && __builtin_amdgcn_readfirstlane(lds_peek(&sSeen)) < geo.nCX - J;
             int peek = 0;                           // wave 0: the count as it is now, there when the staged inputs are
             if (late && wave == 0) peek = __hip_atomic_load(progress + I + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (pI >= 0) flush_bc();                // the tile before this one
             commit(I, J);
             if (late && wave == 0) {
                 seen = __builtin_amdgcn_readfirstlane(peek);
@@ -671,12 +678,24 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 for (int m = PXW; m < 64; m <<= 1) v += __shfl_xor(v, m);
                 if (lane < PXW) sS[spx] = 0.25f * v;
             }
+            // (nothing enters the first row and column of tiles; here and not sooner, since it waits for the checkpoints requested)
+            if (SINGLE || I == 0) {
+#pragma unroll
+                for (int j = 0; j < kCkX; ++j) hu[j] = 0.f;
+                hc = 0.f;
+            }
+            if (SINGLE || J == 0) {
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) { hlft[r] = 0.f; slft[r] = 0.f; }
+                hc = 0.f;
+            }
             // ---- recompute h on the whole tile, and s at column 3 of every row (the sweep takes a row's right half first)
             float hT[TE][TE], smid[TE];
             // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
             // the tile loop (a spilled register is two vector memory instructions per tile, 2 to 4 % of the kernel); the column
-            // segments' bookkeeping leaves room for two.
-            constexpr int KA = TE == 7 ? 4 : SEG ? 2 : 5;
+            // segments' bookkeeping leaves room for two, a 7x7 tile for all (64 x 768 x 14x14 bf16 283 -> 279 us, 32 x 768 x 28x28 564 -> 553;
+            // its pipelined form, 16 x 384 x 21x35 fp32, 178 -> 182: four there).
+            constexpr int KA = TE == 7 ? (PIPE ? 4 : 7) : SEG ? 2 : 5;
             float aT[KA ? TE : 1][KA ? KA : 1];
             {
                 float aprev[8], hprev[8], dlr[4];
@@ -907,7 +926,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 load_col_ckpt(In, Jn);
             }
 
-            pI = I; pJ = J;
+            Part part;
+            flush_read(part);
+            __builtin_amdgcn_sched_barrier(0);
             // ---- once per pixel: du, ddelta (thread that staged the pixel), dD, ddelta_bias
             {
             SND_THREAD_MAPS(NP);
@@ -968,6 +989,7 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             }
             }
+            flush_bc(part, I, J);
         }
         if (SEG && seg + 1 < geo.nSeg) {
             // hand the carried column state to the block of the strip's next segment: stores, each wave waits for its
@@ -985,7 +1007,6 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             strip_signal(segdone + I);
         }
     }
-    if (pI >= 0) flush_bc();
 #undef DL
 #undef AEXP
 #undef EXPA
