@@ -367,11 +367,32 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 if (dead && tid == 0) sDead = 1;
             }
             __syncthreads();
-            if (wave == 0) {                        // read by the output phase, behind the next barrier
-                float t = 0.f;
-                if (VEC) {                          // from the committed tile: sum_n B*C of the pixel
+            // S, read by the output phase behind the next barrier.  DEAL: the pixels dealt over the waves, the states over the lanes of a
+            // pixel; by one wave for all, the others wait for it at that barrier.  us: 256 channels of 512x512 bf16 1138 -> 1087, 8 x 768 x
+            // 56x56 bf16 232 -> 216, 64 x 192 x 56x56 bf16 433 -> 425, fp32 483 -> 478.  Without saved state, whose stores the other waves
+            // do not have either, one wave is as fast or faster (256 x 512x512 900 / 915, 2 x 192 x 200x336 445 / 451).
+            constexpr bool DEAL = VEC && SAVE;
+            constexpr int PXW = kTile / WPB;
+            const int spx = PXW * wave_u + (tid & 63) % PXW, sg = (tid & 63) / PXW;
+            float tb[4], tc[4];
+            if (DEAL) {
 #pragma unroll
-                    for (int k = 0; k < NP; ++k) t = fmaf(sB[k * NSTR + (tid & 63)], sC[k * NSTR + (tid & 63)], t);
+                for (int k = 0; k < 4; ++k) { tb[k] = sB[(sg * 4 + k) * NSTR + spx]; tc[k] = sC[(sg * 4 + k) * NSTR + spx]; }
+            } else if (wave == 0) {
+                float t = 0.f;
+                if (VEC) {                          // (added up in the order of the dealt sum: out does not depend on whether state is saved)
+                    float g4[NP / 4];
+#pragma unroll
+                    for (int q = 0; q < NP / 4; ++q) {
+                        g4[q] = 0.f;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) g4[q] = fmaf(sB[(q * 4 + k) * NSTR + (tid & 63)], sC[(q * 4 + k) * NSTR + (tid & 63)], g4[q]);
+                    }
+#pragma unroll
+                    for (int m = 1; m < NP / 4; m <<= 1)
+#pragma unroll
+                        for (int q = 0; q < NP / 4; q += 2 * m) g4[q] += g4[q + m];
+                    t = g4[0];
                 } else {
 #pragma unroll
                     for (int w = 0; w < WPB; ++w) t += sSp[w * kTile + (tid & 63)];
@@ -401,6 +422,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
                 if (ahead) load_pair(In, Jn);
             } else if (INSIDE) { In = I; Jn = J; }  // (the block's last tile: loads that nobody reads, of a tile that exists)
             const int Jn1 = min(Jn + 1, geo.nCX - 1);
+            if (DEAL) {
+                float t = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) t = fmaf(tb[k], tc[k], t);
+#pragma unroll
+                for (int m = PXW; m < 64; m <<= 1) t += __shfl_xor(t, m);
+                sS[spx] = 0.25f * t;                // (every lane of a pixel the same value)
+            }
             if (handed) {                           // the corner is the previous fetch's last column
                 corner = J > 0 ? xv_last : 0.f;
                 xv_last = hup[TE - 1];
