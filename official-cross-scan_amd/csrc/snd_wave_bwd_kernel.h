@@ -66,7 +66,7 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // 99 -> 68; packed, 32 x 768 x 28x28 92 -> 86; several segments (no ONE) 64 x 96 x 112x112 411 -> 408;
 // one channel per block, 1 x 192 x 56x56 bf16, one state 31 -> 26, 1 x 64 x 56x56 fp32, two 51 -> 35.
 template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1)>
-__global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
+__global__ __launch_bounds__(ONE ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
     static_assert(!EXT || (CHB == (SPL ? 2 : 1) && PK == 1 && CPL == 1 && (!EVEN || SPL)), "column groups: one channel per block, one column per lane");
     static_assert(!SPL || EXT, "a split plane hands over like a column group");
@@ -80,11 +80,14 @@ __global__ __launch_bounds__(64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(con
     // Two buffers, so that one barrier per band is enough - where they leave the CU its blocks: with three states they
     // would be 48 KB, two blocks per CU instead of four (32x12288x7x7: 0.50 ms against 0.31 with one buffer).
     constexpr int kXBuf = CHB == 1 ? 1 : (NS >= 3 || XW > 8) ? 1 : 2;
-    constexpr int kXWaves = CHB == 1 ? 1 : XW;
+    constexpr int kXWaves = CHB == 1 ? 1 : ONE ? CHB : XW;   // (one segment: a wave per channel; 16 x 384 x 28x28, four states, 71.5 -> 70.0 us with half the LDS)
     __shared__ float sX[kXBuf][kXWaves][CHB == 1 ? 1 : kItems][CHB == 1 ? 1 : 64];
     // load a band's inputs one band ahead (with three or four states it measured 20 % slower, and with two columns per
-    // lane the registers are needed elsewhere)
-    constexpr bool PF = NS <= 2 && CPL == 1;
+    // lane the registers are needed elsewhere).  Packed planes have few bands and many waves: without it they take 67 to 88
+    // registers instead of 105 to 113, and with the LDS of a block of four waves (below) a SIMD holds five to seven waves
+    // instead of four.  us: one state, 64 x 1536 x 7x7 31.2 -> 27.4, 64 x 768 x 14x14 49.9 -> 49.2, 32 x 768 x 28x28 merged 82.1 ->
+    // 80.3; two states, 7x7 47.8 -> 45.8, 14x14 73.1 -> 71.8.  (Planes of 33 to 64 columns: no change bf16, +0.6 % fp32.)
+    constexpr bool PF = NS <= 2 && CPL == 1 && PK == 1;
     // The rows' hand-overs behind the band's last row instead of each behind its own: without a branch between the rows the
     // compiler overlaps one row's sums with the next row's scan.  One state, 256 channels of 512x512 398 -> 383 us, 64 channels of
     // 600x900 873 -> 831; two states lose by it (bands of two rows; 2 x 192 x 200x336 381 -> 386).
