@@ -3,7 +3,7 @@
 // read once from it (halos and second passes come from the L2) and written once, in the layout its reader wants - tokens by
 // channels for the linear layers, channels by pixels for the scan - with the transposition done in LDS on the way.
 // Measured on a block of width 96 (inner 192, rank 6) at 8 x 56 x 56, bf16, us forward / backward, against the torch layers
-// they replace: convolution + SiLU 90 / 420 -> 33 / 64 (layout copies, im2col per image for the weight), projections 100 / 400
+// they replace: convolution + SiLU 90 / 420 -> 19 / 49 (layout copies, im2col per image for the weight), projections 100 / 400
 // -> 35 / 95 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 22 / 46,
 // token norm 33 / 70 -> 6 / 13 each, weight gradient of a linear layer 93 + 20 -> 20; the block's training step 2940 -> 1500.
 #include <algorithm>
@@ -137,60 +137,95 @@ __global__ __launch_bounds__(norm_threads(GL)) void norm_bwd_kernel(const TY *dy
 // A block takes 32 channels of 4 rows x 32 columns.  The 6 x 34 pixels around them go through LDS, channels innermost at an
 // odd pitch, so that both sides of the transposition (lanes along channels of a token, along pixels of a channel) are free of
 // bank conflicts.
+// Bound by instructions, most of them for the staging's addresses, and by how many blocks a CU holds: with tiles as fp32 in LDS and
+// indices divided out per element 33 us forward and 64 backward at 8 x 56 x 56, 192 channels, bf16; tiles in 16 bits 22 and 51; rows
+// as scalar bases, all of a thread's loads at once, 19 and 49.
 constexpr int kCvC = 32, kCvR = 4, kCvX = 32, kCvP = kCvC + 1, kCvRow = (kCvX + 2) * kCvP, kCvTile = (kCvR + 2) * kCvRow;
-constexpr int kCvN = (kCvR + 2) * (kCvX + 2) * kCvC, kCvB = 13;     // elements of a tile; loads a thread has in flight
-static_assert((kCvN + 255) / 256 == 2 * kCvB, "two batches of loads per thread");
-// All loads are of valid addresses (clamped coordinates) and unconditional, so that a batch is requested before any is waited
-// for; what lies outside the image becomes zero afterwards.
-template <typename T>
-__device__ __forceinline__ void conv_stage_x(float *sX, const T *xb, int h0, int w0, int c0, int H, int W, int Di) {
+// A tile is kept in LDS in the tensors' type: what is staged are its values, or results that are rounded to it.  A thread's loads are
+// requested together, at valid addresses (clamped coordinates): a row's is the scalar base, a column's and channel's an offset that
+// all rows share (below 2^32 bytes in an image that the scan takes); what lies outside the image becomes zero afterwards.
+constexpr int kCvS = kCvR + 2, kCvJ = (kCvX + 2 + 7) / 8;            // staged rows; staged columns per thread (tokens, channels along lanes)
+template <typename T> struct ConvX {
+    T v[kCvS][kCvJ];
+    __device__ __forceinline__ void load(const T *xb, int h0, int w0, int c0, int H, int W, int Di) {
+        uint32_t off[kCvJ];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        float v[kCvB];
+        for (int j = 0; j < kCvJ; ++j) off[j] = (uint32_t)min(max(w0 + (int)(threadIdx.x >> 5) + 8 * j - 1, 0), W - 1) * (2 * Di) + min(c0 + (int)(threadIdx.x & 31), Di - 1);
 #pragma unroll
-        for (int k = 0; k < kCvB; ++k) {
-            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), ch = i & 31, p = i >> 5, r = p / (kCvX + 2), x = p - r * (kCvX + 2);
-            const int h = min(max(h0 + r - 1, 0), H - 1), q = min(max(w0 + x - 1, 0), W - 1);
-            v[k] = ldg(xb + ((int64_t)h * W + q) * 2 * Di, min(c0 + ch, Di - 1));
-        }
+        for (int r = 0; r < kCvS; ++r) {
+            const T *const row = xb + (int64_t)min(max(h0 + r - 1, 0), H - 1) * W * 2 * Di;
 #pragma unroll
-        for (int k = 0; k < kCvB; ++k) {
-            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), ch = i & 31, p = i >> 5, r = p / (kCvX + 2), x = p - r * (kCvX + 2);
-            const int h = h0 + r - 1, q = w0 + x - 1;
-            sX[r * kCvRow + x * kCvP + ch] = h >= 0 && h < H && q >= 0 && q < W && c0 + ch < Di ? v[k] : 0.f;
+            for (int j = 0; j < kCvJ; ++j) v[r][j] = row[off[j]];
         }
     }
-}
-// dpre = du * silu'(pre); du, pre: the planes of channel c0
-template <typename T>
-__device__ __forceinline__ void conv_stage_d(float *sD, const T *du, const T *pre, int h0, int w0, int c0, int H, int W, int Di) {
+    __device__ __forceinline__ void put(T *sX, int h0, int w0, int c0, int H, int W, int Di) const {
+        const int ch = threadIdx.x & 31, x0 = threadIdx.x >> 5;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        float v[kCvB], a[kCvB];
+        for (int j = 0; j < kCvJ; ++j) {
+            const int x = x0 + 8 * j, q = w0 + x - 1;
+            const bool in = q >= 0 && q < W && c0 + ch < Di;
+            if (x < kCvX + 2)
 #pragma unroll
-        for (int k = 0; k < kCvB; ++k) {
-            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), p = i / (kCvX + 2), x = i - p * (kCvX + 2), ch = p / (kCvR + 2), r = p - ch * (kCvR + 2);
-            const int h = min(max(h0 + r - 1, 0), H - 1), q = min(max(w0 + x - 1, 0), W - 1);
-            const int64_t o = ((int64_t)min(ch, Di - 1 - c0) * H + h) * W + q;
-            v[k] = ldg(du + o, 0);
-            a[k] = ldg(pre + o, 0);
-        }
-#pragma unroll
-        for (int k = 0; k < kCvB; ++k) {
-            const int i = min((int)threadIdx.x + 256 * (half * kCvB + k), kCvN - 1), p = i / (kCvX + 2), x = i - p * (kCvX + 2), ch = p / (kCvR + 2), r = p - ch * (kCvR + 2);
-            const int h = h0 + r - 1, q = w0 + x - 1;
-            sD[r * kCvRow + x * kCvP + ch] = h >= 0 && h < H && q >= 0 && q < W && c0 + ch < Di ? rnd<T>(v[k] * dsilu(a[k])) : 0.f;
+                for (int r = 0; r < kCvS; ++r) sX[r * kCvRow + x * kCvP + ch] = in && h0 + r - 1 >= 0 && h0 + r - 1 < H ? v[r][j] : T{};
         }
     }
-}
+};
+// du and pre (from the planes of channel c0), staged as dpre = du * silu'(pre): lanes along 32 columns, four channels per thread, and the
+// last two columns by themselves
+template <typename T> struct ConvD {
+    T v[kCvS][4], a[kCvS][4], ve[2], ae[2];
+    __device__ __forceinline__ static void edge(int k, int &r, int &x, int &ch) {
+        r = min((int)(threadIdx.x >> 6) + 4 * k, kCvS - 1);
+        x = kCvX + (threadIdx.x & 1);
+        ch = (threadIdx.x >> 1) & 31;
+    }
+    __device__ __forceinline__ void load(const T *du, const T *pre, int h0, int w0, int c0, int H, int W, int Di) {
+        const uint32_t HW = (uint32_t)H * W;
+        uint32_t off[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) off[k] = (uint32_t)min((int)(threadIdx.x >> 5) + 8 * k, Di - 1 - c0) * HW + min(max(w0 + (int)(threadIdx.x & 31) - 1, 0), W - 1);
+#pragma unroll
+        for (int r = 0; r < kCvS; ++r) {
+            const int64_t row = (int64_t)min(max(h0 + r - 1, 0), H - 1) * W;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { v[r][k] = (du + row)[off[k]]; a[r][k] = (pre + row)[off[k]]; }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            int r, x, ch;
+            edge(k, r, x, ch);
+            const uint32_t o = (uint32_t)min(ch, Di - 1 - c0) * HW + (uint32_t)min(max(h0 + r - 1, 0), H - 1) * W + min(w0 + x - 1, W - 1);
+            ve[k] = du[o];
+            ae[k] = pre[o];
+        }
+    }
+    __device__ __forceinline__ void put(T *sD, int h0, int w0, int c0, int H, int W, int Di) const {
+        auto store = [&](int r, int x, int ch, const T &d, const T &p) {
+            const int h = h0 + r - 1, q = w0 + x - 1;
+            stg(sD, r * kCvRow + x * kCvP + ch, h >= 0 && h < H && q >= 0 && q < W && c0 + ch < Di ? ldg(&d, 0) * dsilu(ldg(&p, 0)) : 0.f);
+        };
+#pragma unroll
+        for (int r = 0; r < kCvS; ++r)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) store(r, threadIdx.x & 31, (threadIdx.x >> 5) + 8 * k, v[r][k], a[r][k]);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            int r, x, ch;
+            edge(k, r, x, ch);                      // (rows beyond the last: the last once more)
+            store(r, x, ch, ve[k], ae[k]);
+        }
+    }
+};
 
 template <typename T>
 __global__ __launch_bounds__(256) void conv_fwd_kernel(snd_block_shape s, const T *xz, const float *w, const float *bias, T *pre, T *u) {
-    __shared__ float sX[kCvTile];
+    __shared__ T sX[kCvTile];
     const int H = s.nrows, W = s.ncols, Di = s.inner, t = threadIdx.x;
     const int nX = (W + kCvX - 1) / kCvX, h0 = (blockIdx.x / nX) * kCvR, w0 = (blockIdx.x % nX) * kCvX, c0 = blockIdx.y * kCvC, b = blockIdx.z;
     const T *xb = xz + (int64_t)b * H * W * 2 * Di;
-    conv_stage_x(sX, xb, h0, w0, c0, H, W, Di);
+    ConvX<T> cx;
+    cx.load(xb, h0, w0, c0, H, W, Di);
+    cx.put(sX, h0, w0, c0, H, W, Di);
     __syncthreads();
     const int x = t & 31;
     if (w0 + x >= W) return;
@@ -208,7 +243,7 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(snd_block_shape s, const 
         for (int r = 0; r < kCvR + 2; ++r)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const float v = sX[r * kCvRow + (x + j) * kCvP + ch];
+                const float v = ldg(sX, r * kCvRow + (x + j) * kCvP + ch);
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
                     if (r - i >= 0 && r - i < kCvR) acc[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0] = fmaf(wt[i * 3 + j], v, acc[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0]);
@@ -226,13 +261,19 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(snd_block_shape s, const 
 template <typename T>
 __global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const T *du, const T *pre, const T *xz, const float *w, T *dxz, float *dw,
                                                        float *dbias) {
-    __shared__ float sX[kCvTile], sD[kCvTile];
+    __shared__ __align__(16) T sX[kCvTile];
+    __shared__ T sD[kCvTile];
+    static_assert(sizeof(sX) >= 8 * 10 * 32 * sizeof(float), "the block's sums take the place of the staged x");
     const int H = s.nrows, W = s.ncols, Di = s.inner, t = threadIdx.x;
     const int nX = (W + kCvX - 1) / kCvX, h0 = (blockIdx.x / nX) * kCvR, w0 = (blockIdx.x % nX) * kCvX, c0 = blockIdx.y * kCvC, b = blockIdx.z;
     const T *xb = xz + (int64_t)b * H * W * 2 * Di;
     const int64_t plane = ((int64_t)b * Di + c0) * H * W;
-    conv_stage_x(sX, xb, h0, w0, c0, H, W, Di);
-    conv_stage_d(sD, du + plane, pre + plane, h0, w0, c0, H, W, Di);
+    ConvX<T> cx;
+    ConvD<T> cd;
+    cx.load(xb, h0, w0, c0, H, W, Di);
+    cd.load(du + plane, pre + plane, h0, w0, c0, H, W, Di);
+    cx.put(sX, h0, w0, c0, H, W, Di);
+    cd.put(sD, h0, w0, c0, H, W, Di);
     __syncthreads();
     const int ch = t & 31, c = c0 + ch;
     float wt[9], gw[9], gb = 0.f;
@@ -244,7 +285,7 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const 
         for (int r = 0; r < kCvR + 2; ++r)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {           // dx[h, q] = sum w[i][j] dpre[h - i + 1, q - j + 1]
-                const float d = sD[r * kCvRow + (x + 2 - j) * kCvP + ch];
+                const float d = ldg(sD, r * kCvRow + (x + 2 - j) * kCvP + ch);
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
                     const int o = r - 2 + i;        // r = o + 2 - i
@@ -253,12 +294,12 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const 
             }
         float d[kCvR];
 #pragma unroll
-        for (int r = 0; r < kCvR; ++r) { d[r] = sD[(r + 1) * kCvRow + (x + 1) * kCvP + ch]; gb += d[r]; }
+        for (int r = 0; r < kCvR; ++r) { d[r] = ldg(sD, (r + 1) * kCvRow + (x + 1) * kCvP + ch); gb += d[r]; }
 #pragma unroll
         for (int r = 0; r < kCvR + 2; ++r)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {           // dw[i][j] = sum dpre[h, q] x[h + i - 1, q + j - 1]
-                const float v = sX[r * kCvRow + (x + j) * kCvP + ch];
+                const float v = ldg(sX, r * kCvRow + (x + j) * kCvP + ch);
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
                     if (r - i >= 0 && r - i < kCvR) gw[i * 3 + j] = fmaf(d[r - i < 0 ? 0 : r - i < kCvR ? r - i : 0], v, gw[i * 3 + j]);
@@ -269,7 +310,7 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(snd_block_shape s, const 
                 if (h0 + r < H) stg(dxz + (((int64_t)b * H + h0 + r) * W + w0 + x) * 2 * Di, c, dx[r]);
     }
     __syncthreads();
-    float *red = sX;                                // [8][10][32]
+    float *red = (float *)sX;                       // [8][10][32]
 #pragma unroll
     for (int k = 0; k < 9; ++k) red[((t >> 5) * 10 + k) * 32 + ch] = gw[k];
     red[((t >> 5) * 10 + 9) * 32 + ch] = gb;
