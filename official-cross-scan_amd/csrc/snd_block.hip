@@ -667,55 +667,66 @@ __global__ __launch_bounds__(256) void wgrad_kernel(const T *a, int64_t ab, int6
 // Here the summed axis is the outer one, so stages of 64 tokens x 64 channels of either operand are transposed on their way
 // into LDS: a thread takes two channels of two tokens, swaps the inner halves, and stores two token pairs.  Threads are
 // dealt 8 channel pairs x 8 token pairs to a wave: 32-byte runs of memory, and both the stores and the fragment reads
-// (16 bytes at a pitch of 36 words) spread over all LDS banks.  The next stage's loads are in flight during the products.
-// The library's product has M * N / 4096 blocks and walks all tokens in each (25088 x 384 x 96: 93 us); here the tokens are
-// split over the grid.
+// (16 bytes at a pitch of 36 words) spread over all LDS banks.  The library's product has M * N / 4096 blocks and walks all
+// tokens in each (25088 x 384 x 96: 93 us); here the tokens are split over the grid.
+// Bound by one trip to memory per stage, and by how often the operands cross from the memory side into an L2: the blocks of one
+// split, which read the same tokens, are therefore dealt to one XCD (they used to be neighbours in the grid, on eight), and the loads of
+// two stages are in flight during a third's products.  bf16, tokens x M x N, us: 25088 x 384 x 96 20.5 -> 17.4 on one XCD -> 16.3 with
+// two stages ahead, 25088 x 96 x 192 18.5 -> 13.5 -> 13.7, 6272 x 768 x 192 18.3 -> 16.2 -> 15.4, 250000 x 96 x 96 54.6 -> 37.6 -> 32.3,
+// 32768 x 1024 x 768 215 -> 162 -> 142.  (512 blocks in place of 768: 15.3, 13.7, 16.4, 34.0, 216; halves of a block that take stages in
+// turn and add up in LDS, half the atomics: 20.0, 17.5, 16.4, 59, 238 before the others of these.)
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *c, int64_t tokens, int M, int N, int splits, float *out, float *bias) {
     constexpr int KT = 64, PW = KT / 2 + 4;         // tokens per stage; words per channel row
     __shared__ __align__(16) uint32_t sA[64 * PW], sC[64 * PW];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nN = (N + 63) / 64, m0 = (blockIdx.x / nN) * 64, n0 = (blockIdx.x % nN) * 64;
-    const int64_t per = ((tokens + splits - 1) / splits + KT - 1) / KT * KT, k0 = blockIdx.y * per, k1 = min(k0 + per, tokens);
+    const int nN = (N + 63) / 64, tiles = (M + 63) / 64 * nN, seq = blockIdx.x >> 3;
+    // (blocks go to the eight XCDs in turn)
+    const int tile = splits < 8 ? blockIdx.x % tiles : seq % tiles, split = splits < 8 ? blockIdx.x / tiles : seq / tiles * 8 + (blockIdx.x & 7);
+    const int m0 = tile / nN * 64, n0 = tile % nN * 64;
+    const int64_t per = ((tokens + splits - 1) / splits + KT - 1) / KT * KT, k0 = split * per, k1 = min(k0 + per, tokens);
     if (k0 >= k1) return;
     // item k of this thread: channel pair cp, token pair tp = lane bits 3-5 + 8 * k; the wave index selects 8 of the 32 channel pairs
     const int cp = (lane & 7) + 8 * wave, tb = lane >> 3;
     const int ca = min(m0 + 2 * cp, M - 2), cc = min(n0 + 2 * cp, N - 2);       // (clamped channels: rows of the result that are not stored)
-    uint32_t ra[4][2], rc[4][2];
-    auto load = [&](int64_t k) {
+    struct Stage { uint32_t a[4][2], c[4][2]; } st[2];
+    // the stage at token k: tokens past the last are read as the last (and masked where they are used)
+    auto load = [&](Stage &s, int64_t k) {
+        k = min(k, tokens - 1);
+        const char *const pa = (const char *)(a + k * M + ca), *const pc = (const char *)(c + k * N + cc);
+        const uint32_t last = (uint32_t)min(tokens - 1 - k, (int64_t)KT);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int64_t tok = min(k + 2 * (tb + 8 * i) + h, tokens - 1);
-                ra[i][h] = *(const uint32_t *)(a + tok * M + ca);
-                rc[i][h] = *(const uint32_t *)(c + tok * N + cc);
+                const uint64_t tok = min((uint32_t)(2 * (tb + 8 * i) + h), last);
+                s.a[i][h] = *(const uint32_t *)(pa + tok * (2u * (uint32_t)M));
+                s.c[i][h] = *(const uint32_t *)(pc + tok * (2u * (uint32_t)N));
             }
     };
     f32x4 acc[2][2] = {};
     float bsum[2] = {};
     const bool sums = bias != nullptr && n0 == 0;
-    load(k0);
-    for (int64_t k = k0; k < k1; k += KT) {
+    auto step = [&](Stage &s, int64_t k) {
         __syncthreads();
+        const int left = (int)max(min(k1 - k, (int64_t)KT), (int64_t)0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int tp = tb + 8 * i;
-            const int64_t tok = k + 2 * tp;
-            const uint32_t keep = (tok < k1 ? 0xffffu : 0u) | (tok + 1 < k1 ? 0xffff0000u : 0u);
+            const uint32_t keep = (2 * tp < left ? 0xffffu : 0u) | (2 * tp + 1 < left ? 0xffff0000u : 0u);
             // (low half of each word: the even channel) -> words of two tokens per channel
-            const uint32_t e = ((ra[i][0] & 0xffffu) | (ra[i][1] << 16)) & keep, o = ((ra[i][0] >> 16) | (ra[i][1] & 0xffff0000u)) & keep;
+            const uint32_t e = ((s.a[i][0] & 0xffffu) | (s.a[i][1] << 16)) & keep, o = ((s.a[i][0] >> 16) | (s.a[i][1] & 0xffff0000u)) & keep;
             sA[(2 * cp) * PW + tp] = e;
             sA[(2 * cp + 1) * PW + tp] = o;
-            sC[(2 * cp) * PW + tp] = ((rc[i][0] & 0xffffu) | (rc[i][1] << 16)) & keep;
-            sC[(2 * cp + 1) * PW + tp] = ((rc[i][0] >> 16) | (rc[i][1] & 0xffff0000u)) & keep;
+            sC[(2 * cp) * PW + tp] = ((s.c[i][0] & 0xffffu) | (s.c[i][1] << 16)) & keep;
+            sC[(2 * cp + 1) * PW + tp] = ((s.c[i][0] >> 16) | (s.c[i][1] & 0xffff0000u)) & keep;
             if (sums) {
                 bsum[0] += raw_to_f32((const T *)nullptr, e & 0xffffu) + raw_to_f32((const T *)nullptr, e >> 16);
                 bsum[1] += raw_to_f32((const T *)nullptr, o & 0xffffu) + raw_to_f32((const T *)nullptr, o >> 16);
             }
         }
         __syncthreads();
-        load(min(k + KT, tokens - 1));
+        load(s, k + 2 * KT);
 #pragma unroll
         for (int ks = 0; ks < KT; ks += 32) {
             Frag<T> fa[2], fc[2];
@@ -730,6 +741,12 @@ __global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *
 #pragma unroll
                 for (int j = 0; j < 2; ++j) acc[i][j] = mma(fa[i], fc[j], acc[i][j]);
         }
+    };
+    load(st[0], k0);
+    load(st[1], k0 + KT);
+    for (int64_t k = k0; k < k1; k += 2 * KT) {
+        step(st[0], k);
+        if (k + KT < k1) step(st[1], k + KT);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -955,8 +972,9 @@ int snd_block_linear_wgrad(const void *dy, const void *x, int64_t tokens, int M,
     if (dtype != SND_BF16 && dtype != SND_F16) return SND_ERR_DTYPE;
     const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
     if (tiles >= (int64_t)1 << 31) return SND_ERR_SHAPE;
-    const int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 768 / tiles), (tokens + 255) / 256);
-    const dim3 grid((unsigned)tiles, (unsigned)splits);
+    int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 768 / tiles), (tokens + 255) / 256);
+    if (splits >= 8) splits &= ~7;                  // whole rounds of the eight XCDs
+    const dim3 grid((unsigned)(tiles * splits));
     if (dtype == SND_BF16)
         hipLaunchKernelGGL((wgrad_tokens_kernel<bf16_t>), grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t *)dy, (const bf16_t *)x, tokens, M, N, splits, dw, dbias);
     else
