@@ -644,13 +644,13 @@ at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Te
 // walks all tokens in each, the kernel splits the tokens over the grid and pays with atomics.
 // Kernel / library (product, sum over the tokens, casts), bf16, us, by tokens:
 //     M x N           784        3136       12544        32768       100352       401408
-//     768 x 384     14 / 38    20 / 48    44 /  96     96 / 183    270 / 370   1121 / 1098
-//     1024 x 512    14 / 37    27 / 48    67 / 105    158 / 202    488 / 475   1964 / 1433
-//     1536 x 384    14 / 39    28 / 53    75 / 101    180 / 207    563 / 530   2245 / 1652
-//     1024 x 768    19 / 37    33 / 49    89 / 101    218 / 228    689 / 574   2771 / 1506
-//     1024 x 1024   19 / 37    37 / 49   114 / 107    290 / 232    932 / 578   3726 / 1622
-// Up to 2^19 elements it is the kernel at any number of tokens, the last columns too: its sums are fp32, the library's result
-// is rounded to 16 bits.
+//     768 x 384     11 / 40    19 / 48    37 /  97     75 / 183    215 / 372    872 / 1101
+//     1024 x 512    13 / 44    23 / 50    52 / 106    114 / 203    344 / 476   1349 / 1434
+//     1536 x 384    15 / 41    24 / 53    57 / 102    124 / 209    396 / 533   1739 / 1658
+//     1024 x 768    18 / 42    28 / 49    66 / 102    149 / 231    481 / 574   1945 / 1512
+//     1024 x 1024   19 / 40    31 / 49    85 / 107    204 / 234    654 / 582   2752 / 1646
+// Up to 2^19 elements it is the kernel at any number of tokens: its sums are fp32, the library's result is rounded to 16 bits.
+// (The kernel's column was measured again since the line was drawn, it got faster; the last rows' line is the older one.)
 bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) {
     return M % 2 == 0 && N % 2 == 0 && (M * N <= (int64_t)1 << 19 || (M * N <= (int64_t)3 << 18 && tokens <= 1 << 15));
 }

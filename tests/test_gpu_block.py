@@ -72,6 +72,20 @@ def test_linear_weight_gradient(gpu_device, tokens, M, N):
     assert rel(dw, dy.double().t() @ x.double()) <= 1e-5 and rel(db, dy.double().sum(0)) <= 1e-5
 
 
+# How a weight gradient is cut: fewer than eight splits of the tokens, eight with one token in the last, ten taken as eight, one
+# stage and a bit, many tiles.  A result is a sum in fp32 of up to 2560 exact products: about sqrt(2560) * 2^-24 = 3e-6 of its size.
+@pytest.mark.parametrize("tokens,M,N", [(1700, 64, 64), (1793, 64, 64), (2560, 130, 66), (65, 64, 64), (300, 1024, 512)])
+def test_linear_weight_gradient_splits(gpu_device, tokens, M, N):
+    from selective_nd_scan.interface import ext
+    torch.manual_seed(8)
+    x = torch.randn(tokens, N, device=gpu_device, dtype=torch.bfloat16)
+    dy = torch.randn(tokens, M, device=gpu_device, dtype=torch.bfloat16)
+    w = torch.randn(M, N, device=gpu_device).requires_grad_()
+    b = torch.randn(M, device=gpu_device).requires_grad_()
+    dw, db = torch.autograd.grad(ext().block_linear(x, w, b, x), (w, b), dy)
+    assert rel(dw, dy.double().t() @ x.double()) <= 1e-5 and rel(db, dy.double().sum(0)) <= 1e-5
+
+
 @pytest.mark.parametrize("C,dtype", [(1, torch.float32), (65, torch.float32), (200, torch.bfloat16), (1024, torch.float32)])
 def test_token_norm(gpu_device, C, dtype):
     from selective_nd_scan.interface import ext
