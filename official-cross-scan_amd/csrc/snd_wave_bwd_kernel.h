@@ -65,13 +65,23 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // 64 x 384 x 56x56 bf16, one state 381 -> 336, two 632 -> 542; 8 x 384 x 56x56, four 174 -> 140; 8 x 96 x 56x56 fp32, three
 // 99 -> 68; packed, 32 x 768 x 28x28 92 -> 86; several segments (no ONE) 64 x 96 x 112x112 411 -> 408;
 // one channel per block, 1 x 192 x 56x56 bf16, one state 31 -> 26, 1 x 64 x 56x56 fp32, two 51 -> 35.
-template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1)>
-__global__ __launch_bounds__(ONE ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
+//
+// PF: a band's inputs are loaded one band ahead (with three or four states it measured 20 % slower, and with two columns per lane the
+// registers are needed elsewhere).  Not so for eight planes per wave of one or two bands, 16 bits, one state: there is hardly a
+// band to load ahead, and without it the kernel takes 67 registers instead of 105, seven waves per SIMD instead of four (us, bf16 / f16:
+// 8 x 256 x 7x7 7.7 -> 7.5 / 7.7 -> 7.6, 96 x 512 x 7x7 19.8 -> 15.5 / 22.7 -> 15.8, 64 x 1536 x 7x7 30.9 -> 26.7 / 31.0 -> 27.3, x 8x7
+// 32.4 -> 29.3 / 32.6 -> 29.8).  From three bands on it gains in some launches and loses in others (96 x 512 x 9x7 26.8 -> 23.8, 64 x 512 x
+// 12x7 19.2 -> 20.3, 64 x 512 x 200x5 312 -> 320), and so do the other packed kernels, most of all where there are few waves: one state,
+// 64 x 128 x 28x28 34.3 -> 37.3, 64 x 1536 x 7x7 fp32 37.2 -> 38.4; two states, 4 x 256 x 28x28 24.8 -> 26.2, fp32 24.9 -> 26.7, 64 x 512 x 7x7
+// 17.4 -> 17.9.
+template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1), bool PF = (NS <= 2 && CPL == 1)>
+__global__ __launch_bounds__(PK > 1 ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
     static_assert(!EXT || (CHB == (SPL ? 2 : 1) && PK == 1 && CPL == 1 && (!EVEN || SPL)), "column groups: one channel per block, one column per lane");
     static_assert(!SPL || EXT, "a split plane hands over like a column group");
     static_assert(CHB == 1 || CPL == 1, "shared atomics: one column per lane");
     static_assert(PK == 1 || (CHB > 1 && !EVEN), "packed planes share their atomics");
+    static_assert(!PF || (NS <= 2 && CPL == 1), "loads a band ahead: one or two states, one column per lane");
     static_assert(ONE ? CPL == 1 && !EXT : PK == 1, "one segment: one column per lane; packed planes are one segment wide");
     constexpr int S = 64 / PK;                       // lanes per plane
     constexpr int kItems = R * NS * 2;               // dB and dC rows of a band
@@ -80,14 +90,10 @@ __global__ __launch_bounds__(ONE ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wa
     // Two buffers, so that one barrier per band is enough - where they leave the CU its blocks: with three states they
     // would be 48 KB, two blocks per CU instead of four (32x12288x7x7: 0.50 ms against 0.31 with one buffer).
     constexpr int kXBuf = CHB == 1 ? 1 : (NS >= 3 || XW > 8) ? 1 : 2;
-    constexpr int kXWaves = CHB == 1 ? 1 : ONE ? CHB : XW;   // (one segment: a wave per channel; 16 x 384 x 28x28, four states, 71.5 -> 70.0 us with half the LDS)
+    // (packed planes: the block's four waves.  Planes of 33 to 64 columns keep room for eight: with half the LDS more than four of their
+    // waves share a SIMD, and in fp32, one state, 16 x 384 x 56x56 goes from 95.5 to 102.6 us.)
+    constexpr int kXWaves = CHB == 1 ? 1 : PK > 1 ? CHB : XW;
     __shared__ float sX[kXBuf][kXWaves][CHB == 1 ? 1 : kItems][CHB == 1 ? 1 : 64];
-    // load a band's inputs one band ahead (with three or four states it measured 20 % slower, and with two columns per
-    // lane the registers are needed elsewhere).  Packed planes have few bands and many waves: without it they take 67 to 88
-    // registers instead of 105 to 113, and with the LDS of a block of four waves (below) a SIMD holds five to seven waves
-    // instead of four.  us: one state, 64 x 1536 x 7x7 31.2 -> 27.4, 64 x 768 x 14x14 49.9 -> 49.2, 32 x 768 x 28x28 merged 82.1 ->
-    // 80.3; two states, 7x7 47.8 -> 45.8, 14x14 73.1 -> 71.8.  (Planes of 33 to 64 columns: no change bf16, +0.6 % fp32.)
-    constexpr bool PF = NS <= 2 && CPL == 1 && PK == 1;
     // The rows' hand-overs behind the band's last row instead of each behind its own: without a branch between the rows the
     // compiler overlaps one row's sums with the next row's scan.  One state, 256 channels of 512x512 398 -> 383 us, 64 channels of
     // 600x900 873 -> 831; two states lose by it (bands of two rows; 2 x 192 x 200x336 381 -> 386).
@@ -677,7 +683,7 @@ static inline int wave_bwd_share(const snd_shape &sh, const WaveGeo &wg) {
     return wg.nseg * 4 <= kWaveShareWaves ? 4 : 2;
 }
 
-template <typename T, int NS, int CPL, bool VEC, int CHB, int PK, int XW = kMaxSeg, bool ONE = (PK > 1)>
+template <typename T, int NS, int CPL, bool VEC, int CHB, int PK, int XW = kMaxSeg, bool ONE = (PK > 1), bool PF = (NS <= 2 && CPL == 1)>
 static int launch_wave_bwd_c(const snd_bwd_params &p, const WaveGeo &wg, hipStream_t stream) {
     const snd_shape &sh = p.f.shape;
     const int rg = sh.dim / sh.n_groups;
@@ -688,11 +694,11 @@ static int launch_wave_bwd_c(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     const bool even = NS <= 2 && CPL == 1 && PK == 1 && sh.nrows % R == 0 && sh.ncols % (kSeg * CPL) == 0;
     if (even) {
         constexpr bool E = NS <= 2 && CPL == 1 && PK == 1;
-        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, E, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
-        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, E, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
+        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, E, CHB, PK, XW, false, false, ONE, PF>), grid, block, 0, stream, p, wg);
+        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, E, CHB, PK, XW, false, false, ONE, PF>), grid, block, 0, stream, p, wg);
     } else {
-        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, false, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
-        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, false, CHB, PK, XW, false, false, ONE>), grid, block, 0, stream, p, wg);
+        if (p.dout_dtype == SND_F32) hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, true, false, CHB, PK, XW, false, false, ONE, PF>), grid, block, 0, stream, p, wg);
+        else hipLaunchKernelGGL((wave_bwd_kernel<T, NS, CPL, VEC, F32, false, CHB, PK, XW, false, false, ONE, PF>), grid, block, 0, stream, p, wg);
     }
     return hipGetLastError() == hipSuccess ? SND_OK : SND_ERR_LAUNCH;
 }
@@ -702,6 +708,8 @@ static int launch_wave_bwd_v(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     const int share = CPL == 1 ? wave_bwd_share(p.f.shape, wg) : 1;
     const int pk = CPL == 1 ? wave_pack(wg, p.f.shape.ncols) : 1;
     // (packed planes always in blocks of four waves: the planes of a wave are added up where the waves of a block are)
+    constexpr bool SHORT = CPL == 1 && NS == 1 && sizeof(T) == 2;    // (see PF)
+    if (SHORT && pk == 8 && wg.nBands <= 2) return launch_wave_bwd_c<T, NS, CPL, VEC, SHORT ? 4 : 1, SHORT ? 8 : 1, kMaxSeg, SHORT, NS <= 2 && CPL == 1 && !SHORT>(p, wg, stream);
     if (pk == 8) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 8 : 1>(p, wg, stream);
     if (pk == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 4 : 1>(p, wg, stream);
     if (pk == 2) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 2 : 1>(p, wg, stream);

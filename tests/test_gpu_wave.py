@@ -291,6 +291,10 @@ PACKED = [
     (2, 40, 6, 5, 2, 4, None, torch.float16, {}),
     (2, 24, 7, 7, 1, 4, None, torch.float32, dict(dirs=capi.DIR_CORNERS, decay=0.9)),
     (2, 20, 10, 7, 3, 4, None, torch.float32, dict(dirs=capi.DIR_CORNERS, softplus=False)),
+    # one state, 16 bits, either side of the line between loads at their use and a band ahead: one, two and three bands
+    (2, 72, 4, 7, 1, 4, None, torch.bfloat16, {}),
+    (2, 72, 8, 7, 1, 4, 36, torch.float16, {}),
+    (2, 72, 9, 6, 1, 4, None, torch.bfloat16, {}),
 ]
 
 
