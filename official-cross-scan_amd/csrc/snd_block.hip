@@ -670,19 +670,21 @@ __global__ __launch_bounds__(256) void wgrad_kernel(const T *a, int64_t ab, int6
 // (16 bytes at a pitch of 36 words) spread over all LDS banks.  The library's product has M * N / 4096 blocks and walks all
 // tokens in each (25088 x 384 x 96: 93 us); here the tokens are split over the grid.
 // Bound by one trip to memory per stage, and by how often the operands cross from the memory side into an L2: the blocks of one
-// split, which read the same tokens, are therefore dealt to one XCD (they used to be neighbours in the grid, on eight), and the loads of
-// two stages are in flight during a third's products.  bf16, tokens x M x N, us: 25088 x 384 x 96 20.5 -> 17.4 on one XCD -> 16.3 with
-// two stages ahead, 25088 x 96 x 192 18.5 -> 13.5 -> 13.7, 6272 x 768 x 192 18.3 -> 16.2 -> 15.4, 250000 x 96 x 96 54.6 -> 37.6 -> 32.3,
-// 32768 x 1024 x 768 215 -> 162 -> 142.  (512 blocks in place of 768: 15.3, 13.7, 16.4, 34.0, 216; halves of a block that take stages in
-// turn and add up in LDS, half the atomics: 20.0, 17.5, 16.4, 59, 238 before the others of these.)
+// split, which read the same tokens, are dealt to one XCD where there are eight splits to deal, and the loads of two stages are in
+// flight during a third's products.  Against neighbouring blocks on eight XCDs and one stage ahead, bf16, tokens x M x N, us: 25088 x 384 x
+// 96 20.4 -> 16.1, 25088 x 96 x 192 16.0 -> 11.7, 6272 x 768 x 192 18.3 -> 15.8, 250000 x 96 x 96 54.0 -> 32.7, 12544 x 768 x 384 40.2 -> 29.0;
+// by the second stage and cheaper addresses alone, fewer than eight splits not being placed: 32768 x 1024 x 768 215 -> 142.  (Halves of a
+// block that take stages in turn and add up in LDS, half the atomics, 15 % slower and more; the splits % 8 that remain each on an XCD of its own
+// too instead of spread, 12544 x 768 x 384 29 -> 39, or split counts rounded up, 32.)
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_tokens_kernel(const T *a, const T *c, int64_t tokens, int M, int N, int splits, float *out, float *bias) {
     constexpr int KT = 64, PW = KT / 2 + 4;         // tokens per stage; words per channel row
     __shared__ __align__(16) uint32_t sA[64 * PW], sC[64 * PW];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nN = (N + 63) / 64, tiles = (M + 63) / 64 * nN, seq = blockIdx.x >> 3;
-    // (blocks go to the eight XCDs in turn)
-    const int tile = splits < 8 ? blockIdx.x % tiles : seq % tiles, split = splits < 8 ? blockIdx.x / tiles : seq / tiles * 8 + (blockIdx.x & 7);
+    const int nN = (N + 63) / 64, tiles = (M + 63) / 64 * nN;
+    // blocks go to the eight XCDs in turn: eight splits at a time, each on an XCD of its own; the last splits % 8 spread over all
+    const int whole = (splits & ~7) * tiles, i = blockIdx.x, rest = i - whole;
+    const int tile = rest < 0 ? (i >> 3) % tiles : rest % tiles, split = rest < 0 ? (i >> 3) / tiles * 8 + (i & 7) : (splits & ~7) + rest / tiles;
     const int m0 = tile / nN * 64, n0 = tile % nN * 64;
     const int64_t per = ((tokens + splits - 1) / splits + KT - 1) / KT * KT, k0 = split * per, k1 = min(k0 + per, tokens);
     if (k0 >= k1) return;
@@ -972,8 +974,12 @@ int snd_block_linear_wgrad(const void *dy, const void *x, int64_t tokens, int M,
     if (dtype != SND_BF16 && dtype != SND_F16) return SND_ERR_DTYPE;
     const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
     if (tiles >= (int64_t)1 << 31) return SND_ERR_SHAPE;
+    // Splits of 256 tokens, as many as give 768 blocks.  From 32 splits on they are whole rounds of the XCDs (9984 x 192 x 384, 39 splits,
+    // 15.5 -> 14.9 us; 25088 x 96 x 192, 98, 15.5 -> 13.2), where the last of them only make the others longer; fewer would get
+    // noticeably longer and larger in error (3600 x 64 x 64, 15 splits, 6.0 -> 8.6 us as eight), and so would splits that are few because of the
+    // tiles (25088 x 768 x 192, 21 splits, 29.0 -> 32.9 us and 2.2e-7 -> 2.5e-7 as 16).
     int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 768 / tiles), (tokens + 255) / 256);
-    if (splits >= 8) splits &= ~7;                  // whole rounds of the eight XCDs
+    if (splits >= 32 && splits == (tokens + 255) / 256) splits &= ~7;
     const dim3 grid((unsigned)(tiles * splits));
     if (dtype == SND_BF16)
         hipLaunchKernelGGL((wgrad_tokens_kernel<bf16_t>), grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t *)dy, (const bf16_t *)x, tokens, M, N, splits, dw, dbias);
