@@ -37,9 +37,10 @@ def test_jobs_clear_and_sum(gpu_device, src, dst, outer, rows, cols):
     assert torch.equal(out, want.to(dst))
 
 
-@pytest.mark.parametrize("n", [1, 65536 * 3 + 1])
+@pytest.mark.parametrize("n", [1, 65536 * 3 + 1, 2, 65536 * 3 + 2])
 def test_rounding_to_bfloat16(gpu_device, n):
-    """To nearest even, bit for bit as torch rounds: ties, subnormal values, the largest ones, infinities; a NaN stays one."""
+    """To nearest even, bit for bit as torch rounds: ties, subnormal values, the largest ones, infinities; a NaN stays one.  Stored one by
+    one, and four at a time where the count (n and 22 special values) is a multiple of four."""
     bits = torch.arange(n, device=gpu_device, dtype=torch.int64) * 21845 + (torch.arange(n, device=gpu_device) % 5 - 2) + 0x8000
     special = torch.tensor([0x00008000, 0x00018000, 0x3f808000, 0x3f818000, 0x7f7fffff, 0x7f7f8000, 0x7f800000, 0x7f800001, 0x7fc00000, 1, 0x007fffff],
                            device=gpu_device, dtype=torch.int64)
@@ -101,6 +102,10 @@ def test_jobs_merge_weights(gpu_device, G, rg):
     (1, 16, 40, 24, 16, 2, torch.float32, 2),     # strips: through the workspace
     (1, 64, 14, 14, 16, 4, torch.float32, 0),
     (70, 16, 21, 14, 7, 4, torch.float16, 0),     # 7x7 tiles, 8-lane kernels
+    (66, 16, 17, 12, 8, 4, torch.float32, 0),     # 8-lane kernels, whole four-column chunks
+    (65, 16, 24, 20, 6, 4, torch.bfloat16, 0),
+    (2, 32, 24, 40, 3, 2, torch.float32, 1),      # 8 lanes for three states
+    (1, 32, 40, 24, 4, 2, torch.bfloat16, 2),
     (2, 16, 33, 130, 2, 4, torch.float32, 0),     # row-segment kernels
     (1, 8, 9, 1500, 2, 2, torch.float32, 0),      # wide planes: the column groups hand over through the workspace
 ])
