@@ -1,11 +1,12 @@
 // The passes of a VSS block around its scan: token LayerNorm, depthwise convolution + SiLU, the step-size projection, output
-// LayerNorm + gate, and the weight gradients of the two projections.  All of them are bound by memory: what they move is
-// read once from it (halos and second passes come from the L2) and written once, in the layout its reader wants - tokens by
-// channels for the linear layers, channels by pixels for the scan - with the transposition done in LDS on the way.
+// LayerNorm + gate, and the weight gradients of the two projections.  What they move is
+// read once from memory (halos and second passes come from the L2) and written once, in the layout its reader wants - tokens by
+// channels for the linear layers, channels by pixels for the scan - with the transposition done in LDS on the way.  None is at the
+// rate of memory yet: the convolution's bytes at a copy's rate take 6 / 8 of its 19 / 49 us, the gate's backward's 14 of 39.
 // Measured on a block of width 96 (inner 192, rank 6) at 8 x 56 x 56, bf16, us forward / backward, against the torch layers
 // they replace: convolution + SiLU 90 / 420 -> 19 / 49 (layout copies, im2col per image for the weight), projections 100 / 400
-// -> 35 / 95 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 22 / 46,
-// token norm 33 / 70 -> 6 / 13 each, weight gradient of a linear layer 93 + 20 -> 20; the block's training step 2940 -> 1500.
+// -> 35 / 95 (products with one long side, copies into and out of their layout), output norm + gate 60 / 150 -> 21 / 39,
+// token norm 33 / 70 -> 6 / 13 each, weight gradient of a linear layer 93 + 20 -> 16; the block's training step 2940 -> 1340.
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>
@@ -976,8 +977,8 @@ int snd_block_linear_wgrad(const void *dy, const void *x, int64_t tokens, int M,
     if (tiles >= (int64_t)1 << 31) return SND_ERR_SHAPE;
     // Splits of 256 tokens, as many as give 768 blocks.  From 32 splits on they are whole rounds of the XCDs (9984 x 192 x 384, 39 splits,
     // 15.5 -> 14.9 us; 25088 x 96 x 192, 98, 15.5 -> 13.2), where the last of them only make the others longer; fewer would get
-    // noticeably longer and larger in error (3600 x 64 x 64, 15 splits, 6.0 -> 8.6 us as eight), and so would splits that are few because of the
-    // tiles (25088 x 768 x 192, 21 splits, 29.0 -> 32.9 us and 2.2e-7 -> 2.5e-7 as 16).
+    // noticeably longer and larger in error (3837 x 64 x 64, 15 splits, 6.2 -> 8.6 us and 1.1e-7 -> 1.4e-7 as eight), and so would splits that are
+    // few because of the tiles (32768 x 768 x 192, 21 splits, 34.8 -> 40.0 us and 2.5e-7 -> 2.8e-7 as 16).
     int splits = (int)std::min<int64_t>(std::max<int64_t>(1, 768 / tiles), (tokens + 255) / 256);
     if (splits >= 32 && splits == (tokens + 255) / 256) splits &= ~7;
     const dim3 grid((unsigned)(tiles * splits));

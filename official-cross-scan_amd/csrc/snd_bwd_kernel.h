@@ -487,12 +487,14 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // beside dD, at no cost in the sweep.
     float dw_acc = 0.f;
 
-    // dB, dC of a tile leave the block (summed over its channels) behind its sweep, from the waves' partial sums in LDS.  They are
-    // read (flush_read) ahead of the per-pixel epilogue, which covers the reads' latency, and added up and sent behind it; a wave
-    // alone with its arithmetic is what such a wait costs, two waves per SIMD hide little of it.  Read where they are added up, ahead
-    // of the next tile's commit, us: 64 x 192 x 56x56 fp32 1059 -> 1024, 2 x 192 x 200x336 920 -> 880, 1 x 256 x 512^2 bf16 2020 ->
-    // 1960, 8 x 768 x 56x56 bf16 552 -> 532, 12 x 196 x 65x91 660 -> 631.  (The atomics one state at a time between the rows of the
-    // next recomputation: 1.3 to 4 % slower than all at once, with those of held tiles dropped by their offset.)
+    // dB, dC of a tile leave the block (summed over its channels) behind its sweep and epilogue, from the waves' partial sums in LDS:
+    // a tenth of a tile's time.  One tile late, ahead of the next tile's commit, with the zeros of border tiles ahead of it too and
+    // loads in flight on the way into the tile loop (below), us: 64 x 192 x 56x56 fp32 1080 -> 1049, 2 x 192 x 200x336 922 -> 884, 1 x 256 x
+    // 512^2 bf16 1993 -> 1968, 8 x 768 x 56x56 bf16 556 -> 539, 12 x 196 x 65x91 657 -> 630, 64 x 1536 x 7x7 144 -> 135.  They are read
+    // (flush_read) ahead of the epilogue, under which the reads arrive: 0 to 0.5 % faster than behind it.  (The atomics one state at a time
+    // between the rows of the next recomputation: 1.3 to 4 % slower than all at once, with those of held tiles dropped by their offset.
+    // A column segment's hand-over ahead of the last tile's flush instead of behind it: 2 x 192 x 200x336 fp32 878 -> 885, 4 x 96 x 256x256
+    // 940 -> 939, 2 x 384 x 100x168 fp16 463 -> 493.)
     // The terms in dout*C/4 and bu/4 are left out of the sweep: summed over channels (states) they are products of B or C
     // with per-pixel sums that all states (channels) share,
     //     dB: C * T,  dC: B * T,  T = sum_c dout*delta'*u / 4        sum_n dbu*B: dout * S,  S = sum_n B*C / 4
@@ -589,8 +591,8 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
         load_col_ckpt(I_hi, J_hi);
     }
     // Nothing in flight on the way into the tile loop: the waits that the compiler derives for the staged inputs then count the loop's own
-    // instructions behind them instead of waiting for all of them (64 x 192 x 56x56 1055 -> 1048 us; planes of one tile 144 -> 136,
-    // 64 x 1536 x 7x7).  Whole planes of several tiles lose by it (64 x 768 x 14x14 282 -> 291).
+    // instructions behind them instead of waiting for all of them.  Whole planes of several tiles lose by it (64 x 768 x 14x14 277 ->
+    // 279 us, 32 x 768 x 28x28 541 -> 551).
     if (PIPE || SINGLE) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     for (int I = I_hi; I >= I_lo; --I) {
         const int r0 = I * TE;
@@ -693,8 +695,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(2, 2)))
             float hT[TE][TE], smid[TE];
             // columns whose a is kept from this pass for the sweep: as many as fit under 256 registers without a spill in
             // the tile loop (a spilled register is two vector memory instructions per tile, 2 to 4 % of the kernel); the column
-            // segments' bookkeeping leaves room for two, a 7x7 tile for all (64 x 768 x 14x14 bf16 283 -> 279 us, 32 x 768 x 28x28 564 -> 553;
-            // its pipelined form, 16 x 384 x 21x35 fp32, 178 -> 182: four there).
+            // segments' bookkeeping leaves room for two, a 7x7 tile for all (four / seven, bf16, us: 64 x 768 x 14x14 280 / 277, 32 x 768 x 28x28
+            // 551 / 541, 64 x 1536 x 7x7 137 / 135; in its pipelined form four, with no difference between the two that builds alike do not show,
+            // 16 x 384 x 21x35 fp32 175 to 185).
             constexpr int KA = TE == 7 ? (PIPE ? 4 : 7) : SEG ? 2 : 5;
             float aT[KA ? TE : 1][KA ? KA : 1];
             {

@@ -65,8 +65,8 @@ typedef _Float16 f16_t;
 __device__ __forceinline__ float bf16_to_f32(uint16_t v) { return __builtin_bit_cast(float, (uint32_t)v << 16); }
 // To nearest even, by the hardware's conversion (a NaN stays one): the rounding in integer arithmetic took seven instructions per
 // value, which the kernels that store 16-bit rows and issue nothing but vector instructions felt.  Backward in us: 64 x 384 x 56x56,
-// one state, merged 334 -> 319, 256 channels of 512x512, one state 384 -> 372, 64 x 192 x 56x56, two states 282 -> 273, eight
-// states 708 -> 686; the 16-state kernels -0.5 to -1 %, the same bits.
+// one state, merged 341 -> 325, 256 channels of 512x512, one state 386 -> 377, 64 x 192 x 56x56, two states 288 -> 282, eight
+// states 709 -> 687; the 16-state kernels +0.2 to -1.3 %, the same bits.
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint16_t f32_to_bf16(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }

@@ -54,8 +54,9 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
     __shared__ __align__(16) float sDu[CB * PCH];    // delta' * u
     __shared__ __align__(16) float sY[CB * PCH];     // sum_n C*(h - s)
     // The bu/4 term of the output, sum_n C*B*delta'*u/4, is delta'*u times a per-pixel sum that all
-    // channels share: S/4 = sum_n B*C / 4 is built once per tile (per-wave partial sums at staging, added
-    // up by one wave) instead of one multiply-add per state cell.
+    // channels share: S/4 = sum_n B*C / 4 is built once per tile instead of one multiply-add per state cell - staged element by
+    // element, from per-wave partial sums (sSp) by one wave; staged in chunks, from the committed tile by one wave or (with saved
+    // state) by all of them (DEAL).
     __shared__ __align__(16) float sSp[(NP / 4) * kTile], sS[kTile];
     // out of up to four consecutive tiles of a strip (two in the 8-state kernels, whose blocks have
     // less LDS each), flushed together: a 32-byte run per tile row is a partial line write (measured:
@@ -368,9 +369,10 @@ __global__ __launch_bounds__(16 * NP) __attribute__((amdgpu_waves_per_eu(NP >= 8
             }
             __syncthreads();
             // S, read by the output phase behind the next barrier.  DEAL: the pixels dealt over the waves, the states over the lanes of a
-            // pixel; by one wave for all, the others wait for it at that barrier.  us: 256 channels of 512x512 bf16 1138 -> 1087, 8 x 768 x
-            // 56x56 bf16 232 -> 216, 64 x 192 x 56x56 bf16 433 -> 425, fp32 483 -> 478.  Without saved state, whose stores the other waves
-            // do not have either, one wave is as fast or faster (256 x 512x512 900 / 915, 2 x 192 x 200x336 445 / 451).
+            // pixel; by one wave for all, the others wait for it at that barrier.  us: 256 channels of 512x512 bf16 1127 -> 1085, 8 x 768 x
+            // 56x56 bf16 225 -> 215, 64 x 192 x 56x56 bf16 433 -> 430, fp32 482 -> 479.  Without saved state one wave is faster where a plane is
+            // cut into strips (one / dealt: 256 channels of 512x512 898 / 916, 2 x 192 x 200x336 445 / 455) and slower where it is
+            // not, by less (8 x 768 x 56x56 195 / 192, 64 x 192 x 56x56 fp32 400 / 397).
             constexpr bool DEAL = VEC && SAVE;
             constexpr int PXW = kTile / WPB;
             const int spx = PXW * wave_u + (tid & 63) % PXW, sg = (tid & 63) / PXW;

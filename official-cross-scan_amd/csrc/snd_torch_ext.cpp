@@ -644,13 +644,14 @@ at::Tensor block_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Te
 // walks all tokens in each, the kernel splits the tokens over the grid and pays with atomics.
 // Kernel / library (product, sum over the tokens, casts), bf16, us, by tokens:
 //     M x N           784        3136       12544        32768       100352       401408
-//     768 x 384     11 / 40    19 / 48    37 /  97     75 / 183    215 / 372    872 / 1101
-//     1024 x 512    13 / 44    23 / 50    52 / 106    114 / 203    344 / 476   1349 / 1434
-//     1536 x 384    15 / 41    24 / 53    57 / 102    124 / 209    396 / 533   1739 / 1658
-//     1024 x 768    18 / 42    28 / 49    66 / 102    149 / 231    481 / 574   1945 / 1512
-//     1024 x 1024   19 / 40    31 / 49    85 / 107    204 / 234    654 / 582   2752 / 1646
+//     768 x 384     11 / 41    19 / 48    34 /  97     66 / 183    187 / 372    740 / 1102
+//     1024 x 512    13 / 45    23 / 51    51 / 106    115 / 203    339 / 476   1352 / 1439
+//     1536 x 384    15 / 41    24 / 53    56 / 102    124 / 209    398 / 532   1751 / 1659
+//     1024 x 768    18 / 41    28 / 49    65 / 102    151 / 231    471 / 575   1997 / 1513
+//     1024 x 1024   19 / 40    31 / 49    85 / 107    203 / 233    653 / 585   2765 / 1641
 // Up to 2^19 elements it is the kernel at any number of tokens: its sums are fp32, the library's result is rounded to 16 bits.
-// (The kernel's column was measured again since the line was drawn, it got faster; the last rows' line is the older one.)
+// From there on the line is where a slower kernel met the library (1024 x 768: 218 / 228 at 32768 tokens, 689 / 574 at 100352); as it is now
+// the kernel would be faster beyond it, up to 100352 tokens at 1024 x 768 and up to 32768 at 1024 x 1024.
 bool linear_wgrad_pays(int64_t tokens, int64_t M, int64_t N) {
     return M % 2 == 0 && N % 2 == 0 && (M * N <= (int64_t)1 << 19 || (M * N <= (int64_t)3 << 18 && tokens <= 1 << 15));
 }

@@ -69,11 +69,11 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // PF: a band's inputs are loaded one band ahead (with three or four states it measured 20 % slower, and with two columns per lane the
 // registers are needed elsewhere).  Not so for eight planes per wave of one or two bands, 16 bits, one state: there is hardly a
 // band to load ahead, and without it the kernel takes 67 registers instead of 105, seven waves per SIMD instead of four (us, bf16 / f16:
-// 8 x 256 x 7x7 7.7 -> 7.5 / 7.7 -> 7.6, 96 x 512 x 7x7 19.8 -> 15.5 / 22.7 -> 15.8, 64 x 1536 x 7x7 30.9 -> 26.7 / 31.0 -> 27.3, x 8x7
-// 32.4 -> 29.3 / 32.6 -> 29.8).  From three bands on it gains in some launches and loses in others (96 x 512 x 9x7 26.8 -> 23.8, 64 x 512 x
-// 12x7 19.2 -> 20.3, 64 x 512 x 200x5 312 -> 320), and so do the other packed kernels, most of all where there are few waves: one state,
-// 64 x 128 x 28x28 34.3 -> 37.3, 64 x 1536 x 7x7 fp32 37.2 -> 38.4; two states, 4 x 256 x 28x28 24.8 -> 26.2, fp32 24.9 -> 26.7, 64 x 512 x 7x7
-// 17.4 -> 17.9.
+// 8 x 256 x 7x7 7.7 -> 7.6 / 7.8 -> 7.6, 96 x 512 x 7x7 20.1 -> 15.6 / 20.0 -> 16.0, 64 x 1536 x 7x7 31.0 -> 26.8 / 31.4 -> 27.3, 32 x 1536 x
+// 8x7 bf16 19.4 -> 15.6).  From three bands on it gains in some launches and loses in others (96 x 512 x 9x7 26.8 -> 23.6, 64 x 512 x
+// 12x7 19.2 -> 20.0, 64 x 512 x 200x5 312 -> 319), and so do the other packed kernels, most of all where there are few waves: one state,
+// 64 x 128 x 28x28 35.9 -> 37.7, 64 x 1536 x 7x7 fp32 37.3 -> 38.4; two states, 4 x 256 x 28x28 24.9 -> 26.2, fp32 24.9 -> 26.7, 64 x 512 x 7x7
+// 17.5 -> 17.7, fp16 17.4 -> 20.0.
 template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1), bool PF = (NS <= 2 && CPL == 1)>
 __global__ __launch_bounds__(PK > 1 ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(PK > 1 ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void
     // would be 48 KB, two blocks per CU instead of four (32x12288x7x7: 0.50 ms against 0.31 with one buffer).
     constexpr int kXBuf = CHB == 1 ? 1 : (NS >= 3 || XW > 8) ? 1 : 2;
     // (packed planes: the block's four waves.  Planes of 33 to 64 columns keep room for eight: with half the LDS more than four of their
-    // waves share a SIMD, and in fp32, one state, 16 x 384 x 56x56 goes from 95.5 to 102.6 us.)
+    // waves share a SIMD, and in fp32, one state, 16 x 384 x 56x56 goes from 98.0 to 103.6 us.)
     constexpr int kXWaves = CHB == 1 ? 1 : PK > 1 ? CHB : XW;
     __shared__ float sX[kXBuf][kXWaves][CHB == 1 ? 1 : kItems][CHB == 1 ? 1 : 64];
     // The rows' hand-overs behind the band's last row instead of each behind its own: without a branch between the rows the
