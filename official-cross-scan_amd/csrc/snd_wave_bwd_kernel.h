@@ -67,13 +67,7 @@ __device__ __forceinline__ void wave_glb_add(float *p, float v) {
 // one channel per block, 1 x 192 x 56x56 bf16, one state 31 -> 26, 1 x 64 x 56x56 fp32, two 51 -> 35.
 //
 // PF: a band's inputs are loaded one band ahead (with three or four states it measured 20 % slower, and with two columns per lane the
-// registers are needed elsewhere).  Not so for eight planes per wave of one or two bands, 16 bits, one state: there is hardly a
-// band to load ahead, and without it the kernel takes 67 registers instead of 105, seven waves per SIMD instead of four (us, bf16 / f16:
-// 8 x 256 x 7x7 7.7 -> 7.6 / 7.8 -> 7.6, 96 x 512 x 7x7 20.1 -> 15.6 / 20.0 -> 16.0, 64 x 1536 x 7x7 31.0 -> 26.8 / 31.4 -> 27.3, 32 x 1536 x
-// 8x7 bf16 19.4 -> 15.6).  From three bands on it gains in some launches and loses in others (96 x 512 x 9x7 26.8 -> 23.6, 64 x 512 x
-// 12x7 19.2 -> 20.0, 64 x 512 x 200x5 312 -> 319), and so do the other packed kernels, most of all where there are few waves: one state,
-// 64 x 128 x 28x28 35.9 -> 37.7, 64 x 1536 x 7x7 fp32 37.3 -> 38.4; two states, 4 x 256 x 28x28 24.9 -> 26.2, fp32 24.9 -> 26.7, 64 x 512 x 7x7
-// 17.5 -> 17.7, fp16 17.4 -> 20.0.
+// registers are needed elsewhere) - but not by every packed launch, see wave_bwd_at_use().
 template <typename T, int NS, int CPL, bool VEC, bool DO32, bool EVEN, int CHB, int PK, int XW, bool EXT = false, bool SPL = false, bool ONE = (PK > 1), bool PF = (NS <= 2 && CPL == 1)>
 __global__ __launch_bounds__(PK > 1 ? 64 * CHB : 64 * (XW + (SPL ? 1 : 0))) void wave_bwd_kernel(const snd_bwd_params p, const WaveGeo wg) {
     constexpr int R = wave_band_rows(NS);            // rows per band
@@ -683,6 +677,23 @@ static inline int wave_bwd_share(const snd_shape &sh, const WaveGeo &wg) {
     return wg.nseg * 4 <= kWaveShareWaves ? 4 : 2;
 }
 
+// Whether a packed launch loads a band's inputs where it uses them instead of a band ahead.  Without loads ahead the kernels take 72
+// to 77 registers instead of 105 to 113, six waves per SIMD instead of four.  That pays where there are more waves than four per SIMD
+// - but for one and a half to two rounds of four - and few bands to load ahead: planes no taller than the lanes of a row are wide.  us,
+// ahead / at use:
+//     eight planes per wave, 16 bits: one state at any size, 8 x 256 x 7x7 7.7 / 7.5, 64 x 1536 x 7x7 31.2 / 27.4; two states, 4096 waves
+//         (32 x 1024 x 7x7) 17.8 / 18.2, 5120 25.5 / 21.5, 6656 29.1 / 29.9, 8192 33.5 / 34.8, 12288 50.0 / 46.7; taller, 72 x 1024 x 30x7 fp16 163 / 168
+//     bf16, two and four planes: one state, 5120 waves (40 x 512 x 14x14) 26.1 / 24.4, 6656 30.6 / 32.1, 8192 35.4 / 36.4, 12288 50.8 / 49.6, 96 x
+//         256 x 28x28 84.2 / 81.5; two states, 96 x 256 x 28x28 140.4 / 136.1; few waves, 4 x 256 x 28x28 24.9 / 26.2; taller, 128 x 512 x 28x14,
+//         one state, 124 / 128
+//     fp16: four planes and one state alike (5120 waves 26.0 / 24.5, 12288 51.0 / 50.4), the others mixed (72 x 512 x 14x14, two states, 55.4 /
+//         58.0);  fp32: slower by 1 to 4 % almost everywhere (4 x 256 x 28x28, two states, 24.8 / 26.8)
+template <typename T, int NS> static inline bool wave_bwd_at_use(int pk, int rows, int64_t waves) {
+    if (sizeof(T) != 2 || NS > 2 || rows > 64 / pk) return false;
+    if (pk == 8 && NS == 1) return true;
+    return (pk == 8 || (pk == 4 && NS == 1) || std::is_same<T, bf16_t>::value) && (waves > 8192 || (waves > 4096 && waves <= 6144));
+}
+
 template <typename T, int NS, int CPL, bool VEC, int CHB, int PK, int XW = kMaxSeg, bool ONE = (PK > 1), bool PF = (NS <= 2 && CPL == 1)>
 static int launch_wave_bwd_c(const snd_bwd_params &p, const WaveGeo &wg, hipStream_t stream) {
     const snd_shape &sh = p.f.shape;
@@ -708,8 +719,14 @@ static int launch_wave_bwd_v(const snd_bwd_params &p, const WaveGeo &wg, hipStre
     const int share = CPL == 1 ? wave_bwd_share(p.f.shape, wg) : 1;
     const int pk = CPL == 1 ? wave_pack(wg, p.f.shape.ncols) : 1;
     // (packed planes always in blocks of four waves: the planes of a wave are added up where the waves of a block are)
-    constexpr bool SHORT = CPL == 1 && NS == 1 && sizeof(T) == 2;    // (see PF)
-    if (SHORT && pk == 8 && wg.nBands <= 2) return launch_wave_bwd_c<T, NS, CPL, VEC, SHORT ? 4 : 1, SHORT ? 8 : 1, kMaxSeg, SHORT, NS <= 2 && CPL == 1 && !SHORT>(p, wg, stream);
+    constexpr bool K16 = CPL == 1 && NS <= 2 && sizeof(T) == 2, KB = K16 && std::is_same<T, bf16_t>::value, K4 = KB || (K16 && NS == 1), PF = CPL == 1 && NS <= 2;
+    const snd_shape &sh = p.f.shape;
+    const int64_t waves = (int64_t)sh.batch * sh.n_groups * ((sh.dim / sh.n_groups + 4 * pk - 1) / (4 * pk)) * 4;
+    if (K16 && pk > 1 && wave_bwd_at_use<T, NS>(pk, sh.nrows, waves)) {
+        if (pk == 8) return launch_wave_bwd_c<T, NS, CPL, VEC, K16 ? 4 : 1, K16 ? 8 : 1, kMaxSeg, K16, PF && !K16>(p, wg, stream);
+        if (pk == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, K4 ? 4 : 1, K4 ? 4 : 1, kMaxSeg, K4, PF && !K4>(p, wg, stream);
+        return launch_wave_bwd_c<T, NS, CPL, VEC, KB ? 4 : 1, KB ? 2 : 1, kMaxSeg, KB, PF && !KB>(p, wg, stream);
+    }
     if (pk == 8) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 8 : 1>(p, wg, stream);
     if (pk == 4) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 4 : 1>(p, wg, stream);
     if (pk == 2) return launch_wave_bwd_c<T, NS, CPL, VEC, CPL == 1 ? 4 : 1, CPL == 1 ? 2 : 1>(p, wg, stream);

@@ -291,10 +291,16 @@ PACKED = [
     (2, 40, 6, 5, 2, 4, None, torch.float16, {}),
     (2, 24, 7, 7, 1, 4, None, torch.float32, dict(dirs=capi.DIR_CORNERS, decay=0.9)),
     (2, 20, 10, 7, 3, 4, None, torch.float32, dict(dirs=capi.DIR_CORNERS, softplus=False)),
-    # one state, 16 bits, either side of the line between loads at their use and a band ahead: one, two and three bands
+    # 16 bits, either side of the lines between loads at their use and a band ahead (wave_bwd_at_use): rows, and waves of the launch
     (2, 72, 4, 7, 1, 4, None, torch.bfloat16, {}),
     (2, 72, 8, 7, 1, 4, 36, torch.float16, {}),
     (2, 72, 9, 6, 1, 4, None, torch.bfloat16, {}),
+    (64, 516, 7, 7, 2, 4, None, torch.float16, {}),            # 5120 waves
+    (64, 260, 14, 14, 1, 4, None, torch.bfloat16, {}),         # 5120
+    (64, 260, 9, 11, 1, 4, None, torch.float16, {}),           # 5120
+    (64, 516, 16, 13, 1, 4, None, torch.bfloat16, {}),         # 9216
+    (64, 260, 20, 17, 2, 4, 130, torch.bfloat16, {}),          # 9216
+    (64, 516, 17, 14, 1, 4, None, torch.bfloat16, {}),         # as many, a row too tall
 ]
 
 
