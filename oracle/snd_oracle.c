@@ -1,6 +1,6 @@
 /* CPU restatement of the 2D-CrossScan selective scan in plain C (forward + hand adjoint).
  *
- * TEST INFRASTRUCTURE ONLY: the checker for tests/, __graft_entry__.smoke() and the cpu_baseline
+ * TEST INFRASTRUCTURE ONLY: the oracle of tests/, __graft_entry__.smoke() and the cpu_baseline
  * leg of bench.py.  Nothing in the shipped package links or loads it.
  *
  * Follows the reference cell by cell (same citations as snd_oracle.py):
@@ -10,7 +10,7 @@
  *   scan op  kernels/selective_nd_scan/include/selective_scan_common.h:100-107, constants :13-21
  * It is pinned by tests/test_oracle_c.py against snd_oracle.py (which carries the closed-form,
  * symmetry and autograd pins).  Arithmetic type is SND_REAL (float by default = the reference's
- * fp32 state; build with -DSND_REAL=double for a float64 checker).  Dense row-major fp32 I/O.
+ * fp32 state; build with -DSND_REAL=double for a float64 oracle).  Dense row-major fp32 I/O.
  * Parallel over (batch, group) pairs with OpenMP: each pair owns its dB/dC slice.
  */
 #include <math.h>

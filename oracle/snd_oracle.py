@@ -1,7 +1,7 @@
 """CPU oracle for the 2D-CrossScan selective scan (forward + hand adjoint), float64 numpy.
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package may import this module; it is the
-checker used by tests/, __graft_entry__.smoke() and the cpu_baseline leg of bench.py.
+oracle used by tests/, __graft_entry__.smoke() and the cpu_baseline leg of bench.py.
 
 It restates, cell by cell, what the reference CUDA kernels compute:
 

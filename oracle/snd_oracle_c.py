@@ -2,7 +2,7 @@
 
 fwd / bwd take and return dense float32 numpy arrays with the reference's layouts
 (selective_scan_oflex.cpp:206-229); `real` picks the arithmetic of the state ("f32" = what the
-reference computes in, "f64" = checker).
+reference computes in, "f64" = the oracle).
 """
 import ctypes as C
 import os

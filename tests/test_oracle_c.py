@@ -1,4 +1,4 @@
-"""The C restatement of the oracle (the timed CPU baseline and the checker for large shapes) must
+"""The C restatement of the oracle (the timed CPU baseline and the oracle for large shapes) must
 agree with the pinned numpy oracle."""
 import numpy as np
 import pytest
